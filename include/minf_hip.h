@@ -164,7 +164,24 @@ typedef struct minf_qkvo {
      * output in place. */
     const int32_t *head_list;
     int index_heads;
+    /* Optional scratch memory for split walks, 16-byte aligned: with at least
+     * minf_attn_workspace_bytes() bytes here, launches that would leave the chip idle (few row blocks,
+     * or a few walks far longer than the rest) cut their walks into segments and fold the partial
+     * sums in a second small kernel.  NULL or too small: every walk is made by one workgroup. */
+    void *workspace;
+    size_t workspace_bytes;
 } minf_qkvo;
+
+/*
+ * Bytes of minf_qkvo.workspace that an attention launch of this problem uses (0: it is not split).
+ * op: which entry point; n_init, n_local: of the A-shape / tri-shape entry points, n_last: of tri-shape
+ * (0 for A-shape); ignored otherwise.  A pure host function.
+ */
+#define MINF_OP_VERTICAL_SLASH 0
+#define MINF_OP_BLOCK_SPARSE 1
+#define MINF_OP_ASHAPE 2
+#define MINF_OP_DENSE 3
+size_t minf_attn_workspace_bytes(const minf_qkvo *t, int op, int n_init, int n_local, int n_last);
 
 /*
  * Mixed block-sparse + column-sparse forward over the tensors produced by

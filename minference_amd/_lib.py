@@ -22,6 +22,7 @@ SIGNATURES = {
     "minf_version": (c_int, []),
     "minf_status_string": (ctypes.c_char_p, [c_int]),
     "minf_qkvo_size": (ctypes.c_size_t, []),
+    "minf_attn_workspace_bytes": (ctypes.c_size_t, [c_ptr] + [c_int] * 4),
     "minf_vs_index_build": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr]),
     "minf_vs_index_workspace_bytes": (ctypes.c_size_t, [c_int] * 4),
     "minf_vs_index_build_ws": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
@@ -67,10 +68,13 @@ class QKVO(ctypes.Structure):
         ("sm_scale", c_f32),
         ("head_list", c_ptr),
         ("index_heads", c_int),
+        ("workspace", c_ptr),
+        ("workspace_bytes", ctypes.c_size_t),
     ]
 
 
 MINF_BF16, MINF_F16 = 0, 1
+MINF_OP_VERTICAL_SLASH, MINF_OP_BLOCK_SPARSE, MINF_OP_ASHAPE, MINF_OP_DENSE = 0, 1, 2, 3
 MINF_ROUND_NONE, MINF_ROUND_INPUT_DTYPE = 0, 1
 MINF_BS_FORCE_DIAG_FIRST, MINF_BS_ROUND_INPUT_DTYPE = 1, 2
 

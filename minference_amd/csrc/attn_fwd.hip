@@ -73,7 +73,7 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4_t;
 typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2_t;
 
-enum { MODE_VS = 0, MODE_BS = 1, MODE_ASHAPE = 2, MODE_DENSE = 3 };
+enum { MODE_VS = MINF_OP_VERTICAL_SLASH, MODE_BS = MINF_OP_BLOCK_SPARSE, MODE_ASHAPE = MINF_OP_ASHAPE, MODE_DENSE = MINF_OP_DENSE };
 
 constexpr int BM = 64;        // query rows per workgroup
 constexpr int BN = 64;        // keys per tile
@@ -115,6 +115,21 @@ struct AttnParams {
     // every head is processed and index_heads = hq
     const int *head_list;
     int index_heads;
+    // split walks (see SplitPlan): the row-block pairs >= split_first are walked by up to nseg workgroups,
+    // one segment of the walk each, which leave their share of the sums in `part`
+    int split_first, nseg, seg_len;
+    char *part;
+};
+
+// Split walks.  A launch whose row-block pairs cannot fill the chip, or whose longest walks would outlast
+// everything else, cuts the walks of its pairs >= `first` into segments of about `len` steps (at most
+// `nseg` of them).  One workgroup walks one segment and writes its unnormalised sums -- O^T in fp32 in
+// accumulator layout, row maximum and row sum -- to a slot of the caller's workspace; attn_merge_kernel
+// folds the segments of a pair in ascending order and writes the output rows.
+struct SplitPlan { int first, nseg, len; };
+template <int HD> struct SplitSlot {
+    static constexpr int ACC = 4 * HD * 32 * 4;              // four waves x [HD/32][4][64 lanes] x 16 bytes
+    static constexpr int BYTES = ACC + 4 * 64 * 8;           // ... and (maximum, sum) per lane
 };
 
 typedef const __attribute__((address_space(4))) int *cint_ptr;
@@ -240,11 +255,12 @@ template <int MODE, int HD> struct AttnLds {
     static constexpr int NONLY = VSP ? 2 * VS_ONLY_MAX : 1;
 };
 
-// The whole walk of one workgroup.  EVERY_MAX: the row maximum is computed for every tile; otherwise
+// The whole walk of one workgroup (CUT: or one segment of it, see SplitPlan; a kernel of its own, because
+// the bookkeeping costs the whole walk 2-3 % in scalar registers).  EVERY_MAX: the row maximum is computed for every tile; otherwise
 // only where it is needed (see sm_pv_block), and the function returns true -- for the whole
 // workgroup -- when a row sum left the safe range, i.e. when the walk has to be run again with
 // EVERY_MAX (the output it wrote is then overwritten).
-template <typename T, int MODE, int HD, bool EVERY_MAX>
+template <typename T, int MODE, int HD, bool EVERY_MAX, bool CUT>
 __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[AttnLds<MODE, HD>::NK],
                                           char (&lds_v)[AttnLds<MODE, HD>::NK],
                                           int (&vs_only)[AttnLds<MODE, HD>::NONLY], int (&vs_wsum)[4], int &vs_bad,
@@ -294,8 +310,17 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // faster in ascending order; up to 64K tokens their early row blocks are still growing and the
     // descending order wins for vertical-slash lists (+4 % at 16K, +1.7 % at 32K): the launcher picks.
     const int rows_wg = (p.rows + 1) >> 1;                           // row-block pairs per (batch, head)
-    const int mi = (int)(rest % (unsigned)rows_wg); rest /= (unsigned)rows_wg;
-    const int mslot = p.descending ? rows_wg - 1 - mi : mi;
+    const int split_units = (rows_wg - p.split_first) * p.nseg;      // (no split: split_first == rows_wg)
+    const unsigned units = (unsigned)(p.split_first + split_units);
+    const int mi = (int)(rest % units); rest /= units;
+    int mslot, seg = -1;                             // row-block pair, segment of its walk (-1: the whole walk)
+    if (CUT && mi < split_units) {                    // the split pairs, longest walks first
+        mslot = rows_wg - 1 - mi / p.nseg;
+        seg = mi % p.nseg;
+    } else {
+        mslot = p.descending ? rows_wg - 1 - mi : mi - split_units;
+        if (p.descending) mslot += split_units - (rows_wg - p.split_first);
+    }
     int hkv, b, h, hs;                               // hs: head position in the index tensors
     if (p.head_list) {
         // the selected heads in chunks of `group` consecutive list entries take the place of the kv
@@ -333,7 +358,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // half may still have work, so this half stays for the copies and barriers without tiles
     const bool have_rows = m < p.rows && row0 < seqlen;
     if (!have_rows) {
-        if (m < p.rows)
+        if (m < p.rows && !(CUT && seg >= 0))         // (rows of a split pair are written by the merge)
             for (int i = tid & (NTHREADS - 1); i < BM * NCH; i += NTHREADS) {
                 int r = row0 + i / NCH;
                 if (r < p.n) *reinterpret_cast<u32x4_t *>(o_base + (long long)r * p.os[2] * 2 + (i % NCH) * 16) = u32x4_t{0u, 0u, 0u, 0u};
@@ -475,7 +500,23 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     }
     else
         ntiles = pair_tile_count<MODE>(p, mA, mB, nblk);
-    auto more_tiles = [&](int it) -> bool { return it < ntiles; };   // is there a tile number `it` ?
+    // the part of the walk this workgroup makes: all of it, or one segment
+    int it_begin = 0, it_end = ntiles;
+    char *slot = nullptr;
+    if (CUT && seg >= 0) {
+        const int ns = max(1, min(p.nseg, (ntiles + p.seg_len - 1) / p.seg_len));
+        const int len = (ntiles + ns - 1) / ns;
+        it_begin = min(seg * len, ntiles);
+        it_end = seg < ns ? min(it_begin + len, ntiles) : it_begin;
+        const int heads = p.head_list ? p.index_heads : p.hq;
+        slot = p.part + (((long long)(b * heads + hs) * (rows_wg - p.split_first) + (mslot - p.split_first)) * p.nseg + seg) * SplitSlot<HD>::BYTES;
+        if (it_begin >= it_end) {                       // (workgroup-uniform) nothing to add: a row sum of zero says so
+            float2 *ml = reinterpret_cast<float2 *>(slot + SplitSlot<HD>::ACC) + tid;
+            *ml = make_float2(-INFINITY, 0.f);
+            return false;
+        }
+    }
+    auto more_tiles = [&](int it) -> bool { return it < it_end; };   // is there a tile number `it` ?
     // paired vertical-slash: entry it+1 of the common list sits in a scalar when step `it` starts; the
     // LDS read of entry it+2 is issued at the top of step `it` (no tile copy is in flight there: the
     // list shares an LDS object with the V tiles and must not wait for one) and turns into the next
@@ -484,7 +525,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // this row block's own list in global memory (walked directly when the lists were not split)
     [[maybe_unused]] const cint_ptr sp_list = as_const(list_base) + (((long long)b * p.index_heads + hs) * list_rows + min(m, p.rows - 1)) * list_w;
     auto vs_list = [&](int i) -> int { return reinterpret_cast<const int *>(lds_v1)[min(i, 2 * VS_PAIR_MAX - 1)]; };
-    auto tile_of = [&](int it) -> Tile {      // called with it = 0, 1, 2, ... in order
+    auto tile_of = [&](int it) -> Tile {      // called with it = it_begin, it_begin + 1, ... in order
         if constexpr (VSP) {
             Tile t;
             t.gathered = 0;
@@ -829,11 +870,11 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     Tile cur, nxt;
     int gt_cur = 0, gt_nxt = 0;
     [[maybe_unused]] bool vs_shifted = false;
-    bool have_cur = more_tiles(0);
+    bool have_cur = more_tiles(it_begin);
     if (have_cur) {
-        if constexpr (VSP) vs_entry = __builtin_amdgcn_readfirstlane(vs_list(0));
-        cur = tile_of(0);
-        if constexpr (VSP) vs_entry = __builtin_amdgcn_readfirstlane(vs_list(1));
+        if constexpr (VSP) vs_entry = __builtin_amdgcn_readfirstlane(vs_list(it_begin));
+        cur = tile_of(it_begin);
+        if constexpr (VSP) vs_entry = __builtin_amdgcn_readfirstlane(vs_list(it_begin + 1));
         gt_cur = gather_ids(cur);
         copy_tile(cur, k_base, k_row, std::false_type{}, gt_cur, lds_k);
     }
@@ -915,19 +956,20 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         gt_cur = gt_nxt;
         have_cur = have_nxt;
     };
-    int it = 0;
+    int it = it_begin;
     if constexpr (VSP) {
         // (a first step exists whenever there is a common entry; steps 0 .. vs_nc-2 have a common successor)
-        for (; it + 1 < vs_nc; ++it) step(it, std::integral_constant<int, 1>{});
+        const int common_end = min(vs_nc, it_end);
+        for (; it + 1 < common_end; ++it) step(it, std::integral_constant<int, 1>{});
         // block entries of their own that both row blocks still have (leftovers of the split, or the
         // whole lists when they were not split): these steps run in the SPLIT form
-        const int nb_both = min(vs_na, vs_nb) - vs_nc;
-        if (nb_both >= 3 && have_cur) {
-            if (vs_nc > 0) {                               // from the last common tile to the first split step
+        const int split_end = min(min(vs_na, vs_nb), it_end);
+        if (split_end - max(it_begin, vs_nc) >= 3 && have_cur) {
+            if (it < vs_nc) {                              // from the last common tile to the first split step
                 step(it, std::integral_constant<int, 0>{});
                 ++it;
             }
-            // cur is now each row block's entry 0, its K copy is on the way
+            // cur is now an entry of each row block's own list, its K copy is on the way
             if (!vs_shifted) {
                 vs_shifted = true;
 #pragma unroll
@@ -935,8 +977,9 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
 #pragma unroll
                 for (int db = 0; db < NDB; ++db) v_rd_off[db] += half * TILE_BYTES;
             }
-            sp_entry = vs_merged ? __builtin_amdgcn_readfirstlane(vs_only[half * VS_ONLY_MAX + 1]) : sp_list[1] * LIST_SCALE;
-            for (; it - vs_nc + 1 < nb_both; ++it) step(it, std::integral_constant<int, 2>{});
+            const int j1 = it - vs_nc + 1;
+            sp_entry = vs_merged ? __builtin_amdgcn_readfirstlane(vs_only[half * VS_ONLY_MAX + j1]) : sp_list[j1] * LIST_SCALE;
+            for (; it + 1 < split_end; ++it) step(it, std::integral_constant<int, 2>{});
         }
     }
     for (; have_cur; ++it) step(it, std::integral_constant<int, 0>{});
@@ -963,6 +1006,18 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
                 for (int r = 0; r < 16; ++r) obits = max(obits, __float_as_uint(oacc[i][r]) & 0x7fffffffu);
             const bool suspect = (__float_as_uint(l_tot) & 0x7fffffffu) >= __float_as_uint(0x1p100f) || obits >= 0x7f800000u;
             if (__any(suspect) && lane == 0) lds_redo = 1;
+        }
+        if (CUT && slot) {                               // a segment: the sums as they are (16 bytes per lane, contiguous)
+            char *acc = slot + (wave_wg * NDB * 4 * 64 + lane) * 16;
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int rq = 0; rq < 4; ++rq)
+                    *reinterpret_cast<float4 *>(acc + (db * 4 + rq) * 1024) =
+                        make_float4(oacc[db][rq * 4], oacc[db][rq * 4 + 1], oacc[db][rq * 4 + 2], oacc[db][rq * 4 + 3]);
+            *(reinterpret_cast<float2 *>(slot + SplitSlot<HD>::ACC) + tid) = make_float2(m_i, l_tot);
+            __syncthreads();
+            return !every_max && lds_redo != 0;           // (workgroup-uniform)
         }
         __syncthreads();                                  // K/V tiles no longer needed
         char *ot = (half ? lds_v : lds_k) + wave * 32 * OP;    // 32 rows per wave
@@ -992,7 +1047,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
 
 // (head_dim 256: O^T, Q and the V^T fragments of a wave need more than 256 registers, so that form
 // runs one wave per SIMD with the accumulators in the second half of the register file)
-template <typename T, int MODE, int HD>
+template <typename T, int MODE, int HD, bool CUT>
 __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kernel(const AttnParams p) {
     typedef AttnLds<MODE, HD> L;
     __shared__ __attribute__((aligned(16))) char lds_k[L::NK];
@@ -1003,13 +1058,93 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
     __shared__ int lds_redo;
     if (threadIdx.x == 0) lds_redo = 0;      // (ordered before its readers by the barriers of the walk)
     if constexpr (std::is_same<T, __bf16>::value) {
-        if (attn_walk<T, MODE, HD, false>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo)) {
+        if (attn_walk<T, MODE, HD, false, CUT>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo)) {
             __syncthreads();                 // everyone has read the flag and is done with LDS
-            attn_walk<T, MODE, HD, true>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
+            attn_walk<T, MODE, HD, true, CUT>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
         }
     } else {
         // f16 probabilities have no headroom above the lazy threshold: the maximum of every tile
-        attn_walk<T, MODE, HD, true>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
+        attn_walk<T, MODE, HD, true, CUT>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
+    }
+}
+
+// Folds the segments of a split pair: one workgroup per (batch, head position, pair, 32 query rows), a
+// wave per 32-column block of O^T (same lane layout as the walk's accumulators), segments in ascending
+// order.  The weights are exp2(m_s - M) with M the largest m_s + log2(l_s), so that no product leaves the
+// fp32 range whatever a segment's (lazily raised) maximum was.  Latency-bound and small: it reads what the
+// segments wrote (66 KB each at head_dim 128, from L2) and writes the rows once.
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
+    constexpr int NDB = HD / 32, ROW_BYTES = HD * 2, NCH = ROW_BYTES / 16;
+    __shared__ __attribute__((aligned(16))) char lds_o[32 * ROW_BYTES];
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    const int l32 = lane & 31, g = lane >> 5;
+    const int heads = p.head_list ? p.index_heads : p.hq;
+    const int rows_wg = (p.rows + 1) >> 1, npairs = rows_wg - p.split_first;
+    unsigned rest = blockIdx.x;
+    const int part = (int)(rest & 3u); rest >>= 2;                     // 32-row part of the pair
+    const int pair = (int)(rest % (unsigned)npairs); rest /= (unsigned)npairs;
+    const int hs = (int)(rest % (unsigned)heads), b = (int)(rest / (unsigned)heads);
+    const int h = p.head_list ? p.head_list[hs] : hs;
+    const int seqlen = p.seqlens ? min(p.seqlens[b], p.n) : p.n;
+    const int row0 = (p.split_first + pair) * 2 * BM + part * 32;
+    if (row0 >= p.n) return;
+    char *o_base = p.o + ((long long)b * p.os[0] + (long long)h * p.os[1]) * 2;
+    const char *slots = p.part + ((long long)(b * heads + hs) * npairs + pair) * p.nseg * SplitSlot<HD>::BYTES;
+    // (a pair that starts past the sequence was not walked at all)
+    const int nseg = (p.split_first + pair) * 2 * BM < seqlen ? p.nseg : 0;
+    auto stat = [&](int s) { return *(reinterpret_cast<const float2 *>(slots + (long long)s * SplitSlot<HD>::BYTES + SplitSlot<HD>::ACC) + part * 64 + lane); };
+    float top = -INFINITY;
+    for (int s = 0; s < nseg; ++s) {
+        const float2 ml = stat(s);
+        if (ml.y > 0.f) top = fmaxf(top, ml.x + __builtin_amdgcn_logf(ml.y));
+    }
+    const bool live = row0 + l32 < seqlen;
+    float l_tot = 0.f;
+    float4 acc[NDB > 4 ? 2 : 1][4];
+#pragma unroll
+    for (int i = 0; i < (NDB > 4 ? 2 : 1); ++i)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) acc[i][rq] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s = 0; s < nseg; ++s) {
+        const float2 ml = stat(s);
+        const float w = ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - top) : 0.f;
+        if (!__any(w > 0.f)) continue;                                  // an unused slot holds nothing
+        l_tot += w * ml.y;
+#pragma unroll
+        for (int i = 0; i < (NDB > 4 ? 2 : 1); ++i) {
+            const int db = wave + 4 * i;
+            if (db < NDB) {
+                const char *src = slots + (long long)s * SplitSlot<HD>::BYTES + ((part * NDB + db) * 4 * 64 + lane) * 16;
+#pragma unroll
+                for (int rq = 0; rq < 4; ++rq) {
+                    const float4 x = *reinterpret_cast<const float4 *>(src + rq * 1024);
+                    acc[i][rq].x = fmaf(w, x.x, acc[i][rq].x); acc[i][rq].y = fmaf(w, x.y, acc[i][rq].y);
+                    acc[i][rq].z = fmaf(w, x.z, acc[i][rq].z); acc[i][rq].w = fmaf(w, x.w, acc[i][rq].w);
+                }
+            }
+        }
+    }
+    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+#pragma unroll
+    for (int i = 0; i < (NDB > 4 ? 2 : 1); ++i) {
+        const int db = wave + 4 * i;
+        if (db < NDB)
+#pragma unroll
+            for (int rq = 0; rq < 4; ++rq) {
+                union { T e[4]; u32x2_t u; } out4;
+                const float x[4] = {acc[i][rq].x, acc[i][rq].y, acc[i][rq].z, acc[i][rq].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) out4.e[e] = live ? (T)(x[e] * inv) : (T)0.f;
+                *reinterpret_cast<u32x2_t *>(lds_o + l32 * ROW_BYTES + (32 * db + 8 * rq + 4 * g) * 2) = out4.u;
+            }
+    }
+    __syncthreads();
+    for (int c = (int)threadIdx.x; c < 32 * NCH; c += 256) {
+        const int r = c / NCH, ch = c % NCH;
+        if (row0 + r < p.n)
+            *reinterpret_cast<u32x4_t *>(o_base + (long long)(row0 + r) * p.os[2] * 2 + ch * 16) =
+                *reinterpret_cast<const u32x4_t *>(lds_o + r * ROW_BYTES + ch * 16);
     }
 }
 
@@ -1056,30 +1191,101 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.index_heads = t->head_list ? t->index_heads : t->heads_q;
     p.total_wg = 0;          // set by the launcher
     p.descending = 0;
+    p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
 }
 
-template <int MODE, int HD> int launch_hd(AttnParams p, int dtype, void *stream) {
+// Which walks to split.  `slots` workgroups fit the chip at once.
+//  * Dense walks (dense attention, the last rows of tri-shape) grow with the row block: they are split when
+//    the longest one takes more than half of the steps a slot of the full chip gets, into segments as long
+//    as a slot's share (one head, 16384 tokens: 300 -> 128 us; shares of 0.25, 0.5 and 2: 175, 145, 125 us;
+//    tri-shape, 16 heads of 64, fp16, 24000 tokens, last 128 rows dense: 444 -> 131 us; 147, 138, 152 us).
+//    Below half, the descending order hides the longest walk behind the others.
+//  * Everything else has walks of bounded length and is split only when the launch has at most 64
+//    row-block pairs, i.e. gives at most a quarter of the compute units a workgroup.  The segments then
+//    have SEG_MIN steps whatever else the launch holds, and launches of more than 64 pairs are not split
+//    for one head or for many, so that such a head's bits do not depend on the heads it is launched with.
+// SEG_MIN weighs the fixed cost of a workgroup (about five steps) and of the fold against the chain of
+// steps.  One head: dense 4096 tokens 78 us whole; 45, 35, 31, 27.5, 28.5, 30.5 us with 3, 4, 6, 8, 12, 16
+// steps; vertical-slash 500 + 700, 4096 tokens, the whole path 177 us whole; 157, 152, 148, 145, 147, 150 us.
+constexpr int SEG_MIN = 8;
+SplitPlan plan_split(int mode, const AttnParams &p, int head_dim) {
+    const int pairs = (p.rows + 1) / 2;
+    const SplitPlan none{pairs, 1, 1};
+    const long long heads = (long long)p.batch * (p.head_list ? p.index_heads : p.hq);
+    const int slots = head_dim == 256 ? 256 : (head_dim == 128 ? 512 : 768);
+    auto capped = [&](int first, int longest, int len) -> SplitPlan {
+        const int nseg = (longest + len - 1) / len;
+        return nseg < 2 ? none : SplitPlan{first, nseg < 64 ? nseg : 64, len};
+    };
+    const bool dense = mode == MODE_DENSE;
+    const int first_dense = dense ? 0 : (mode == MODE_ASHAPE && p.dense_from < p.n ? p.dense_from / (2 * BM) : pairs);
+    if (first_dense < pairs) {
+        // steps of the dense pairs first_dense .. pairs-1 (pair i: 2 i + 2) and of the pairs before them
+        double total = (double)pairs * (pairs + 1) - (double)first_dense * (first_dense + 1);
+        if (first_dense > 0) {
+            const double window = (p.n_local + BM - 1) / BN + 2 + (p.n_init + BN - 1) / BN;
+            const double grown = window / 2 < first_dense ? window / 2 : first_dense;
+            total += grown * grown + (first_dense - grown) * window;
+        }
+        const double per_slot = total * (double)heads / slots;
+        const int longest = p.rows;
+        if (2.0 * longest > per_slot) {
+            return capped(first_dense, longest, per_slot > SEG_MIN ? (int)per_slot : SEG_MIN);
+        }
+        if (dense) return none;
+    }
+    if (heads * pairs > 64) return none;
+    return capped(0, 2 * pairs + SEG_MIN, SEG_MIN);
+}
+
+size_t split_bytes(const SplitPlan &s, const AttnParams &p, int head_dim) {
+    const size_t pairs = (size_t)((p.rows + 1) / 2 - s.first) * p.batch * (p.head_list ? p.index_heads : p.hq);
+    const size_t slot = head_dim == 256 ? SplitSlot<256>::BYTES : (head_dim == 128 ? SplitSlot<128>::BYTES : SplitSlot<64>::BYTES);
+    return pairs * s.nseg * slot;
+}
+
+template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void *stream) {
     if (p.batch == 0 || p.rows == 0) return MINF_OK;
+    const int dtype = t->dtype;
+    if (t->workspace && ((uintptr_t)t->workspace & 15) == 0) {
+        const SplitPlan s = plan_split(MODE, p, HD);
+        if (s.nseg > 1 && split_bytes(s, p, HD) <= t->workspace_bytes) {
+            p.split_first = s.first; p.nseg = s.nseg; p.seg_len = s.len;
+            p.part = (char *)t->workspace;
+        }
+    }
     // heads of the grid: all of them, or the selected ones rounded up to whole chunks of hq / hk
     const int group = p.hq / p.hk;
     const long long grid_heads = p.head_list ? (long long)((p.index_heads + group - 1) / group) * group : p.hq;
-    p.total_wg = (long long)p.batch * grid_heads * ((p.rows + 1) / 2);
+    const int split_pairs = (p.rows + 1) / 2 - p.split_first;
+    p.total_wg = (long long)p.batch * grid_heads * (p.split_first + (long long)split_pairs * p.nseg);
     p.descending = MODE == MODE_DENSE || (MODE == MODE_VS && p.rows <= 1024);
     const long long per_xcd = (p.total_wg + 7) >> 3;
     const long long grid = per_xcd * 8;
     if (grid > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
     const dim3 block(2 * NTHREADS);
     hipStream_t st = (hipStream_t)stream;
-    if (dtype == MINF_BF16) hipLaunchKernelGGL((attn_fwd_kernel<__bf16, MODE, HD>), dim3((unsigned)grid), block, 0, st, p);
-    else hipLaunchKernelGGL((attn_fwd_kernel<_Float16, MODE, HD>), dim3((unsigned)grid), block, 0, st, p);
+#define MINF_LAUNCH_ATTN(T)                                                                                      \
+    do {                                                                                                         \
+        if (p.nseg > 1) hipLaunchKernelGGL((attn_fwd_kernel<T, MODE, HD, true>), dim3((unsigned)grid), block, 0, st, p); \
+        else hipLaunchKernelGGL((attn_fwd_kernel<T, MODE, HD, false>), dim3((unsigned)grid), block, 0, st, p);   \
+    } while (0)
+    if (dtype == MINF_BF16) MINF_LAUNCH_ATTN(__bf16);
+    else MINF_LAUNCH_ATTN(_Float16);
+#undef MINF_LAUNCH_ATTN
+    const int status = minf_launch_status();
+    if (status != MINF_OK || p.nseg == 1) return status;
+    const unsigned merge_wgs = (unsigned)(4ll * split_pairs * p.batch * (p.head_list ? p.index_heads : p.hq));
+    if (dtype == MINF_BF16) hipLaunchKernelGGL((attn_merge_kernel<__bf16, HD>), dim3(merge_wgs), dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((attn_merge_kernel<_Float16, HD>), dim3(merge_wgs), dim3(256), 0, st, p);
     return minf_launch_status();
 }
 
 template <int MODE> int launch(const AttnParams &p, const minf_qkvo *t, void *stream) {
     if constexpr (MODE == MODE_ASHAPE || MODE == MODE_DENSE)
-        if (t->head_dim == 256) return launch_hd<MODE, 256>(p, t->dtype, stream);
+        if (t->head_dim == 256) return launch_hd<MODE, 256>(p, t, stream);
     if (t->head_dim == 256) return MINF_ERR_UNSUPPORTED;
-    return t->head_dim == 64 ? launch_hd<MODE, 64>(p, t->dtype, stream) : launch_hd<MODE, 128>(p, t->dtype, stream);
+    return t->head_dim == 64 ? launch_hd<MODE, 64>(p, t, stream) : launch_hd<MODE, 128>(p, t, stream);
 }
 
 }  // namespace
@@ -1145,4 +1351,16 @@ extern "C" int minf_dense_attn_fwd(const minf_qkvo *t, void *stream) {
     AttnParams p;
     fill_params(p, t);
     return launch<MODE_DENSE>(p, t, stream);
+}
+
+extern "C" size_t minf_attn_workspace_bytes(const minf_qkvo *t, int op, int n_init, int n_local, int n_last) {
+    if (!t || t->batch <= 0 || t->n <= 0 || t->heads_q <= 0 || op < MINF_OP_VERTICAL_SLASH || op > MINF_OP_DENSE) return 0;
+    AttnParams p;
+    fill_params(p, t);
+    if (op == MINF_OP_ASHAPE) {
+        p.n_init = n_init; p.n_local = n_local;
+        p.dense_from = n_last > 0 ? (n_last < t->n ? t->n - n_last : 0) : p.dense_from;
+    }
+    const SplitPlan s = plan_split(op, p, t->head_dim);
+    return s.nseg > 1 ? split_bytes(s, p, t->head_dim) : 0;
 }

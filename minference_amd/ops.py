@@ -127,6 +127,14 @@ class _Call:
         self.struct.head_list = head_list.data_ptr() if head_list is not None else None
         self.struct.index_heads = int(head_list.numel()) if head_list is not None else 0
 
+    def scratch(self, op, n_init=0, n_local=0, n_last=0):
+        """Give the next launch of ``op`` the scratch memory its split walks use (none for most)."""
+        nbytes = _lib.load().minf_attn_workspace_bytes(self.ref, op, int(n_init), int(n_local), int(n_last))
+        # (a block freed here is reused only by later work on the same stream)
+        self._scratch = torch.empty(nbytes, dtype=torch.uint8, device=self.q.device) if nbytes else None
+        self.struct.workspace = self._scratch.data_ptr() if nbytes else None
+        self.struct.workspace_bytes = nbytes
+
     def result(self):
         o = self.o
         if self.head_dim != self.kernel_dim:
@@ -150,6 +158,7 @@ def vertical_slash_attention_from_index(query, key, value, block_count, block_of
         raise ValueError("index tensors must be [batch, heads_q, ceil(n/64), ...]")
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
+        c.scratch(_lib.MINF_OP_VERTICAL_SLASH)
         st = lib.minf_vs_attn_fwd(c.ref, block_count.data_ptr(), block_offset.data_ptr(),
                                   column_count.data_ptr(), column_index.data_ptr(), rows,
                                   block_offset.shape[-1], column_index.shape[-1],
@@ -187,6 +196,7 @@ def block_sparse_attention_from_index(query, key, value, block_index):
         raise ValueError("block_index has the wrong batch/head/row sizes")
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
+        c.scratch(_lib.MINF_OP_BLOCK_SPARSE)
         st = lib.minf_bs_attn_fwd(c.ref, block_index.data_ptr(), block_index.shape[2],
                                   block_index.shape[3], _lib.stream_ptr(c.q.device))
     _lib.check(st, "minf_bs_attn_fwd")
@@ -252,6 +262,7 @@ def streaming_forward(q, k, v, n_init: int, n_local: int):
     c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, sm_scale=_streaming_scale(q.shape[-1]))
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
+        c.scratch(_lib.MINF_OP_ASHAPE, n_init, n_local)
         st = lib.minf_ashape_attn_fwd(c.ref, int(n_init), int(n_local), _lib.stream_ptr(c.q.device))
     _lib.check(st, "minf_ashape_attn_fwd")
     return c.result()
@@ -266,6 +277,7 @@ def tri_shape_forward(q, k, v, n_init: int, n_local: int, n_last: int = 100):
     n_last = min(int(n_last), c.N - 1)                   # reference: min(n_last, q.size(2) - 1)
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
+        c.scratch(_lib.MINF_OP_ASHAPE, n_init, n_local, max(n_last, 0))
         st = lib.minf_trishape_attn_fwd(c.ref, int(n_init), int(n_local), max(n_last, 0),
                                         float(c.head_dim) ** -0.5, _lib.stream_ptr(c.q.device))
     _lib.check(st, "minf_trishape_attn_fwd")
@@ -277,6 +289,7 @@ def dense_causal_attention(q, k, v):
     c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING)
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
+        c.scratch(_lib.MINF_OP_DENSE)
         st = lib.minf_dense_attn_fwd(c.ref, _lib.stream_ptr(c.q.device))
     _lib.check(st, "minf_dense_attn_fwd")
     return c.result()

@@ -193,6 +193,7 @@ def _mixed_layer(query_states, key_states, value_states, lp):
                 bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, 64, 64, zero_fill=False)
                 c.struct.seqlens = seqlens.data_ptr()
                 c.select_heads(slot)
+                c.scratch(_lib.MINF_OP_VERTICAL_SLASH)
                 st = lib.minf_vs_attn_fwd(c.ref, bc.data_ptr(), bo.data_ptr(), cc.data_ptr(), ci.data_ptr(), rows,
                                           smax, vmax, stream)
                 c.struct.seqlens = None
@@ -212,6 +213,7 @@ def _mixed_layer(query_states, key_states, value_states, lp):
                                                    ws.data_ptr(), ws_bytes, stream)
                 _lib.check(st, "minf_bs_block_index_heads")
                 c.select_heads(slot)
+                c.scratch(_lib.MINF_OP_BLOCK_SPARSE)
                 st = lib.minf_bs_attn_fwd(c.ref, bi.data_ptr(), brows, kk, stream)
                 _lib.check(st, "minf_bs_attn_fwd")
                 keep += [ws, bi]
@@ -220,6 +222,7 @@ def _mixed_layer(query_states, key_states, value_states, lp):
             for (n_init, n_local), slot in dt["stream_heads"].items():
                 c.select_heads(slot)
                 if N > 0:
+                    c.scratch(_lib.MINF_OP_ASHAPE, n_init, n_local)
                     st = lib.minf_ashape_attn_fwd(c.ref, int(n_init), int(n_local), stream)
                     _lib.check(st, "minf_ashape_attn_fwd")
     finally:

@@ -1,0 +1,75 @@
+"""Split walks (few row blocks, or a few walks far longer than the rest): segments of a walk on several
+workgroups and the fold of their sums, against the fp32 masked-dense oracle.  Sizes: one step, exactly one
+segment (8 steps), one step more, a ragged end, a lone row block in the last pair, rows past seqlen.
+Tolerance: that of the tile engine (the fold adds fp32 roundings only)."""
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests import gen
+from tests.test_gpu_attention import check, expand, make, sdpa_causal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16), (256, torch.bfloat16)])
+@pytest.mark.parametrize("n,hq,hk,b", [(1, 1, 1, 1), (512, 2, 1, 1), (576, 1, 1, 2), (1300, 4, 2, 1)])
+def test_split_walks_match_the_oracle(gpu, n, hq, hk, b, d, dtype):
+    import minference_amd as M
+    print(f"case split n={n} hq={hq} b={b} d={d} {dtype}", flush=True)
+    q, k, v = make(b, hq, hk, n, n + d, dtype, d)
+    qg, kg, vg, ke, ve = q.to(gpu), k.to(gpu), v.to(gpu), expand(k, hq), expand(v, hq)
+    check(M.dense_causal_attention(qg, kg, vg), sdpa_causal(q, ke, ve), "dense")
+    check(M.streaming_forward(qg, kg, vg, 70, 300), O.streaming_forward(q, ke, ve, 70, 300), "a-shape")
+    if n > 1:
+        check(M.tri_shape_forward(qg, kg, vg, 8, 130, 100), O.tri_shape_forward(q, ke, ve, 8, 130, 100), "tri-shape")
+    if d <= 128:
+        check(M.block_sparse_attention(qg, kg, vg, 1000), sdpa_causal(q, ke, ve), "block-sparse")
+        v_idx, s_idx = M.estimate_vertical_slash(qg, kg, 40, 300)
+        check(M.vertical_slash_sparse_attention(qg, kg, vg, v_idx, s_idx),
+              O.vertical_slash_sparse_attention(q, ke, ve, v_idx.cpu(), s_idx.cpu()), "vertical-slash")
+
+
+def test_split_walks_with_short_sequences_and_many_leftovers(gpu):
+    """seqlens below n in the middle of a pair, before one and in the first tile (rows past them are zero),
+    with lists whose leftovers differ between the row blocks of a pair (scattered slashes)."""
+    import minference_amd as M
+    n, b = 1100, 3
+    q, k, v = make(b, 1, 1, n, 5, torch.bfloat16)
+    qg, kg, vg = q.to(gpu), k.to(gpu), v.to(gpu)
+    vi, si = gen.vs_index_inputs(1, n, 60, 40, seed=9, batch=b)
+    lens = torch.tensor([900, 1024, 10], dtype=torch.int32)
+    idx = M.convert_vertical_slash_indexes(lens.to(gpu), torch.from_numpy(vi).to(gpu), torch.from_numpy(si.copy()).to(gpu), n)
+    out = M.vertical_slash_attention_from_index(qg, kg, vg, *idx, lens.to(gpu))
+    bc, bo, cc, ci = (x.cpu().numpy() for x in idx)
+    for i in range(b):
+        mask = O.vs_mask(bc[i, 0], bo[i, 0], cc[i, 0], ci[i, 0], n, int(lens[i]))
+        check(out[i:i + 1, :1], O.masked_attention(q[i, 0], k[i, 0], v[i, 0], mask)[None, None], f"batch {i}")
+        assert (out[i, 0, int(lens[i]):] == 0).all()
+
+
+def test_split_segments_with_scores_past_the_fp32_range(gpu):
+    """A segment whose sums overflow under its lazy maximum walks again; segments whose maxima lie
+    hundreds of powers of two apart fold to the last one."""
+    import minference_amd as M
+    n = 2048
+    q, k, v, _ = gen.planted_layer(n, 1, 1, seed=100, dtype=torch.bfloat16, decay_per_token=80 * 2.0 ** -7 / 128 ** 0.5)
+    qg, kg, vg = q.to(gpu), k.to(gpu), v.to(gpu)
+    check(M.dense_causal_attention(qg, kg, vg), sdpa_causal(q, k, v), "rising dense")
+    assert (M.dense_causal_attention(qg, kg, torch.ones_like(vg)).float() - 1).abs().max().item() <= 2.0 ** -8
+
+
+def test_which_launches_are_split():
+    """The rule, on the host: short single heads and long dense walks are, full layers are not."""
+    import ctypes
+    from minference_amd import _lib
+    lib = _lib.load()
+
+    def nbytes(op, n, hq, *sizes, d=128):
+        t = _lib.QKVO()
+        t.batch, t.heads_q, t.heads_kv, t.n, t.head_dim = 1, hq, 1, n, d
+        return lib.minf_attn_workspace_bytes(ctypes.byref(t), op, *(sizes or (0, 0, 0)))
+    vs, ashape, dense = _lib.MINF_OP_VERTICAL_SLASH, _lib.MINF_OP_ASHAPE, _lib.MINF_OP_DENSE
+    assert nbytes(vs, 4096, 1) > 0 and nbytes(vs, 8192, 1) > 0 and nbytes(vs, 8193, 1) == 0 and nbytes(vs, 4096, 32) == 0
+    assert nbytes(dense, 16384, 1) > 0 and nbytes(dense, 6144, 64) == 0 and nbytes(dense, 64, 1) == 0
+    assert nbytes(ashape, 24000, 16, 8, 512, 128, d=64) > 0 and nbytes(ashape, 24000, 16, 8, 512, 0, d=64) == 0
