@@ -110,6 +110,7 @@ struct AttnParams {
     int n_init, n_local, dense_from;
     long long total_wg;
     int descending;          // row blocks are handed out from the last one down
+    int stripes;             // the row-block pairs of a kv group are dealt to this many XCD ranges (see launch_hd)
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
     // every head is processed and index_heads = hq
@@ -312,7 +313,10 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     const int rows_wg = (p.rows + 1) >> 1;                           // row-block pairs per (batch, head)
     const int split_units = (rows_wg - p.split_first) * p.nseg;      // (no split: split_first == rows_wg)
     const unsigned units = (unsigned)(p.split_first + split_units);
-    const int mi = (int)(rest % units); rest /= units;
+    const unsigned per_stripe = (units + (unsigned)p.stripes - 1u) / (unsigned)p.stripes;
+    const unsigned in_stripe = rest % per_stripe; rest /= per_stripe;
+    const int mi = (int)(in_stripe * (unsigned)p.stripes + rest % (unsigned)p.stripes); rest /= (unsigned)p.stripes;
+    if (mi >= (int)units) return false;              // padding of the last round (workgroup-uniform)
     int mslot, seg = -1;                             // row-block pair, segment of its walk (-1: the whole walk)
     if (CUT && mi < split_units) {                    // the split pairs, longest walks first
         mslot = rows_wg - 1 - mi / p.nseg;
@@ -1190,6 +1194,7 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.head_list = t->head_list;
     p.index_heads = t->head_list ? t->index_heads : t->heads_q;
     p.total_wg = 0;          // set by the launcher
+    p.stripes = 1;
     p.descending = 0;
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
 }
@@ -1258,7 +1263,24 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
     const int group = p.hq / p.hk;
     const long long grid_heads = p.head_list ? (long long)((p.index_heads + group - 1) / group) * group : p.hq;
     const int split_pairs = (p.rows + 1) / 2 - p.split_first;
-    p.total_wg = (long long)p.batch * grid_heads * (p.split_first + (long long)split_pairs * p.nseg);
+    const long long units = p.split_first + (long long)split_pairs * p.nseg;
+    // Every XCD works through one contiguous eighth of the logical order.  When the kv groups do not
+    // divide evenly among the XCDs, an eighth is a stretch of one group's row blocks, and where the work
+    // grows with the row block the XCD with the last ones is left working alone.  The row blocks are then
+    // dealt to the XCDs in turn, as many stripes per group as make the count divisible by eight: dense,
+    // 16384 tokens, 8 / 2 heads 750 -> 480 us, 28 / 4 heads 2.11 -> 1.69 ms.  The list walks and A-shape
+    // grow only at the start of the sequence and share tiles with their neighbours, which the stripes
+    // part: vertical-slash 28 / 4 heads 16384 tokens 1.63 -> 1.39 ms, 60000 tokens 6.27 -> 5.85, 8 / 2
+    // heads 16384 tokens 698 -> 645 us; but 4 / 4 heads 32768 tokens 546 -> 577 us, one head 65536 tokens
+    // 366 -> 381, A-shape 4 / 4 heads 16384 tokens 129 -> 134: so from eight heads and two rounds of
+    // workgroups on, up to 64K tokens.
+    const long long groups = (long long)p.batch * (grid_heads / group);
+    const bool grows = MODE == MODE_DENSE || split_pairs > 0 ||
+                       (p.rows <= 1024 && groups * group >= 8 && groups * group * units >= 1024);
+    p.stripes = 1;
+    if (grows)
+        while (p.stripes < 8 && groups * p.stripes % 8) p.stripes *= 2;
+    p.total_wg = groups * group * p.stripes * ((units + p.stripes - 1) / p.stripes);
     p.descending = MODE == MODE_DENSE || (MODE == MODE_VS && p.rows <= 1024);
     const long long per_xcd = (p.total_wg + 7) >> 3;
     const long long grid = per_xcd * 8;

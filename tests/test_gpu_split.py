@@ -73,3 +73,17 @@ def test_which_launches_are_split():
     assert nbytes(vs, 4096, 1) > 0 and nbytes(vs, 8192, 1) > 0 and nbytes(vs, 8193, 1) == 0 and nbytes(vs, 4096, 32) == 0
     assert nbytes(dense, 16384, 1) > 0 and nbytes(dense, 6144, 64) == 0 and nbytes(dense, 64, 1) == 0
     assert nbytes(ashape, 24000, 16, 8, 512, 128, d=64) > 0 and nbytes(ashape, 24000, 16, 8, 512, 0, d=64) == 0
+
+
+@pytest.mark.parametrize("hq,hk,n,b", [(3, 1, 900, 1), (6, 3, 700, 2), (10, 5, 13400, 1)])
+def test_striped_row_blocks_cover_every_row(gpu, hq, hk, n, b):
+    """Head counts that do not divide among the eight XCDs: the row-block pairs are dealt out in stripes
+    with a padded last round; with V = 1 every row of every head must come out as exactly 1 (the last
+    size also reaches the striped list walks: ten heads, 105 pairs)."""
+    import minference_amd as M
+    q, k, _ = make(b, hq, hk, n, 3, torch.bfloat16)
+    qg, kg = q.to(gpu), k.to(gpu)
+    ones = torch.ones_like(kg)
+    for out in (M.dense_causal_attention(qg, kg, ones), M.streaming_forward(qg, kg, ones, 64, 500),
+                M.block_sparse_attention(qg, kg, ones, 20), M.vertical_slash_prefill(qg, kg, ones, 100, 300)):
+        assert (out.float() - 1).abs().max().item() <= 2.0 ** -8
