@@ -12,7 +12,7 @@
 // memory too when the waves of a workgroup score different kv heads, and otherwise fetched once
 // per workgroup into LDS (LDS-DMA, double buffered) and read from there by all four waves:
 //   stats  : S^T = K.Q^T  -> lane <-> query row: running max / sum-of-exp in
-//            registers, one (max, sum) pair per row per 2048-key chunk;
+//            registers, one (max, sum) pair per row per chunk of keys;
 //   (every workgroup of the second sweep first combines the chunk pairs of its heads into the row
 //   constants M_i = max_i + log2(sum_i): no kernel in between)
 //   scores : S = Q.K^T    -> lane <-> key: p = exp2(s - M_row); column sums are
@@ -21,7 +21,7 @@
 //            LDS tile, no atomics); the per-chunk window is written out whole;
 //   finalize: stitch the chunk windows together (each diagonal gets at most two
 //            pieces, added in a fixed order) and apply the forced +inf entries.
-// Work split: a workgroup owns one 2048-key chunk of one group of up to four query heads that are
+// Work split: a workgroup owns one chunk of keys of one group of up to four query heads that are
 // neighbours in head order (with grouped-query attention: heads that read the same K): wave w
 // scores head w % gw over key sub-range w / gw of the chunk (gw = heads per workgroup: 4, 2 or 1),
 // so the K fragments that the four waves fetch are the same cache lines at the same time -- one
@@ -44,20 +44,24 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4_t;
 
 constexpr int LQ = 64;          // query rows held per head (last_q <= LQ)
-#ifndef EST_KC
-#define EST_KC 2048
-#endif
-constexpr int KC = EST_KC;      // keys per workgroup
+// Keys per workgroup (a chunk), by the number of tokens alone: short chunks give short prompts enough
+// workgroups, long ones keep the per-chunk work (row constants, window) small: a workgroup walks its blocks
+// one after the other, 1.35 us each over both sweeps.  Whole estimate, us, with 128 / 256 / 512 / 1024 / 2048
+// keys: 4096 tokens, 1 head 17 / 19 / 24 / 34 / 53, 32 heads 28 / 36 / 56 / 95 / 174; 16384 tokens, 32 heads
+// 87 / 60 / 61 / 98 / 176; 32768 tokens, 8 heads 63 / 45 / 60 / 97 / 175, 32 heads 206 / 115 / 93 / 104 / 177;
+// 50000 tokens, 8 heads 142 / 72 / 63 / 99 / 176, 32 heads 418 / 203 / 162 / 152 / 181; 131072 tokens, 8 heads
+// - / 194 / 108 / 105 / 179, 32 heads - / 705 / 360 / 288 / 281.
+constexpr int KC_MAX = 2048;
+__host__ __device__ inline int chunk_keys(int n) {
+    return n > 131072 ? 2048 : (n > 57344 ? 1024 : (n > 20480 ? 512 : (n > 6144 ? 256 : 128)));
+}
 constexpr int EST_THREADS = 256;
-constexpr int WIN = KC + LQ;    // diagonal window of one chunk
-// A chunk is always summed as four pieces of KC/4 keys, each piece by one wave from its first key to
+// A chunk is always summed as four pieces of a quarter of its keys, each piece by one wave from its first key to
 // its last, and the pieces are combined in ascending order -- whether one wave walks the whole chunk
 // (four heads per workgroup) or four waves a piece each (one head per workgroup).  The scores of a
 // head therefore do not depend, not even in the last bit, on which other heads share its launch.
-constexpr int PIECE = KC / 4;
-constexpr int PB = PIECE / 32;  // 32-key blocks per piece
-constexpr int PWIN = PIECE + LQ;
-static_assert(KC % 128 == 0, "a chunk is four pieces of whole 32-key blocks");
+constexpr int PWIN_MAX = KC_MAX / 4 + LQ;      // diagonal window of a piece
+static_assert(KC_MAX % 128 == 0, "a chunk is four pieces of whole 32-key blocks");
 
 struct EstParams {
     const char *q, *k;
@@ -66,8 +70,9 @@ struct EstParams {
     float scale_log2;
     float scale;                // sm_scale itself (the rounded form scales in the natural-log domain)
     int nchunks;
+    int kc;                     // keys per chunk (chunk_keys)
     float *stats;               // [B, Hq, nchunks, LQ, 2]
-    float *win;                 // [B, Hq, nchunks, WIN]
+    float *win;                 // [B, Hq, nchunks, kc + LQ]
     float *vertical, *slash;    // [B, Hq, N]
     int force_v, force_s;
     long long total_wg;
@@ -242,8 +247,9 @@ __global__ __launch_bounds__(EST_THREADS, 3) void est_stats_kernel(const EstPara
     const WgId w = decode_wg(p, wave, false);
     if (!w.valid) return;
     const int l32 = lane & 31, g = lane >> 5;
+    const int KC = p.kc, PB = KC / 128;               // keys per chunk, 32-key blocks per piece
     const int nq = 4 / p.gw, klen = KC / nq;          // key sub-ranges per head, keys per wave
-    const int ppw = p.gw;                             // pieces per wave (klen / PIECE)
+    const int ppw = p.gw;                             // pieces per wave
     const int piece0 = (wave % p.gw) * 4 + w.kq * ppw; // this wave's first (head, piece) slot
 
     // lane <-> query rows i = l32 and 32 + l32; regs <-> keys 8*(r/4) + 4*g + r%4 of the block
@@ -338,7 +344,7 @@ __global__ __launch_bounds__(EST_THREADS, 3) void est_stats_kernel(const EstPara
                 ks_.template frags<KS>(blk & 1, lane, kf);
                 score_block(c0, kf);
             }
-            if (w.wave_valid && (blk + 1) % PB == 0) flush_piece();
+            if (w.wave_valid && ((blk + 1) & (PB - 1)) == 0) flush_piece();
         }
     } else if (w.wave_valid) {
         const char *kb = p.k + ((long long)w.b * p.ks[0] + (long long)w.hkv * p.ks[1]) * 2;
@@ -351,7 +357,7 @@ __global__ __launch_bounds__(EST_THREADS, 3) void est_stats_kernel(const EstPara
             for (int ks = 0; ks < KS; ++ks) kf[ks] = kn[ks];
             load_k(p, kb, min(c0 + 32, p.n - 1), lane, kn);      // next block, in flight during this one
             score_block(c0, kf);
-            if ((blk + 1) % PB == 0) flush_piece();
+            if (((blk + 1) & (PB - 1)) == 0) flush_piece();
         }
     }
     // (pieces past the end of the sequence: what is left of the running pair, then empty pairs)
@@ -397,16 +403,18 @@ __device__ __forceinline__ float wave_shr1(float x) {      // lane L <- lane L -
 template <typename T, int HD, bool RR>
 __global__ __launch_bounds__(EST_THREADS, 2) void est_scores_kernel(const EstParams p) {
     constexpr int KS = HD / 16;
-    __shared__ float lds_pwin[16][PWIN];               // [head of the workgroup * 4 + piece][slot]
+    __shared__ float lds_pwin[16 * PWIN_MAX];          // [head of the workgroup * 4 + piece][PWIN]
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // wave-uniform: addresses built from it stay scalar
     const WgId w = decode_wg(p, wave, true);
     if (!w.valid) return;
     const int l32 = lane & 31, g = lane >> 5;
+    const int KC = p.kc, PIECE = KC / 4, PB = PIECE / 32, PWIN = PIECE + LQ, WIN = KC + LQ;
+    const int pb_shift = __builtin_ctz(PB);
     const int nq = 4 / p.gw, klen = KC / nq;          // key sub-ranges per head, keys per wave
-    const int ppw = p.gw;                             // pieces per wave (klen / PIECE)
+    const int ppw = p.gw;                             // pieces per wave
     const long long bh = (long long)w.b * p.index_heads + w.slot;
-    float *const wwin0 = lds_pwin[(wave % p.gw) * 4 + w.kq * ppw];   // this wave's ppw piece windows, contiguous
+    float *const wwin0 = lds_pwin + ((wave % p.gw) * 4 + w.kq * ppw) * PWIN;   // this wave's ppw piece windows, contiguous
 
     for (int i = lane; i < ppw * PWIN; i += 64) wwin0[i] = 0.f;
     __syncthreads();
@@ -463,8 +471,9 @@ __global__ __launch_bounds__(EST_THREADS, 2) void est_scores_kernel(const EstPar
         // The block adds to 95 slots of the diagonal window, as two disjoint ranges: s1 + (0..63) and,
         // in lanes 32..62, s2 = s1 + 32.  Their old values are read now, a block's work ahead of the
         // add (window slot of lane L, row half mb: 32*blk + L + 32 - 32*mb - rshift = key - row + 63 - rshift).
-        float *const wwin = wwin0 + (blk / PB) * PWIN;                  // the window of this block's piece
-        const int s1 = 32 * (blk % PB) + lane - rshift, s2 = s1 + 32;
+        const int piece = blk >> pb_shift;
+        float *const wwin = wwin0 + piece * PWIN;                       // the window of this block's piece
+        const int s1 = 32 * (blk & (PB - 1)) + lane - rshift, s2 = s1 + 32;
         const bool ok1 = s1 >= 0, ok2 = lane >= 32 && lane < 63 && s2 >= 0;
         const float w1 = ok1 ? wwin[s1] : 0.f;
         const float w2 = ok2 ? wwin[s2] : 0.f;
@@ -583,7 +592,7 @@ __global__ __launch_bounds__(EST_THREADS, 2) void est_scores_kernel(const EstPar
         float acc = 0.f;
         for (int pc = 0; pc < 4; ++pc) {
             const int sl = q - pc * PIECE;
-            if (sl >= 0 && sl < PWIN) acc += lds_pwin[hsub * 4 + pc][sl];
+            if (sl >= 0 && sl < PWIN) acc += lds_pwin[(hsub * 4 + pc) * PWIN + sl];
         }
         p.win[(((long long)wh.b * p.index_heads + wh.slot) * p.nchunks + wh.chunk) * WIN + q] = acc;
     }
@@ -594,6 +603,7 @@ __global__ __launch_bounds__(256) void est_finalize_kernel(const EstParams p) {
     const long long bh = blockIdx.y;
     const int j = (int)(blockIdx.x * 256 + threadIdx.x);
     if (j >= p.n) return;
+    const int KC = p.kc, WIN = KC + LQ;
     const int c = j / KC, off = j - c * KC;
     const float *wbase = p.win + bh * p.nchunks * WIN;
     // diagonal j lives at window position `off` of chunk c and, when off < LQ, also at
@@ -624,10 +634,11 @@ int fill(EstParams &p, const void *q, const void *k, const int64_t *q_stride, co
     p.last_q = last_q < n ? last_q : n;
     p.scale_log2 = sm_scale * 1.4426950408889634f;
     p.scale = sm_scale;
-    p.nchunks = (n + KC - 1) / KC;
+    p.kc = chunk_keys(n);
+    p.nchunks = (n + p.kc - 1) / p.kc;
     const long long bh = (long long)batch * index_heads;
     const size_t stats_b = (size_t)bh * p.nchunks * LQ * 2 * sizeof(float);
-    const size_t win_b = (size_t)bh * p.nchunks * WIN * sizeof(float);
+    const size_t win_b = (size_t)bh * p.nchunks * (p.kc + LQ) * sizeof(float);
     if (ws_bytes < stats_b + win_b) return MINF_ERR_WORKSPACE;
     if ((uintptr_t)ws & 15) return MINF_ERR_ALIGNMENT;
     p.stats = (float *)ws;
@@ -649,8 +660,8 @@ int fill(EstParams &p, const void *q, const void *k, const int64_t *q_stride, co
 extern "C" size_t minf_vs_estimate_workspace_bytes(int batch, int heads_q, int n) {
     if (batch <= 0 || heads_q <= 0 || n <= 0) return 0;
     const size_t bh = (size_t)batch * heads_q;
-    const size_t nchunks = ((size_t)n + KC - 1) / KC;
-    return bh * nchunks * LQ * 2 * sizeof(float) + bh * nchunks * WIN * sizeof(float);
+    const size_t kc = chunk_keys(n), nchunks = ((size_t)n + kc - 1) / kc;
+    return bh * nchunks * LQ * 2 * sizeof(float) + bh * nchunks * (kc + LQ) * sizeof(float);
 }
 
 static int estimate_launch(const void *q, const void *k, const int64_t *q_stride, const int64_t *k_stride,

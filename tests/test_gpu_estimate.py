@@ -158,3 +158,17 @@ def test_a_heads_scores_do_not_depend_on_the_heads_it_is_launched_with(gpu, hq, 
         if group > 1:      # ... and two heads of a group launched as a pair
             v2, s2 = vertical_slash_scores(qg[:, :2], kg[:, :1], reference_rounding=rounded)
             assert torch.equal(v2[0], vert[0, :2]) and torch.equal(s2[0], slash[0, :2]), rounded
+
+
+@pytest.mark.parametrize("n", [31, 128, 129, 6144, 6145, 20480, 20481 + 31, 57344 + 1])
+def test_scores_at_the_edges_of_the_chunk_lengths(gpu, n):
+    """The chunk length depends on the number of tokens: one short of a change, at it and past it, ragged
+    last chunks and pieces, fewer tokens than the 64 scored rows.  fp32 arithmetic on both sides (sums in
+    another order: 1e-3, the bound of the score test above)."""
+    from minference_amd.estimate import vertical_slash_scores
+    q, k, _ = gen.qkv(1, 4, 1, n, 128, seed=n, scale=1.0)
+    q, k = q.bfloat16(), k.bfloat16()
+    vert, slash = vertical_slash_scores(q.to(gpu), k.to(gpu), force_vertical=0, force_slash=0, reference_rounding=False)
+    rv, rs = O.estimate_scores(q, expand(k, 4))
+    assert torch.allclose(vert.cpu(), rv, rtol=1e-3, atol=1e-6)
+    assert torch.allclose(slash.cpu(), rs, rtol=1e-3, atol=1e-6)
