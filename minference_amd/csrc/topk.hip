@@ -23,6 +23,7 @@ namespace {
 
 constexpr int TK_THREADS = 1024;
 constexpr int TK_WAVES = TK_THREADS / 64;
+constexpr int TK_FEW_ROWS = 1024;     // up to here a workgroup per row beats a wavefront per row (see topk_regs_kernel)
 constexpr int TK_DEPTH = 16;          // independent 16-byte loads per thread in the sweeps
 
 __device__ __forceinline__ unsigned order_key(float x) {
@@ -453,7 +454,177 @@ __global__ __launch_bounds__(TKW_WAVES * 64, ITEMS >= 64 ? 3 : (ITEMS >= 40 ? 5 
     }
 }
 
+// One radix pass' digit: the workgroup's histogram of the current bucket -> the bin that holds the
+// `need`-th largest key.  Threads 0..255 fold the COPIES copies of one bin each (rotated: one bank per
+// thread), bin 255 - tid, so that an inclusive prefix scan over the threads counts the entries in this
+// bin and above.  (All threads call it after the barrier that ends the tally.)
+struct TopkShared {
+    unsigned bins[4];                        // bin counts of waves 0..3
+    unsigned prefix, need, count;            // the threshold's digits so far, rank inside the bucket, its size
+    unsigned listed;
+    int last;
+    int wave_gt[TK_WAVES], wave_eq[TK_WAVES];
+};
+template <int COPIES>
+__device__ __forceinline__ void topk_digit(const unsigned *hist, TopkShared &sh, unsigned &prefix, unsigned &need, int shift) {
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    unsigned cnt = 0, incl = 0;
+    const int b = 255 - tid;
+    if (tid < 256) {
+#pragma unroll
+        for (int c = 0; c < COPIES; ++c) cnt += hist[b * COPIES + ((c + b) & (COPIES - 1))];
+        incl = cnt;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        if (lane == 63) sh.bins[wave] = incl;
+    }
+    __syncthreads();
+    if (tid < 256) {
+        for (int wv = 0; wv < wave; ++wv) incl += sh.bins[wv];
+        const unsigned excl = incl - cnt;
+        if ((excl < need && need <= incl) || (b == 0 && incl < need)) {
+            sh.prefix = prefix | ((unsigned)b << shift);
+            sh.need = need - excl;
+            sh.count = cnt;
+        }
+    }
+    if (tid == 0) sh.listed = 0;
+    __syncthreads();
+    prefix = sh.prefix;
+    need = sh.need;
+}
+
+// The end of the selection once the bucket is small: its m <= TK_LIST keys are in `list` (then zeros up to a
+// multiple of four); every thread ranks one of them against all.  -> T (the key of the k-th largest entry), need (entries equal to T that
+// are taken).
+constexpr int TK_LIST = 128;             // (512: ranking 500 keys takes longer than a radix pass, 10 against 6 us)
+__device__ __forceinline__ void topk_rank(unsigned *list, int m, TopkShared &sh, unsigned &T, unsigned &need) {
+    const int tid = (int)threadIdx.x;
+    if (tid < 4) list[m + tid] = 0u;
+    __syncthreads();
+    if (tid < m) {
+        const unsigned mine = list[tid];
+        unsigned gt = 0, ge = 0;
+        for (int i = 0; i < m; i += 4) {
+            const uint4 other = *reinterpret_cast<const uint4 *>(list + i);
+            gt += (other.x > mine) + (other.y > mine) + (other.z > mine) + (other.w > mine);
+            ge += (other.x >= mine) + (other.y >= mine) + (other.z >= mine) + (other.w >= mine);
+        }
+        if (gt < need && need <= ge) {           // (every thread with this key writes the same)
+            sh.prefix = mine;
+            sh.need = need - gt;
+        }
+    }
+    __syncthreads();
+    T = sh.prefix;
+    need = sh.need;
+}
+
+// Rows of up to 16384 entries (from the number of rows on at which one wavefront per row fills the chip:
+// only rows longer than topk_wave_kernel takes): one 1024-thread workgroup per row that holds the row's
+// keys in registers (ITEMS per thread; wave w owns the contiguous slice of 64 * ITEMS entries from
+// 64 * ITEMS * w on, item j of a lane is entry 64 j + lane of it), so that the row is read once where
+// topk_kernel sweeps it six times, and every pass after the load is LDS and register work.  Same selection,
+// with 8-bit radix passes from the top digit only until the bucket is small enough to be ranked at once.
+// Two selections in a launch, 32 rows each, us, before (wave kernel up to 4096 entries, else topk_kernel) and
+// now: 2048 entries 18.3 / 6.4, 4096 31.5 / 7.0, 5000 11.9 / 9.2, 8192 13.2 / 10.4, 16001 26.3 / 13.8; 32768
+// in 32 registers per thread 25.6 / 26.0 (and 64 spill), so longer rows are swept.  Rows of 2048 entries:
+// 512 of them 18.7 / 8.1, 1024 18.8 / 13.9, 2048 21.4 / 37 -- hence TK_FEW_ROWS.
+template <int ITEMS>
+__global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem p0, const TopkProblem p1, int n) {
+    const TopkProblem &pr = blockIdx.y == 0 ? p0 : p1;
+    const int kmax = pr.k, reverse_base = pr.reverse_base;
+    const int k = pr.k_rows ? max(1, min(pr.k_rows[blockIdx.x], kmax)) : kmax;
+    constexpr int COPIES = ITEMS > 4 ? 32 : 8;       // copies of the histogram: the fewer keys, the fewer collisions
+    __shared__ unsigned hist[256 * COPIES];
+    __shared__ __attribute__((aligned(16))) unsigned list[TK_LIST + 4];
+    __shared__ TopkShared sh;
+    const float *__restrict__ x = pr.scores + (long long)blockIdx.x * pr.row_stride;
+    int32_t *__restrict__ o = pr.out + (long long)blockIdx.x * pr.out_stride;
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (k >= n) {                    // everything is selected
+        for (int i = tid; i < n; i += TK_THREADS) o[i] = reverse_base >= 0 ? reverse_base - i : i;
+        return;
+    }
+    const int begin = wave * 64 * ITEMS;
+    unsigned key[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const int i = begin + 64 * j + lane;
+        key[j] = i < n ? order_key(x[i]) : 0u;               // padding sorts below every score
+    }
+    unsigned prefix = 0, need = (unsigned)k;
+    int shift = 32;
+    do {
+        const unsigned above = shift == 32 ? 0u : prefix >> shift;
+        const int top = shift;
+        shift -= 8;
+#pragma unroll
+        for (int i = 0; i < 256 * COPIES / TK_THREADS; ++i) hist[i * TK_THREADS + tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j)
+            if (top == 32 || key[j] >> top == above)
+                atomicAdd(&hist[((key[j] >> shift) & 255u) * COPIES + (lane & (COPIES - 1))], 1u);
+        __syncthreads();
+        topk_digit<COPIES>(hist, sh, prefix, need, shift);
+    } while (shift > 0 && sh.count > TK_LIST);
+    unsigned T = prefix;
+    if (shift > 0) {                                          // (workgroup-uniform) the bucket fits the list
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j)
+            if (key[j] >> shift == prefix >> shift && begin + 64 * j + lane < n) list[atomicAdd(&sh.listed, 1u)] = key[j];
+        __syncthreads();
+        topk_rank(list, (int)sh.listed, sh, T, need);        // (the bucket's count may hold padding)
+    }
+    const int r = (int)need;                                  // entries equal to T that are taken
+    int cgt = 0, ceq = 0;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        cgt += __builtin_popcountll(__ballot(key[j] > T));
+        ceq += __builtin_popcountll(__ballot(key[j] == T));
+    }
+    if (lane == 0) { sh.wave_gt[wave] = cgt; sh.wave_eq[wave] = ceq; }
+    __syncthreads();
+    int gt_before = 0, eq_before = 0;
+    for (int wv = 0; wv < wave; ++wv) { gt_before += sh.wave_gt[wv]; eq_before += sh.wave_eq[wv]; }
+    const uint64_t lt = minf_lanemask_lt();
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const int i = begin + 64 * j + lane;
+        const bool gt = key[j] > T, eq = key[j] == T && i < n;
+        const uint64_t mg = __ballot(gt), me = __ballot(eq);
+        if (mg | me) {                                        // (wave-uniform)
+            const int e_here = eq_before + __builtin_popcountll(me & lt);
+            if (gt || (eq && e_here < r)) {
+                const int pos = gt_before + __builtin_popcountll(mg & lt) + min(e_here, r);
+                const int val = reverse_base >= 0 ? reverse_base - i : i;
+                o[pos] = val;
+                if (pos == k - 1) sh.last = val;
+            }
+            gt_before += __builtin_popcountll(mg);
+            eq_before += __builtin_popcountll(me);
+        }
+    }
+    if (k < kmax && pr.pad_mode) {                            // (workgroup-uniform)
+        __syncthreads();
+        const int pad = pr.pad_mode == 2 ? sh.last : pr.pad_value;
+        for (int i = k + tid; i < kmax; i += TK_THREADS) o[i] = pad;
+    }
+}
+
 void launch_topk(const TopkProblem &pa, const TopkProblem &pb, int problems, int rows, int n, hipStream_t st) {
+    const dim3 grid((unsigned)rows, (unsigned)problems);
+    if (pa.causal_rows == 0 && n > 256 && n <= 16 * TK_THREADS && (n > 64 * 64 || (long long)rows * problems <= TK_FEW_ROWS)) {
+        if (n <= 4 * TK_THREADS) hipLaunchKernelGGL(topk_regs_kernel<4>, grid, dim3(TK_THREADS), 0, st, pa, pb, n);
+        else if (n <= 8 * TK_THREADS) hipLaunchKernelGGL(topk_regs_kernel<8>, grid, dim3(TK_THREADS), 0, st, pa, pb, n);
+        else hipLaunchKernelGGL(topk_regs_kernel<16>, grid, dim3(TK_THREADS), 0, st, pa, pb, n);
+        return;
+    }
     const dim3 grid_w((unsigned)((rows + TKW_WAVES - 1) / TKW_WAVES), (unsigned)problems);
     if (n <= 64 * 4)
         hipLaunchKernelGGL(topk_wave_kernel<4>, grid_w, dim3(TKW_WAVES * 64), 0, st, pa, pb, n, rows);
@@ -464,7 +635,7 @@ void launch_topk(const TopkProblem &pa, const TopkProblem &pb, int problems, int
     else if (n <= 64 * 64)
         hipLaunchKernelGGL(topk_wave_kernel<64>, grid_w, dim3(TKW_WAVES * 64), 0, st, pa, pb, n, rows);
     else
-        hipLaunchKernelGGL(topk_kernel, dim3((unsigned)rows, (unsigned)problems), dim3(TK_THREADS), 0, st, pa, pb, n);
+        hipLaunchKernelGGL(topk_kernel, grid, dim3(TK_THREADS), 0, st, pa, pb, n);
 }
 
 }  // namespace

@@ -172,3 +172,36 @@ def test_scores_at_the_edges_of_the_chunk_lengths(gpu, n):
     rv, rs = O.estimate_scores(q, expand(k, 4))
     assert torch.allclose(vert.cpu(), rv, rtol=1e-3, atol=1e-6)
     assert torch.allclose(slash.cpu(), rs, rtol=1e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("n", [257, 4096, 4097, 8192, 8193, 16384, 16385])
+@pytest.mark.parametrize("kind", ["random", "ties", "masked"])
+def test_topk_rows_held_in_registers(gpu, n, kind):
+    """Few rows of up to 16384 entries (one workgroup per row, keys in registers) at the edges of the register
+    counts: random scores, a handful of distinct values (threshold ties, buckets that never get small) and
+    rows that are -inf but for a few entries (fewer than k: the -inf ties take part), ragged k with both
+    paddings.  Exact against the lowest-index rule."""
+    from minference_amd import _lib
+    from minference_amd.estimate import topk_indices
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(3, n, generator=g)
+    if kind == "ties":
+        x = torch.randint(0, 4, (3, n), generator=g).float()
+    elif kind == "masked":
+        keep = torch.rand(3, n, generator=g) < 0.01
+        x = torch.where(keep, x, torch.tensor(-torch.inf))
+    xg = x.to(gpu)
+    for k in (1, 100, n // 2, n - 1):
+        want = O.topk_lowest_index(x, k).sort(-1)[0].int()
+        assert torch.equal(topk_indices(xg, k).cpu(), want), k
+        assert torch.equal(topk_indices(xg, k, reverse_base=n - 1).cpu(), n - 1 - want), k
+    kmax, rows = 200, torch.tensor([200, 7, 64], dtype=torch.int32, device=gpu)
+    a, b = (torch.empty(3, kmax, dtype=torch.int32, device=gpu) for _ in range(2))
+    st = _lib.load().minf_topk_indices_pair_ragged(xg.data_ptr(), rows.data_ptr(), kmax, a.data_ptr(), kmax, -1, 1, 12345,
+                                                   xg.data_ptr(), rows.data_ptr(), kmax, b.data_ptr(), kmax, n - 1, 2, 0,
+                                                   3, n, n, _lib.stream_ptr(gpu))
+    assert st == 0
+    for r, k in enumerate((200, 7, 64)):
+        want = O.topk_lowest_index(x[r], k).sort(-1)[0].int()
+        assert torch.equal(a[r, :k].cpu(), want) and (a[r, k:] == 12345).all()
+        assert torch.equal(b[r, :k].cpu(), n - 1 - want) and (b[r, k:].cpu() == n - 1 - want[-1]).all()
