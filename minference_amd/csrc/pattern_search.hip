@@ -9,13 +9,12 @@
 //   block_flags[R][C]   bit t set: candidate t keeps the 32 x 32 block (R, C)  (block-sparse)
 // and element (r, c), c <= r, belongs to candidate t iff any of its three bits t is set.
 //
-//   pattern_recall_kernel  one workgroup per (head, 64 query rows), heavy row tiles first; its 4
-//                     waves split the causal key blocks (32 keys each).  S^T = K.Q^T on
+//   pattern_recall_kernel  one workgroup per (head, 128 query rows), heavy row tiles first: 2 waves per
+//                     64 rows, which take every second causal key block (32 keys each).  S^T = K.Q^T on
 //                     v_mfma_f32_32x32x16 with fragments read straight from global memory in
-//                     operand layout: lane <-> query row, registers <-> keys, so the running
-//                     maximum, the running sum of exponentials and the 8 running masked sums are
-//                     per-lane registers (online softmax, rescaled whenever the maximum grows).
-//                     Lanes, then waves, are merged through LDS; the row tile's sum of
+//                     operand layout: lane <-> query row, registers <-> keys; online softmax with a
+//                     running maximum per row.  The row sum and the masked sums are matrix products
+//                     too (see the kernel).  Waves are merged through LDS; a 64-row tile's sum of
 //                     masked/total ratios over its rows >= row_begin goes to a partial buffer.
 //   pattern_recall_finalize  sums the partials of a head in a fixed order and divides by the
 //                     number of rows (deterministic; no atomics).
@@ -27,12 +26,13 @@ namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
+typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4_t;
 
 constexpr int HD = 128;
 constexpr int NC = 8;            // candidates per sweep (bits of a flag byte)
-constexpr int TILE = 64;         // query rows per workgroup
+constexpr int TILE = 64;         // query rows per wave pair (two tiles per workgroup)
 constexpr int KB = 32;           // keys per block
 
 union Frag {
@@ -52,12 +52,14 @@ template <> __device__ __forceinline__ f32x16_t mma<_Float16>(const Frag &a, con
 struct RecallParams {
     const char *q, *k;
     long long qs[3], ks[3];      // element strides batch, head, token
-    int hq, hk, n;
+    int batch, hq, hk, n;
     float scale_log2;
     const unsigned char *col, *diag, *blk;   // blk may be null
     long long flag_pitch;        // bytes between heads of col / diag (>= n rounded up to 64)
     long long blk_pitch;         // bytes between block rows; a head has ceil(n/32) block rows
     int row_begin, tiles;
+    int stripes;                 // the row tiles of a kv group are dealt to this many XCD ranges
+    unsigned total_wg;
     float *partial;              // [batch*hq, tiles, NC]
 };
 
@@ -77,6 +79,24 @@ __device__ __forceinline__ unsigned load_u32_unaligned(const unsigned char *p) {
     return w;
 }
 
+// (see copy16_to_lds in attn_fwd.hip: assembly keeps the LDS read counter in order)
+__device__ __forceinline__ void copy16_to_lds(const char *src, char *dst) {
+    const int lds = (int)(unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)dst;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
+}
+
+// x - (float)h.lo / x - (float)h.hi in one instruction each
+__device__ __forceinline__ float sub_lo(float x, unsigned h) {
+    float r;
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    return r;
+}
+__device__ __forceinline__ float sub_hi(float x, unsigned h) {
+    float r;
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
+    return r;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 struct RowState {
@@ -93,138 +113,295 @@ __device__ __forceinline__ void merge_into(RowState &a, float m, float z, const 
     a.m = mn;
 }
 
+// What all 63 diagonals of a 32 x 32 block have in common, per candidate: the block at distance d (in
+// blocks) from the diagonal holds the offsets 32 d - 31 .. 32 d + 31.  Per aligned group of 32 offsets the
+// table holds the OR and the AND of its flag bytes, and the same without the group's first offset.
+constexpr int DIAG_GROUPS = 8192;            // (262144 tokens; farther blocks are treated as mixed)
+
+// The masked sums as matrix products.  Per 32-key block and row,  Z_t += sum_c mask_t(c) e(c)  with e the
+// block's exponentials in B-operand layout straight from the S^T accumulators and the masks as the A
+// operand: row t of A is candidate t (t < 8), row 8 is all ones (the row sum itself).  That covers the
+// columns, and -- by setting a candidate's whole row -- the blocks and those blocks all of whose diagonals
+// a candidate keeps (most of a window, of a run of slashes).  Only candidates with SOME of a block's
+// diagonals are added element by element (their columns left out: those are in the product already).  The
+// exponentials enter as a sum of two f16 terms (22 bits; the row's largest is scaled to 2^7 .. 2^13, so that
+// what f16 cannot hold lies 2^-31 below it), the sums are fp32.
+// Bound by its vector instructions (70 % of the issue slots): about 115 per 32 x 32 block (fma and exp 32,
+// conversions 32, maximum 14, masks) and 40 per candidate with mixed diagonals, beside 12 MFMAs, where
+// testing a bit per element and candidate took about 550.  32 / 8 heads, 16384 tokens, the six candidates of
+// the reference: 6.50 ms -> 3.05 (products) -> 2.70 (K shared through LDS instead of fragments from global
+// memory) -> 2.45 (mixed-precision subtraction, scalar descriptors) -> 2.34 ms (dot products for mixed
+// diagonals); the score products alone take 0.44 ms at the nominal rate.
 template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_kernel(const RecallParams p) {
+    __shared__ unsigned dtab[DIAG_GROUPS];             // bytes: OR, AND, OR without the first, AND without the first
     __shared__ float lds[4][TILE][NC + 2];
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // two steps of two 32-key blocks each (one per key parity), 256-byte rows whose 16-byte chunks are
+    // XOR-permuted (chunk ^ row % 16) so that the fragment reads of 32 rows hit distinct banks
+    __shared__ __attribute__((aligned(16))) char kt[2][2 * KB * HD * 2];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
-    const int head_lin = (int)blockIdx.y;                          // batch*hq + h
-    const int rt = p.tiles - 1 - (int)blockIdx.x;                  // heavy (late) row tiles first
-    const int b = head_lin / p.hq, h = head_lin % p.hq;
-    const int hkv = h / (p.hq / p.hk);
+    // XCD-aware order: every XCD works through one contiguous eighth of (batch, kv head, stripe, row tile,
+    // query head in the group), so that the tiles and heads that read one kv head share an L2
+    const unsigned per_xcd = p.total_wg >> 3;
+    unsigned rest = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+    const int group = p.hq / p.hk, tps = (p.tiles + 1) / 2, per_stripe = (tps + p.stripes - 1) / p.stripes;
+    const int hin = (int)(rest % (unsigned)group); rest /= (unsigned)group;
+    const int in_stripe = (int)(rest % (unsigned)per_stripe); rest /= (unsigned)per_stripe;
+    const int ti = in_stripe * p.stripes + (int)(rest % (unsigned)p.stripes); rest /= (unsigned)p.stripes;
+    if (ti >= tps || rest >= (unsigned)(p.batch * p.hk)) return;   // padding
+    const int tp = tps - 1 - ti;                                   // heavy (late) row tiles first
+    const int hkv = (int)(rest % (unsigned)p.hk), b = (int)(rest / (unsigned)p.hk), h = hkv * group + hin;
+    const int head_lin = b * p.hq + h;
+    const int half = wave & 1, kpar = wave >> 1;
+    const int rt = 2 * tp + half;                                  // this wave's 64-row tile
     const char *qb = p.q + ((long long)b * p.qs[0] + (long long)h * p.qs[1]) * 2;
     const char *kbase = p.k + ((long long)b * p.ks[0] + (long long)hkv * p.ks[1]) * 2;
     const unsigned char *col = p.col + (long long)head_lin * p.flag_pitch;
     const unsigned char *diag = p.diag + (long long)head_lin * p.flag_pitch;
     const int brows = (p.n + KB - 1) / KB;
     const unsigned char *blk = p.blk ? p.blk + (long long)head_lin * brows * p.blk_pitch : nullptr;
+    float *const out = p.partial + ((long long)head_lin * p.tiles + rt) * NC;
+    if ((tp + 1) * 2 * TILE <= p.row_begin) {                      // no row of the tiles counts
+        if (kpar == 0 && rt < p.tiles && lane < NC) out[lane] = 0.f;
+        return;
+    }
+
+    const int groups = min(min(4 * tp + 4, brows), DIAG_GROUPS);
+    for (int i = tid; i < groups; i += 256) {
+        const unsigned *w = reinterpret_cast<const unsigned *>(diag + 32ll * i);
+        unsigned o = 0u, an = 0xffffffffu, w0 = w[0];
+#pragma unroll
+        for (int j = 1; j < 8; ++j) { const unsigned x = w[j]; o |= x; an &= x; }
+        auto fold_or = [](unsigned x) { x |= x >> 16; return (x | (x >> 8)) & 0xffu; };
+        auto fold_and = [](unsigned x) { x &= x >> 16; return (x & (x >> 8)) & 0xffu; };
+        dtab[i] = fold_or(o | w0) | (fold_and(an & w0) << 8) | (fold_or(o | (w0 & ~0xffu)) << 16) | (fold_and(an & (w0 | 0xffu)) << 24);
+    }
+    __syncthreads();
 
     Frag qf[2][8];
     load_frag(qb, p.qs[2], rt * TILE, p.n, lane, qf[0]);
     load_frag(qb, p.qs[2], rt * TILE + 32, p.n, lane, qf[1]);
 
-    RowState st[2];
+    constexpr float BIAS = 7.f, LAZY = 6.f;            // exponentials reach 2^BIAS .. 2^(BIAS + LAZY) < 2^16
+    float m[2] = {-INFINITY, -INFINITY};               // running maximum of the lane's row (same in both lane halves)
+    f32x16_t zacc[2];                                  // rows t = 8 (r / 4) + 4 g + r % 4: r 0..3 candidates 4 g + r, r 4 (g 0) the sum
+    float zx[2][NC];                                   // this lane's share of the element-wise sums
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
-        st[nb].m = -INFINITY;
-        st[nb].z = 0.f;
 #pragma unroll
-        for (int t = 0; t < NC; ++t) st[nb].zm[t] = 0.f;
+        for (int r = 0; r < 16; ++r) zacc[nb][r] = 0.f;
+#pragma unroll
+        for (int t = 0; t < NC; ++t) zx[nb][t] = 0.f;
     }
+    // A operand: lane l holds row t = l % 32, contraction index 8 g + e <-> key 16 s + 8 (e / 4) + 4 g + e % 4
+    const unsigned a_and = l32 < NC ? 0x01010101u : 0u, a_or = l32 == NC ? 0x01010101u : 0u;
+    const int a_shift = l32 & 7;
 
-    const int last_kb = min(2 * rt + 1, brows - 1);               // last key block any row of the tile sees
-    Frag kf[8], kn[8];
-    if (wave <= last_kb) load_frag(kbase, p.ks[2], wave * KB, p.n, lane, kn);
-    for (int kb = wave; kb <= last_kb; kb += 4) {
-        const int n0 = kb * KB;
+    const bool counts = rt < p.tiles && (rt + 1) * TILE > p.row_begin;
+    const int last_kb = counts ? min(2 * rt + 1, brows - 1) : -1;  // last key block any row of the tile sees
+    const int last_any = min(4 * tp + 3, brows - 1);               // ... and any row of the workgroup
+    // the 64 keys of a step, copied by the four waves together (16 rows each, 4 per instruction; rows past
+    // the sequence read a valid row instead: no row of a head sees those keys)
+    const int cp_r = lane >> 4, cp_c = lane & 15;
+    const int row_bytes = (int)p.ks[2] * 2;
+    int cp_off[4];
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) kf[ks] = kn[ks];
-        if (kb + 4 <= last_kb) load_frag(kbase, p.ks[2], (kb + 4) * KB, p.n, lane, kn);
+    for (int j = 0; j < 4; ++j) cp_off[j] = cp_r * row_bytes + ((cp_c ^ (4 * j + cp_r)) << 4);
+    auto copy_k = [&](int kb0, int buf) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the builtins do not exist in the host pass)
+        if ((kb0 + 2) * KB <= p.n && p.ks[2] <= (1 << 22)) {       // (the copies' offsets are 32-bit)
+            const __amdgpu_buffer_rsrc_t srd = __builtin_amdgcn_make_buffer_rsrc((void *)(kbase + (long long)kb0 * KB * row_bytes), 0, 2 * KB * row_bytes, 0x00020000);
+            const int lds0 = (int)(unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)kt[buf] + 16 * wave * HD * 2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(srd, (__attribute__((address_space(3))) void *)(unsigned long long)(unsigned)(lds0 + 4 * j * HD * 2),
+                                                         16, cp_off[j], (16 * wave + 4 * j) * row_bytes, 0, 0);
+            return;
+        }
+#endif
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = 16 * wave + 4 * j + cp_r;
+            const char *src = kbase + (long long)min(kb0 * KB + r, p.n - 1) * p.ks[2] * 2 + ((cp_c ^ (r & 15)) << 4);
+            copy16_to_lds(src, kt[buf] + (16 * wave + 4 * j) * HD * 2);
+        }
+    };
+    // flags of this wave's key block: column words of the lane's 16 keys (keys n0 + 8j + 4g + i, one aligned
+    // word per j) and the block bytes of its two row blocks; fetched a step ahead
+    unsigned cw[4], bb[2] = {0u, 0u}, cw_next[4], bb_next[2] = {0u, 0u};
+    auto fetch_flags = [&](int kb, unsigned (&c)[4], unsigned (&bk)[2]) {
+        const int at = min(kb, brows - 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c[j] = *reinterpret_cast<const unsigned *>(col + at * KB + 8 * j + 4 * g);
+        if (blk)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) bk[nb] = blk[(long long)min(2 * rt + nb, brows - 1) * p.blk_pitch + at];
+    };
+    copy_k(0, 0);
+    fetch_flags(kpar, cw_next, bb_next);
+    for (int kb0 = 0; kb0 <= last_any; kb0 += 2) {
+        const int buf = (kb0 >> 1) & 1, kb = kb0 + kpar, n0 = kb * KB;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) cw[j] = cw_next[j];
+        bb[0] = bb_next[0]; bb[1] = bb_next[1];
+        __builtin_amdgcn_s_waitcnt(0x0f70);            // vmcnt(0): this wave's share of the step is in LDS
+        __syncthreads();                               // ... and everybody's; everyone is done with the step before
+        if (kb0 + 2 <= last_any) {
+            copy_k(kb0 + 2, buf ^ 1);
+            fetch_flags(kb + 2, cw_next, bb_next);
+        }
+        if (kb > last_kb) continue;                    // (wave-uniform; no barrier below)
+        unsigned full[2], mixed[2];                    // candidates that keep all / some of a block, by its row block
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            const int rb = min(2 * rt + nb, brows - 1), d = max(rb - kb, 0);
+            const unsigned here = __builtin_amdgcn_readfirstlane(dtab[min(d, DIAG_GROUPS - 1)]);
+            unsigned before = __builtin_amdgcn_readfirstlane(dtab[min(max(d - 1, 0), DIAG_GROUPS - 1)]) >> 16;
+            if (d == 0) before = 0xff00u;              // (nothing before the main diagonal)
+            unsigned any = (here | before) & 0xffu, all = (here & before) >> 8;
+            if (d >= DIAG_GROUPS) { any = 0xffu; all = 0u; }
+            full[nb] = __builtin_amdgcn_readfirstlane(bb[nb]) | (all & 0xffu);
+            mixed[nb] = any & ~full[nb];
+        }
+        f32x16_t acc[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { acc[0][r] = 0.f; acc[1][r] = 0.f; }
+        const char *krow = kt[buf] + (kpar * KB + l32) * HD * 2;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            Frag kf;
+            kf.u = *reinterpret_cast<const u32x4_t *>(krow + (((2 * ks + g) ^ (l32 & 15)) << 4));
+            acc[0] = mma<T>(kf, qf[0][ks], acc[0]);
+            acc[1] = mma<T>(kf, qf[1][ks], acc[1]);
+        }
 
-        // column flags of the lane's 16 keys: keys n0 + 8j + 4g + i, one aligned word per j
-        unsigned cw[4];
+        Frag am[2];                                    // the columns' masks, shared by both row blocks
 #pragma unroll
-        for (int j = 0; j < 4; ++j) cw[j] = *reinterpret_cast<const unsigned *>(col + n0 + 8 * j + 4 * g);
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj) {
+                const unsigned x = ((cw[2 * s + jj] >> a_shift) & a_and) | a_or;
+                am[s].u[2 * jj] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c010c00u), 0x3c00u);
+                am[s].u[2 * jj + 1] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c030c02u), 0x3c00u);
+            }
 
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
             const int rb = 2 * rt + nb;                            // 32-row block of this half
             if (kb > rb) continue;                                 // wholly above the diagonal
-            f32x16_t acc;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-#pragma unroll
-            for (int ks = 0; ks < 8; ++ks) acc = mma<T>(kf[ks], qf[nb][ks], acc);
-
             const int row = rb * 32 + l32;
-            const unsigned bb = blk ? (unsigned)blk[(long long)min(rb, brows - 1) * p.blk_pitch + kb] : 0u;
-            // diagonal flags: key i of group j has offset o0 - i, o0 = row - (n0 + 8j + 4g); the word
-            // read at o0-3 holds it in byte 3-i.  Near the diagonal o0-3 may be negative: read at
-            // 0 and shift the bytes up (offsets < 0 are above the diagonal and masked anyway).
-            unsigned dw[4];
+            if (kb == rb) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int o0 = row - (n0 + 8 * j + 4 * g);
-                const int base = min(max(o0 - 3, 0), (int)p.flag_pitch - 4);
-                unsigned w = load_u32_unaligned(diag + base);
-                const int up = base - (o0 - 3);                    // > 0 only when o0 < 3
-                w = up >= 4 ? 0u : (w << (8 * max(up, 0)));
-                dw[j] = w;
+                for (int r = 0; r < 16; ++r)
+                    if (n0 + 8 * (r >> 2) + 4 * g + (r & 3) > row) acc[nb][r] = -INFINITY;
             }
-            const bool on_diag = kb == rb;
-            float s[16];
-            float mx = -INFINITY;
+            float mx = fmaxf(fmaxf(acc[nb][0], acc[nb][1]), acc[nb][2]);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int key = n0 + 8 * (r >> 2) + 4 * g + (r & 3);
-                float x = acc[r] * p.scale_log2;
-                if (on_diag && key > row) x = -INFINITY;
-                s[r] = x;
-                mx = fmaxf(mx, x);
+            for (int r = 3; r + 1 < 16; r += 2) mx = fmaxf(fmaxf(mx, acc[nb][r]), acc[nb][r + 1]);
+            mx = fmaxf(mx, acc[nb][15]);
+            { const unsigned u = __float_as_uint(mx); auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false); mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])); }
+            const float cand = mx * p.scale_log2;
+            const bool grow = cand > m[nb] + LAZY;                 // (raised only when it has to be)
+            if (__any(grow)) {
+                const float alpha = grow ? fast_exp2(m[nb] - cand) : 1.0f;
+                m[nb] = grow ? cand : m[nb];
+#pragma unroll
+                for (int r = 0; r < 5; ++r) zacc[nb][r] *= alpha;
+#pragma unroll
+                for (int t = 0; t < NC; ++t) zx[nb][t] *= alpha;
             }
-            const float mn = fmaxf(st[nb].m, mx);
-            const float mu = mn == -INFINITY ? 0.f : mn;
-            const float alpha = fast_exp2(st[nb].m - mu);
-            float z = st[nb].z * alpha;
-            float zm[NC];
+            float e[16];
+            const float off = BIAS - m[nb];
 #pragma unroll
-            for (int t = 0; t < NC; ++t) zm[t] = st[nb].zm[t] * alpha;
+            for (int r = 0; r < 16; ++r) e[r] = fast_exp2(fmaf(acc[nb][r], p.scale_log2, off));
+            Frag a0 = am[0], a1 = am[1];
+            if (full[nb]) {                                            // candidates that keep the whole block
+                const bool mine = (full[nb] >> a_shift) & a_and & 1u;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int j = r >> 2, i = r & 3;
-                const float e = fast_exp2(s[r] - mu);
-                const unsigned bits = (cw[j] >> (8 * i)) | (dw[j] >> (8 * (3 - i))) | bb;
-                z += e;
-#pragma unroll
-                for (int t = 0; t < NC; ++t) zm[t] += (bits >> t) & 1u ? e : 0.f;
+                for (int i = 0; i < 4; ++i) {
+                    a0.u[i] = mine ? 0x3c003c00u : a0.u[i];
+                    a1.u[i] = mine ? 0x3c003c00u : a1.u[i];
+                }
             }
-            st[nb].m = mn;
-            st[nb].z = z;
+            Frag hi[2], lo[2];
 #pragma unroll
-            for (int t = 0; t < NC; ++t) st[nb].zm[t] = zm[t];
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x = e[8 * s + 2 * i], y = e[8 * s + 2 * i + 1];
+                    hi[s].u[i] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(x, y));
+                    lo[s].u[i] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(sub_lo(x, hi[s].u[i]), sub_hi(y, hi[s].u[i])));
+                }
+                zacc[nb] = mma<_Float16>(s ? a1 : a0, hi[s], zacc[nb]);
+                zacc[nb] = mma<_Float16>(s ? a1 : a0, lo[s], zacc[nb]);
+            }
+            if (mixed[nb]) {
+                // diagonal flags: key i of group j has offset o0 - i, o0 = row - (n0 + 8j + 4g); the word
+                // read at o0-3 holds it in byte 3-i
+                unsigned pm[4];
+                const int first = row - n0 - 4 * g - 3;
+                if (kb != rb) {                                    // every offset is positive
+                    const unsigned char *dp = diag + first;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) pm[j] = __builtin_bswap32(load_u32_unaligned(dp - 8 * j)) & ~cw[j];
+                } else {
+                    // on the main diagonal o0-3 may be negative: read at 0 and shift the bytes up (offsets < 0
+                    // are above the diagonal, their exponentials are 0 anyway)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int at = first - 8 * j, base = max(at, 0), up = base - at;
+                        const unsigned w = load_u32_unaligned(diag + base);
+                        pm[j] = __builtin_bswap32(up >= 4 ? 0u : (w << (8 * up))) & ~cw[j];
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < NC; ++t)
+                    if ((mixed[nb] >> t) & 1u) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const unsigned x = (pm[j] >> t) & 0x01010101u;
+                            const f16x2_t k0 = __builtin_bit_cast(f16x2_t, __umul24(__builtin_amdgcn_perm(0u, x, 0x0c010c00u), 0x3c00u));
+                            const f16x2_t k1 = __builtin_bit_cast(f16x2_t, __umul24(__builtin_amdgcn_perm(0u, x, 0x0c030c02u), 0x3c00u));
+                            const unsigned h0 = hi[j >> 1].u[2 * (j & 1)], h1 = hi[j >> 1].u[2 * (j & 1) + 1];
+                            const unsigned l0 = lo[j >> 1].u[2 * (j & 1)], l1 = lo[j >> 1].u[2 * (j & 1) + 1];
+                            float z = zx[nb][t];
+                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, h0), k0, z, false);
+                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, l0), k0, z, false);
+                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, h1), k1, z, false);
+                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, l1), k1, z, false);
+                            zx[nb][t] = z;
+                        }
+                    }
+            }
         }
     }
 
-    // merge the two lanes of a row (keys 4g + ...), then the four waves
+    // merge the two lanes of a row and the element-wise sums, then the two waves
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
-        const float om = __shfl_xor(st[nb].m, 32);
-        const float oz = __shfl_xor(st[nb].z, 32);
-        float ozm[NC];
-#pragma unroll
-        for (int t = 0; t < NC; ++t) ozm[t] = __shfl_xor(st[nb].zm[t], 32);
-        merge_into(st[nb], om, oz, ozm);
+        float *dst = lds[wave][nb * 32 + l32];
         if (g == 0) {
-            float *dst = lds[wave][nb * 32 + l32];
-            dst[0] = st[nb].m;
-            dst[1] = st[nb].z;
-#pragma unroll
-            for (int t = 0; t < NC; ++t) dst[2 + t] = st[nb].zm[t];
+            dst[0] = m[nb];
+            dst[1] = zacc[nb][4];
         }
+        float own[NC];
+#pragma unroll
+        for (int t = 0; t < NC; ++t) own[t] = zx[nb][t] + __shfl_xor(zx[nb][t], 32);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dst[2 + 4 * g + r] = zacc[nb][r] + (g ? own[4 + r] : own[r]);
     }
     __syncthreads();
-    if (wave == 0) {
+    if (kpar == 0 && rt < p.tiles) {
         RowState a;
-        a.m = lds[0][lane][0];
-        a.z = lds[0][lane][1];
+        a.m = lds[wave][lane][0];
+        a.z = lds[wave][lane][1];
 #pragma unroll
-        for (int t = 0; t < NC; ++t) a.zm[t] = lds[0][lane][2 + t];
+        for (int t = 0; t < NC; ++t) a.zm[t] = lds[wave][lane][2 + t];
+        float zm[NC];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) {
-            float zm[NC];
-#pragma unroll
-            for (int t = 0; t < NC; ++t) zm[t] = lds[w][lane][2 + t];
-            merge_into(a, lds[w][lane][0], lds[w][lane][1], zm);
-        }
+        for (int t = 0; t < NC; ++t) zm[t] = lds[wave + 2][lane][2 + t];
+        merge_into(a, lds[wave + 2][lane][0], lds[wave + 2][lane][1], zm);
         const int row = rt * TILE + lane;
         const bool counted = row < p.n && row >= p.row_begin && a.z > 0.f;
         const float inv = counted ? 1.0f / a.z : 0.f;
@@ -233,7 +410,7 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
             float x = a.zm[t] * inv;
 #pragma unroll
             for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d);     // fixed butterfly order
-            if (lane == 0) p.partial[((long long)head_lin * p.tiles + rt) * NC + t] = x;
+            if (lane == 0) out[t] = x;
         }
     }
 }
@@ -302,7 +479,6 @@ extern "C" int minf_pattern_recall(const void *q, const void *k, const int64_t *
     if (((uintptr_t)col_flags | (uintptr_t)diag_flags) & 3) return MINF_ERR_ALIGNMENT;
     if (block_flags && block_pitch < (n + KB - 1) / KB) return MINF_ERR_INVALID_ARG;
     if (batch == 0) return MINF_OK;
-    if ((long long)batch * heads_q > 65535) return MINF_ERR_UNSUPPORTED;
     const size_t need = minf_pattern_recall_workspace_bytes(batch, heads_q, n);
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 3)) return MINF_ERR_WORKSPACE;
 
@@ -313,6 +489,7 @@ extern "C" int minf_pattern_recall(const void *q, const void *k, const int64_t *
         p.qs[i] = q_stride[i];
         p.ks[i] = k_stride[i];
     }
+    p.batch = batch;
     p.hq = heads_q;
     p.hk = heads_kv;
     p.n = n;
@@ -326,7 +503,14 @@ extern "C" int minf_pattern_recall(const void *q, const void *k, const int64_t *
     p.tiles = tiles;
     p.partial = (float *)workspace;
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid(tiles, batch * heads_q);
+    const long long groups = (long long)batch * heads_kv;
+    p.stripes = 1;
+    while (p.stripes < 8 && groups * p.stripes % 8) p.stripes *= 2;
+    const long long per_stripe = ((tiles + 1) / 2 + p.stripes - 1) / p.stripes;
+    const long long wgs = (groups * p.stripes * per_stripe * (heads_q / heads_kv) + 7) / 8 * 8;
+    if (wgs > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
+    p.total_wg = (unsigned)wgs;
+    const dim3 grid((unsigned)wgs);
     if (dtype == MINF_BF16)
         hipLaunchKernelGGL(pattern_recall_kernel<__bf16>, grid, dim3(256), 0, st, p);
     else

@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .estimate import _prep16, topk_indices, vertical_slash_scores
+from .estimate import _prep16, topk_vertical_slash, vertical_slash_scores
 from .ops import _check_qkv
 
 ROW_BEGIN = 2500                  # minference_forward.py:161: attn_weights_x[:, :, 2500:]
@@ -71,6 +71,8 @@ def pattern_recall(q, k, candidates=CANDIDATES, row_begin=ROW_BEGIN):
     _check_qkv(q, k, k)
     head_dim = q.shape[-1]
     q16, k16 = _prep16(q, k)
+    if q16.shape[-1] < 128:                            # the sweep is built for 128 dims: zero columns add nothing
+        q16, k16 = (torch.nn.functional.pad(t, [0, 128 - t.shape[-1]]) for t in (q16, k16))
     B, H, N, _ = q16.shape
     Hk = k16.shape[1]
     dev = q16.device
@@ -94,8 +96,7 @@ def pattern_recall(q, k, candidates=CANDIDATES, row_begin=ROW_BEGIN):
             elif ty == "vertical_and_slash":
                 if scores is None:
                     scores = vertical_slash_scores(q, k, 64, SEARCH_FORCE, SEARCH_FORCE, reference_rounding=False)
-                v_idx = topk_indices(scores[0], min(a, N))
-                s_idx = topk_indices(scores[1], min(b, N), reverse_base=N - 1)
+                v_idx, s_idx = topk_vertical_slash(scores[0], scores[1], a, b)
                 for idx, flags in ((v_idx, col), (s_idx, diag)):
                     kk = idx.shape[-1]
                     _lib.check(lib.minf_flags_set_indices(idx.data_ptr(), B * H, kk, kk, bit, flags.data_ptr(),

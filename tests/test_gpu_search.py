@@ -153,3 +153,21 @@ def test_search_mode_of_the_dispatcher_writes_the_pattern_file(gpu, tmp_path):
         minference_prefill_forward(qg, kg, vg, {"layer_idx": 0, "num_hidden_layers": 2, "attn_forward_config": cfg})
     sparse = minference_prefill_forward(qg, kg, vg, {"layer_idx": 1, "attn_forward_config": {"best_pattern": table}})
     assert sparse.shape == dense.shape and torch.isfinite(sparse.float()).all()
+
+
+@pytest.mark.parametrize("n,hq,hk,begin", [(33, 1, 1, 0), (128, 3, 1, 0), (129, 2, 2, 128), (1000, 2, 1, 64), (700, 2, 1, 690)])
+@pytest.mark.parametrize("d", [128, 64])
+def test_recall_tiles_stripes_and_flag_mixes(gpu, n, hq, hk, begin, d):
+    """Edges of the 128-row workgroups, counted rows that start inside a tile, head counts that do not divide
+    among the XCDs, head_dim 64 (padded), and candidates that share bits in one flag byte: windows that fill
+    whole blocks, single diagonals, every second column, all eight candidates in use.  Flags are set through
+    the public candidate list; the oracle multiplies N x N masks."""
+    from minference_amd import pattern_recall
+    q, k, _ = gen.qkv(1, hq, hk, n, d, 7 + n, dtype=torch.float32, scale=1.0)
+    q, k = q.bfloat16(), k.bfloat16()
+    cands = [("stream_llm", 4, 70), ("stream_llm", n // 2, 3), ("vertical_and_slash", 40, 60), ("vertical_and_slash", 31, 100),
+             ("vertical_and_slash", 200, 51), ("block_sparse", 2, 1), ("block_sparse", 3, 1), ("stream_llm", 1, n)]
+    got = pattern_recall(q.to(gpu), k.to(gpu), cands, begin)[0].cpu().numpy()
+    want = np.array(oracle_scores(q, k, cands, begin))
+    assert np.abs(got - want).max() <= TOL, (got, want)
+    assert np.abs(got[:, 7] - 1.0).max() <= 1e-6             # a window of all offsets keeps everything
