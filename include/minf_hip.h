@@ -36,6 +36,7 @@ extern "C" {
 
 #define MINF_BF16 0
 #define MINF_F16 1
+#define MINF_F32 2                  /* the decoder-layer passes at the end of this header only */
 
 /* Rounding of the two index selectors (pattern estimation, block index).  MINF_ROUND_NONE: fp32
  * arithmetic on the 16-bit inputs.  MINF_ROUND_INPUT_DTYPE: round every intermediate that the
@@ -426,6 +427,25 @@ int minf_search_block_index(const void *q, const void *k, const int64_t *q_strid
                             const int64_t *k_stride, int batch, int heads_q, int heads_kv, int n,
                             int head_dim, int dtype, int top_k, int32_t *block_index,
                             void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * The element-wise passes of a decoder layer around the attention path (reference
+ * minference/patch.py:500-558, :688-693, as chains of torch ops); dtype MINF_BF16, MINF_F16 or
+ * MINF_F32, contiguous tensors (minf_rope, minf_silu_mul: 16-byte aligned).  Values are rounded to
+ * dtype where those chains round.
+ *
+ * minf_rms_norm: x [rows, dim] (+ delta, if not NULL: the sum is written back to x); out [rows, dim] =
+ *   round(x * rsqrt(mean(x^2) + eps)) * weight.
+ * minf_rope: q [tokens, heads_q, head_dim] and k [tokens, heads_kv, head_dim] in place; pairs
+ *   (i, i + head_dim/2) are rotated by the angles whose cosines / sines are row `token` of the fp32
+ *   tables [tokens, head_dim/2].
+ * minf_silu_mul: gate[i] = round(silu(gate[i])) * up[i] for i < n.
+ */
+int minf_rms_norm(void *x, const void *delta, const void *weight, void *out, int64_t rows, int dim,
+                  float eps, int dtype, void *stream);
+int minf_rope(void *q, void *k, const float *cos_table, const float *sin_table, int64_t tokens,
+              int heads_q, int heads_kv, int head_dim, int dtype, void *stream);
+int minf_silu_mul(void *gate, const void *up, int64_t n, int dtype, void *stream);
 
 #ifdef __cplusplus
 }

@@ -6,11 +6,12 @@ minference/modules/forward.py:22-234 attention forward that hands [B,H,N,D] q/k/
 ``prefill_forwards["minference"]``) as a self-contained block stack instead of a monkey patch of
 a particular transformers version.  Linear layers are plain library GEMMs (torch matmul ->
 hipBLASLt); everything between the q/k/v projections and o_proj is
-``minference_prefill_forward``.  K/V keep their own (fewer) heads: no repeat_kv copy.
+``minference_prefill_forward``; norms (with the residual add before them), rotary embedding and
+SiLU * up are one kernel each (csrc/decoder.hip).  K/V keep their own (fewer) heads: no repeat_kv copy.
 
-Memory layout for 262144 tokens of Llama-3-8B on one 288 GB GPU: weights 16 GB, hidden state
-2 GiB, q 2 GiB, k/v 0.5 GiB each per layer; norms, projections, RoPE and the MLP are applied over
-token chunks so no intermediate is larger than ``chunk x intermediate_size``.
+Memory layout for 262144 tokens of Llama-3-8B on one 288 GB GPU: weights 16 GB, hidden state and its
+norm 2 GiB each, q and the attention output 2 GiB each, k/v 0.5 GiB each per layer; projections and
+the MLP are applied over token chunks so no intermediate is larger than ``chunk x intermediate_size``.
 """
 from __future__ import annotations
 
@@ -18,6 +19,7 @@ from dataclasses import dataclass
 
 import torch
 
+from . import _lib
 from .prefill import minference_prefill_forward
 
 
@@ -41,6 +43,7 @@ class LlamaPrefill:
 
     def __init__(self, config: LlamaConfig, device="cuda", dtype=torch.bfloat16, seed=0, std=0.02):
         self.cfg, self.device, self.dtype = config, torch.device(device), dtype
+        self._dt = {torch.bfloat16: _lib.MINF_BF16, torch.float16: _lib.MINF_F16, torch.float32: _lib.MINF_F32}[dtype]
         c = config
         g = torch.Generator(device=self.device).manual_seed(seed)
 
@@ -79,23 +82,38 @@ class LlamaPrefill:
         self.lm_head = get("lm_head.weight") if "lm_head.weight" in sd else self.embed_tokens
 
     # ---- pieces ---------------------------------------------------------------------------
-    def _rms(self, x, weight):
-        xf = x.float()
-        xf = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.cfg.rms_eps)
-        return (xf.to(self.dtype)) * weight
+    def _rms(self, x, weight, delta=None, out=None):
+        """RMSNorm of the rows of x (contiguous); with ``delta`` x += delta first, in place."""
+        out = torch.empty_like(x) if out is None else out
+        lib = _lib.load()
+        with torch.cuda.device(x.device):
+            st = lib.minf_rms_norm(x.data_ptr(), delta.data_ptr() if delta is not None else None, weight.data_ptr(),
+                                   out.data_ptr(), x.shape[0], x.shape[1], self.cfg.rms_eps, self._dt, _lib.stream_ptr(x.device))
+        _lib.check(st, "minf_rms_norm")
+        return out
 
-    def _rope_tables(self, start, stop):
+    def _rope_tables(self, n):
+        """cos, sin [n, D/2] fp32 (rotate_half convention: pairs (i, i + D/2) share an angle)."""
         c = self.cfg
         inv = 1.0 / (c.rope_theta ** (torch.arange(0, c.head_dim, 2, device=self.device, dtype=torch.float32) / c.head_dim))
-        ang = torch.arange(start, stop, device=self.device, dtype=torch.float32)[:, None] * inv[None, :]
-        ang = torch.cat([ang, ang], dim=-1)              # rotate_half convention: pairs (i, i + D/2)
-        return ang.cos()[:, None, :], ang.sin()[:, None, :]
+        ang = torch.arange(n, device=self.device, dtype=torch.float32)[:, None] * inv[None, :]
+        return ang.cos(), ang.sin()
 
-    @staticmethod
-    def _rotate(x, cos, sin):
-        half = x.shape[-1] // 2
-        xr = torch.cat([-x[..., half:], x[..., :half]], dim=-1)
-        return (x.float() * cos + xr.float() * sin).to(x.dtype)
+    def _rotate(self, q, k, cos, sin):
+        """Rotary embedding of q [n, Hq, D] and k [n, Hk, D] in place."""
+        lib = _lib.load()
+        with torch.cuda.device(q.device):
+            st = lib.minf_rope(q.data_ptr(), k.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.shape[0], q.shape[1],
+                               k.shape[1], q.shape[2], self._dt, _lib.stream_ptr(q.device))
+        _lib.check(st, "minf_rope")
+
+    def _silu_mul(self, gate, up):
+        """gate <- silu(gate) * up."""
+        lib = _lib.load()
+        with torch.cuda.device(gate.device):
+            st = lib.minf_silu_mul(gate.data_ptr(), up.data_ptr(), gate.numel(), self._dt, _lib.stream_ptr(gate.device))
+        _lib.check(st, "minf_silu_mul")
+        return gate
 
     # ---- prefill --------------------------------------------------------------------------
     @torch.no_grad()
@@ -108,36 +126,38 @@ class LlamaPrefill:
         n = ids.numel()
         cfg = attn_forward_config if attn_forward_config is not None else {"best_pattern": None}
         hidden = self.embed_tokens[ids]                                    # [N, hidden]
-        q = torch.empty((n, c.num_heads, c.head_dim), device=self.device, dtype=self.dtype)
+        cos, sin = self._rope_tables(n)
+        new = lambda *shape: torch.empty(shape, device=self.device, dtype=self.dtype)
+        q, attn = new(n, c.num_heads, c.head_dim), new(n, c.num_heads, c.head_dim)
+        # the norm that comes next is taken together with the residual add before it: `normed` holds the
+        # input of the next projections
+        normed = self._rms(hidden, self.layers[0]["input_layernorm"]) if self.layers else None
         kv_cache = [] if keep_kv else None
         k = v = None
         for li, L in enumerate(self.layers):
             if k is None or keep_kv:
-                k = torch.empty((n, c.num_kv_heads, c.head_dim), device=self.device, dtype=self.dtype)
-                v = torch.empty((n, c.num_kv_heads, c.head_dim), device=self.device, dtype=self.dtype)
+                k, v = new(n, c.num_kv_heads, c.head_dim), new(n, c.num_kv_heads, c.head_dim)
             for s in range(0, n, chunk):
                 e = min(s + chunk, n)
-                x = self._rms(hidden[s:e], L["input_layernorm"])
-                cos, sin = self._rope_tables(s, e)
-                q[s:e] = self._rotate((x @ L["q_proj"].T).view(e - s, c.num_heads, c.head_dim), cos, sin)
-                k[s:e] = self._rotate((x @ L["k_proj"].T).view(e - s, c.num_kv_heads, c.head_dim), cos, sin)
-                v[s:e] = (x @ L["v_proj"].T).view(e - s, c.num_kv_heads, c.head_dim)
+                for dst, w in ((q, "q_proj"), (k, "k_proj"), (v, "v_proj")):
+                    torch.mm(normed[s:e], L[w].T, out=dst[s:e].view(e - s, -1))
+            self._rotate(q, k, cos, sin)
             # [N, H, D] storage viewed as [1, H, N, D]: the kernels take strides, nothing is copied
-            attn = minference_prefill_forward(q.permute(1, 0, 2)[None], k.permute(1, 0, 2)[None],
-                                              v.permute(1, 0, 2)[None],
-                                              {"layer_idx": li, "attn_forward_config": cfg})
-            attn = attn[0].permute(1, 0, 2)                                 # [N, H, D] view
+            minference_prefill_forward(q.permute(1, 0, 2)[None], k.permute(1, 0, 2)[None], v.permute(1, 0, 2)[None],
+                                       {"layer_idx": li, "attn_forward_config": cfg, "out": attn.permute(1, 0, 2)[None]})
+            nxt = self.layers[li + 1]["input_layernorm"] if li + 1 < len(self.layers) else None
             for s in range(0, n, chunk):
                 e = min(s + chunk, n)
-                a = attn[s:e].reshape(e - s, c.num_heads * c.head_dim)
-                h = hidden[s:e] + a @ L["o_proj"].T
-                x = self._rms(h, L["post_attention_layernorm"])
-                mlp = (torch.nn.functional.silu(x @ L["gate_proj"].T) * (x @ L["up_proj"].T)) @ L["down_proj"].T
-                hidden[s:e] = h + mlp
-            del attn
+                o = attn[s:e].view(e - s, -1) @ L["o_proj"].T
+                x = self._rms(hidden[s:e], L["post_attention_layernorm"], delta=o, out=normed[s:e])
+                mlp = self._silu_mul(x @ L["gate_proj"].T, x @ L["up_proj"].T) @ L["down_proj"].T
+                if nxt is not None:
+                    self._rms(hidden[s:e], nxt, delta=mlp, out=normed[s:e])
+                else:
+                    hidden[s:e] += mlp
             if keep_kv:
                 kv_cache.append((k, v))
-        last = self._rms(hidden[-1:], self.norm)
+        last = self._rms(hidden[-1:].clone(), self.norm)
         logits = (last @ self.lm_head.T).float()[0]
         return logits, kv_cache
 

@@ -72,7 +72,7 @@ class _Call:
     """Holds the (possibly cast/padded) tensors of one operator call and the
     filled ``minf_qkvo`` struct."""
 
-    def __init__(self, q, k, v, seqlens=None, need_out=True, native_dims=_NATIVE_D, sm_scale=None):
+    def __init__(self, q, k, v, seqlens=None, need_out=True, native_dims=_NATIVE_D, sm_scale=None, out=None):
         _check_qkv(q, k, v)
         self.out_dtype = q.dtype
         self.head_dim = q.shape[-1]
@@ -100,8 +100,15 @@ class _Call:
         self.q, self.k, self.v = _prep(q), _prep(k), _prep(v)
         B, H, N, _ = self.q.shape
         self.B, self.H, self.N, self.Hk = B, H, N, self.k.shape[1]
-        self.o = torch.empty((B, H, N, Dk) if need_out else (1, 1, 1, Dk),
-                             dtype=self.q.dtype, device=q.device)
+        # `out` (the caller's [B, H, N, D] buffer, any strides the kernels take) is written in place when
+        # it has the kernels' own shape and dtype, else copied into at the end
+        self.out = out
+        if out is not None and tuple(out.shape) == (B, H, N, Dk) and out.dtype == self.q.dtype == self.out_dtype \
+                and out.device == q.device and out.stride(2) >= Dk and _prep(out) is out:
+            self.o = out
+        else:
+            self.o = torch.empty((B, H, N, Dk) if need_out else (1, 1, 1, Dk),
+                                 dtype=self.q.dtype, device=q.device)
         s = _lib.QKVO()
         s.q, s.k, s.v, s.o = self.q.data_ptr(), self.k.data_ptr(), self.v.data_ptr(), self.o.data_ptr()
         for name, t in (("q_stride", self.q), ("k_stride", self.k), ("v_stride", self.v), ("o_stride", self.o)):
@@ -139,16 +146,18 @@ class _Call:
         o = self.o
         if self.head_dim != self.kernel_dim:
             o = o[..., : self.head_dim]
+        if self.out is not None:
+            return self.out if o is self.out else self.out.copy_(o)
         if o.dtype != self.out_dtype:
             o = o.to(self.out_dtype)
         return o
 
 
 def vertical_slash_attention_from_index(query, key, value, block_count, block_offset,
-                                        column_count, column_index, seqlens=None):
+                                        column_count, column_index, seqlens=None, out=None):
     """Mixed block + column sparse attention over prebuilt index tensors
     (counterpart of _triton_mixed_sparse_attention, pit_sparse_flash_attention_v2.py:156-192)."""
-    c = _Call(query, key, value, seqlens)
+    c = _Call(query, key, value, seqlens, out=out)
     rows = (c.N + 63) // 64
     for t in (block_count, block_offset, column_count, column_index):
         if t.dtype != torch.int32 or not t.is_contiguous():
@@ -186,10 +195,10 @@ def vertical_slash_sparse_attention(query, key, value, v_idx, s_idx, block_size_
     return vertical_slash_attention_from_index(query, key, value, bc, bo, cc, ci, seqlens)
 
 
-def block_sparse_attention_from_index(query, key, value, block_index):
+def block_sparse_attention_from_index(query, key, value, block_index, out=None):
     """Block-sparse attention over a prebuilt [batch, heads, rows, max_blocks] int32 block
     list (counterpart of _triton_block_sparse_attention, block_sparse_flash_attention.py:115-148)."""
-    c = _Call(query, key, value)
+    c = _Call(query, key, value, out=out)
     if block_index.dtype != torch.int32 or not block_index.is_contiguous() or block_index.dim() != 4:
         raise ValueError("block_index must be a contiguous int32 [batch, heads, rows, max_blocks] tensor")
     if block_index.shape[0] != c.B or block_index.shape[1] != c.H or block_index.shape[2] < (c.N + 63) // 64:
@@ -236,13 +245,14 @@ def _build_block_index(query, key, top_k, block_size_M=64, block_size_N=64, forc
     return out
 
 
-def block_sparse_attention(query, key, value, top_k: int, block_size_M: int = 64, block_size_N: int = 64):
+def block_sparse_attention(query, key, value, top_k: int, block_size_M: int = 64, block_size_N: int = 64,
+                           out=None):
     """Top-k block-sparse attention (block_sparse_flash_attention.py:169-186)."""
     if block_size_M != 64 or block_size_N != 64:
         raise ValueError("only 64x64 blocks are supported")
     _check_qkv(query, key, value)
     block_index = _build_block_index(query, key, top_k, block_size_M, block_size_N)
-    return block_sparse_attention_from_index(query, key, value, block_index)
+    return block_sparse_attention_from_index(query, key, value, block_index, out)
 
 
 def _streaming_scale(head_dim: int) -> float:
@@ -255,11 +265,11 @@ def _streaming_scale(head_dim: int) -> float:
     return float(d) ** -0.5
 
 
-def streaming_forward(q, k, v, n_init: int, n_local: int):
+def streaming_forward(q, k, v, n_init: int, n_local: int, out=None):
     """A-shape attention: n_init sink tokens + a sliding window of n_local
     (streaming_kernel.py:611-646), in one pass.  head_dim up to 256 like the reference (:429); the
     scale follows the reference's padded head_dim (see _streaming_scale)."""
-    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, sm_scale=_streaming_scale(q.shape[-1]))
+    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, sm_scale=_streaming_scale(q.shape[-1]), out=out)
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
         c.scratch(_lib.MINF_OP_ASHAPE, n_init, n_local)
@@ -284,9 +294,9 @@ def tri_shape_forward(q, k, v, n_init: int, n_local: int, n_last: int = 100):
     return c.result()
 
 
-def dense_causal_attention(q, k, v):
+def dense_causal_attention(q, k, v, out=None):
     """Dense causal attention on the same tile engine (comparator for speed-up figures)."""
-    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING)
+    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, out=out)
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
         c.scratch(_lib.MINF_OP_DENSE)

@@ -26,14 +26,14 @@ from .ops import (block_sparse_attention, dense_causal_attention, streaming_forw
 DEFAULT_PATTERN = ("vertical_and_slash", 1000, 6096, 1)   # minference_forward.py:621
 
 
-def vertical_slash_prefill(q, k, v, vertical_size=1000, slash_size=6096):
+def vertical_slash_prefill(q, k, v, vertical_size=1000, slash_size=6096, out=None):
     """estimate -> top-k -> index build -> mixed sparse attention for all heads of ``q``
     (``vertical_and_slash_kernel``, minference_forward.py:599-614)."""
     B, H, N, _ = q.shape
     v_idx, s_idx = estimate_vertical_slash(q, k, vertical_size, slash_size)
     seqlens = torch.full((B,), N, dtype=torch.int32, device=q.device)
     bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, 64, 64, zero_fill=False)
-    return vertical_slash_attention_from_index(q, k, v, bc, bo, cc, ci, seqlens)
+    return vertical_slash_attention_from_index(q, k, v, bc, bo, cc, ci, seqlens, out)
 
 
 def load_best_pattern(path):
@@ -139,7 +139,7 @@ def _head_list(heads, device):
     return torch.tensor(sorted(heads), dtype=torch.int32).to(device)
 
 
-def _mixed_layer(query_states, key_states, value_states, lp):
+def _mixed_layer(query_states, key_states, value_states, lp, out=None):
     """All heads of a layer whose pattern table mixes types and sizes (``lp``: its _LayerPlan): q/k/v
     are prepared once, the output is one shared buffer, and every pattern type is ONE launch chain
     over the original tensors with a head selection -- no gathered copies of Q, no scattered writes
@@ -158,7 +158,7 @@ def _mixed_layer(query_states, key_states, value_states, lp):
     B, H, N, D = query_states.shape
     rounded = reference_rounding_for(query_states.dtype)     # the reference's rounding points on 16-bit inputs
     dev = query_states.device
-    c = _Call(query_states, key_states, value_states)
+    c = _Call(query_states, key_states, value_states, out=out)
     lib = _lib.load()
     stream = _lib.stream_ptr(dev)
     i64x3 = _lib.c_i64 * 3
@@ -236,15 +236,15 @@ def _mixed_layer(query_states, key_states, value_states, lp):
     return out
 
 
-def minference_prefill_kernel(q, k, v, pattern, vertical_size, slash_size):
+def minference_prefill_kernel(q, k, v, pattern, vertical_size, slash_size, out=None):
     """One pattern for all heads of q (minference_forward.py:626-631; for ``stream_llm`` the
     two sizes are n_init and n_local, as in the reference)."""
     if pattern == "stream_llm":
-        return streaming_forward(q, k, v, vertical_size, slash_size)
+        return streaming_forward(q, k, v, vertical_size, slash_size, out)
     if pattern == "vertical_and_slash":
-        return vertical_slash_prefill(q, k, v, vertical_size, slash_size)
+        return vertical_slash_prefill(q, k, v, vertical_size, slash_size, out)
     if pattern == "block_sparse":
-        return block_sparse_attention(q, k, v, 100)     # top_k fixed at 100 (:616-618)
+        return block_sparse_attention(q, k, v, 100, out=out)     # top_k fixed at 100 (:616-618)
     raise KeyError(pattern)
 
 
@@ -270,12 +270,15 @@ def _search_layer(query_states, key_states, value_states, prefill_kwargs):
             config_list.append(new_config)
             with open(config_path, "w") as f:
                 json.dump(config_list, f, indent=2)
-    return dense_causal_attention(query_states, key_states, value_states)
+    return dense_causal_attention(query_states, key_states, value_states, prefill_kwargs.get("out"))
 
 
 def minference_prefill_forward(query_states, key_states, value_states, prefill_kwargs):
-    """Sparse prefill attention of one layer: [B,Hq,N,D] x [B,Hk,N,D] -> [B,Hq,N,D]."""
+    """Sparse prefill attention of one layer: [B,Hq,N,D] x [B,Hk,N,D] -> [B,Hq,N,D].  An optional
+    ``out`` in prefill_kwargs is a [B,Hq,N,D] tensor the result is written to (a transposed view of the
+    layout the caller wants, for instance); it is then what is returned."""
     config = prefill_kwargs["attn_forward_config"]
+    out = prefill_kwargs.get("out")
     layer_idx = prefill_kwargs["layer_idx"]
     starting_layer = config.get("starting_layer", 0)
     B, H, N, D = query_states.shape
@@ -283,12 +286,12 @@ def minference_prefill_forward(query_states, key_states, value_states, prefill_k
     if config.get("is_search", False):
         return _search_layer(query_states, key_states, value_states, prefill_kwargs)
     if layer_idx < starting_layer:
-        return dense_causal_attention(query_states, key_states, value_states)
+        return dense_causal_attention(query_states, key_states, value_states, out)
     lp = _layer_plan(config, layer_idx, H)
     if len(lp.plan) == 1:
         (ty, vs, ss), _ = next(iter(lp.plan.items()))
-        return minference_prefill_kernel(query_states, key_states, value_states, ty, vs, ss)
-    return _mixed_layer(query_states, key_states, value_states, lp)
+        return minference_prefill_kernel(query_states, key_states, value_states, ty, vs, ss, out)
+    return _mixed_layer(query_states, key_states, value_states, lp, out)
 
 
 def a_shape_kernel(query_states, key_states, value_states, prefill_kwargs):
