@@ -319,8 +319,12 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     if (mi >= (int)units) return false;              // padding of the last round (workgroup-uniform)
     int mslot, seg = -1;                             // row-block pair, segment of its walk (-1: the whole walk)
     if (CUT && mi < split_units) {                    // the split pairs, longest walks first
-        mslot = rows_wg - 1 - mi / p.nseg;
-        seg = mi % p.nseg;
+        // first segments of all of them, then second segments, ...: a walk's own segments side by side, of
+        // which only every nseg-th exists where walks are short, all went to the same shader engines
+        // (workgroups are dealt to them in turn: dense, 12000 tokens, 16 heads of 64, two segments: 450 us)
+        const int split_pairs = rows_wg - p.split_first;
+        mslot = rows_wg - 1 - mi % split_pairs;
+        seg = mi / split_pairs;
     } else {
         mslot = p.descending ? rows_wg - 1 - mi : mi - split_units;
         if (p.descending) mslot += split_units - (rows_wg - p.split_first);
@@ -376,40 +380,6 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     const long long k_row = p.ks[2] * 2, v_row = p.vs[2] * 2;
     const long long ridx = ((long long)b * p.index_heads + hs) * p.rows + min(m, p.rows - 1);
 
-    constexpr bool every_max = EVERY_MAX;
-    // log2-domain scale of this lane's query row: one value per launch, except for the dense rows of a
-    // tri-shape launch (the reference scales its A-shape rows by the padded head_dim and its last
-    // rows by the unpadded one, streaming_kernel.py:575 against :826)
-    float sc_l2 = p.scale_log2;
-    if constexpr (MODE == MODE_ASHAPE) sc_l2 = qrow >= p.dense_from ? p.scale_log2_dense : p.scale_log2;
-    // ---- Q fragments (B operand of S^T): row qrow, d = 16*ks + 8*g + 0..7 ----
-    Frag qf[KS];
-    {
-        const bool ok = qrow < seqlen;
-        const char *qp = q_base + (long long)(ok ? qrow : min(row0, seqlen - 1)) * p.qs[2] * 2 + g * 16;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            qf[ks].u = *reinterpret_cast<const u32x4_t *>(qp + ks * 32);
-            if (!ok) qf[ks].u = u32x4_t{0u, 0u, 0u, 0u};
-        }
-    }
-
-    int nblk = 0;
-    // Paired list walks (vertical-slash block lists, block-sparse lists scaled to key starts): the
-    // block lists of the two row blocks (ascending key starts; vertical-slash lists of
-    // neighbouring row blocks are each other's translate by 64 keys wherever no entry is clipped, so
-    // runs of blocks share all but their ends) are split ONCE, by all 256 threads, before the tile
-    // loop: both lists are staged in LDS, every entry looks itself up in the other list by binary
-    // search, and a workgroup prefix sum over the hits places it either in the list of COMMON
-    // entries (tiles that both row blocks visit: copied once by four waves, one LDS word per step)
-    // or in its row block's list of entries the other one lacks (run ends).  The walk is then
-    //   common tiles, both halves computing;
-    //   split steps: every half visits its own leftover tiles -- the entries the other list lacks,
-    //   then its gathered column tiles -- with the K/V buffers of its own half,
-    // i.e. exactly max(tiles of A, tiles of B) steps, never more than the longer list alone.
-    // Lists that are too long for LDS or not strictly ascending are not split: each half then walks
-    // its whole list in split steps (still in lockstep with its neighbour, which is what keeps the
-    // neighbour's tiles in L2 when the lists are long and scattered).
     // where the block lists live: [batch, heads, list_rows, list_w]
     [[maybe_unused]] const int *const list_base = MODE == MODE_BS ? p.bidx : p.bo;
     [[maybe_unused]] const int list_w = MODE == MODE_BS ? p.max_blocks : p.nnz_s;
@@ -431,6 +401,62 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             vs_nb = b_exists ? max(0, min(as_const(p.bc)[vs_rb], p.nnz_s)) : 0;
             vs_ccb = b_exists ? max(0, min(as_const(p.cc)[vs_rb], p.nnz_v)) : 0;
         }
+    }
+    // steps of the walk (splitting the lists into common and leftover entries does not change their number)
+    int nblk = 0, ntiles;
+    if constexpr (VSP) ntiles = max(vs_na + ((vs_cca + BN - 1) >> 6), vs_nb + ((vs_ccb + BN - 1) >> 6));
+    else ntiles = pair_tile_count<MODE>(p, mA, mB, nblk);
+    // the part of the walk this workgroup makes: all of it, or one segment
+    int it_begin = 0, it_end = ntiles;
+    char *slot = nullptr;
+    if (CUT && seg >= 0) {
+        const int ns = max(1, min(p.nseg, (ntiles + p.seg_len - 1) / p.seg_len));
+        const int len = (ntiles + ns - 1) / ns;
+        it_begin = min(seg * len, ntiles);
+        it_end = seg < ns ? min(it_begin + len, ntiles) : it_begin;
+        const int heads = p.head_list ? p.index_heads : p.hq;
+        slot = p.part + (((long long)(b * heads + hs) * (rows_wg - p.split_first) + (mslot - p.split_first)) * p.nseg + seg) * SplitSlot<HD>::BYTES;
+        if (it_begin >= it_end) {                       // (workgroup-uniform) nothing to add: a row sum of zero says so, before any of the walk's set-up
+            float2 *ml = reinterpret_cast<float2 *>(slot + SplitSlot<HD>::ACC) + tid;
+            *ml = make_float2(-INFINITY, 0.f);
+            return false;
+        }
+    }
+
+    constexpr bool every_max = EVERY_MAX;
+    // log2-domain scale of this lane's query row: one value per launch, except for the dense rows of a
+    // tri-shape launch (the reference scales its A-shape rows by the padded head_dim and its last
+    // rows by the unpadded one, streaming_kernel.py:575 against :826)
+    float sc_l2 = p.scale_log2;
+    if constexpr (MODE == MODE_ASHAPE) sc_l2 = qrow >= p.dense_from ? p.scale_log2_dense : p.scale_log2;
+    // ---- Q fragments (B operand of S^T): row qrow, d = 16*ks + 8*g + 0..7 ----
+    Frag qf[KS];
+    {
+        const bool ok = qrow < seqlen;
+        const char *qp = q_base + (long long)(ok ? qrow : min(row0, seqlen - 1)) * p.qs[2] * 2 + g * 16;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            qf[ks].u = *reinterpret_cast<const u32x4_t *>(qp + ks * 32);
+            if (!ok) qf[ks].u = u32x4_t{0u, 0u, 0u, 0u};
+        }
+    }
+
+    // Paired list walks (vertical-slash block lists, block-sparse lists scaled to key starts): the
+    // block lists of the two row blocks (ascending key starts; vertical-slash lists of
+    // neighbouring row blocks are each other's translate by 64 keys wherever no entry is clipped, so
+    // runs of blocks share all but their ends) are split ONCE, by all 256 threads, before the tile
+    // loop: both lists are staged in LDS, every entry looks itself up in the other list by binary
+    // search, and a workgroup prefix sum over the hits places it either in the list of COMMON
+    // entries (tiles that both row blocks visit: copied once by four waves, one LDS word per step)
+    // or in its row block's list of entries the other one lacks (run ends).  The walk is then
+    //   common tiles, both halves computing;
+    //   split steps: every half visits its own leftover tiles -- the entries the other list lacks,
+    //   then its gathered column tiles -- with the K/V buffers of its own half,
+    // i.e. exactly max(tiles of A, tiles of B) steps, never more than the longer list alone.
+    // Lists that are too long for LDS or not strictly ascending are not split: each half then walks
+    // its whole list in split steps (still in lockstep with its neighbour, which is what keeps the
+    // neighbour's tiles in L2 when the lists are long and scattered).
+    if constexpr (VSP) {
         if (vs_na <= VS_PAIR_MAX && vs_nb <= VS_PAIR_MAX && vs_na > 0 && vs_nb > 0) {
             int *rawA = reinterpret_cast<int *>(lds_k1), *rawB = rawA + VS_PAIR_MAX;
             int *common = reinterpret_cast<int *>(lds_v1);
@@ -488,7 +514,6 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             }
         }
     }
-    int ntiles = 0;
     // paired vertical-slash: vs_nc common steps, then the split steps: per half its leftover block
     // entries (from LDS when the lists were split, else its whole list from global memory) and its
     // gathered column tiles.  The barriers are the workgroup's: both halves make max(A, B) split
@@ -500,25 +525,6 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         vs_nb_mine = half ? nb_b : nb_a;
         vs_cc_mine = half ? vs_ccb : vs_cca;
         vs_nt_mine = have_rows ? (half ? nt_b : nt_a) : 0;
-        ntiles = vs_nc + max(nt_a, nt_b);
-    }
-    else
-        ntiles = pair_tile_count<MODE>(p, mA, mB, nblk);
-    // the part of the walk this workgroup makes: all of it, or one segment
-    int it_begin = 0, it_end = ntiles;
-    char *slot = nullptr;
-    if (CUT && seg >= 0) {
-        const int ns = max(1, min(p.nseg, (ntiles + p.seg_len - 1) / p.seg_len));
-        const int len = (ntiles + ns - 1) / ns;
-        it_begin = min(seg * len, ntiles);
-        it_end = seg < ns ? min(it_begin + len, ntiles) : it_begin;
-        const int heads = p.head_list ? p.index_heads : p.hq;
-        slot = p.part + (((long long)(b * heads + hs) * (rows_wg - p.split_first) + (mslot - p.split_first)) * p.nseg + seg) * SplitSlot<HD>::BYTES;
-        if (it_begin >= it_end) {                       // (workgroup-uniform) nothing to add: a row sum of zero says so
-            float2 *ml = reinterpret_cast<float2 *>(slot + SplitSlot<HD>::ACC) + tid;
-            *ml = make_float2(-INFINITY, 0.f);
-            return false;
-        }
     }
     auto more_tiles = [&](int it) -> bool { return it < it_end; };   // is there a tile number `it` ?
     // paired vertical-slash: entry it+1 of the common list sits in a scalar when step `it` starts; the
@@ -1199,48 +1205,64 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
 }
 
-// Which walks to split.  `slots` workgroups fit the chip at once.
-//  * Dense walks (dense attention, the last rows of tri-shape) grow with the row block: they are split when
-//    the longest one takes more than half of the steps a slot of the full chip gets, into segments as long
-//    as a slot's share (one head, 16384 tokens: 300 -> 128 us; shares of 0.25, 0.5 and 2: 175, 145, 125 us;
-//    tri-shape, 16 heads of 64, fp16, 24000 tokens, last 128 rows dense: 444 -> 131 us; 147, 138, 152 us).
-//    Below half, the descending order hides the longest walk behind the others.
-//  * Everything else has walks of bounded length and is split only when the launch has at most 64
-//    row-block pairs, i.e. gives at most a quarter of the compute units a workgroup.  The segments then
-//    have SEG_MIN steps whatever else the launch holds, and launches of more than 64 pairs are not split
-//    for one head or for many, so that such a head's bits do not depend on the heads it is launched with.
-// SEG_MIN weighs the fixed cost of a workgroup (about five steps) and of the fold against the chain of
-// steps.  One head: dense 4096 tokens 78 us whole; 45, 35, 31, 27.5, 28.5, 30.5 us with 3, 4, 6, 8, 12, 16
-// steps; vertical-slash 500 + 700, 4096 tokens, the whole path 177 us whole; 157, 152, 148, 145, 147, 150 us.
+// Which walks to split, and how.  `slots` workgroups fit the chip at once, a slot's share of the launch is
+// `share` steps.  The longest walk sets the time of a launch whose share is much smaller; cut, it costs a
+// fixed part per segment (about five steps), and its sums travel through memory to the fold (0.02 us per
+// segment of a full chip).  Segments of 1.4 shares were the best or within 5 % of it wherever splitting
+// paid at all (lengths 8 .. 128 swept): dense, 8 / 2 heads 8192 tokens 180 -> 162 us, 4 heads 16384 tokens
+// 350 -> 301, one head 24000 tokens 439 -> 175, 8 heads of 64, 6000 tokens 87 -> 61; vertical-slash,
+// 4 heads 5000 tokens 95 -> 56, 4 heads 8000 tokens 177 -> 95, 16 heads 2570 tokens 68 -> 62; block-sparse
+// 8 heads 6000 tokens 145 -> 100; A-shape 8 heads 6000 tokens 117 -> 97.  Where a share is nearly the
+// longest walk the whole walks win, longest first (dense: 16 heads of 64, 12000 tokens 310 against 345 us,
+// 16 heads 6000 tokens 161 : 174), and so they do where a walk is too short for what a cut costs (dense,
+// 32 / 8 heads 2048 tokens 53 : 58; 32 heads 1000 tokens 26 : 32; block-sparse, 28 heads 2000 tokens 57 :
+// 64): the steps saved have to be worth it.
+//  * Dense walks and the dense last rows of tri-shape have any number of steps.
+//  * Lists are not known on the host and are taken as dense, A-shape walks end at their window.  Both
+//    are split up to 64 row-block pairs per head only: beyond, a head has the same bits whatever heads it
+//    is launched with, which per-head dispatch relies on.  Up to 64 pairs in all, segments have SEG_MIN
+//    steps whatever else the launch holds.
 constexpr int SEG_MIN = 8;
 SplitPlan plan_split(int mode, const AttnParams &p, int head_dim) {
     const int pairs = (p.rows + 1) / 2;
     const SplitPlan none{pairs, 1, 1};
     const long long heads = (long long)p.batch * (p.head_list ? p.index_heads : p.hq);
     const int slots = head_dim == 256 ? 256 : (head_dim == 128 ? 512 : 768);
-    auto capped = [&](int first, int longest, int len) -> SplitPlan {
-        const int nseg = (longest + len - 1) / len;
-        return nseg < 2 ? none : SplitPlan{first, nseg < 64 ? nseg : 64, len};
+    // walks of pairs 0 .. k-1: pair i has 2 i + 2 steps, at most `most`
+    const int window = mode == MODE_ASHAPE ? (int)(((long long)p.n_local + BM - 1) / BN + 2 + ((long long)p.n_init + BN - 1) / BN) : 0x7fffffff;
+    auto steps = [&](int k, int most) -> double {
+        const double grown = most / 2 < k ? most / 2 : k;
+        return grown * (grown + 1) + (k - grown) * most;
     };
-    const bool dense = mode == MODE_DENSE;
-    const int first_dense = dense ? 0 : (mode == MODE_ASHAPE && p.dense_from < p.n ? p.dense_from / (2 * BM) : pairs);
-    if (first_dense < pairs) {
-        // steps of the dense pairs first_dense .. pairs-1 (pair i: 2 i + 2) and of the pairs before them
-        double total = (double)pairs * (pairs + 1) - (double)first_dense * (first_dense + 1);
-        if (first_dense > 0) {
-            const double window = (p.n_local + BM - 1) / BN + 2 + (p.n_init + BN - 1) / BN;
-            const double grown = window / 2 < first_dense ? window / 2 : first_dense;
-            total += grown * grown + (first_dense - grown) * window;
-        }
-        const double per_slot = total * (double)heads / slots;
-        const int longest = p.rows;
-        if (2.0 * longest > per_slot) {
-            return capped(first_dense, longest, per_slot > SEG_MIN ? (int)per_slot : SEG_MIN);
-        }
-        if (dense) return none;
+    const int first_dense = mode == MODE_DENSE ? 0 : (mode == MODE_ASHAPE && p.dense_from < p.n ? p.dense_from / (2 * BM) : pairs);
+    const bool dense = first_dense < pairs;
+    if (!dense && pairs > 64) return none;
+    const int first = dense ? first_dense : 0;
+    const int longest = dense ? p.rows : (p.rows < window ? p.rows : window);
+    const int others = first > 0 ? (2 * first < window ? 2 * first : window) : 0;      // longest of the walks that stay whole
+    const double total = dense ? steps(pairs, 0x7fffffff) - steps(first, 0x7fffffff) + (first > 0 ? steps(first, window) : 0.) : steps(pairs, window);
+    const double share = total * (double)heads / slots;
+    if (!dense && heads * pairs <= 64) {
+        const int most = longest + (mode == MODE_VS ? SEG_MIN : 0);                    // (gathered columns)
+        const int nseg = (most + SEG_MIN - 1) / SEG_MIN;
+        return longest < 2 * SEG_MIN ? none : SplitPlan{0, nseg, SEG_MIN};
     }
-    if (heads * pairs > 64) return none;
-    return capped(0, 2 * pairs + SEG_MIN, SEG_MIN);
+    double want = 1.4 * share + 2;
+    // dense rows at the end of a launch of shorter walks would finish last: segments of one share (16 heads of
+    // 64, fp16, 24000 tokens, 128 dense rows: whole 434 us; 145, 133, 129, 152 us with 16, 48, 64, 96 steps)
+    // and at least two (32 / 8 heads, 8000 tokens, window 3968: 550 -> 460 us)
+    if (others > 0) want = share;
+    if (others > 0 && want > (longest + 1) / 2) want = (longest + 1) / 2 > window ? (longest + 1) / 2 : window;
+    if (want >= longest) return none;
+    const int len = want > SEG_MIN ? (int)want : SEG_MIN;
+    int nseg = (longest + (mode == MODE_VS ? SEG_MIN : 0) + len - 1) / len;
+    if (nseg > 64) nseg = 64;
+    const int cut = (longest + nseg - 1) / nseg;
+    // (a launch of more than 400 workgroups fills most of the chip already: vertical-slash, 16 heads of scattered
+    // lists, 4096 tokens, 512 workgroups, 32 of 64 steps saved: 110 -> 116 us)
+    const long long wgs = heads * (pairs - first);
+    if (longest - (cut > others ? cut : others) < (wgs <= 400 ? 4 + wgs / 24 : wgs / 13)) return none;
+    return SplitPlan{first, nseg, len};
 }
 
 size_t split_bytes(const SplitPlan &s, const AttnParams &p, int head_dim) {
@@ -1275,13 +1297,23 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
     // 366 -> 381, A-shape 4 / 4 heads 16384 tokens 129 -> 134: so from eight heads and two rounds of
     // workgroups on, up to 64K tokens.
     const long long groups = (long long)p.batch * (grid_heads / group);
+    // (block-sparse, 50000 tokens, 28 / 4 heads: top-100 4.19 -> 4.00 ms, top-50 2.12 -> 2.16: where the walks
+    // grow over less than a fourteenth of the rows the stripes do not pay)
+    const int most = MODE == MODE_BS ? p.max_blocks :
+                     MODE == MODE_ASHAPE ? (int)(((long long)p.n_local + p.n_init) / BN) + 2 : p.rows;    // steps of a full walk (lists: unknown)
     const bool grows = MODE == MODE_DENSE || split_pairs > 0 ||
-                       (p.rows <= 1024 && groups * group >= 8 && groups * group * units >= 1024);
+                       (p.rows <= 1024 && p.rows <= 14ll * most && groups * group >= 8 && groups * group * units >= 1024);
     p.stripes = 1;
     if (grows)
         while (p.stripes < 8 && groups * p.stripes % 8) p.stripes *= 2;
     p.total_wg = groups * group * p.stripes * ((units + p.stripes - 1) / p.stripes);
-    p.descending = MODE == MODE_DENSE || (MODE == MODE_VS && p.rows <= 1024);
+    // Longest walks first wherever they grow with the row block over much of the sequence.  A-shape and
+    // block-sparse, 32 / 8 heads: 3000 tokens 107 -> 91 and 118 -> 92 us, 6000 tokens 336 -> 315 (6824) and
+    // 333 -> 308, 12000 tokens 702 -> 677 and 921 -> 897, 24000 tokens 1508 -> 1487 and (32768) 2947 -> 2920;
+    // neither order wins past 60000 tokens, and with fewer than two rounds of workgroups and walks that are
+    // full-length early the first rows finish last (A-shape, 8 / 2 heads, 12000 tokens 227 -> 234 us).
+    p.descending = MODE == MODE_DENSE || (MODE == MODE_VS ? p.rows <= 1024 :
+                   p.rows <= most || (p.rows <= 8ll * most && groups * group * units >= 1024));
     const long long per_xcd = (p.total_wg + 7) >> 3;
     const long long grid = per_xcd * 8;
     if (grid > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;

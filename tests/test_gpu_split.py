@@ -30,6 +30,25 @@ def test_split_walks_match_the_oracle(gpu, n, hq, hk, b, d, dtype):
               O.vertical_slash_sparse_attention(q, ke, ve, v_idx.cpu(), s_idx.cpu()), "vertical-slash")
 
 
+@pytest.mark.parametrize("n,hq,hk,b", [(2111, 12, 3, 1), (4033, 4, 4, 2)])
+def test_half_full_launches_are_split_by_their_share(gpu, n, hq, hk, b):
+    """More than 64 row-block pairs, too few to fill the chip: segments of 1.4 shares (lone last row block,
+    ragged end), several heads and batches; the oracle on one head of each batch."""
+    import minference_amd as M
+    q, k, v = make(b, hq, hk, n, n, torch.bfloat16)
+    qg, kg, vg = q.to(gpu), k.to(gpu), v.to(gpu)
+    h = hq - 1
+    one = (slice(None), slice(h, h + 1))
+    qo, ko, vo = q[one], expand(k, hq)[one], expand(v, hq)[one]
+    check(M.dense_causal_attention(qg, kg, vg)[one], sdpa_causal(qo, ko, vo), "dense")
+    check(M.block_sparse_attention(qg, kg, vg, 1000)[one], sdpa_causal(qo, ko, vo), "block-sparse")
+    check(M.streaming_forward(qg, kg, vg, 70, 4000)[one], O.streaming_forward(qo, ko, vo, 70, 4000), "a-shape")
+    check(M.tri_shape_forward(qg, kg, vg, 8, 130, 300)[one], O.tri_shape_forward(qo, ko, vo, 8, 130, 300), "tri-shape")
+    v_idx, s_idx = M.estimate_vertical_slash(qg, kg, 200, 500)
+    check(M.vertical_slash_sparse_attention(qg, kg, vg, v_idx, s_idx)[one],
+          O.vertical_slash_sparse_attention(qo, ko, vo, v_idx[one].cpu(), s_idx[one].cpu()), "vertical-slash")
+
+
 def test_split_walks_with_short_sequences_and_many_leftovers(gpu):
     """seqlens below n in the middle of a pair, before one and in the first tile (rows past them are zero),
     with lists whose leftovers differ between the row blocks of a pair (scattered slashes)."""
@@ -70,6 +89,14 @@ def test_which_launches_are_split():
         t.batch, t.heads_q, t.heads_kv, t.n, t.head_dim = 1, hq, 1, n, d
         return lib.minf_attn_workspace_bytes(ctypes.byref(t), op, *(sizes or (0, 0, 0)))
     vs, ashape, dense = _lib.MINF_OP_VERTICAL_SLASH, _lib.MINF_OP_ASHAPE, _lib.MINF_OP_DENSE
+    bs = _lib.MINF_OP_BLOCK_SPARSE
+    # half a chip of long walks is split, a full one and one of short walks are not
+    assert nbytes(vs, 8192, 4) > 0 and nbytes(bs, 6000, 8) > 0 and nbytes(ashape, 6000, 8, 128, 3968, 0) > 0
+    assert nbytes(vs, 4096, 16) == 0 and nbytes(bs, 2000, 28) == 0 and nbytes(ashape, 6000, 8, 64, 1000, 0) == 0
+    assert nbytes(dense, 16384, 4) > 0 and nbytes(dense, 6000, 16) == 0 and nbytes(dense, 12000, 16, d=64) == 0
+    assert nbytes(dense, 2048, 32) == 0 and nbytes(vs, 400, 2) == 0
+    # the dense rows of tri-shape: where they outlast the windows, in two segments at least
+    assert nbytes(ashape, 8000, 32, 128, 3968, 100) > 0 and nbytes(ashape, 523, 32, 128, 3968, 100) == 0
     assert nbytes(vs, 4096, 1) > 0 and nbytes(vs, 8192, 1) > 0 and nbytes(vs, 8193, 1) == 0 and nbytes(vs, 4096, 32) == 0
     assert nbytes(dense, 16384, 1) > 0 and nbytes(dense, 6144, 64) == 0 and nbytes(dense, 64, 1) == 0
     assert nbytes(ashape, 24000, 16, 8, 512, 128, d=64) > 0 and nbytes(ashape, 24000, 16, 8, 512, 0, d=64) == 0
