@@ -56,6 +56,7 @@ __host__ __device__ inline int chunk_keys(int n) {
     return n > 131072 ? 2048 : (n > 57344 ? 1024 : (n > 20480 ? 512 : (n > 6144 ? 256 : 128)));
 }
 constexpr int EST_THREADS = 256;
+constexpr int EST_WHOLE_MIN = 160;   // workgroups from which a wave walks a chunk of its own (see fill)
 // A chunk is always summed as four pieces of a quarter of its keys, each piece by one wave from its first key to
 // its last, and the pieces are combined in ascending order -- whether one wave walks the whole chunk
 // (four heads per workgroup) or four waves a piece each (one head per workgroup).  The scores of a
@@ -82,6 +83,8 @@ struct EstParams {
     int index_heads;
     int gw;                     // query heads per workgroup (waves w % gw), 4 / gw key sub-ranges each
     int nhc;                    // head groups: ceil(index_heads / gw)
+    int cw;                     // chunks per workgroup: 1 (the waves of a head share it), or 4 / gw (a wave walks a chunk of its own)
+    int nwc;                    // ceil(nchunks / cw)
 };
 
 union Frag {
@@ -124,11 +127,12 @@ template <typename T> __device__ __forceinline__ void ref_logit_pair(float &a, f
 }
 constexpr float LOG2E = 1.4426950408889634f;
 
-struct WgId { int b, h, hkv, chunk, slot, kq; bool valid, wave_valid; };
+struct WgId { int b, h, hkv, chunk, slot, kq; bool valid, wave_valid; };      // kq: which quarter / half of the chunk this wave walks
 
 // Workgroup order: (batch, head group, chunk), contiguous per XCD: the chunks of one head group --
 // i.e. of (mostly) one kv head -- are swept by consecutive workgroups of one XCD.  `reverse` flips
-// the order (second sweep).  Wave `wave` of the workgroup gets head hc * gw + wave % gw.
+// the order (second sweep).  Wave `wave` of the workgroup gets head hc * gw + wave % gw, and with
+// several chunks per workgroup chunk wave / gw of them.
 __device__ __forceinline__ WgId decode_wg(const EstParams &p, int wave, bool reverse) {
     WgId w;
     const long long per_xcd = (p.total_wg + 7) >> 3;
@@ -137,12 +141,13 @@ __device__ __forceinline__ WgId decode_wg(const EstParams &p, int wave, bool rev
     if (reverse) logical = p.total_wg - 1 - logical;
     const int group = p.hq / p.hk;
     long long rest = logical;
-    w.chunk = (int)(rest % p.nchunks); rest /= p.nchunks;
+    w.chunk = (int)(rest % p.nwc) * p.cw; rest /= p.nwc;
     const int hc = (int)(rest % p.nhc);
     w.b = (int)(rest / p.nhc);
-    w.kq = wave / p.gw;
+    w.kq = p.cw > 1 ? 0 : wave / p.gw;
+    if (p.cw > 1) w.chunk += wave / p.gw;
     w.slot = hc * p.gw + wave % p.gw;
-    w.wave_valid = w.valid && w.slot < p.index_heads;
+    w.wave_valid = w.valid && w.slot < p.index_heads && w.chunk < p.nchunks;
     w.h = w.wave_valid ? (p.head_list ? p.head_list[w.slot] : w.slot) : 0;
     w.hkv = w.h / group;
     return w;
@@ -241,16 +246,18 @@ __device__ __forceinline__ int common_kv_head(const EstParams &p, const WgId &w,
 template <typename T, int HD, bool RR>
 __global__ __launch_bounds__(EST_THREADS, 3) void est_stats_kernel(const EstParams p) {
     constexpr int KS = HD / 16;       // k-steps of one 32x32 score block
-    __shared__ float lds_m[16][LQ], lds_l[16][LQ];     // [head of the workgroup * 4 + piece][row]
+    __shared__ float lds_m[16][LQ], lds_l[16][LQ];     // [unit of the workgroup * 4 + piece][row]
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // wave-uniform: addresses built from it stay scalar
     const WgId w = decode_wg(p, wave, false);
     if (!w.valid) return;
     const int l32 = lane & 31, g = lane >> 5;
     const int KC = p.kc, PB = KC / 128;               // keys per chunk, 32-key blocks per piece
-    const int nq = 4 / p.gw, klen = KC / nq;          // key sub-ranges per head, keys per wave
-    const int ppw = p.gw;                             // pieces per wave
-    const int piece0 = (wave % p.gw) * 4 + w.kq * ppw; // this wave's first (head, piece) slot
+    const int nq = p.cw > 1 ? 1 : 4 / p.gw, klen = KC / nq;          // key sub-ranges per chunk, keys per wave
+    const int ppw = 4 / nq;                           // pieces per wave
+    const int units = p.gw * p.cw;                    // (head, chunk) pairs of the workgroup: unit u is wave u's
+    const int unit = p.cw > 1 ? wave : wave % p.gw;
+    const int piece0 = unit * 4 + w.kq * ppw;         // this wave's first (unit, piece) slot
 
     // lane <-> query rows i = l32 and 32 + l32; regs <-> keys 8*(r/4) + 4*g + r%4 of the block
     float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
@@ -332,7 +339,7 @@ __global__ __launch_bounds__(EST_THREADS, 3) void est_stats_kernel(const EstPara
     };
     if (kv_common >= 0) {
         KShare<HD> ks_;
-        ks_.init(p, p.k + ((long long)w.b * p.ks[0] + (long long)kv_common * p.ks[1]) * 2, lds_kt[w.kq & 1], lane, wave % p.gw);
+        ks_.init(p, p.k + ((long long)w.b * p.ks[0] + (long long)kv_common * p.ks[1]) * 2, lds_kt[(wave / p.gw) & 1], lane, wave % p.gw);
         ks_.copy(key_begin, 0);
         for (int blk = 0; blk < nblk; ++blk) {
             const int c0 = key_begin + blk * 32;
@@ -364,9 +371,9 @@ __global__ __launch_bounds__(EST_THREADS, 3) void est_stats_kernel(const EstPara
     if (w.wave_valid)
         while (pieces_done < ppw) flush_piece();
     __syncthreads();
-    // thread (hsub, row) folds the four pieces of head hsub's row in ascending order
+    // thread (hsub, row) folds the four pieces of unit hsub's row in ascending order
     const int hsub = tid / LQ, row = tid % LQ;
-    if (hsub < p.gw) {
+    if (hsub < units) {
         const WgId wh = decode_wg(p, hsub, false);
         if (wh.wave_valid) {
             float m = lds_m[hsub * 4][row], l = lds_l[hsub * 4][row];
@@ -403,7 +410,7 @@ __device__ __forceinline__ float wave_shr1(float x) {      // lane L <- lane L -
 template <typename T, int HD, bool RR>
 __global__ __launch_bounds__(EST_THREADS, 2) void est_scores_kernel(const EstParams p) {
     constexpr int KS = HD / 16;
-    __shared__ float lds_pwin[16 * PWIN_MAX];          // [head of the workgroup * 4 + piece][PWIN]
+    __shared__ float lds_pwin[16 * PWIN_MAX];          // [unit of the workgroup * 4 + piece][PWIN]
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // wave-uniform: addresses built from it stay scalar
     const WgId w = decode_wg(p, wave, true);
@@ -411,10 +418,12 @@ __global__ __launch_bounds__(EST_THREADS, 2) void est_scores_kernel(const EstPar
     const int l32 = lane & 31, g = lane >> 5;
     const int KC = p.kc, PIECE = KC / 4, PB = PIECE / 32, PWIN = PIECE + LQ, WIN = KC + LQ;
     const int pb_shift = __builtin_ctz(PB);
-    const int nq = 4 / p.gw, klen = KC / nq;          // key sub-ranges per head, keys per wave
-    const int ppw = p.gw;                             // pieces per wave
+    const int nq = p.cw > 1 ? 1 : 4 / p.gw, klen = KC / nq;          // key sub-ranges per chunk, keys per wave
+    const int ppw = 4 / nq;                           // pieces per wave
+    const int units = p.gw * p.cw;                    // (head, chunk) pairs of the workgroup: unit u is wave u's
+    const int unit = p.cw > 1 ? wave : wave % p.gw;
     const long long bh = (long long)w.b * p.index_heads + w.slot;
-    float *const wwin0 = lds_pwin + ((wave % p.gw) * 4 + w.kq * ppw) * PWIN;   // this wave's ppw piece windows, contiguous
+    float *const wwin0 = lds_pwin + (unit * 4 + w.kq * ppw) * PWIN;   // this wave's ppw piece windows, contiguous
 
     for (int i = lane; i < ppw * PWIN; i += 64) wwin0[i] = 0.f;
     __syncthreads();
@@ -549,7 +558,7 @@ __global__ __launch_bounds__(EST_THREADS, 2) void est_scores_kernel(const EstPar
     };
     if (kv_common >= 0) {
         KShare<HD> ks_;
-        ks_.init(p, p.k + ((long long)w.b * p.ks[0] + (long long)kv_common * p.ks[1]) * 2, lds_kt[w.kq & 1], lane, wave % p.gw);
+        ks_.init(p, p.k + ((long long)w.b * p.ks[0] + (long long)kv_common * p.ks[1]) * 2, lds_kt[(wave / p.gw) & 1], lane, wave % p.gw);
         ks_.copy(key_begin, 0);
         float cs_prev = 0.f;                         // column sum of the previous block, stored a block later
         int c_prev = -1;                             // (so that no store is waited for with the copies)
@@ -583,9 +592,9 @@ __global__ __launch_bounds__(EST_THREADS, 2) void est_scores_kernel(const EstPar
         }
     }
     __syncthreads();
-    // chunk window of head hsub, position q = (key - chunk0) + (last_q - 1 - i): piece pc contributes
+    // chunk window of unit hsub, position q = (key - chunk0) + (last_q - 1 - i): piece pc contributes
     // its slot q - pc * PIECE; the pieces are added in ascending order
-    for (int idx = tid; idx < p.gw * WIN; idx += EST_THREADS) {
+    for (int idx = tid; idx < units * WIN; idx += EST_THREADS) {
         const int hsub = idx / WIN, q = idx - hsub * WIN;
         const WgId wh = decode_wg(p, hsub, true);
         if (!wh.wave_valid) continue;
@@ -649,7 +658,16 @@ int fill(EstParams &p, const void *q, const void *k, const int64_t *q_stride, co
     const int group = heads_q / heads_kv;
     p.gw = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
     p.nhc = (index_heads + p.gw - 1) / p.gw;
-    p.total_wg = (long long)batch * p.nhc * p.nchunks;
+    // Waves that share a chunk each repeat what a workgroup does once per head (the row constants from every
+    // chunk's statistics, the windows): four heads in a workgroup amortise that over a whole chunk per
+    // wave, one head over a quarter.  With enough of them to fill the chip, workgroups of one or two
+    // heads take one chunk per wave as well.  Whole estimate, us, waves sharing / not: 28 / 4 heads 34806
+    // tokens 161 / 105, 16384 106 / 66, 8000 (224 workgroups) 60 / 40, 2570 (168) 38 / 30; 16 heads 53720
+    // 155 / 111, 4096 (128) 30 / 31; 4 heads 100000 (100) 71 / 108; one head 131072 45 / 107.
+    p.cw = 4 / p.gw;
+    p.nwc = (p.nchunks + p.cw - 1) / p.cw;
+    if ((long long)batch * p.nhc * p.nwc < EST_WHOLE_MIN) { p.cw = 1; p.nwc = p.nchunks; }
+    p.total_wg = (long long)batch * p.nhc * p.nwc;
     p.head_list = head_list;
     p.index_heads = index_heads;
     return MINF_OK;

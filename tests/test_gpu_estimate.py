@@ -139,7 +139,10 @@ def test_ragged_topk_pads_with_noop_entries(gpu, n):
 
 
 @pytest.mark.parametrize("hq,hk,n,dtype,d", [(4, 1, 20000 + 37, torch.bfloat16, 128), (8, 2, 9000, torch.float16, 64),
-                                              (2, 1, 5000, torch.bfloat16, 128), (6, 2, 2048 * 3, torch.bfloat16, 64)])
+                                              (2, 1, 5000, torch.bfloat16, 128), (6, 2, 2048 * 3, torch.bfloat16, 64),
+                                              # enough heads for a wave per chunk: one and two heads per workgroup, a last
+                                              # workgroup with waves past the last chunk
+                                              (14, 2, 40001, torch.bfloat16, 64), (16, 8, 20481, torch.float16, 128)])
 def test_a_heads_scores_do_not_depend_on_the_heads_it_is_launched_with(gpu, hq, hk, n, dtype, d):
     """Grouped-query launches score four (or two) heads per workgroup, one wave per head over a whole
     2048-key chunk; a head on its own is scored by four waves of 512 keys.  Both sum a chunk as the same
