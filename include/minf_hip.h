@@ -128,6 +128,17 @@ int minf_vs_index_build_static(const int32_t *seqlens, const int32_t *vertical_i
                                void *stream);
 
 /*
+ * Sorts index rows for the index builder: vertical [rows, nnz_v] ascending, slash [rows, nnz_s] descending,
+ * both contiguous, int32 or (is64 != 0) int64 truncated to 32 bits, into int32 outputs of the same shapes;
+ * input and output may not overlap.  Values may repeat and be negative.  Rows of up to MINF_INDEX_SORT_MAX values
+ * (reference minference/ops/pit_sparse_flash_attention_v2.py:224-225 sorts with torch).
+ */
+#define MINF_INDEX_SORT_MAX 16384
+int minf_index_sort_pair(const void *vertical, int vertical_is64, int nnz_v, int32_t *vertical_out,
+                         const void *slash, int slash_is64, int nnz_s, int32_t *slash_out, int rows,
+                         void *stream);
+
+/*
  * Sparse flash-attention forward on one shared 64x64 bf16/f16 MFMA tile
  * engine.  Common arguments of the four entry points below:
  *

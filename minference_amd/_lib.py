@@ -27,6 +27,7 @@ SIGNATURES = {
     "minf_vs_index_workspace_bytes": (ctypes.c_size_t, [c_int] * 4),
     "minf_vs_index_build_ws": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
     "minf_vs_index_build_static": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr]),
+    "minf_index_sort_pair": (c_int, [c_ptr, c_int, c_int, c_ptr] * 2 + [c_int, c_ptr]),
     "minf_vs_attn_fwd": (c_int, [c_ptr] * 5 + [c_int] * 3 + [c_ptr]),
     "minf_bs_attn_fwd": (c_int, [c_ptr, c_ptr, c_int, c_int, c_ptr]),
     "minf_ashape_attn_fwd": (c_int, [c_ptr, c_int, c_int, c_ptr]),
@@ -78,6 +79,7 @@ class QKVO(ctypes.Structure):
 
 MINF_BF16, MINF_F16, MINF_F32 = 0, 1, 2
 MINF_OP_VERTICAL_SLASH, MINF_OP_BLOCK_SPARSE, MINF_OP_ASHAPE, MINF_OP_DENSE = 0, 1, 2, 3
+MINF_INDEX_SORT_MAX = 16384
 MINF_ROUND_NONE, MINF_ROUND_INPUT_DTYPE = 0, 1
 MINF_BS_FORCE_DIAG_FIRST, MINF_BS_ROUND_INPUT_DTYPE = 1, 2
 

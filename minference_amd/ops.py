@@ -176,6 +176,24 @@ def vertical_slash_attention_from_index(query, key, value, block_count, block_of
     return c.result()
 
 
+def _sorted_indices(v_idx, s_idx, B, H):
+    """[B, H, nnz] int32: v_idx ascending, s_idx descending (one kernel; rows longer than its LDS are left
+    to torch)."""
+    v = v_idx if v_idx.dtype in (torch.int32, torch.int64) else v_idx.to(torch.int32)
+    s = s_idx if s_idx.dtype in (torch.int32, torch.int64) else s_idx.to(torch.int32)
+    v, s = v.reshape((B, H, -1)).contiguous(), s.reshape((B, H, -1)).contiguous()
+    nv, ns = v.shape[-1], s.shape[-1]
+    if not (v.is_cuda and s.device == v.device) or max(nv, ns) > _lib.MINF_INDEX_SORT_MAX:
+        return (v.to(torch.int32).sort(dim=-1, descending=False)[0], s.to(torch.int32).sort(dim=-1, descending=True)[0])
+    vo, so = (torch.empty(t.shape, dtype=torch.int32, device=t.device) for t in (v, s))
+    with torch.cuda.device(v.device):
+        st = _lib.load().minf_index_sort_pair(v.data_ptr(), v.dtype == torch.int64, nv, vo.data_ptr(),
+                                              s.data_ptr(), s.dtype == torch.int64, ns, so.data_ptr(), B * H,
+                                              _lib.stream_ptr(v.device))
+    _lib.check(st, "minf_index_sort_pair")
+    return vo, so
+
+
 def vertical_slash_sparse_attention(query, key, value, v_idx, s_idx, block_size_M: int = 64,
                                     block_size_N: int = 64):
     """Vertical-slash sparse attention (pit_sparse_flash_attention_v2.py:195-242).
@@ -187,8 +205,7 @@ def vertical_slash_sparse_attention(query, key, value, v_idx, s_idx, block_size_
         raise ValueError("only 64x64 blocks are supported")
     _check_qkv(query, key, value)
     B, H, N, _ = query.shape
-    v_idx = v_idx.to(torch.int32).reshape((B, H, -1)).sort(dim=-1, descending=False)[0]
-    s_idx = s_idx.to(torch.int32).reshape((B, H, -1)).sort(dim=-1, descending=True)[0]
+    v_idx, s_idx = _sorted_indices(v_idx, s_idx, B, H)
     seqlens = torch.full((B,), N, dtype=torch.int32, device=query.device)
     bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, block_size_M,
                                                     block_size_N, zero_fill=False)
