@@ -36,6 +36,7 @@ extern "C" {
 
 #define MINF_BF16 0
 #define MINF_F16 1
+#define MINF_16BIT_SELECT 3         /* attention entry points only: see minf_qkvo.dtype_select */
 #define MINF_F32 2                  /* the decoder-layer passes at the end of this header only */
 
 /* Rounding of the two index selectors (pattern estimation, block index).  MINF_ROUND_NONE: fp32
@@ -182,7 +183,21 @@ typedef struct minf_qkvo {
      * sums in a second small kernel.  NULL or too small: every walk is made by one workgroup. */
     void *workspace;
     size_t workspace_bytes;
+    /* With dtype MINF_16BIT_SELECT: device word that holds MINF_BF16 or MINF_F16, what q, k, v and o
+     * are (minf_narrow_qkv writes it); read by the kernels, never by the host. */
+    const int32_t *dtype_select;
 } minf_qkvo;
+
+/*
+ * fp32 q, k, v (t->q/k/v with their strides in elements, rows of dim_in values, multiples of 4, 16-byte aligned)
+ * to contiguous 16-bit tensors [batch, heads, n, t->head_dim], zero-padded from dim_in to t->head_dim: fp16
+ * when the largest |value| of all three lies in [2^-10, 32768], else bf16.  workspace: MINF_NARROW_WORKSPACE_INTS
+ * ints; workspace[0] becomes the dtype code (minf_qkvo.dtype_select).
+ * minf_widen_out: 16-bit rows of dim_in values -> fp32 rows of their first dim, both contiguous.
+ */
+#define MINF_NARROW_WORKSPACE_INTS 769
+int minf_narrow_qkv(const minf_qkvo *t, int dim_in, void *q16, void *k16, void *v16, int32_t *workspace, void *stream);
+int minf_widen_out(const void *o16, float *out, int64_t rows, int dim, int dim_in, const int32_t *dtype_code, void *stream);
 
 /*
  * Bytes of minf_qkvo.workspace that an attention launch of this problem uses (0: it is not split).

@@ -28,6 +28,8 @@ SIGNATURES = {
     "minf_vs_index_build_ws": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
     "minf_vs_index_build_static": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr]),
     "minf_index_sort_pair": (c_int, [c_ptr, c_int, c_int, c_ptr] * 2 + [c_int, c_ptr]),
+    "minf_narrow_qkv": (c_int, [c_ptr, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),
+    "minf_widen_out": (c_int, [c_ptr, c_ptr, c_i64, c_int, c_int, c_ptr, c_ptr]),
     "minf_vs_attn_fwd": (c_int, [c_ptr] * 5 + [c_int] * 3 + [c_ptr]),
     "minf_bs_attn_fwd": (c_int, [c_ptr, c_ptr, c_int, c_int, c_ptr]),
     "minf_ashape_attn_fwd": (c_int, [c_ptr, c_int, c_int, c_ptr]),
@@ -74,10 +76,12 @@ class QKVO(ctypes.Structure):
         ("index_heads", c_int),
         ("workspace", c_ptr),
         ("workspace_bytes", ctypes.c_size_t),
+        ("dtype_select", c_ptr),
     ]
 
 
-MINF_BF16, MINF_F16, MINF_F32 = 0, 1, 2
+MINF_BF16, MINF_F16, MINF_F32, MINF_16BIT_SELECT = 0, 1, 2, 3
+MINF_NARROW_WORKSPACE_INTS = 769
 MINF_OP_VERTICAL_SLASH, MINF_OP_BLOCK_SPARSE, MINF_OP_ASHAPE, MINF_OP_DENSE = 0, 1, 2, 3
 MINF_INDEX_SORT_MAX = 16384
 MINF_ROUND_NONE, MINF_ROUND_INPUT_DTYPE = 0, 1

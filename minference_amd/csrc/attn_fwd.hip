@@ -120,6 +120,8 @@ struct AttnParams {
     // one segment of the walk each, which leave their share of the sums in `part`
     int split_first, nseg, seg_len;
     char *part;
+    int dtype;               // MINF_BF16, MINF_F16 or MINF_16BIT_SELECT
+    const int *select;       // not null: this launch is one of two, and only the one for dtype *select does anything
 };
 
 // Split walks.  A launch whose row-block pairs cannot fill the chip, or whose longest walks would outlast
@@ -1057,9 +1059,11 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
 
 // (head_dim 256: O^T, Q and the V^T fragments of a wave need more than 256 registers, so that form
 // runs one wave per SIMD with the accumulators in the second half of the register file)
+template <typename T> constexpr int dtype_code() { return std::is_same<T, __bf16>::value ? MINF_BF16 : MINF_F16; }
 template <typename T, int MODE, int HD, bool CUT>
 __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kernel(const AttnParams p) {
     typedef AttnLds<MODE, HD> L;
+    if (p.select && *as_const(p.select) != dtype_code<T>()) return;
     __shared__ __attribute__((aligned(16))) char lds_k[L::NK];
     __shared__ __attribute__((aligned(16))) char lds_v[L::NK];
     __shared__ int vs_only[L::NONLY];        // paired list walks: [row block][entries the other list lacks]
@@ -1083,10 +1087,11 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
 // order.  The weights are exp2(m_s - M) with M the largest m_s + log2(l_s), so that no product leaves the
 // fp32 range whatever a segment's (lazily raised) maximum was.  Latency-bound and small: it reads what the
 // segments wrote (66 KB each at head_dim 128, from L2) and writes the rows once.
-template <typename T, int HD>
+template <int HD>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     constexpr int NDB = HD / 32, ROW_BYTES = HD * 2, NCH = ROW_BYTES / 16;
     __shared__ __attribute__((aligned(16))) char lds_o[32 * ROW_BYTES];
+    const bool to_bf16 = (p.select ? *as_const(p.select) : p.dtype) == MINF_BF16;
     const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
     const int l32 = lane & 31, g = lane >> 5;
     const int heads = p.head_list ? p.index_heads : p.hq;
@@ -1142,10 +1147,13 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
         if (db < NDB)
 #pragma unroll
             for (int rq = 0; rq < 4; ++rq) {
-                union { T e[4]; u32x2_t u; } out4;
+                union { __bf16 b[4]; _Float16 h[4]; u32x2_t u; } out4;
                 const float x[4] = {acc[i][rq].x, acc[i][rq].y, acc[i][rq].z, acc[i][rq].w};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) out4.e[e] = live ? (T)(x[e] * inv) : (T)0.f;
+                for (int e = 0; e < 4; ++e) {
+                    const float y = live ? x[e] * inv : 0.f;
+                    if (to_bf16) out4.b[e] = (__bf16)y; else out4.h[e] = (_Float16)y;
+                }
                 *reinterpret_cast<u32x2_t *>(lds_o + l32 * ROW_BYTES + (32 * db + 8 * rq + 4 * g) * 2) = out4.u;
             }
     }
@@ -1167,7 +1175,8 @@ int check_tensors(const minf_qkvo *t, bool allow_256 = false) {
     if (t->heads_q % t->heads_kv != 0) return MINF_ERR_INVALID_ARG;
     if (t->head_list && t->index_heads <= 0) return MINF_ERR_INVALID_ARG;
     if (t->head_dim != 128 && t->head_dim != 64 && !(allow_256 && t->head_dim == 256)) return MINF_ERR_UNSUPPORTED;
-    if (t->dtype != MINF_BF16 && t->dtype != MINF_F16) return MINF_ERR_UNSUPPORTED;
+    if (t->dtype == MINF_16BIT_SELECT) { if (!empty && !t->dtype_select) return MINF_ERR_INVALID_ARG; }
+    else if (t->dtype != MINF_BF16 && t->dtype != MINF_F16) return MINF_ERR_UNSUPPORTED;
     const void *ptrs[4] = {t->q, t->k, t->v, t->o};
     const int64_t *strides[4] = {t->q_stride, t->k_stride, t->v_stride, t->o_stride};
     for (int i = 0; i < 4; ++i) {
@@ -1203,6 +1212,8 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.stripes = 1;
     p.descending = 0;
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
+    p.dtype = t->dtype;
+    p.select = t->dtype == MINF_16BIT_SELECT ? t->dtype_select : nullptr;
 }
 
 // Which walks to split, and how.  `slots` workgroups fit the chip at once, a slot's share of the launch is
@@ -1324,14 +1335,13 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
         if (p.nseg > 1) hipLaunchKernelGGL((attn_fwd_kernel<T, MODE, HD, true>), dim3((unsigned)grid), block, 0, st, p); \
         else hipLaunchKernelGGL((attn_fwd_kernel<T, MODE, HD, false>), dim3((unsigned)grid), block, 0, st, p);   \
     } while (0)
-    if (dtype == MINF_BF16) MINF_LAUNCH_ATTN(__bf16);
-    else MINF_LAUNCH_ATTN(_Float16);
+    if (dtype != MINF_F16) MINF_LAUNCH_ATTN(__bf16);
+    if (dtype != MINF_BF16) MINF_LAUNCH_ATTN(_Float16);
 #undef MINF_LAUNCH_ATTN
     const int status = minf_launch_status();
     if (status != MINF_OK || p.nseg == 1) return status;
     const unsigned merge_wgs = (unsigned)(4ll * split_pairs * p.batch * (p.head_list ? p.index_heads : p.hq));
-    if (dtype == MINF_BF16) hipLaunchKernelGGL((attn_merge_kernel<__bf16, HD>), dim3(merge_wgs), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((attn_merge_kernel<_Float16, HD>), dim3(merge_wgs), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((attn_merge_kernel<HD>), dim3(merge_wgs), dim3(256), 0, st, p);
     return minf_launch_status();
 }
 

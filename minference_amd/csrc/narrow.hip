@@ -1,0 +1,164 @@
+// fp32 tensors on 16-bit matrix operands, without a host read in between.
+//
+// The attention kernels compute on 16-bit operands with fp32 accumulation (the reference picks fp16 operands for
+// every input that is not bf16, pit_sparse_flash_attention_v2.py:175).  fp32 q/k/v become fp16 when the
+// largest |value| of the three lies in [2^-10, 32768], else bf16 (fp16 would overflow, or flush most of
+// the tensor).  The choice is made here, on the device: a first kernel leaves the largest |value| of each
+// of its workgroups, every workgroup of the second one folds those, converts its share and one of them
+// leaves the dtype code that the attention launches and the widening kernel read
+// (minf_qkvo.dtype_select).  Bound by bytes: q, k and v are read twice (the second time mostly from the
+// Infinity Cache) and written once at half the size.  With the choice read back by the host (three
+// reductions, a synchronisation, three conversions) the GPU idled about 60 us per call.
+#include "minf_common.h"
+
+namespace {
+
+constexpr int NARROW_THREADS = 256;
+constexpr int NARROW_PARTIALS = MINF_NARROW_WORKSPACE_INTS - 1;      // amax workgroups, a third per tensor
+constexpr int NARROW_WGS = NARROW_PARTIALS / 3;
+static_assert(NARROW_WGS * 3 == NARROW_PARTIALS, "the same number of workgroups for each tensor");
+
+struct NarrowTensor {
+    const float *in;
+    char *out;                   // [batch, heads, n, dim_out] 16-bit, contiguous
+    long long stride[3];         // elements: batch, head, token
+    long long rows;              // batch * heads * n
+    int heads;
+};
+struct NarrowParams {
+    NarrowTensor t[3];
+    int n, dim, dim_out;
+    int *ws;                     // [0]: the dtype code, then the partial maxima (bit patterns)
+};
+
+// (I: 32-bit numbers of vectors wherever they fit; 64-bit divisions cost more than the loads they place)
+template <typename I> __device__ __forceinline__ const float *row_ptr(const NarrowTensor &t, int n, I row) {
+    const unsigned bh = (unsigned)(row / (I)n), at = (unsigned)(row - (I)bh * (I)n);
+    return t.in + (long long)(bh / (unsigned)t.heads) * t.stride[0] + (long long)(bh % (unsigned)t.heads) * t.stride[1] + (long long)at * t.stride[2];
+}
+
+// largest bit pattern of |x| (NaN above infinity above every number) over the workgroup, in thread 0 .. 255
+__device__ __forceinline__ unsigned wg_max(unsigned m, unsigned (&part)[NARROW_THREADS / 64]) {
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, s));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NARROW_THREADS / 64; ++w) m = max(m, part[w]);
+    return m;
+}
+
+template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_amax_kernel(const NarrowParams p) {
+    __shared__ unsigned part[NARROW_THREADS / 64];
+    const NarrowTensor t = p.t[blockIdx.y];
+    const unsigned per_row = (unsigned)p.dim / 4u;
+    const I total = (I)(t.rows * per_row);
+    unsigned m = 0;
+    for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += (I)NARROW_WGS * NARROW_THREADS) {
+        const I row = i / per_row;
+        const uint4 x = *reinterpret_cast<const uint4 *>(row_ptr<I>(t, p.n, row) + 4 * (int)(i - row * per_row));
+        m = max(max(max(m, x.x & 0x7fffffffu), x.y & 0x7fffffffu), max(x.z & 0x7fffffffu, x.w & 0x7fffffffu));
+    }
+    m = wg_max(m, part);
+    if (threadIdx.x == 0) p.ws[1 + blockIdx.y * NARROW_WGS + blockIdx.x] = (int)m;
+}
+
+template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_kernel(const NarrowParams p) {
+    __shared__ unsigned part[NARROW_THREADS / 64];
+    unsigned m = 0;
+    for (int i = (int)threadIdx.x; i < NARROW_PARTIALS; i += NARROW_THREADS) m = max(m, (unsigned)p.ws[1 + i]);
+    m = wg_max(m, part);
+    const bool f16 = m >= __float_as_uint(0x1p-10f) && m <= __float_as_uint(32768.0f);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.ws[0] = f16 ? MINF_F16 : MINF_BF16;
+    const NarrowTensor t = p.t[blockIdx.y];
+    const unsigned per_row = (unsigned)p.dim_out / 8u;                   // 8 output elements per thread and step
+    const I total = (I)(t.rows * per_row);
+    for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += (I)gridDim.x * NARROW_THREADS) {
+        const I row = i / per_row;
+        const int d = 8 * (int)(i - row * per_row);
+        const float *src = row_ptr<I>(t, p.n, row) + d;
+        float4 x[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) x[h] = d + 4 * h < p.dim ? *reinterpret_cast<const float4 *>(src + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float v[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
+        union { _Float16 h[8]; __bf16 b[8]; uint4 u; } o;
+        if (f16) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o.h[e] = (_Float16)v[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o.b[e] = (__bf16)v[e];
+        }
+        *reinterpret_cast<uint4 *>(t.out + (long long)i * 16) = o.u;
+    }
+}
+
+__global__ __launch_bounds__(NARROW_THREADS) void widen_kernel(const char *__restrict__ in, float *__restrict__ out, long long rows,
+                                                              int dim, int dim_in, const int *__restrict__ code) {
+    const bool f16 = *code == MINF_F16;
+    const unsigned per_row = (unsigned)dim / 4u;
+    const long long total = rows * per_row;
+    for (long long i = (long long)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += (long long)gridDim.x * NARROW_THREADS) {
+        const long long row = i / per_row;
+        const int d = 4 * (int)(i - row * per_row);
+        union { _Float16 h[4]; __bf16 b[4]; uint2 u; } x;
+        x.u = *reinterpret_cast<const uint2 *>(in + (row * dim_in + d) * 2);
+        float4 o;
+        if (f16) o = make_float4((float)x.h[0], (float)x.h[1], (float)x.h[2], (float)x.h[3]);
+        else o = make_float4((float)x.b[0], (float)x.b[1], (float)x.b[2], (float)x.b[3]);
+        *reinterpret_cast<float4 *>(out + i * 4) = o;
+    }
+}
+
+unsigned narrow_grid(long long vectors) {
+    const long long wgs = (vectors + 4 * NARROW_THREADS - 1) / (4 * NARROW_THREADS);
+    return (unsigned)(wgs < 1 ? 1 : (wgs > 2048 ? 2048 : wgs));
+}
+
+}  // namespace
+
+extern "C" int minf_narrow_qkv(const minf_qkvo *t, int dim_in, void *q16, void *k16, void *v16, int32_t *workspace, void *stream) {
+    if (!t || !t->q || !t->k || !t->v || !q16 || !k16 || !v16 || !workspace) return MINF_ERR_INVALID_ARG;
+    if (t->batch <= 0 || t->heads_q <= 0 || t->heads_kv <= 0 || t->n <= 0 || dim_in <= 0 || t->head_dim < dim_in) return MINF_ERR_INVALID_ARG;
+    if ((dim_in & 3) || (t->head_dim & 7)) return MINF_ERR_ALIGNMENT;
+    if ((long long)t->batch * t->heads_q > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
+    NarrowParams p;
+    const void *in[3] = {t->q, t->k, t->v};
+    void *out[3] = {q16, k16, v16};
+    const int64_t *strides[3] = {t->q_stride, t->k_stride, t->v_stride};
+    for (int i = 0; i < 3; ++i) {
+        if ((((uintptr_t)in[i]) | ((uintptr_t)out[i])) & 15) return MINF_ERR_ALIGNMENT;
+        for (int j = 0; j < 3; ++j) {
+            if (strides[i][j] < 0 || (strides[i][j] & 3)) return MINF_ERR_ALIGNMENT;
+            p.t[i].stride[j] = strides[i][j];
+        }
+        p.t[i].in = (const float *)in[i];
+        p.t[i].out = (char *)out[i];
+        p.t[i].heads = i == 0 ? t->heads_q : t->heads_kv;
+        p.t[i].rows = (long long)t->batch * p.t[i].heads * t->n;
+    }
+    p.n = t->n; p.dim = dim_in; p.dim_out = t->head_dim;
+    p.ws = workspace;
+    hipStream_t st = (hipStream_t)stream;
+    // (a margin below 2^32 for the last step past the end)
+    const long long most = p.t[0].rows > p.t[1].rows ? p.t[0].rows : p.t[1].rows;
+    const bool small = most * (dim_in / 4 > p.dim_out / 8 ? dim_in / 4 : p.dim_out / 8) < 0xf0000000LL;
+    if (small) hipLaunchKernelGGL(narrow_amax_kernel<unsigned>, dim3(NARROW_WGS, 3), dim3(NARROW_THREADS), 0, st, p);
+    else hipLaunchKernelGGL(narrow_amax_kernel<unsigned long long>, dim3(NARROW_WGS, 3), dim3(NARROW_THREADS), 0, st, p);
+    const int status = minf_launch_status();
+    if (status != MINF_OK) return status;
+    const dim3 grid(narrow_grid(p.t[0].rows * (p.dim_out / 8)), 3);
+    if (small) hipLaunchKernelGGL(narrow_kernel<unsigned>, grid, dim3(NARROW_THREADS), 0, st, p);
+    else hipLaunchKernelGGL(narrow_kernel<unsigned long long>, grid, dim3(NARROW_THREADS), 0, st, p);
+    return minf_launch_status();
+}
+
+extern "C" int minf_widen_out(const void *o16, float *out, int64_t rows, int dim, int dim_in, const int32_t *dtype_code, void *stream) {
+    if (rows < 0 || dim <= 0 || dim_in < dim) return MINF_ERR_INVALID_ARG;
+    if (rows == 0) return MINF_OK;
+    if (!o16 || !out || !dtype_code) return MINF_ERR_INVALID_ARG;
+    if ((dim & 3) || (dim_in & 3) || ((uintptr_t)o16 & 15) || ((uintptr_t)out & 15)) return MINF_ERR_ALIGNMENT;
+    hipLaunchKernelGGL(widen_kernel, dim3(narrow_grid(rows * (dim / 4))), dim3(NARROW_THREADS), 0, (hipStream_t)stream,
+                       (const char *)o16, out, (long long)rows, dim, dim_in, dtype_code);
+    return minf_launch_status();
+}

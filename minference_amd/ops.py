@@ -72,11 +72,19 @@ class _Call:
     """Holds the (possibly cast/padded) tensors of one operator call and the
     filled ``minf_qkvo`` struct."""
 
-    def __init__(self, q, k, v, seqlens=None, need_out=True, native_dims=_NATIVE_D, sm_scale=None, out=None):
+    def __init__(self, q, k, v, seqlens=None, need_out=True, native_dims=_NATIVE_D, sm_scale=None, out=None,
+                 attention_only=False):
         _check_qkv(q, k, v)
         self.out_dtype = q.dtype
         self.head_dim = q.shape[-1]
-        if q.dtype == torch.float32:
+        # fp32 tensors of a call that only makes attention launches: narrowed by a kernel that leaves the
+        # choice of operand dtype on the device (no host read)
+        self.select = None
+        select = attention_only and q.dtype == torch.float32 and q.shape[-1] % 4 == 0 and q.numel() and k.numel() \
+            and q.device == k.device == v.device
+        if select:
+            pass
+        elif q.dtype == torch.float32:
             # the tile engine computes on 16-bit operands with fp32 accumulation
             q, k, v = _narrow_fp32(q, k, v)
         elif q.dtype not in (torch.bfloat16, torch.float16):
@@ -90,7 +98,9 @@ class _Call:
         # the reference runs head_dim 16, 32, 64, 128 (pit_sparse_flash_attention_v2.py:172); here 64 and
         # 128 (and 256 for the streaming operators) are native, anything else is zero-padded to the next
         Dk = min(d for d in native_dims if d >= D)
-        if D < Dk:
+        if select:
+            q, k, v = self._narrow(q, k, v, Dk)
+        elif D < Dk:
             # zero columns change neither q.k nor the first D output columns
             pad = Dk - D
             q = torch.nn.functional.pad(q, [0, pad])
@@ -116,10 +126,32 @@ class _Call:
         s.batch, s.heads_q, s.heads_kv, s.n = B, H, self.Hk, N
         s.head_dim = Dk
         s.dtype = _lib.MINF_BF16 if self.q.dtype == torch.bfloat16 else _lib.MINF_F16
+        if self.select is not None:
+            s.dtype, s.dtype_select = _lib.MINF_16BIT_SELECT, self.select.data_ptr()
         self.seqlens = seqlens
         s.seqlens = seqlens.data_ptr() if seqlens is not None else None
         s.sm_scale = float(self.head_dim) ** -0.5 if sm_scale is None else float(sm_scale)
         self.struct = s
+
+    def _narrow(self, q, k, v, Dk):
+        """The operands of fp32 q, k, v (see _narrow_fp32), zero-padded to head_dim Dk; which of the two 16-bit
+        formats they hold is known to the device only (``self.select``)."""
+        def rows(t):       # whole 16-byte vectors of unit-stride rows
+            bad = t.stride(-1) != 1 or any(s % 4 or s < 0 for s in t.stride()[:-1]) or t.data_ptr() % 16
+            return t.clone(memory_format=torch.contiguous_format) if bad else t
+        q, k, v = rows(q), rows(k), rows(v)
+        s = _lib.QKVO()
+        s.q, s.k, s.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
+        s.q_stride[:], s.k_stride[:], s.v_stride[:] = q.stride()[:3], k.stride()[:3], v.stride()[:3]
+        s.batch, s.heads_q, s.heads_kv, s.n, s.head_dim = q.shape[0], q.shape[1], k.shape[1], q.shape[2], Dk
+        dev = q.device
+        narrowed = [torch.empty(t.shape[:3] + (Dk,), dtype=torch.float16, device=dev) for t in (q, k, v)]
+        self.select = torch.empty(_lib.MINF_NARROW_WORKSPACE_INTS, dtype=torch.int32, device=dev)
+        with torch.cuda.device(dev):
+            st = _lib.load().minf_narrow_qkv(ctypes.byref(s), q.shape[-1], *(t.data_ptr() for t in narrowed),
+                                             self.select.data_ptr(), _lib.stream_ptr(dev))
+        _lib.check(st, "minf_narrow_qkv")
+        return narrowed
 
     @property
     def ref(self):
@@ -144,6 +176,17 @@ class _Call:
 
     def result(self):
         o = self.o
+        if self.select is not None:
+            # (always contiguous: an fp32 call never writes its 16-bit result into the caller's buffer)
+            wide = self.out
+            if wide is None or wide.dtype != torch.float32 or not wide.is_contiguous() or wide.data_ptr() % 16 \
+                    or wide.shape != o.shape[:3] + (self.head_dim,) or wide.device != o.device or wide.requires_grad:
+                wide = torch.empty(o.shape[:3] + (self.head_dim,), dtype=torch.float32, device=o.device)
+            with torch.cuda.device(o.device):
+                st = _lib.load().minf_widen_out(o.data_ptr(), wide.data_ptr(), self.B * self.H * self.N, self.head_dim,
+                                                self.kernel_dim, self.select.data_ptr(), _lib.stream_ptr(o.device))
+            _lib.check(st, "minf_widen_out")
+            return wide if self.out is None or wide is self.out else self.out.copy_(wide)
         if self.head_dim != self.kernel_dim:
             o = o[..., : self.head_dim]
         if self.out is not None:
@@ -157,7 +200,7 @@ def vertical_slash_attention_from_index(query, key, value, block_count, block_of
                                         column_count, column_index, seqlens=None, out=None):
     """Mixed block + column sparse attention over prebuilt index tensors
     (counterpart of _triton_mixed_sparse_attention, pit_sparse_flash_attention_v2.py:156-192)."""
-    c = _Call(query, key, value, seqlens, out=out)
+    c = _Call(query, key, value, seqlens, out=out, attention_only=True)
     rows = (c.N + 63) // 64
     for t in (block_count, block_offset, column_count, column_index):
         if t.dtype != torch.int32 or not t.is_contiguous():
@@ -215,7 +258,7 @@ def vertical_slash_sparse_attention(query, key, value, v_idx, s_idx, block_size_
 def block_sparse_attention_from_index(query, key, value, block_index, out=None):
     """Block-sparse attention over a prebuilt [batch, heads, rows, max_blocks] int32 block
     list (counterpart of _triton_block_sparse_attention, block_sparse_flash_attention.py:115-148)."""
-    c = _Call(query, key, value, out=out)
+    c = _Call(query, key, value, out=out, attention_only=True)
     if block_index.dtype != torch.int32 or not block_index.is_contiguous() or block_index.dim() != 4:
         raise ValueError("block_index must be a contiguous int32 [batch, heads, rows, max_blocks] tensor")
     if block_index.shape[0] != c.B or block_index.shape[1] != c.H or block_index.shape[2] < (c.N + 63) // 64:
@@ -286,7 +329,8 @@ def streaming_forward(q, k, v, n_init: int, n_local: int, out=None):
     """A-shape attention: n_init sink tokens + a sliding window of n_local
     (streaming_kernel.py:611-646), in one pass.  head_dim up to 256 like the reference (:429); the
     scale follows the reference's padded head_dim (see _streaming_scale)."""
-    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, sm_scale=_streaming_scale(q.shape[-1]), out=out)
+    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, sm_scale=_streaming_scale(q.shape[-1]), out=out,
+              attention_only=True)
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
         c.scratch(_lib.MINF_OP_ASHAPE, n_init, n_local)
@@ -300,7 +344,7 @@ def tri_shape_forward(q, k, v, n_init: int, n_local: int, n_last: int = 100):
     n_last query rows, dense causal attention for those (streaming_kernel.py:820-833,
     minference_forward.py:444-455), in one launch.  Like the reference, the A-shape rows are scaled
     by the padded head_dim (see _streaming_scale) and the last rows by head_dim^-0.5 (:826)."""
-    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, sm_scale=_streaming_scale(q.shape[-1]))
+    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, sm_scale=_streaming_scale(q.shape[-1]), attention_only=True)
     n_last = min(int(n_last), c.N - 1)                   # reference: min(n_last, q.size(2) - 1)
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
@@ -313,7 +357,7 @@ def tri_shape_forward(q, k, v, n_init: int, n_local: int, n_last: int = 100):
 
 def dense_causal_attention(q, k, v, out=None):
     """Dense causal attention on the same tile engine (comparator for speed-up figures)."""
-    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, out=out)
+    c = _Call(q, k, v, native_dims=_NATIVE_D_STREAMING, out=out, attention_only=True)
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
         c.scratch(_lib.MINF_OP_DENSE)

@@ -1,0 +1,78 @@
+"""fp32 tensors narrowed on the device: the same bits as the caller's own conversion to the 16-bit format the rule
+names (fp16 when the largest |value| of q, k and v lies in [2^-10, 32768], else bf16), for padded head dims,
+strided and unaligned tensors and an output buffer; outputs compared with torch.equal (one kernel, one plan)."""
+import pytest
+import torch
+
+from tests import gen
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(dev, n, hq, hk, d, scale=1.0):
+    q, k, v = gen.qkv(2, hq, hk, n, d, seed=n + d, dtype=torch.float32, scale=scale)
+    return q.to(dev), k.to(dev), v.to(dev)
+
+
+@pytest.mark.parametrize("n,hq,hk,d", [(1, 1, 1, 64), (65, 2, 1, 128), (700, 4, 2, 96), (130, 3, 3, 20), (517, 2, 2, 256), (300, 2, 1, 66)])
+@pytest.mark.parametrize("amax,dtype", [(None, torch.float16), (32768.0, torch.float16), (32769.0, torch.bfloat16), (1e30, torch.bfloat16), ("tiny", torch.bfloat16)])
+def test_same_bits_as_the_callers_conversion(gpu, n, hq, hk, d, amax, dtype):
+    import minference_amd as M
+    q, k, v = _inputs(gpu, n, hq, hk, d)
+    if amax == "tiny":
+        q, k, v = (t * 2.0 ** -14 / 4 for t in (q, k, v))
+    elif amax is not None:
+        v[1, hk - 1, n - 1, d - 1] = -amax
+    got = M.dense_causal_attention(q, k, v)
+    want = M.dense_causal_attention(q.to(dtype), k.to(dtype), v.to(dtype)).float()
+    assert got.dtype == torch.float32 and got.shape == q.shape and torch.equal(got, want)
+    got = M.streaming_forward(q, k, v, 16, 100)
+    assert torch.equal(got, M.streaming_forward(q.to(dtype), k.to(dtype), v.to(dtype), 16, 100).float())
+
+
+def test_strided_unaligned_and_caller_owned_tensors(gpu):
+    import minference_amd as M
+    q, k, v = _inputs(gpu, 400, 4, 2, 128)
+    want = M.dense_causal_attention(q.half(), k.half(), v.half()).float()
+    t = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in (q, k, v)]
+    assert torch.equal(M.dense_causal_attention(*t), want)
+    flat = torch.empty(q.numel() + 1, device=gpu)
+    shifted = flat[1:].view(q.shape)
+    shifted.copy_(q)
+    assert torch.equal(M.dense_causal_attention(shifted, k, v), want)
+    for out in (torch.empty_like(q), torch.empty_like(t[0]), torch.empty_like(q, dtype=torch.float16)):
+        assert M.dense_causal_attention(q, k, v, out) is out and torch.equal(out.float(), want)
+    assert torch.equal(M.dense_causal_attention(q, k[:, :1].expand(2, 2, 400, 128), v),
+                       M.dense_causal_attention(q.half(), k[:, :1].expand(2, 2, 400, 128).half(), v.half()).float())
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_values_that_are_no_numbers_choose_bf16(gpu, bad):
+    import minference_amd as M
+    q, k, v = _inputs(gpu, 100, 1, 1, 64)
+    v[0, 0, 99, 3] = bad
+    got = M.dense_causal_attention(q, k, v)
+    want = M.dense_causal_attention(q.bfloat16(), k.bfloat16(), v.bfloat16()).float()
+    assert torch.equal(got[1], want[1]) and torch.equal(got[0, 0, :64], want[0, 0, :64])
+
+
+def test_a_call_on_fp32_tensors_does_not_wait_for_the_gpu(gpu):
+    """Recorded into a graph (a host read would end the capture) and replayed on inputs of the other format."""
+    import minference_amd as M
+    q, k, v = _inputs(gpu, 600, 4, 2, 128)
+    vi = torch.arange(0, 40, device=gpu).expand(2, 4, 40).contiguous()
+    si = torch.arange(0, 150, device=gpu).expand(2, 4, 150).contiguous()
+    f = lambda: M.vertical_slash_sparse_attention(q, k, v, vi, si)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        f()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = f()
+    for scale in (1.0, 1e6, 1.0, 3.0):
+        v.mul_(scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, f()), scale
