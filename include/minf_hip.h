@@ -103,6 +103,11 @@ int minf_vs_index_build_ws(const int32_t *seqlens, const int32_t *vertical_idx,
                            int32_t *column_index, int batch, int heads, int rows,
                            int nnz_v, int nnz_s, int zero_fill, int32_t *error_flag,
                            void *workspace, size_t workspace_bytes, void *stream);
+/* The same where every sequence fills the context (rows row blocks are live): no seqlens. */
+int minf_vs_index_build_full_ws(const int32_t *vertical_idx, const int32_t *slash_idx, int32_t *block_count,
+                                int32_t *block_offset, int32_t *column_count, int32_t *column_index, int batch,
+                                int heads, int rows, int nnz_v, int nnz_s, int zero_fill, int32_t *error_flag,
+                                void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * minf_vs_index_build_ws without a workspace argument and without any allocation: the tables and

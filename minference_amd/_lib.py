@@ -26,6 +26,7 @@ SIGNATURES = {
     "minf_vs_index_build": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr]),
     "minf_vs_index_workspace_bytes": (ctypes.c_size_t, [c_int] * 4),
     "minf_vs_index_build_ws": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
+    "minf_vs_index_build_full_ws": (c_int, [c_ptr] * 6 + [c_int] * 6 + [c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
     "minf_vs_index_build_static": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr]),
     "minf_index_sort_pair": (c_int, [c_ptr, c_int, c_int, c_ptr] * 2 + [c_int, c_ptr]),
     "minf_narrow_qkv": (c_int, [c_ptr, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(IDX_WAVES *MINF_WAVE) void vs_index_kernel(
     const int32_t *vert = vertical + bh * (long long)nnz_v;
     const int32_t *sl = slash + bh * (long long)nnz_s;
 
-    const int seqlen = seqlens[b];
+    const int seqlen = seqlens ? seqlens[b] : INT_MAX;
     const int start_m = m * 64;
     const int end_m = start_m + 64;
 
@@ -220,11 +220,9 @@ __global__ __launch_bounds__(IDX_WAVES *MINF_WAVE) void vs_index_kernel(
         }
     }
 
-    if (zero_fill || live) {
-        if (lane == 0) {
-            block_count[ro] = nb;
-            column_count[ro] = ncol;
-        }
+    if (lane == 0) {                 // (rows past the sequence and rows without an entry: zero)
+        block_count[ro] = nb;
+        column_count[ro] = ncol;
     }
     if (zero_fill) {
         zero_range(bo_row, nb, nnz_s, lane);
@@ -504,7 +502,7 @@ __global__ __launch_bounds__(IDX_WAVES *MINF_WAVE, ZERO_FILL ? 8 : 1) void vs_in
     const int32_t *run_a = crun + nnz_s, *run_e = run_a + nnz_s, *cgaps = run_e + nnz_s, *glist = cgaps + nnz_s;
     const uint32_t *bm = reinterpret_cast<const uint32_t *>(glist + nnz_s);
 
-    const int seqlen = seqlens[b];
+    const int seqlen = seqlens ? seqlens[b] : INT_MAX;
     const int start_m = m * 64;
     const int end_m = start_m + 64;
     const uint64_t lt = minf_lanemask_lt();
@@ -711,11 +709,9 @@ __global__ __launch_bounds__(IDX_WAVES *MINF_WAVE, ZERO_FILL ? 8 : 1) void vs_in
         }
     }
 
-    if (zero_fill || live) {
-        if (lane == 0) {
-            block_count[ro] = nb;
-            column_count[ro] = ncol;
-        }
+    if (lane == 0) {                 // (rows past the sequence and rows without an entry: zero)
+        block_count[ro] = nb;
+        column_count[ro] = ncol;
     }
     if (zero_fill) {
         zero_range(bo_row, nb, nnz_s, lane);
@@ -785,13 +781,12 @@ static int index_build_tables(const int32_t *seqlens, const int32_t *vertical_id
     return minf_launch_status();
 }
 
-extern "C" int minf_vs_index_build_ws(const int32_t *seqlens, const int32_t *vertical_idx,
-                                      const int32_t *slash_idx, int32_t *block_count,
-                                      int32_t *block_offset, int32_t *column_count,
-                                      int32_t *column_index, int batch, int heads, int rows,
-                                      int nnz_v, int nnz_s, int zero_fill, int32_t *error_flag,
-                                      void *workspace, size_t workspace_bytes, void *stream) {
-    if (!seqlens || !vertical_idx || !slash_idx || !block_count || !block_offset ||
+// (seqlens NULL: every sequence fills the context)
+static int index_build_ws(const int32_t *seqlens, const int32_t *vertical_idx, const int32_t *slash_idx, int32_t *block_count,
+                          int32_t *block_offset, int32_t *column_count, int32_t *column_index, int batch, int heads, int rows,
+                          int nnz_v, int nnz_s, int zero_fill, int32_t *error_flag,
+                          void *workspace, size_t workspace_bytes, void *stream) {
+    if (!vertical_idx || !slash_idx || !block_count || !block_offset ||
         !column_count || !column_index)
         return MINF_ERR_INVALID_ARG;
     if (batch < 0 || heads < 0 || rows < 0 || nnz_v < 1 || nnz_s < 1) return MINF_ERR_INVALID_ARG;
@@ -803,6 +798,25 @@ extern "C" int minf_vs_index_build_ws(const int32_t *seqlens, const int32_t *ver
     return index_build_tables(seqlens, vertical_idx, slash_idx, block_count, block_offset, column_count,
                               column_index, batch, heads, rows, nnz_v, nnz_s, zero_fill, error_flag,
                               (int32_t *)workspace, total, (hipStream_t)stream);
+}
+
+extern "C" int minf_vs_index_build_ws(const int32_t *seqlens, const int32_t *vertical_idx,
+                                      const int32_t *slash_idx, int32_t *block_count,
+                                      int32_t *block_offset, int32_t *column_count,
+                                      int32_t *column_index, int batch, int heads, int rows,
+                                      int nnz_v, int nnz_s, int zero_fill, int32_t *error_flag,
+                                      void *workspace, size_t workspace_bytes, void *stream) {
+    if (!seqlens) return MINF_ERR_INVALID_ARG;
+    return index_build_ws(seqlens, vertical_idx, slash_idx, block_count, block_offset, column_count, column_index, batch, heads,
+                          rows, nnz_v, nnz_s, zero_fill, error_flag, workspace, workspace_bytes, stream);
+}
+
+extern "C" int minf_vs_index_build_full_ws(const int32_t *vertical_idx, const int32_t *slash_idx, int32_t *block_count,
+                                           int32_t *block_offset, int32_t *column_count, int32_t *column_index, int batch,
+                                           int heads, int rows, int nnz_v, int nnz_s, int zero_fill, int32_t *error_flag,
+                                           void *workspace, size_t workspace_bytes, void *stream) {
+    return index_build_ws(nullptr, vertical_idx, slash_idx, block_count, block_offset, column_count, column_index, batch, heads,
+                          rows, nnz_v, nnz_s, zero_fill, error_flag, workspace, workspace_bytes, stream);
 }
 
 // ---- the entry point that allocates nothing ---------------------------------------------------

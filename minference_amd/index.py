@@ -38,12 +38,17 @@ def convert_vertical_slash_indexes(seqlens, vertical_indexes, slash_indexes, con
         raise RuntimeError("convert_vertical_slash_indexes needs GPU tensors (no CPU path)")
     if vertical_indexes.dim() != 3 or slash_indexes.dim() != 3:
         raise ValueError("vertical_indexes / slash_indexes must be [B, H, nnz]")
-    seqlens = _i32_contig(seqlens)
+    return _build(_i32_contig(seqlens), vertical_indexes, slash_indexes, context_size, zero_fill, error_flag, use_tables)
+
+
+def _build(seqlens, vertical_indexes, slash_indexes, context_size, zero_fill, error_flag=None, use_tables=True):
+    """convert_vertical_slash_indexes after its argument checks; ``seqlens`` None (tables only): every
+    sequence fills the context."""
     v = _i32_contig(vertical_indexes)
     s = _i32_contig(slash_indexes)
     B, H, S = s.shape
     V = v.shape[2]
-    if v.shape[0] != B or v.shape[1] != H or seqlens.numel() != B:
+    if v.shape[0] != B or v.shape[1] != H or (seqlens is not None and seqlens.numel() != B):
         raise ValueError("batch/head sizes of seqlens, vertical_indexes, slash_indexes differ")
     rows = (int(context_size) + 63) // 64
     dev = v.device
@@ -52,12 +57,8 @@ def convert_vertical_slash_indexes(seqlens, vertical_indexes, slash_indexes, con
     block_offset = alloc((B, H, rows, S), dtype=torch.int32, device=dev)
     column_count = alloc((B, H, rows), dtype=torch.int32, device=dev)
     column_index = alloc((B, H, rows, V), dtype=torch.int32, device=dev)
-    if not zero_fill:
-        # counts of rows past seqlen are not written by the kernel in this mode
-        block_count.zero_()
-        column_count.zero_()
     lib = _lib.load()
-    args = (seqlens.data_ptr(), v.data_ptr(), s.data_ptr(), block_count.data_ptr(),
+    args = (v.data_ptr(), s.data_ptr(), block_count.data_ptr(),
             block_offset.data_ptr(), column_count.data_ptr(), column_index.data_ptr(),
             B, H, rows, V, S, 1 if zero_fill else 0,
             error_flag.data_ptr() if error_flag is not None else None)
@@ -65,8 +66,11 @@ def convert_vertical_slash_indexes(seqlens, vertical_indexes, slash_indexes, con
         if use_tables:
             ws_bytes = lib.minf_vs_index_workspace_bytes(B, H, S, rows)
             ws = torch.empty(max(ws_bytes, 4), dtype=torch.uint8, device=dev)
-            st = lib.minf_vs_index_build_ws(*args, ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev))
+            if seqlens is None:
+                st = lib.minf_vs_index_build_full_ws(*args, ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev))
+            else:
+                st = lib.minf_vs_index_build_ws(seqlens.data_ptr(), *args, ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev))
         else:
-            st = lib.minf_vs_index_build(*args, _lib.stream_ptr(dev))
+            st = lib.minf_vs_index_build(seqlens.data_ptr(), *args, _lib.stream_ptr(dev))
     _lib.check(st, "minf_vs_index_build")
     return [block_count, block_offset, column_count, column_index]

@@ -21,7 +21,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .index import convert_vertical_slash_indexes
+from .index import _build as _build_index
 
 _NATIVE_D = (64, 128)         # head_dims every kernel is instantiated for; others are zero-padded up
 _NATIVE_D_STREAMING = (64, 128, 256)   # ... and the A-shape / tri-shape / dense kernels also for 256
@@ -249,10 +249,10 @@ def vertical_slash_sparse_attention(query, key, value, v_idx, s_idx, block_size_
     _check_qkv(query, key, value)
     B, H, N, _ = query.shape
     v_idx, s_idx = _sorted_indices(v_idx, s_idx, B, H)
-    seqlens = torch.full((B,), N, dtype=torch.int32, device=query.device)
-    bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, block_size_M,
-                                                    block_size_N, zero_fill=False)
-    return vertical_slash_attention_from_index(query, key, value, bc, bo, cc, ci, seqlens)
+    if not v_idx.is_cuda:
+        raise RuntimeError("vertical_slash_sparse_attention needs GPU tensors (no CPU path)")
+    bc, bo, cc, ci = _build_index(None, v_idx, s_idx, N, zero_fill=False)
+    return vertical_slash_attention_from_index(query, key, value, bc, bo, cc, ci)
 
 
 def block_sparse_attention_from_index(query, key, value, block_index, out=None):

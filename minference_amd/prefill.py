@@ -19,6 +19,7 @@ from collections import OrderedDict
 import torch
 
 from .estimate import estimate_vertical_slash
+from .index import _build as _build_index
 from .index import convert_vertical_slash_indexes
 from .ops import (block_sparse_attention, dense_causal_attention, streaming_forward, tri_shape_forward,
                   vertical_slash_attention_from_index, vertical_slash_sparse_attention)
@@ -29,11 +30,10 @@ DEFAULT_PATTERN = ("vertical_and_slash", 1000, 6096, 1)   # minference_forward.p
 def vertical_slash_prefill(q, k, v, vertical_size=1000, slash_size=6096, out=None):
     """estimate -> top-k -> index build -> mixed sparse attention for all heads of ``q``
     (``vertical_and_slash_kernel``, minference_forward.py:599-614)."""
-    B, H, N, _ = q.shape
+    N = q.shape[2]
     v_idx, s_idx = estimate_vertical_slash(q, k, vertical_size, slash_size)
-    seqlens = torch.full((B,), N, dtype=torch.int32, device=q.device)
-    bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, 64, 64, zero_fill=False)
-    return vertical_slash_attention_from_index(q, k, v, bc, bo, cc, ci, seqlens, out)
+    bc, bo, cc, ci = _build_index(None, v_idx, s_idx, N, zero_fill=False)
+    return vertical_slash_attention_from_index(q, k, v, bc, bo, cc, ci, out=out)
 
 
 def load_best_pattern(path):
@@ -99,6 +99,7 @@ class _LayerPlan:
                 d["vs_heads"] = _head_list([h for h, _, _ in self.vs], dev)
                 d["vs_kv"] = torch.tensor(kv * B, dtype=torch.int32).to(dev)
                 d["vs_ks"] = torch.tensor(ksl * B, dtype=torch.int32).to(dev)
+                d["seqlens"] = torch.tensor([N] * B, dtype=torch.int32).to(dev)
                 d["vs_max"] = (max(kv), max(ksl))
             if self.bs:
                 d["bs_heads"] = _head_list(self.bs, dev)
@@ -189,16 +190,14 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
                                                        slash.data_ptr(), ks_t.data_ptr(), smax, s_idx.data_ptr(), smax, N - 1, 2, 0,
                                                        B * nh, N, N, stream)
                 _lib.check(st, "minf_topk_indices_pair_ragged")
-                seqlens = torch.full((B,), N, dtype=torch.int32, device=dev)
+                seqlens = dt["seqlens"]
                 bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, 64, 64, zero_fill=False)
-                c.struct.seqlens = seqlens.data_ptr()
                 c.select_heads(slot)
                 c.scratch(_lib.MINF_OP_VERTICAL_SLASH)
                 st = lib.minf_vs_attn_fwd(c.ref, bc.data_ptr(), bo.data_ptr(), cc.data_ptr(), ci.data_ptr(), rows,
                                           smax, vmax, stream)
-                c.struct.seqlens = None
                 _lib.check(st, "minf_vs_attn_fwd")
-                keep += [vertical, slash, ws, v_idx, s_idx, seqlens, bc, bo, cc, ci]
+                keep += [vertical, slash, ws, v_idx, s_idx, bc, bo, cc, ci]
             if lp.bs:
                 nh = len(lp.bs)
                 slot = dt["bs_heads"]
@@ -226,7 +225,6 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
                     st = lib.minf_ashape_attn_fwd(c.ref, int(n_init), int(n_local), stream)
                     _lib.check(st, "minf_ashape_attn_fwd")
     finally:
-        c.struct.seqlens = None
         c.struct.sm_scale = float(D) ** -0.5
         c.select_heads(None)
     out = c.result()

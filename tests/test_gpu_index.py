@@ -214,3 +214,23 @@ def test_config3_shape_bit_exact(gpu):
         assert np.array_equal(g[:, :2], r)
     bc, bo, cc, ci = got
     assert (bc >= 1).all() and (bc <= 6096).all() and (cc <= 1000).all()
+
+
+@pytest.mark.parametrize("n,batch", [(64, 1), (1000, 2), (4097, 3)])
+def test_counts_are_written_for_every_row_and_full_sequences_need_no_lengths(gpu, n, batch):
+    """Payload-only builds into memory that holds other values: row blocks past a sequence get zero counts from
+    the kernel itself (both builders), and a build without sequence lengths equals one with full ones."""
+    from minference_amd.index import _build
+    v, s = gen.vs_index_inputs(2, n, min(n, 60), min(n, 90), seed=n, batch=batch)
+    vg, sg = torch.from_numpy(v).to(gpu), torch.from_numpy(s.copy()).to(gpu)
+    lens = torch.tensor([n, max(1, n // 2), 1][:batch], dtype=torch.int32, device=gpu)
+    full = torch.full((batch,), n, dtype=torch.int32, device=gpu)
+    junk = torch.full((4, 1 << 16), 77, dtype=torch.int32, device=gpu)
+    del junk                                                   # (the caching allocator hands it out again)
+    for seqlens in (lens, full):
+        want = convert_vertical_slash_indexes(seqlens, vg, sg, n)
+        for tables in (True, False):
+            got = convert_vertical_slash_indexes(seqlens, vg, sg, n, zero_fill=False, use_tables=tables)
+            assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2]), tables
+    got = _build(None, vg, sg, n, zero_fill=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
