@@ -94,7 +94,18 @@ template <typename T> __global__ __launch_bounds__(256) void bs_pool_kernel(cons
     }
 }
 
-constexpr int SCORE_CHUNK = 16;
+// Key tiles a workgroup scores one after the other, 64 matrix instructions of 64 cycles each: a chain that
+// nothing else on its SIMD fills when there are few workgroups.  Chunks are halved until there are SCORE_WGS of
+// them.  Whole block index, us, with 16 / 8 / 4 / 2 / 1 tiles: 32 / 8 heads 32768 tokens 181 / 154 / 140 / 138 /
+// 135, 16384 tokens 93 / 93 / 85 / 77 / 75, 100000 tokens 607 / 491 / 485 / 498 / 516; 8 / 2 heads 12000
+// tokens 40 / 40 / 34 / 28 / 25; one head 100000 tokens 97 / 69 / 55 / 52 / 47.
+constexpr int SCORE_CHUNK_MAX = 16;
+constexpr int SCORE_WGS = 5000;
+inline int score_chunk(long long groups, int ntiles) {
+    int chunk = SCORE_CHUNK_MAX;
+    while (chunk > 1 && groups * ((ntiles + chunk - 1) / chunk) < SCORE_WGS) chunk /= 2;
+    return chunk;
+}
 
 struct ScoreParams {
     const float *qp, *kp;     // pooled [batch*heads_q, rows, 128], [batch*heads_kv, rows, 128]
@@ -102,7 +113,7 @@ struct ScoreParams {
     int heads_q, heads_kv, rows, pitch, force;
     int mtiles, ntiles;
     int mquads;               // groups of four query tiles (one workgroup each per chunk)
-    int nchunks;              // chunks of SCORE_CHUNK key tiles per group
+    int chunk, nchunks;       // key tiles per chunk, chunks per group
     int skip_masked;
     const int *head_list;     // as in PoolParams; qp and scores have index_heads heads
     int index_heads;
@@ -118,7 +129,7 @@ __device__ __forceinline__ void load_operand(const float *base, int row, int row
 }
 
 // One workgroup: four query tiles (one per wave, A operand held in registers) against one chunk of
-// SCORE_CHUNK key tiles.  A key tile (32 pooled rows = 16 KB, contiguous in memory) is loaded once
+// p.chunk key tiles.  A key tile (32 pooled rows = 16 KB, contiguous in memory) is loaded once
 // per workgroup with coalesced 16-byte loads, staged in LDS (two buffers, rows padded by 16 bytes so
 // that the operand reads spread over the banks) and read from there by all four waves in MFMA
 // layout: the matrix instructions then wait for LDS, whose latency two reads in flight cover, and
@@ -130,7 +141,7 @@ __global__ __launch_bounds__(256, 3) void bs_scores_kernel(const ScoreParams p) 
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, g = lane >> 5;
     const int mq = p.mquads - 1 - (int)blockIdx.x / p.nchunks;    // heavy (late) query tiles first
-    const int nt_begin = ((int)blockIdx.x % p.nchunks) * SCORE_CHUNK;
+    const int nt_begin = ((int)blockIdx.x % p.nchunks) * p.chunk;
     const int bh = blockIdx.y;
     const int b = bh / p.index_heads, slot = bh % p.index_heads;   // (grid: batch x index_heads)
     const int h = p.head_list ? p.head_list[slot] : slot;
@@ -146,7 +157,7 @@ __global__ __launch_bounds__(256, 3) void bs_scores_kernel(const ScoreParams p) 
     // (rows of at most 4096 scores), they are neither computed nor stored; otherwise they are stored
     // without arithmetic.  The workgroup walks up to the last tile any of its waves needs.
     const int last_any = min(p.ntiles - 1, (min(4 * mq + 3, p.mtiles - 1) * 32 + 31) / 32);
-    const int nt_stop = min(nt_begin + SCORE_CHUNK, p.skip_masked ? last_any + 1 : p.ntiles);
+    const int nt_stop = min(nt_begin + p.chunk, p.skip_masked ? last_any + 1 : p.ntiles);
     if (nt_begin >= nt_stop) return;                               // (workgroup-uniform)
     const int last_mine = (m0 + 31) / 32;                          // last tile this wave computes
 
@@ -270,9 +281,10 @@ int block_index_impl(const void *q, const void *k, const int64_t *q_stride, cons
     if (status != MINF_OK) return status;
 
     const bool causal_topk = rows <= 64 * 64;      // one wave per row: reads only the stored prefix of a row
+    const int mtiles = (rows + 31) / 32, ntiles = (pitch + 31) / 32, mquads = (mtiles + 3) / 4;
+    const int chunk = score_chunk((long long)batch * index_heads * mquads, ntiles);
     ScoreParams sp{qp, kp, scores, heads_q, heads_kv, rows, pitch, force_diag_first ? 1 : 0,
-                   (rows + 31) / 32, (pitch + 31) / 32, ((rows + 31) / 32 + 3) / 4,
-                   ((pitch + 31) / 32 + SCORE_CHUNK - 1) / SCORE_CHUNK, causal_topk ? 1 : 0, head_list, index_heads,
+                   mtiles, ntiles, mquads, chunk, (ntiles + chunk - 1) / chunk, causal_topk ? 1 : 0, head_list, index_heads,
                    rounded ? dtype : -1};
     hipLaunchKernelGGL(bs_scores_kernel, dim3(sp.mquads * sp.nchunks, batch * index_heads), dim3(256), 0, st, sp);
     status = minf_launch_status();

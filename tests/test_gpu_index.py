@@ -220,7 +220,7 @@ def test_config3_shape_bit_exact(gpu):
 def test_counts_are_written_for_every_row_and_full_sequences_need_no_lengths(gpu, n, batch):
     """Payload-only builds into memory that holds other values: row blocks past a sequence get zero counts from
     the kernel itself (both builders), and a build without sequence lengths equals one with full ones."""
-    from minference_amd.index import _build
+    from minference_amd.index import _build, convert_vertical_slash_indexes
     v, s = gen.vs_index_inputs(2, n, min(n, 60), min(n, 90), seed=n, batch=batch)
     vg, sg = torch.from_numpy(v).to(gpu), torch.from_numpy(s.copy()).to(gpu)
     lens = torch.tensor([n, max(1, n // 2), 1][:batch], dtype=torch.int32, device=gpu)
