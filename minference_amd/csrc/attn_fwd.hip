@@ -1085,7 +1085,9 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
 // Folds the segments of a split pair: one workgroup per (batch, head position, pair, 32 query rows), a
 // wave per 32-column block of O^T (same lane layout as the walk's accumulators), segments in ascending
 // order.  The weights are exp2(m_s - M) with M the largest m_s + log2(l_s), so that no product leaves the
-// fp32 range whatever a segment's (lazily raised) maximum was.  Latency-bound and small: it reads what the
+// fp32 range whatever a segment's (lazily raised) maximum was.  A segment is left out only where its row sum
+// is the zero of an unused or fully masked one, by bit pattern: a NaN among the keys makes the row sum NaN,
+// and the row is to be NaN, as a whole walk leaves it.  Latency-bound and small: it reads what the
 // segments wrote (66 KB each at head_dim 128, from L2) and writes the rows once.
 template <int HD>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
@@ -1112,7 +1114,8 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     float top = -INFINITY;
     for (int s = 0; s < nseg; ++s) {
         const float2 ml = stat(s);
-        if (ml.y > 0.f) top = fmaxf(top, ml.x + __builtin_amdgcn_logf(ml.y));
+        const bool number = (__float_as_uint(ml.y) & 0x7fffffffu) <= 0x7f800000u;
+        if (__float_as_uint(ml.y) != 0 && number) top = fmaxf(top, ml.x + __builtin_amdgcn_logf(ml.y));
     }
     const bool live = row0 + l32 < seqlen;
     float l_tot = 0.f;
@@ -1123,8 +1126,9 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
         for (int rq = 0; rq < 4; ++rq) acc[i][rq] = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int s = 0; s < nseg; ++s) {
         const float2 ml = stat(s);
-        const float w = ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - top) : 0.f;
-        if (!__any(w > 0.f)) continue;                                  // an unused slot holds nothing
+        const bool used = __float_as_uint(ml.y) != 0;
+        const float w = used ? __builtin_amdgcn_exp2f(ml.x - top) : 0.f;
+        if (!__any(used)) continue;                                     // an unused slot holds nothing
         l_tot += w * ml.y;
 #pragma unroll
         for (int i = 0; i < (NDB > 4 ? 2 : 1); ++i) {

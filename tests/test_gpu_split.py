@@ -114,3 +114,20 @@ def test_striped_row_blocks_cover_every_row(gpu, hq, hk, n, b):
     for out in (M.dense_causal_attention(qg, kg, ones), M.streaming_forward(qg, kg, ones, 64, 500),
                 M.block_sparse_attention(qg, kg, ones, 20), M.vertical_slash_prefill(qg, kg, ones, 100, 300)):
         assert (out.float() - 1).abs().max().item() <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+def test_a_nan_key_reaches_every_row_that_attends_to_it(gpu, d, dtype):
+    """The row sum of a segment with a NaN score is NaN: the fold keeps it, as a whole walk's rows are NaN,
+    and rows that do not attend to the key (other segments, masked entries of its tile) stay numbers."""
+    import minference_amd as M
+    n, at, window = 1300, 600, 300
+    q, k, v = (t.to(gpu) for t in make(1, 1, 1, n, 17, dtype, d))
+    clean, bad = M.dense_causal_attention(q, k, v), k.clone()
+    bad[0, 0, at] = float("nan")
+    out = M.dense_causal_attention(q, bad, v)
+    assert torch.isnan(out[0, 0, at:]).all() and torch.isfinite(out[0, 0, :at]).all()
+    check(out[:, :, :at], clean[:, :, :at].cpu(), "rows before the key")
+    out = M.streaming_forward(q, bad, v, 64, window)
+    assert torch.isnan(out[0, 0, at:at + window]).all()
+    assert torch.isfinite(out[0, 0, :at]).all() and torch.isfinite(out[0, 0, at + window + 1:]).all()
