@@ -60,3 +60,14 @@ def test_silu_mul(gpu, dtype, n):
     gate, up = (4 * torch.randn(n, device=gpu, generator=g).to(dtype) for _ in range(2))
     want = torch.nn.functional.silu(gate) * up
     assert close(m._silu_mul(gate.clone(), up), want, dtype, 3)
+
+
+def test_silu_mul_fp32_far_from_zero(gpu):
+    """fp32 tensors, x in [-80, 80], against fp64: a few roundings (exponential, sum, quotient, product: 2^-21),
+    not the 2^-19 that rounding x log2(e) to fp32 would leave at the ends."""
+    m = model(16, torch.float32, gpu)
+    gate = torch.linspace(-80, 80, 4097, device=gpu)
+    up = torch.full_like(gate, 1.5)
+    got = m._silu_mul(gate.clone(), up).double()
+    want = torch.nn.functional.silu(gate.double()) * up.double()
+    assert ((got - want).abs() <= 2.0 ** -21 * want.abs()).all()
