@@ -97,6 +97,14 @@ __device__ __forceinline__ float sub_hi(float x, unsigned h) {
     return r;
 }
 
+// two f16 values, rounded to nearest
+__device__ __forceinline__ unsigned pack_f16(float x, float y) {
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+    const f32x2_t v = {x, y};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, h2_t));
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 struct RowState {
@@ -124,14 +132,16 @@ constexpr int DIAG_GROUPS = 8192;            // (262144 tokens; farther blocks a
 // columns, and -- by setting a candidate's whole row -- the blocks and those blocks all of whose diagonals
 // a candidate keeps (most of a window, of a run of slashes).  Only candidates with SOME of a block's
 // diagonals are added element by element (their columns left out: those are in the product already).  The
-// exponentials enter as a sum of two f16 terms (22 bits; the row's largest is scaled to 2^7 .. 2^13, so that
-// what f16 cannot hold lies 2^-31 below it), the sums are fp32.
+// exponentials enter as a sum of two f16 terms, each rounded to nearest (24 bits; the row's largest is scaled
+// to 2^8 .. 2^15, so that what f16 cannot hold lies 2^-32 below it), the sums are fp32.  Scores against fp64
+// sums, 4096 .. 16384 tokens: relative error up to 7.4e-8 (fp32 sums element by element 1.2e-7; terms rounded
+// towards zero 4.6e-7).
 // Bound by its vector instructions (70 % of the issue slots): about 115 per 32 x 32 block (fma and exp 32,
 // conversions 32, maximum 14, masks) and 40 per candidate with mixed diagonals, beside 12 MFMAs, where
 // testing a bit per element and candidate took about 550.  32 / 8 heads, 16384 tokens, the six candidates of
 // the reference: 6.50 ms -> 3.05 (products) -> 2.70 (K shared through LDS instead of fragments from global
 // memory) -> 2.45 (mixed-precision subtraction, scalar descriptors) -> 2.34 ms (dot products for mixed
-// diagonals); the score products alone take 0.44 ms at the nominal rate.
+// diagonals), 2.36 with the terms rounded to nearest; the score products alone take 0.44 ms at the nominal rate.
 template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_kernel(const RecallParams p) {
     __shared__ unsigned dtab[DIAG_GROUPS];             // bytes: OR, AND, OR without the first, AND without the first
     __shared__ float lds[4][TILE][NC + 2];
@@ -183,7 +193,7 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
     load_frag(qb, p.qs[2], rt * TILE, p.n, lane, qf[0]);
     load_frag(qb, p.qs[2], rt * TILE + 32, p.n, lane, qf[1]);
 
-    constexpr float BIAS = 7.f, LAZY = 6.f;            // exponentials reach 2^BIAS .. 2^(BIAS + LAZY) < 2^16
+    constexpr float BIAS = 9.f, LAZY = 6.f;            // exponentials reach 2^(BIAS - 1) .. 2^(BIAS + LAZY) < 2^16
     float m[2] = {-INFINITY, -INFINITY};               // running maximum of the lane's row (same in both lane halves)
     f32x16_t zacc[2];                                  // rows t = 8 (r / 4) + 4 g + r % 4: r 0..3 candidates 4 g + r, r 4 (g 0) the sum
     float zx[2][NC];                                   // this lane's share of the element-wise sums
@@ -304,8 +314,10 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
             const float cand = mx * p.scale_log2;
             const bool grow = cand > m[nb] + LAZY;                 // (raised only when it has to be)
             if (__any(grow)) {
-                const float alpha = grow ? fast_exp2(m[nb] - cand) : 1.0f;
-                m[nb] = grow ? cand : m[nb];
+                // (a whole number: BIAS - m and the rescale are exact, so that what was summed under one maximum
+                // and what is summed under the next are in proportion to the last bit)
+                const float up = ceilf(cand), alpha = grow ? fast_exp2(m[nb] - up) : 1.0f;
+                m[nb] = grow ? up : m[nb];
 #pragma unroll
                 for (int r = 0; r < 5; ++r) zacc[nb][r] *= alpha;
 #pragma unroll
@@ -330,8 +342,8 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float x = e[8 * s + 2 * i], y = e[8 * s + 2 * i + 1];
-                    hi[s].u[i] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(x, y));
-                    lo[s].u[i] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(sub_lo(x, hi[s].u[i]), sub_hi(y, hi[s].u[i])));
+                    hi[s].u[i] = pack_f16(x, y);
+                    lo[s].u[i] = pack_f16(sub_lo(x, hi[s].u[i]), sub_hi(y, hi[s].u[i]));
                 }
                 zacc[nb] = mma<_Float16>(s ? a1 : a0, hi[s], zacc[nb]);
                 zacc[nb] = mma<_Float16>(s ? a1 : a0, lo[s], zacc[nb]);
@@ -420,14 +432,14 @@ __global__ __launch_bounds__(64) void pattern_recall_finalize(const float *parti
     const int head_lin = (int)blockIdx.x, lane = (int)threadIdx.x;
     const float *src = partial + (long long)head_lin * tiles * NC;
     for (int t = 0; t < NC; ++t) {
-        float x = 0.f;
-        for (int i = lane; i < tiles; i += 64) x += src[(long long)i * NC + t];
+        double x = 0.;
+        for (int i = lane; i < tiles; i += 64) x += (double)src[(long long)i * NC + t];
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d);
         // no rows to average over -> NaN, like the mean of an empty slice in the reference
         // (written as a bit pattern: the library is built without NaN semantics, under which the constant
         // itself is undefined)
-        if (lane == 0) recall[head_lin * NC + t] = n > row_begin ? x / (float)(n - max(row_begin, 0)) : __uint_as_float(0x7fc00000u);
+        if (lane == 0) recall[head_lin * NC + t] = n > row_begin ? (float)(x / (double)(n - max(row_begin, 0))) : __uint_as_float(0x7fc00000u);
     }
 }
 

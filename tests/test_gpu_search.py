@@ -171,3 +171,21 @@ def test_recall_tiles_stripes_and_flag_mixes(gpu, n, hq, hk, begin, d):
     want = np.array(oracle_scores(q, k, cands, begin))
     assert np.abs(got - want).max() <= TOL, (got, want)
     assert np.abs(got[:, 7] - 1.0).max() <= 1e-6             # a window of all offsets keeps everything
+
+
+@pytest.mark.parametrize("n,dtype", [(1500, torch.bfloat16), (3001, torch.float16)])
+def test_recall_keeps_fp32_accuracy(gpu, n, dtype):
+    """Against fp64 sums on the same operands: exponentials of 24 bits, fp32 row sums whose roundings average
+    out over the rows, one rounding of the result (2^-24): 2^-23 in all."""
+    import minference_amd as M
+    g = torch.Generator(device=gpu).manual_seed(n)
+    q, k = ((2 * torch.randn(1, 2, n, 128, device=gpu, generator=g)).to(dtype) for _ in range(2))
+    cands = [("stream_llm", 1, 5), ("stream_llm", 40, 77), ("stream_llm", 3, 300), ("stream_llm", 300, 10)]
+    got = M.pattern_recall(q, k, cands, row_begin=0)[0].double()
+    r, c = torch.arange(n, device=gpu)[:, None], torch.arange(n, device=gpu)[None]
+    for h in range(2):
+        s = q[0, h].double() @ k[0, h].double().t().contiguous() * 128 ** -0.5
+        p = torch.softmax(s.masked_fill(c > r, float("-inf")), -1)
+        for t, (_, v, w) in enumerate(cands):
+            want = (p * ((c < v) | (r - c <= w))).sum() / n
+            assert abs(got[h, t] - want) <= 2.0 ** -23 * want, (h, t)
