@@ -45,8 +45,8 @@ def _narrow_fp32(*tensors):
     do not fit that format: when some |value| exceeds 32768 (fp16 would overflow) or the largest
     |value| is below 2^-10 (fp16 would flush most of the tensor to zero or to subnormals) they are
     narrowed to bf16 instead, which has fp32's exponent range and 8 mantissa bits.  The decision
-    costs one max-abs reduction and ONE HOST READ (a stream synchronisation) per call: the fp32 path
-    is the reference's CPU-checkable case, not the serving path.  Accumulation, softmax statistics
+    costs one max-abs reduction and ONE HOST READ (a stream synchronisation) per call; the attention
+    operators make it on the device instead (_Call._narrow).  Accumulation, softmax statistics
     and the scale stay fp32 either way."""
     amax = torch.stack([torch.linalg.vector_norm(t.reshape(-1).float(), float("inf")) if t.numel() else
                         torch.ones((), device=t.device) for t in tensors]).max().item()
