@@ -220,8 +220,11 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
     for (int j = 0; j < 4; ++j) cp_off[j] = cp_r * row_bytes + ((cp_c ^ (4 * j + cp_r)) << 4);
     auto copy_k = [&](int kb0, int buf) {
 #if defined(__HIP_DEVICE_COMPILE__)      // (the builtins do not exist in the host pass)
-        if ((kb0 + 2) * KB <= p.n && p.ks[2] <= (1 << 22)) {       // (the copies' offsets are 32-bit)
-            const __amdgpu_buffer_rsrc_t srd = __builtin_amdgcn_make_buffer_rsrc((void *)(kbase + (long long)kb0 * KB * row_bytes), 0, 2 * KB * row_bytes, 0x00020000);
+        if ((kb0 + 2) * KB <= p.n && p.ks[2] >= 0 && p.ks[2] <= (1 << 22)) {       // (the copies' offsets are 32-bit and unsigned)
+            // the extent of 64 rows: the last one ends HD elements past its start, however close the rows lie (rows
+            // that overlap, one row for every key: token stride 0)
+            const int extent = (2 * KB - 1) * row_bytes + HD * 2;
+            const __amdgpu_buffer_rsrc_t srd = __builtin_amdgcn_make_buffer_rsrc((void *)(kbase + (long long)kb0 * KB * row_bytes), 0, extent, 0x00020000);
             const int lds0 = (int)(unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)kt[buf] + 16 * wave * HD * 2;
 #pragma unroll
             for (int j = 0; j < 4; ++j)

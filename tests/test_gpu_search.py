@@ -189,3 +189,48 @@ def test_recall_keeps_fp32_accuracy(gpu, n, dtype):
         for t, (_, v, w) in enumerate(cands):
             want = (p * ((c < v) | (r - c <= w))).sum() / n
             assert abs(got[h, t] - want) <= 2.0 ** -23 * want, (h, t)
+
+
+def _recall_of(q, k_ptr, k_strides, hk, n, cands):
+    """minf_pattern_recall through the C ABI on stream_llm candidates: K by pointer and strides."""
+    from minference_amd import _lib
+    lib, dev, hq = _lib.load(), q.device, q.shape[1]
+    pitch, i64x3, stream = (n + 63) // 64 * 64, _lib.c_i64 * 3, _lib.stream_ptr(q.device)
+    col, diag = (torch.zeros(hq, pitch, dtype=torch.uint8, device=dev) for _ in range(2))
+    for bit, (_, v, s) in enumerate(cands):
+        col[:, :v] |= 1 << bit
+        diag[:, :s + 1] |= 1 << bit
+    recall = torch.empty(hq, 8, dtype=torch.float32, device=dev)
+    nbytes = lib.minf_pattern_recall_workspace_bytes(1, hq, n)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    _lib.check(lib.minf_pattern_recall(q.data_ptr(), k_ptr, i64x3(*q.stride()[:3]), i64x3(*k_strides), 1, hq, hk, n, 128,
+                                       _lib.MINF_BF16, 128.0 ** -0.5, col.data_ptr(), diag.data_ptr(), pitch, None, 0, 0,
+                                       recall.data_ptr(), ws.data_ptr(), nbytes, stream), "minf_pattern_recall")
+    return recall[:, :len(cands)]
+
+
+@pytest.mark.parametrize("n", [64, 300, 1025])
+@pytest.mark.parametrize("stride", [0, 8, 64, 136])
+def test_recall_reads_every_row_of_k_whatever_its_token_stride(gpu, n, stride):
+    """Views whose rows coincide (stride 0: one key for every position), overlap or have gaps: the same bits as
+    a contiguous copy of the view."""
+    from minference_amd import pattern_recall
+    q = heads(n, 2, 1, 60 + n, planted=False)[0].to(gpu)
+    store = torch.randn((n - 1) * stride + 128, generator=torch.Generator().manual_seed(n)).bfloat16().to(gpu)
+    k = store.as_strided((1, 1, n, 128), (store.numel(), store.numel(), stride, 1))
+    k = store.expand(1, 1, n, 128) if stride == 0 else k
+    cands = [("stream_llm", 4, 60), ("stream_llm", 30, 0), ("vertical_and_slash", 40, 60)]
+    got = pattern_recall(q, k, cands, 0)
+    assert torch.equal(got, pattern_recall(q, k.contiguous(), cands, 0))
+    assert torch.equal(_recall_of(q, k.data_ptr(), (0, 0, stride), 1, n, cands[:2]),
+                       _recall_of(q, k.contiguous().data_ptr(), (0, 0, 128), 1, n, cands[:2]))
+
+
+def test_recall_with_k_stored_backwards(gpu):
+    """A negative token stride (C ABI): the rows are addressed from the last one down."""
+    n = 500
+    q, k = (t.to(gpu) for t in heads(n, 1, 1, 9, planted=False))
+    cands = [("stream_llm", 4, 60), ("stream_llm", 30, 0)]
+    back = k.flip(2).contiguous()
+    last = back.data_ptr() + (n - 1) * 128 * 2
+    assert torch.equal(_recall_of(q, last, (0, 0, -128), 1, n, cands), _recall_of(q, k.data_ptr(), (0, 0, 128), 1, n, cands))
