@@ -327,7 +327,7 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
                 for (int t = 0; t < NC; ++t) zx[nb][t] *= alpha;
             }
             float e[16];
-            const float off = BIAS - m[nb];
+            const float off = m[nb] == -INFINITY ? 0.f : BIAS - m[nb];     // (no key yet whose score is above -inf)
 #pragma unroll
             for (int r = 0; r < 16; ++r) e[r] = fast_exp2(fmaf(acc[nb][r], p.scale_log2, off));
             Frag a0 = am[0], a1 = am[1];

@@ -234,3 +234,22 @@ def test_recall_with_k_stored_backwards(gpu):
     back = k.flip(2).contiguous()
     last = back.data_ptr() + (n - 1) * 128 * 2
     assert torch.equal(_recall_of(q, last, (0, 0, -128), 1, n, cands), _recall_of(q, k.data_ptr(), (0, 0, 128), 1, n, cands))
+
+
+@pytest.mark.parametrize("n,masked", [(400, 64), (700, 33), (300, 290)])
+def test_scores_of_minus_infinity_keep_nothing(gpu, n, masked):
+    """Products that leave the fp32 range downwards in a row's first key blocks: such keys have no mass, and rows
+    that see no other key count as zero; the rest against an fp64 softmax without those keys."""
+    from minference_amd import pattern_recall
+    g = torch.Generator().manual_seed(n)
+    q, k = (torch.randn(1, 1, n, 128, generator=g).bfloat16() for _ in range(2))
+    q[..., 0], k[..., 0] = 2.0 ** 70, 0.0
+    k[:, :, :masked, 0] = -2.0 ** 70
+    cands = [("stream_llm", 5, 40), ("stream_llm", masked + 9, 3), ("stream_llm", 1, n)]
+    got = pattern_recall(q.to(gpu), k.to(gpu), cands, 0)[0, 0].double().cpu()
+    s = q[0, 0, :, 1:].double() @ k[0, 0, :, 1:].double().t() * 128 ** -0.5
+    r, c = torch.arange(n)[:, None], torch.arange(n)[None]
+    p = torch.softmax(s.masked_fill((c > r) | (c < masked), float("-inf")), -1).nan_to_num(0.0)
+    for t, (_, v, w) in enumerate(cands):
+        want = (p * ((c < v) | (r - c <= w))).sum() / n
+        assert abs(got[t] - want) <= 2.0 ** -22 * want, (t, got[t].item(), want.item())
