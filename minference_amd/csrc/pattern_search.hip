@@ -53,7 +53,8 @@ struct RecallParams {
     const char *q, *k;
     long long qs[3], ks[3];      // element strides batch, head, token
     int batch, hq, hk, n;
-    float scale_log2;
+    float scale_log2;            // of |sm_scale|: the maximum is taken before the scale,
+    unsigned q_flip;             // and the sign bits of Q are turned for a negative one
     const unsigned char *col, *diag, *blk;   // blk may be null
     long long flag_pitch;        // bytes between heads of col / diag (>= n rounded up to 64)
     long long blk_pitch;         // bytes between block rows; a head has ceil(n/32) block rows
@@ -192,6 +193,14 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
     Frag qf[2][8];
     load_frag(qb, p.qs[2], rt * TILE, p.n, lane, qf[0]);
     load_frag(qb, p.qs[2], rt * TILE + 32, p.n, lane, qf[1]);
+    if (p.q_flip)
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                qf[0][ks].u[i] ^= p.q_flip;
+                qf[1][ks].u[i] ^= p.q_flip;
+            }
 
     constexpr float BIAS = 9.f, LAZY = 6.f;            // exponentials reach 2^(BIAS - 1) .. 2^(BIAS + LAZY) < 2^16
     float m[2] = {-INFINITY, -INFINITY};               // running maximum of the lane's row (same in both lane halves)
@@ -508,7 +517,8 @@ extern "C" int minf_pattern_recall(const void *q, const void *k, const int64_t *
     p.hq = heads_q;
     p.hk = heads_kv;
     p.n = n;
-    p.scale_log2 = sm_scale * 1.4426950408889634f;
+    p.scale_log2 = fabsf(sm_scale) * 1.4426950408889634f;
+    p.q_flip = sm_scale < 0.f ? 0x80008000u : 0u;
     p.col = col_flags;
     p.diag = diag_flags;
     p.blk = block_flags;

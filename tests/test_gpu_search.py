@@ -191,7 +191,7 @@ def test_recall_keeps_fp32_accuracy(gpu, n, dtype):
             assert abs(got[h, t] - want) <= 2.0 ** -23 * want, (h, t)
 
 
-def _recall_of(q, k_ptr, k_strides, hk, n, cands):
+def _recall_of(q, k_ptr, k_strides, hk, n, cands, sm_scale=128.0 ** -0.5):
     """minf_pattern_recall through the C ABI on stream_llm candidates: K by pointer and strides."""
     from minference_amd import _lib
     lib, dev, hq = _lib.load(), q.device, q.shape[1]
@@ -204,7 +204,7 @@ def _recall_of(q, k_ptr, k_strides, hk, n, cands):
     nbytes = lib.minf_pattern_recall_workspace_bytes(1, hq, n)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     _lib.check(lib.minf_pattern_recall(q.data_ptr(), k_ptr, i64x3(*q.stride()[:3]), i64x3(*k_strides), 1, hq, hk, n, 128,
-                                       _lib.MINF_BF16, 128.0 ** -0.5, col.data_ptr(), diag.data_ptr(), pitch, None, 0, 0,
+                                       _lib.MINF_BF16, sm_scale, col.data_ptr(), diag.data_ptr(), pitch, None, 0, 0,
                                        recall.data_ptr(), ws.data_ptr(), nbytes, stream), "minf_pattern_recall")
     return recall[:, :len(cands)]
 
@@ -253,3 +253,13 @@ def test_scores_of_minus_infinity_keep_nothing(gpu, n, masked):
     for t, (_, v, w) in enumerate(cands):
         want = (p * ((c < v) | (r - c <= w))).sum() / n
         assert abs(got[t] - want) <= 2.0 ** -22 * want, (t, got[t].item(), want.item())
+
+
+def test_recall_with_a_negative_scale(gpu):
+    """sm_scale < 0 (C ABI) is the positive one on -Q, bit for bit."""
+    n = 900
+    q, k = (4 * t.to(gpu) for t in heads(n, 2, 1, 12))
+    cands = [("stream_llm", 4, 60), ("stream_llm", 30, 0), ("stream_llm", 1, n - 1)]
+    got = _recall_of(q, k.data_ptr(), k.stride()[:3], 1, n, cands, -128.0 ** -0.5)
+    assert torch.equal(got, _recall_of(-q, k.data_ptr(), k.stride()[:3], 1, n, cands))
+    assert (got[:, 2] - 1).abs().max() <= 2.0 ** -22
