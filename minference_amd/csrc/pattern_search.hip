@@ -11,7 +11,7 @@
 //
 //   pattern_recall_kernel  one workgroup per (head, 128 query rows), heavy row tiles first: 2 waves per
 //                     64 rows, which take every second causal key block (32 keys each).  S^T = K.Q^T on
-//                     v_mfma_f32_32x32x16 with fragments read straight from global memory in
+//                     v_mfma_f32_32x32x16, K copied to LDS and read from there in
 //                     operand layout: lane <-> query row, registers <-> keys; online softmax with a
 //                     running maximum per row.  The row sum and the masked sums are matrix products
 //                     too (see the kernel).  Waves are merged through LDS; a 64-row tile's sum of
@@ -26,7 +26,8 @@ namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
-typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2_t;
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4_t;
 
@@ -86,25 +87,22 @@ __device__ __forceinline__ void copy16_to_lds(const char *src, char *dst) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
 }
 
-// x - (float)h.lo / x - (float)h.hi in one instruction each
-__device__ __forceinline__ float sub_lo(float x, unsigned h) {
-    float r;
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
-    return r;
-}
-__device__ __forceinline__ float sub_hi(float x, unsigned h) {
-    float r;
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(x));
-    return r;
-}
-
-// two f16 values, rounded to nearest
-__device__ __forceinline__ unsigned pack_f16(float x, float y) {
-    typedef float f32x2_t __attribute__((ext_vector_type(2)));
-    typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+// two values rounded to bf16 (nearest), and what the rounding left of each: one instruction per value
+__device__ __forceinline__ unsigned pack_bf16(float x, float y) {
     const f32x2_t v = {x, y};
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, h2_t));
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2_t));
 }
+__device__ __forceinline__ float left_of(float x, unsigned rounded, unsigned minus_one) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, rounded), __builtin_bit_cast(bf16x2_t, minus_one), x, false);
+#else
+    return x;
+#endif
+}
+// bf16 -1 in the low / high half, 0 in the other, in a register: as an inline constant of the instruction, the
+// compiler's form of the first, -1 stands in the high half
+__device__ __forceinline__ unsigned minus_one_lo() { unsigned x; asm("s_mov_b32 %0, 0x0000bf80" : "=s"(x)); return x; }
+__device__ __forceinline__ unsigned minus_one_hi() { unsigned x; asm("s_mov_b32 %0, 0xbf800000" : "=s"(x)); return x; }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -133,16 +131,17 @@ constexpr int DIAG_GROUPS = 8192;            // (262144 tokens; farther blocks a
 // columns, and -- by setting a candidate's whole row -- the blocks and those blocks all of whose diagonals
 // a candidate keeps (most of a window, of a run of slashes).  Only candidates with SOME of a block's
 // diagonals are added element by element (their columns left out: those are in the product already).  The
-// exponentials enter as a sum of two f16 terms, each rounded to nearest (24 bits; the row's largest is scaled
-// to 2^8 .. 2^15, so that what f16 cannot hold lies 2^-32 below it), the sums are fp32.  Scores against fp64
-// sums, 4096 .. 16384 tokens: relative error up to 7.4e-8 (fp32 sums element by element 1.2e-7; terms rounded
-// towards zero 4.6e-7).
-// Bound by its vector instructions (70 % of the issue slots): about 115 per 32 x 32 block (fma and exp 32,
-// conversions 32, maximum 14, masks) and 40 per candidate with mixed diagonals, beside 12 MFMAs, where
-// testing a bit per element and candidate took about 550.  32 / 8 heads, 16384 tokens, the six candidates of
-// the reference: 6.50 ms -> 3.05 (products) -> 2.70 (K shared through LDS instead of fragments from global
-// memory) -> 2.45 (mixed-precision subtraction, scalar descriptors) -> 2.34 ms (dot products for mixed
-// diagonals), 2.36 with the terms rounded to nearest; the score products alone take 0.44 ms at the nominal rate.
+// exponentials enter as the sum of three bf16 terms, which is exact (8 + 8 + 8 bits) and has the exponents of
+// fp32: what lies far below a row's maximum -- every other key, where a head has a sink -- keeps its 24 bits for
+// the candidates that leave the maximum out.  (Two f16 terms, of 24 bits near the maximum only, had lost 4e-4 of
+// such a candidate's score under a sink 22 nats above the rest, and all of it under one of 26.)  The sums are fp32.
+// Relative error of the scores against fp64 sums, 4096 .. 16384 tokens: up to 7.6e-8; 6000 tokens under a sink of
+// 14 .. 30 nats up to 1.3e-6, of 80 nats 1.9e-6 (fp32 sums element by element: 1.2e-7, 4.8e-6, 1.9e-6).
+// Bound by its vector instructions: about 140 per 32 x 32 block (fma and exp 32, conversions 56, maximum 14,
+// masks) and 40 per candidate with mixed diagonals, beside 14 MFMAs, where testing a bit per element and
+// candidate took about 550.  32 / 8 heads, 16384 tokens, the six candidates of the reference: 7.00 ms (bits)
+// -> 2.86; with two f16 terms, which this replaces, 2.46.  K shared through LDS instead of fragments from global
+// memory is worth 0.35 ms of it; the score products alone take 0.44 ms at the nominal rate.
 template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_kernel(const RecallParams p) {
     __shared__ unsigned dtab[DIAG_GROUPS];             // bytes: OR, AND, OR without the first, AND without the first
     __shared__ float lds[4][TILE][NC + 2];
@@ -202,7 +201,8 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
                 qf[1][ks].u[i] ^= p.q_flip;
             }
 
-    constexpr float BIAS = 9.f, LAZY = 6.f;            // exponentials reach 2^(BIAS - 1) .. 2^(BIAS + LAZY) < 2^16
+    const unsigned neg_lo = minus_one_lo(), neg_hi = minus_one_hi();
+    constexpr float LAZY = 6.f;                        // exponentials reach 2^-1 .. 2^LAZY
     float m[2] = {-INFINITY, -INFINITY};               // running maximum of the lane's row (same in both lane halves)
     f32x16_t zacc[2];                                  // rows t = 8 (r / 4) + 4 g + r % 4: r 0..3 candidates 4 g + r, r 4 (g 0) the sum
     float zx[2][NC];                                   // this lane's share of the element-wise sums
@@ -304,8 +304,8 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
 #pragma unroll
             for (int jj = 0; jj < 2; ++jj) {
                 const unsigned x = ((cw[2 * s + jj] >> a_shift) & a_and) | a_or;
-                am[s].u[2 * jj] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c010c00u), 0x3c00u);
-                am[s].u[2 * jj + 1] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c030c02u), 0x3c00u);
+                am[s].u[2 * jj] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c010c00u), 0x3f80u);
+                am[s].u[2 * jj + 1] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c030c02u), 0x3f80u);
             }
 
 #pragma unroll
@@ -326,7 +326,7 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
             const float cand = mx * p.scale_log2;
             const bool grow = cand > m[nb] + LAZY;                 // (raised only when it has to be)
             if (__any(grow)) {
-                // (a whole number: BIAS - m and the rescale are exact, so that what was summed under one maximum
+                // (a whole number: the rescale is exact, so that what was summed under one maximum
                 // and what is summed under the next are in proportion to the last bit)
                 const float up = ceilf(cand), alpha = grow ? fast_exp2(m[nb] - up) : 1.0f;
                 m[nb] = grow ? up : m[nb];
@@ -336,7 +336,7 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
                 for (int t = 0; t < NC; ++t) zx[nb][t] *= alpha;
             }
             float e[16];
-            const float off = m[nb] == -INFINITY ? 0.f : BIAS - m[nb];     // (no key yet whose score is above -inf)
+            const float off = m[nb] == -INFINITY ? 0.f : -m[nb];           // (no key yet whose score is above -inf)
 #pragma unroll
             for (int r = 0; r < 16; ++r) e[r] = fast_exp2(fmaf(acc[nb][r], p.scale_log2, off));
             Frag a0 = am[0], a1 = am[1];
@@ -344,21 +344,24 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
                 const bool mine = (full[nb] >> a_shift) & a_and & 1u;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    a0.u[i] = mine ? 0x3c003c00u : a0.u[i];
-                    a1.u[i] = mine ? 0x3c003c00u : a1.u[i];
+                    a0.u[i] = mine ? 0x3f803f80u : a0.u[i];
+                    a1.u[i] = mine ? 0x3f803f80u : a1.u[i];
                 }
             }
-            Frag hi[2], lo[2];
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
+                Frag hi, mid, lo;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float x = e[8 * s + 2 * i], y = e[8 * s + 2 * i + 1];
-                    hi[s].u[i] = pack_f16(x, y);
-                    lo[s].u[i] = pack_f16(sub_lo(x, hi[s].u[i]), sub_hi(y, hi[s].u[i]));
+                    hi.u[i] = pack_bf16(x, y);
+                    const float x1 = left_of(x, hi.u[i], neg_lo), y1 = left_of(y, hi.u[i], neg_hi);
+                    mid.u[i] = pack_bf16(x1, y1);
+                    lo.u[i] = pack_bf16(left_of(x1, mid.u[i], neg_lo), left_of(y1, mid.u[i], neg_hi));
                 }
-                zacc[nb] = mma<_Float16>(s ? a1 : a0, hi[s], zacc[nb]);
-                zacc[nb] = mma<_Float16>(s ? a1 : a0, lo[s], zacc[nb]);
+                zacc[nb] = mma<__bf16>(s ? a1 : a0, hi, zacc[nb]);
+                zacc[nb] = mma<__bf16>(s ? a1 : a0, mid, zacc[nb]);
+                zacc[nb] = mma<__bf16>(s ? a1 : a0, lo, zacc[nb]);
             }
             if (mixed[nb]) {
                 // diagonal flags: key i of group j has offset o0 - i, o0 = row - (n0 + 8j + 4g); the word
@@ -385,15 +388,9 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             const unsigned x = (pm[j] >> t) & 0x01010101u;
-                            const f16x2_t k0 = __builtin_bit_cast(f16x2_t, __umul24(__builtin_amdgcn_perm(0u, x, 0x0c010c00u), 0x3c00u));
-                            const f16x2_t k1 = __builtin_bit_cast(f16x2_t, __umul24(__builtin_amdgcn_perm(0u, x, 0x0c030c02u), 0x3c00u));
-                            const unsigned h0 = hi[j >> 1].u[2 * (j & 1)], h1 = hi[j >> 1].u[2 * (j & 1) + 1];
-                            const unsigned l0 = lo[j >> 1].u[2 * (j & 1)], l1 = lo[j >> 1].u[2 * (j & 1) + 1];
                             float z = zx[nb][t];
-                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, h0), k0, z, false);
-                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, l0), k0, z, false);
-                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, h1), k1, z, false);
-                            z = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, l1), k1, z, false);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) z = fmaf((float)((x >> (8 * i)) & 0xffu), e[4 * j + i], z);
                             zx[nb][t] = z;
                         }
                     }

@@ -175,7 +175,7 @@ def test_recall_tiles_stripes_and_flag_mixes(gpu, n, hq, hk, begin, d):
 
 @pytest.mark.parametrize("n,dtype", [(1500, torch.bfloat16), (3001, torch.float16)])
 def test_recall_keeps_fp32_accuracy(gpu, n, dtype):
-    """Against fp64 sums on the same operands: exponentials of 24 bits, fp32 row sums whose roundings average
+    """Against fp64 sums on the same operands, all candidates with the largest keys: exponentials of 24 bits, fp32 row sums whose roundings average
     out over the rows, one rounding of the result (2^-24): 2^-23 in all."""
     import minference_amd as M
     g = torch.Generator(device=gpu).manual_seed(n)
@@ -191,8 +191,8 @@ def test_recall_keeps_fp32_accuracy(gpu, n, dtype):
             assert abs(got[h, t] - want) <= 2.0 ** -23 * want, (h, t)
 
 
-def _recall_of(q, k_ptr, k_strides, hk, n, cands, sm_scale=128.0 ** -0.5):
-    """minf_pattern_recall through the C ABI on stream_llm candidates: K by pointer and strides."""
+def _recall_of(q, k_ptr, k_strides, hk, n, cands, sm_scale=128.0 ** -0.5, flags=None):
+    """minf_pattern_recall through the C ABI: K by pointer and strides, stream_llm candidates or (col, diag) flags."""
     from minference_amd import _lib
     lib, dev, hq = _lib.load(), q.device, q.shape[1]
     pitch, i64x3, stream = (n + 63) // 64 * 64, _lib.c_i64 * 3, _lib.stream_ptr(q.device)
@@ -200,13 +200,14 @@ def _recall_of(q, k_ptr, k_strides, hk, n, cands, sm_scale=128.0 ** -0.5):
     for bit, (_, v, s) in enumerate(cands):
         col[:, :v] |= 1 << bit
         diag[:, :s + 1] |= 1 << bit
+    col, diag = (col, diag) if flags is None else flags
     recall = torch.empty(hq, 8, dtype=torch.float32, device=dev)
     nbytes = lib.minf_pattern_recall_workspace_bytes(1, hq, n)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     _lib.check(lib.minf_pattern_recall(q.data_ptr(), k_ptr, i64x3(*q.stride()[:3]), i64x3(*k_strides), 1, hq, hk, n, 128,
                                        _lib.MINF_BF16, sm_scale, col.data_ptr(), diag.data_ptr(), pitch, None, 0, 0,
                                        recall.data_ptr(), ws.data_ptr(), nbytes, stream), "minf_pattern_recall")
-    return recall[:, :len(cands)]
+    return recall[:, :len(cands)] if flags is None else recall
 
 
 @pytest.mark.parametrize("n", [64, 300, 1025])
@@ -263,3 +264,31 @@ def test_recall_with_a_negative_scale(gpu):
     got = _recall_of(q, k.data_ptr(), k.stride()[:3], 1, n, cands, -128.0 ** -0.5)
     assert torch.equal(got, _recall_of(-q, k.data_ptr(), k.stride()[:3], 1, n, cands))
     assert (got[:, 2] - 1).abs().max() <= 2.0 ** -22
+
+
+@pytest.mark.parametrize("nats", [14, 22, 30, 60])
+def test_candidates_without_the_sink_keep_their_accuracy(gpu, nats):
+    """One key far above all others in every row: the candidates that leave it out keep a share of e^-nats, all
+    of it from small exponentials (columns and diagonals in and outside the sink's own block, whole blocks, single
+    diagonals).  Bound: a score at distance D (powers of two) from the maximum is rounded there and scaled by a
+    rounded factor, 2^-24 D each, beside fp32 sums of about 5 roundings each way: 2^-23 (D + 32) of the share."""
+    n = 1500
+    g = torch.Generator().manual_seed(nats)
+    q, k = (torch.randn(1, 1, n, 128, generator=g) for _ in range(2))
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[0, 0, 0, 0] = nats * 128 ** 0.5 / 8
+    q, k = q.bfloat16().to(gpu), k.bfloat16().to(gpu)
+    col, diag = (torch.zeros(1, (n + 63) // 64 * 64, dtype=torch.uint8, device=gpu) for _ in range(2))
+    col[:, 1:21] |= 1
+    col[:, 40:300:3] |= 2
+    col[:, 1:] |= 4
+    diag[:, :300] |= 8
+    diag[:, 5:200:7] |= 16
+    got = _recall_of(q, k.data_ptr(), k.stride()[:3], 1, n, (), flags=(col, diag))[0].double()
+    r, c = torch.arange(n, device=gpu)[:, None], torch.arange(n, device=gpu)[None]
+    s = q[0, 0].double() @ k[0, 0].double().t().contiguous() * 128 ** -0.5
+    p = torch.softmax(s.masked_fill(c > r, float("-inf")), -1)
+    keep = col[0, :n][None] | diag[0][(r - c).clamp(min=0)]
+    for t in range(5):
+        want = (p * ((keep >> t) & 1)).sum() / n
+        assert abs(got[t] - want) <= 2.0 ** -23 * (nats * 1.4427 + 10 + 32) * want, (t, got[t].item(), want.item())
