@@ -71,3 +71,14 @@ def test_silu_mul_fp32_far_from_zero(gpu):
     got = m._silu_mul(gate.clone(), up).double()
     want = torch.nn.functional.silu(gate.double()) * up.double()
     assert ((got - want).abs() <= 2.0 ** -21 * want.abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_silu_mul_of_every_gate(gpu, dtype):
+    """Every finite 16-bit gate: the bits of the torch chain, whose fp32 exponential, sum and quotient are the
+    same operations."""
+    m = model(16, dtype, gpu)
+    gate = torch.arange(-32768, 32768, device=gpu).to(torch.int16).view(dtype)
+    gate = gate[torch.isfinite(gate)].contiguous()
+    up = torch.ones_like(gate)
+    assert torch.equal(m._silu_mul(gate.clone(), up), torch.nn.functional.silu(gate) * up)
