@@ -43,7 +43,7 @@ class LlamaPrefill:
 
     def __init__(self, config: LlamaConfig, device="cuda", dtype=torch.bfloat16, seed=0, std=0.02):
         self.cfg, self.device, self.dtype = config, torch.device(device), dtype
-        self._dt = {torch.bfloat16: _lib.MINF_BF16, torch.float16: _lib.MINF_F16, torch.float32: _lib.MINF_F32}[dtype]
+        self._dt = {torch.bfloat16: _lib.MINF_BF16, torch.float16: _lib.MINF_F16, torch.float32: _lib.MINF_F32}.get(dtype)
         c = config
         g = torch.Generator(device=self.device).manual_seed(seed)
 
@@ -115,6 +115,23 @@ class LlamaPrefill:
         _lib.check(st, "minf_silu_mul")
         return gate
 
+    def _as_configured(self, hidden):
+        """Whether every weight (and the embedded tokens) has the dtype, device and shape that the configuration
+        says, the norms' one after the other in memory: what the kernels above take by pointer.  Weights a caller
+        filled in otherwise go through torch ops, which promote, broadcast or refuse them."""
+        c = self.cfg
+        qd, kd, inter = c.num_heads * c.head_dim, c.num_kv_heads * c.head_dim, c.intermediate_size
+        shapes = {"input_layernorm": (c.hidden_size,), "post_attention_layernorm": (c.hidden_size,),
+                  "q_proj": (qd, c.hidden_size), "k_proj": (kd, c.hidden_size), "v_proj": (kd, c.hidden_size),
+                  "o_proj": (c.hidden_size, qd), "gate_proj": (inter, c.hidden_size), "up_proj": (inter, c.hidden_size),
+                  "down_proj": (c.hidden_size, inter)}
+
+        def fits(t, shape):
+            return t.dtype == self.dtype and t.device == hidden.device and tuple(t.shape) == shape \
+                and (t.dim() > 1 or t.is_contiguous())
+        return self._dt is not None and hidden.is_cuda and fits(hidden, (hidden.shape[0], c.hidden_size)) \
+            and fits(self.norm, (c.hidden_size,)) and all(fits(L[k], shape) for L in self.layers for k, shape in shapes.items())
+
     # ---- prefill --------------------------------------------------------------------------
     @torch.no_grad()
     def prefill(self, input_ids, attn_forward_config=None, chunk=32768, keep_kv=False):
@@ -126,6 +143,8 @@ class LlamaPrefill:
         n = ids.numel()
         cfg = attn_forward_config if attn_forward_config is not None else {"best_pattern": None}
         hidden = self.embed_tokens[ids]                                    # [N, hidden]
+        if not self._as_configured(hidden):
+            return self._prefill_torch(hidden, cfg, chunk, keep_kv)
         cos, sin = self._rope_tables(n)
         new = lambda *shape: torch.empty(shape, device=self.device, dtype=self.dtype)
         q, attn = new(n, c.num_heads, c.head_dim), new(n, c.num_heads, c.head_dim)
@@ -160,6 +179,41 @@ class LlamaPrefill:
         last = self._rms(hidden[-1:].clone(), self.norm)
         logits = (last @ self.lm_head.T).float()[0]
         return logits, kv_cache
+
+    def _prefill_torch(self, hidden, cfg, chunk, keep_kv):
+        """The same for weights that are not as configured (_as_configured): torch ops around the attention path."""
+        c, n = self.cfg, hidden.shape[0]
+
+        def rms(x, weight):
+            xf = x.float()
+            return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + c.rms_eps)).to(self.dtype) * weight
+
+        def rotate(x, cos, sin):
+            half = c.head_dim // 2
+            return (x.float() * cos + torch.cat([-x[..., half:], x[..., :half]], dim=-1).float() * sin).to(x.dtype)
+        cos, sin = (torch.cat([t, t], dim=-1)[:, None] for t in self._rope_tables(n))
+        new = lambda heads: torch.empty((n, heads, c.head_dim), device=self.device, dtype=self.dtype)
+        q, k, v, kv_cache = new(c.num_heads), None, None, [] if keep_kv else None
+        for li, L in enumerate(self.layers):
+            if k is None or keep_kv:
+                k, v = new(c.num_kv_heads), new(c.num_kv_heads)
+            for s in range(0, n, chunk):
+                e = min(s + chunk, n)
+                x = rms(hidden[s:e], L["input_layernorm"])
+                q[s:e] = rotate((x @ L["q_proj"].T).view(e - s, c.num_heads, c.head_dim), cos[s:e], sin[s:e])
+                k[s:e] = rotate((x @ L["k_proj"].T).view(e - s, c.num_kv_heads, c.head_dim), cos[s:e], sin[s:e])
+                v[s:e] = (x @ L["v_proj"].T).view(e - s, c.num_kv_heads, c.head_dim)
+            attn = minference_prefill_forward(q.permute(1, 0, 2)[None], k.permute(1, 0, 2)[None], v.permute(1, 0, 2)[None],
+                                              {"layer_idx": li, "attn_forward_config": cfg})[0].permute(1, 0, 2)
+            for s in range(0, n, chunk):
+                e = min(s + chunk, n)
+                h = hidden[s:e] + attn[s:e].reshape(e - s, -1) @ L["o_proj"].T
+                x = rms(h, L["post_attention_layernorm"])
+                mlp = (torch.nn.functional.silu(x @ L["gate_proj"].T) * (x @ L["up_proj"].T)) @ L["down_proj"].T
+                hidden[s:e] = h + mlp
+            if keep_kv:
+                kv_cache.append((k, v))
+        return (rms(hidden[-1:], self.norm) @ self.lm_head.T).float()[0], kv_cache
 
     def flops_linear(self, n):
         """FLOPs of the GEMMs of one prefill of n tokens (attention excluded, lm_head on one token)."""

@@ -109,3 +109,51 @@ def test_seeded_pattern_mix_matches_config5_description():
     assert abs(frac["vertical_and_slash"] - 0.7) < 0.05 and abs(frac["block_sparse"] - 0.2) < 0.05
     assert abs(frac["stream_llm"] - 0.1) < 0.05
     assert t == seeded_pattern_mix(32, 32, seed=501)
+
+
+def test_weights_that_are_not_as_configured(gpu):
+    """Weights a caller filled in: an fp32 residual stream, norm weights that broadcast or are strided, an fp32
+    norm + lm_head and another MLP width are computed (the values of the plain model within bf16 roundings, or of
+    the same model with the weights laid out), shapes and dtypes that do not go together are refused."""
+    from minference_amd.llama import LlamaConfig, LlamaPrefill
+
+    def model():
+        m = LlamaPrefill(LlamaConfig(**TINY), device=gpu, seed=3)
+        for L in m.layers:
+            for w in ("input_layernorm", "post_attention_layernorm"):
+                L[w] = 1 + 0.25 * torch.randn(256, generator=torch.Generator().manual_seed(5)).to(gpu, m.dtype)
+        return m
+    ids = torch.randint(0, 500, (300,), generator=torch.Generator().manual_seed(1))
+    run = lambda m: m.prefill(ids, chunk=128)[0]
+    near = lambda a, b: (a - b).norm() <= 3e-2 * b.norm()
+    plain = run(model())
+    m = model()
+    assert near(m._prefill_torch(m.embed_tokens[ids.to(gpu)], {"best_pattern": None}, 128, False)[0], plain)
+    m = model()
+    m.embed_tokens = m.embed_tokens.float()                 # residuals in fp32
+    assert near(run(m), plain)
+    m = model()
+    wide = torch.zeros(256, 2, device=gpu, dtype=m.dtype)   # a column of a wider tensor
+    wide[:, 0] = m.layers[1]["input_layernorm"]
+    m.layers[1]["input_layernorm"] = wide[:, 0]
+    assert near(run(m), plain)
+    m, b = model(), model()                                 # one weight for all dims
+    m.layers[0]["input_layernorm"] = torch.full((1,), 1.5, device=gpu, dtype=m.dtype)
+    b.layers[0]["input_layernorm"] = torch.full((256,), 1.5, device=gpu, dtype=m.dtype)
+    assert near(run(m), run(b))
+    m = model()
+    m.norm, m.lm_head = m.norm.float(), m.lm_head.float()
+    assert near(run(m), plain)
+    m = model()
+    for L in m.layers:                                      # half of the MLP
+        L["gate_proj"], L["up_proj"], L["down_proj"] = L["gate_proj"][:256], L["up_proj"][:256], L["down_proj"][:, :256]
+    assert torch.isfinite(run(m)).all()
+    for name, cut in (("up_proj", slice(0, 256)), ("o_proj", slice(0, 128)), ("q_proj", slice(0, 128)), ("input_layernorm", slice(0, 128))):
+        m = model()
+        m.layers[0][name] = m.layers[0][name][cut]
+        with pytest.raises(RuntimeError):
+            run(m)
+    m = model()
+    m.layers[1]["post_attention_layernorm"] = m.layers[1]["post_attention_layernorm"].float()
+    with pytest.raises(RuntimeError):
+        run(m)
