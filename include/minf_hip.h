@@ -163,6 +163,8 @@ int minf_index_sort_pair(const void *vertical, int vertical_is64, int nnz_v, int
  *   sm_scale multiplies q.k before the softmax (reference: head_dim^-0.5).
  *   Every o element of every row < n (of every selected head) is written; nothing else is.
  *   Token strides must be at least head_dim (rows must not overlap).
+ *   o must not share memory with q, k or v: keys are read by workgroups that start after others have
+ *   written their rows, and q is read again where a walk is made a second time.
  */
 typedef struct minf_qkvo {
     const void *q, *k, *v;

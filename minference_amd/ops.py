@@ -34,6 +34,17 @@ def _prep(t: torch.Tensor) -> torch.Tensor:
     return t
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the stretches of memory from the first to the last element of a and b meet (views that only
+    interleave, like the thirds of one [B, N, 3 H, D] projection, count as meeting)."""
+    def span(t):
+        return t.data_ptr(), t.data_ptr() + (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride()))) * t.element_size()
+    if not a.numel() or not b.numel() or a.device != b.device:
+        return False
+    (a0, a1), (b0, b1) = span(a), span(b)
+    return a0 < b1 and b0 < a1
+
+
 _F16_SAFE_ABS = 32768.0
 _F16_TINY_ABS = 2.0 ** -10
 
@@ -111,10 +122,13 @@ class _Call:
         B, H, N, _ = self.q.shape
         self.B, self.H, self.N, self.Hk = B, H, N, self.k.shape[1]
         # `out` (the caller's [B, H, N, D] buffer, any strides the kernels take) is written in place when
-        # it has the kernels' own shape and dtype, else copied into at the end
+        # it has the kernels' own shape and dtype and shares no memory with the operands, else copied into at the
+        # end: keys are read by workgroups that start after others have written, queries by a walk that is made
+        # twice and by the launches of other pattern types
         self.out = out
         if out is not None and tuple(out.shape) == (B, H, N, Dk) and out.dtype == self.q.dtype == self.out_dtype \
-                and out.device == q.device and out.stride(2) >= Dk and _prep(out) is out:
+                and out.device == q.device and out.stride(2) >= Dk and _prep(out) is out \
+                and not any(_overlap(out, t) for t in (self.q, self.k, self.v)):
             self.o = out
         else:
             self.o = torch.empty((B, H, N, Dk) if need_out else (1, 1, 1, Dk),
