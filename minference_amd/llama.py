@@ -118,7 +118,10 @@ class LlamaPrefill:
     def _as_configured(self, hidden):
         """Whether every weight (and the embedded tokens) has the dtype, device and shape that the configuration
         says, the norms' one after the other in memory: what the kernels above take by pointer.  Weights a caller
-        filled in otherwise go through torch ops, which promote, broadcast or refuse them."""
+        filled in otherwise go through torch ops, which promote, broadcast or refuse them; so does a call under
+        autocast, whose products come in autocast's dtype."""
+        if torch.is_autocast_enabled(self.device.type):
+            return False
         c = self.cfg
         qd, kd, inter = c.num_heads * c.head_dim, c.num_kv_heads * c.head_dim, c.intermediate_size
         shapes = {"input_layernorm": (c.hidden_size,), "post_attention_layernorm": (c.hidden_size,),

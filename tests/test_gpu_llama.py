@@ -157,3 +157,17 @@ def test_weights_that_are_not_as_configured(gpu):
     m.layers[1]["post_attention_layernorm"] = m.layers[1]["post_attention_layernorm"].float()
     with pytest.raises(RuntimeError):
         run(m)
+
+
+@pytest.mark.parametrize("dtype,cast", [(torch.bfloat16, torch.float16), (torch.float32, torch.bfloat16)])
+def test_prefill_under_autocast(gpu, dtype, cast):
+    """The products of a call under autocast come in autocast's dtype, which is not what the fused passes are told
+    their operands have: the call runs through torch ops.  (3e-2: two layers on operands of 8 bits.)"""
+    from minference_amd.llama import LlamaConfig, LlamaPrefill
+    m = LlamaPrefill(LlamaConfig(**TINY), device=gpu, dtype=dtype, seed=3)
+    ids = torch.randint(0, 500, (300,), generator=torch.Generator().manual_seed(1))
+    plain = m.prefill(ids, chunk=128)[0]
+    with torch.autocast("cuda", cast):
+        assert not m._as_configured(m.embed_tokens[ids.to(gpu)])
+        got = m.prefill(ids, chunk=128)[0]
+    assert (got - plain).norm() <= 3e-2 * plain.norm()
