@@ -46,7 +46,9 @@ extern "C" {
 #define MINF_ROUND_NONE 0
 #define MINF_ROUND_INPUT_DTYPE 1
 
-/* Library version as major*10000 + minor*100 + patch. */
+/* Library version as major*10000 + minor*100 + patch: minf_version() is that of the library, MINF_VERSION
+ * that of this header.  A change of a signature or of minf_qkvo changes it. */
+#define MINF_VERSION 400
 int minf_version(void);
 
 /* sizeof(minf_qkvo) as this library was compiled.  A caller built against another revision of this

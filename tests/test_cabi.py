@@ -41,6 +41,18 @@ def test_version_and_status_strings(lib):
         assert lib.minf_status_string(code) not in (b"ok", b"unknown status")
 
 
+def test_version_names_the_struct(lib):
+    """The version is the header's and the package's, and belongs to one size of minf_qkvo: a struct that grows
+    without a new version would be read past a caller's end."""
+    import minference_amd
+    from minference_amd import _lib
+    with open(os.path.join(ROOT, "include", "minf_hip.h")) as f:
+        header = int(re.search(r"#define MINF_VERSION (\d+)", f.read()).group(1))
+    major, minor, patch = (int(x) for x in minference_amd.__version__.split("."))
+    assert lib.minf_version() == header == major * 10000 + minor * 100 + patch
+    assert (header, lib.minf_qkvo_size(), ctypes.sizeof(_lib.QKVO)) == (400, 208, 208)
+
+
 def test_argument_validation_needs_no_gpu(lib):
     from minference_amd import _lib
     # null pointers / bad sizes are rejected before any HIP call
