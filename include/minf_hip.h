@@ -211,7 +211,9 @@ int minf_widen_out(const void *o16, float *out, int64_t rows, int dim, int dim_i
 /*
  * Bytes of minf_qkvo.workspace that an attention launch of this problem uses (0: it is not split).
  * op: which entry point; n_init, n_local: of the A-shape / tri-shape entry points, n_last: of tri-shape
- * (0 for A-shape); ignored otherwise.  A pure host function.
+ * (0 for A-shape); vertical-slash: n_init = nnz_v, n_local = nnz_s, block-sparse: n_local = max_blocks (n_local 0: as
+ * many as there are; a launch whose lists are narrower may then use less, or nothing); ignored
+ * otherwise.  A pure host function.
  */
 #define MINF_OP_VERTICAL_SLASH 0
 #define MINF_OP_BLOCK_SPARSE 1

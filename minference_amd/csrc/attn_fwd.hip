@@ -1233,18 +1233,33 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
 // 32 / 8 heads 2048 tokens 53 : 58; 32 heads 1000 tokens 26 : 32; block-sparse, 28 heads 2000 tokens 57 :
 // 64): the steps saved have to be worth it.
 //  * Dense walks and the dense last rows of tri-shape have any number of steps.
-//  * Lists are not known on the host and are taken as dense, A-shape walks end at their window.  Both
-//    are split up to 64 row-block pairs per head only: beyond, a head has the same bits whatever heads it
-//    is launched with, which per-head dispatch relies on.  Up to 64 pairs in all, segments have SEG_MIN
-//    steps whatever else the launch holds.
+//  * Lists are not known on the host, only their widths: a walk is taken to be as long as its list is wide, up to
+//    the diagonal.  Up to 100 slashes are taken to be neighbours (the estimation always selects the last 100
+//    diagonals first): two or three blocks.  A longer walk than was taken is cut into the same number of segments.
+//    Taken as dense, short lists paid for segments that do not exist and for the fold: block-sparse, top-10,
+//    one head 8192 tokens 24 whole, 30 split, 4 heads 25 : 34 us; top-20, 4 heads 6000 tokens 39 : 47; 50
+//    slashes and 30 columns, one head 8192 tokens 18 : 27.
+//  * A-shape walks end at their window.
+//  * Lists and A-shape are split up to 64 row-block pairs per head only: beyond, a head has the same bits
+//    whatever heads it is launched with.  Up to there the number of segments follows the launch's load, and a head's
+//    bits (the order of its fp32 sums) with it.  Up to 64 pairs in all, segments have SEG_MIN steps
+//    whatever else the launch holds.
 constexpr int SEG_MIN = 8;
+constexpr int ADJACENT_SLASHES = 100;
 SplitPlan plan_split(int mode, const AttnParams &p, int head_dim) {
     const int pairs = (p.rows + 1) / 2;
     const SplitPlan none{pairs, 1, 1};
     const long long heads = (long long)p.batch * (p.head_list ? p.index_heads : p.hq);
     const int slots = head_dim == 256 ? 256 : (head_dim == 128 ? 512 : 768);
     // walks of pairs 0 .. k-1: pair i has 2 i + 2 steps, at most `most`
-    const int window = mode == MODE_ASHAPE ? (int)(((long long)p.n_local + BM - 1) / BN + 2 + ((long long)p.n_init + BN - 1) / BN) : 0x7fffffff;
+    int window = 0x7fffffff;
+    if (mode == MODE_ASHAPE) window = (int)(((long long)p.n_local + BM - 1) / BN + 2 + ((long long)p.n_init + BN - 1) / BN);
+    if (mode == MODE_BS && p.max_blocks > 0) window = p.max_blocks;
+    if (mode == MODE_VS && p.nnz_s > 0) {
+        const long long blocks = p.nnz_s <= ADJACENT_SLASHES ? (p.nnz_s + BN - 1) / BN + 1 : p.nnz_s;
+        const long long both = blocks + ((long long)p.nnz_v + BN - 1) / BN;
+        window = both < 0x7fffffff ? (int)both : 0x7fffffff;
+    }
     auto steps = [&](int k, int most) -> double {
         const double grown = most / 2 < k ? most / 2 : k;
         return grown * (grown + 1) + (k - grown) * most;
@@ -1429,6 +1444,8 @@ extern "C" size_t minf_attn_workspace_bytes(const minf_qkvo *t, int op, int n_in
         p.n_init = n_init; p.n_local = n_local;
         p.dense_from = n_last > 0 ? (n_last < t->n ? t->n - n_last : 0) : p.dense_from;
     }
+    if (op == MINF_OP_BLOCK_SPARSE) p.max_blocks = n_local;
+    if (op == MINF_OP_VERTICAL_SLASH) { p.nnz_v = n_init > 0 ? n_init : 0; p.nnz_s = n_local; }
     const SplitPlan s = plan_split(op, p, t->head_dim);
     return s.nseg > 1 ? split_bytes(s, p, t->head_dim) : 0;
 }

@@ -181,7 +181,8 @@ class _Call:
         self.struct.index_heads = int(head_list.numel()) if head_list is not None else 0
 
     def scratch(self, op, n_init=0, n_local=0, n_last=0):
-        """Give the next launch of ``op`` the scratch memory its split walks use (none for most)."""
+        """Give the next launch of ``op`` the scratch memory its split walks use (none for most).  List operators:
+        n_init / n_local are the widths of the column / block lists."""
         nbytes = _lib.load().minf_attn_workspace_bytes(self.ref, op, int(n_init), int(n_local), int(n_last))
         # (a block freed here is reused only by later work on the same stream)
         self._scratch = torch.empty(nbytes, dtype=torch.uint8, device=self.q.device) if nbytes else None
@@ -224,7 +225,7 @@ def vertical_slash_attention_from_index(query, key, value, block_count, block_of
         raise ValueError("index tensors must be [batch, heads_q, ceil(n/64), ...]")
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
-        c.scratch(_lib.MINF_OP_VERTICAL_SLASH)
+        c.scratch(_lib.MINF_OP_VERTICAL_SLASH, column_index.shape[-1], block_offset.shape[-1])
         st = lib.minf_vs_attn_fwd(c.ref, block_count.data_ptr(), block_offset.data_ptr(),
                                   column_count.data_ptr(), column_index.data_ptr(), rows,
                                   block_offset.shape[-1], column_index.shape[-1],
@@ -279,7 +280,7 @@ def block_sparse_attention_from_index(query, key, value, block_index, out=None):
         raise ValueError("block_index has the wrong batch/head/row sizes")
     lib = _lib.load()
     with torch.cuda.device(c.q.device):
-        c.scratch(_lib.MINF_OP_BLOCK_SPARSE)
+        c.scratch(_lib.MINF_OP_BLOCK_SPARSE, 0, block_index.shape[3])
         st = lib.minf_bs_attn_fwd(c.ref, block_index.data_ptr(), block_index.shape[2],
                                   block_index.shape[3], _lib.stream_ptr(c.q.device))
     _lib.check(st, "minf_bs_attn_fwd")

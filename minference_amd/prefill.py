@@ -193,7 +193,7 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
                 seqlens = dt["seqlens"]
                 bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, 64, 64, zero_fill=False)
                 c.select_heads(slot)
-                c.scratch(_lib.MINF_OP_VERTICAL_SLASH)
+                c.scratch(_lib.MINF_OP_VERTICAL_SLASH, vmax, smax)
                 st = lib.minf_vs_attn_fwd(c.ref, bc.data_ptr(), bo.data_ptr(), cc.data_ptr(), ci.data_ptr(), rows,
                                           smax, vmax, stream)
                 _lib.check(st, "minf_vs_attn_fwd")
@@ -212,7 +212,7 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
                                                    ws.data_ptr(), ws_bytes, stream)
                 _lib.check(st, "minf_bs_block_index_heads")
                 c.select_heads(slot)
-                c.scratch(_lib.MINF_OP_BLOCK_SPARSE)
+                c.scratch(_lib.MINF_OP_BLOCK_SPARSE, 0, kk)
                 st = lib.minf_bs_attn_fwd(c.ref, bi.data_ptr(), brows, kk, stream)
                 _lib.check(st, "minf_bs_attn_fwd")
                 keep += [ws, bi]

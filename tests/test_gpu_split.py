@@ -102,6 +102,42 @@ def test_which_launches_are_split():
     assert nbytes(ashape, 24000, 16, 8, 512, 128, d=64) > 0 and nbytes(ashape, 24000, 16, 8, 512, 0, d=64) == 0
 
 
+def test_short_lists_are_not_split():
+    """The rule knows how wide the lists are: too few blocks for what a cut costs, or neighbouring slashes (two
+    or three blocks), are walked whole where full lists are split; lists as wide as the rows as if not known."""
+    import ctypes
+    from minference_amd import _lib
+    lib = _lib.load()
+
+    def nbytes(op, n, hq, wide_v, wide):
+        t = _lib.QKVO()
+        t.batch, t.heads_q, t.heads_kv, t.n, t.head_dim = 1, hq, 1, n, 128
+        return lib.minf_attn_workspace_bytes(ctypes.byref(t), op, wide_v, wide, 0)
+    vs, bs = _lib.MINF_OP_VERTICAL_SLASH, _lib.MINF_OP_BLOCK_SPARSE
+    for n, hq in ((1500, 1), (4000, 4), (8192, 1), (8192, 4)):
+        assert nbytes(bs, n, hq, 0, 10) == 0 and nbytes(vs, n, hq, 30, 50) == 0
+        assert nbytes(bs, n, hq, 0, (n + 63) // 64) == nbytes(bs, n, hq, 0, 0) > 0
+        assert nbytes(vs, n, hq, 1000, 6096) == nbytes(vs, n, hq, 0, 0) > 0
+    assert nbytes(bs, 6000, 4, 0, 20) == 0 < nbytes(bs, 6000, 1, 0, 20)
+    assert nbytes(vs, 4096, 4, 3500, 100) > 0                # a few blocks, 55 column tiles
+
+
+@pytest.mark.parametrize("n,hq,top_k,nv,ns", [(2111, 2, 17, 1000, 100), (4033, 1, 33, 600, 90)])
+def test_split_walks_of_narrow_lists(gpu, n, hq, top_k, nv, ns):
+    """Segments cut for the width of the list: block lists that end inside a segment's length, and scattered
+    slashes whose walks are longer than the neighbouring ones that the cut assumes."""
+    import minference_amd as M
+    q, k, v = make(1, hq, hq, n, n, torch.bfloat16)
+    qg, kg, vg = q.to(gpu), k.to(gpu), v.to(gpu)
+    bi = M.ops._build_block_index(qg, kg, top_k)
+    ref = torch.stack([O.masked_attention(q[0, h], k[0, h], v[0, h], O.bs_mask(bi[0, h].cpu().numpy(), n)) for h in range(hq)])
+    check(M.block_sparse_attention(qg, kg, vg, top_k), ref[None], "block-sparse")
+    vi, si = gen.vs_index_inputs(hq, n, nv, ns, seed=9)
+    vi, si = torch.from_numpy(vi), torch.from_numpy(si.copy())
+    check(M.vertical_slash_sparse_attention(qg, kg, vg, vi.to(gpu), si.to(gpu)),
+          O.vertical_slash_sparse_attention(q, k, v, vi, si), "vertical-slash")
+
+
 @pytest.mark.parametrize("hq,hk,n,b", [(3, 1, 900, 1), (6, 3, 700, 2), (10, 5, 13400, 1)])
 def test_striped_row_blocks_cover_every_row(gpu, hq, hk, n, b):
     """Head counts that do not divide among the eight XCDs: the row-block pairs are dealt out in stripes
