@@ -189,7 +189,9 @@ typedef struct minf_qkvo {
     /* Optional scratch memory for split walks, 16-byte aligned: with at least
      * minf_attn_workspace_bytes() bytes here, launches that would leave the chip idle (few row blocks,
      * or a few walks far longer than the rest) cut their walks into segments and fold the partial
-     * sums in a second small kernel.  NULL or too small: every walk is made by one workgroup. */
+     * sums in a second small kernel.  The number of segments depends on the launch (batch, heads, n, list
+     * widths), and with it the order of a head's fp32 sums: other heads in the launch, other last bits.
+     * NULL or too small: every walk is made by one workgroup, in one order. */
     void *workspace;
     size_t workspace_bytes;
     /* With dtype MINF_16BIT_SELECT: device word that holds MINF_BF16 or MINF_F16, what q, k, v and o

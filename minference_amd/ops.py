@@ -8,11 +8,18 @@ Same callables, argument names and defaults as the reference package
 * ``streaming_forward``                minference/ops/streaming_kernel.py:611-646
 
 Inputs are ``[batch, heads, n, head_dim]`` GPU tensors (any strides); the
-result is a new tensor of the query's shape and dtype.  In addition to the
-reference, K/V may have fewer heads than Q (grouped-query attention) and are
-then read in place instead of being expanded.  All arithmetic runs in
-libminf_hip.so on the caller's current stream; torch is only used for memory,
-and the index sort of the vertical-slash wrapper.
+result is a new tensor of the query's shape and dtype, or ``out`` where an
+operator takes one.  In addition to the reference, K/V may have fewer heads than
+Q (grouped-query attention) and are then read in place instead of being expanded.
+All arithmetic runs in libminf_hip.so on the caller's current stream; torch is
+only used for memory, for padding and casts of operands the kernels do not take as
+they are, and for index rows of more than 16384 values.
+
+Calls are deterministic.  A launch that would leave the chip idle cuts its walks
+over the keys into segments, as many as its load asks for: dense attention and the
+dense rows of tri-shape at any length, the others up to 8192 tokens.  There a head
+that shares its call with other heads or batches may differ in its last bits from the
+same head on its own.
 """
 from __future__ import annotations
 

@@ -445,3 +445,24 @@ def test_mixed_layer_replays_from_a_hip_graph(gpu):
         torch.cuda.synchronize()
         assert torch.isfinite(got.float()).all()
         assert torch.equal(got, eager), f"replay {rep} differs from the eager call"
+
+
+@pytest.mark.parametrize("n,hq,hk", [(1000, 8, 2), (2300, 8, 2), (4096, 32, 8), (8192, 16, 4)])
+def test_short_mixed_layers_against_per_head_calls(gpu, n, hq, hk):
+    """Up to 8192 tokens the walks of a launch are cut by its load and its list widths, so a head of a mixed layer
+    and the same head on its own may sum the same keys in another order.  Its selections are the same; each
+    side is within 3 x 2^-9 of sum p |v| of the exact rows (numerator, row sum and result rounded to 8 bits),
+    so the two are within 3 x 2^-8 of it (2^-6 with the rounding of that sum itself)."""
+    import minference_amd as M
+    q, k, v, _ = gen.planted_layer(n, hq, hk, seed=n, dtype=torch.bfloat16)
+    qg, kg, vg = q.to(gpu), k.to(gpu), v.to(gpu)
+    layer = _ragged_table(hq)
+    layer["6"] = ["stream_llm", 100, 800, 1.0]
+    kwargs = {"layer_idx": 0, "attn_forward_config": {"best_pattern": [layer]}}
+    out, mass = (M.minference_prefill_forward(qg, kg, x, kwargs).float() for x in (vg, vg.abs()))
+    for h in range(hq):
+        one = lambda x: x[:, h // (hq // hk):h // (hq // hk) + 1]
+        ty, a, b, _ = layer[str(h)]
+        got = M.minference_prefill_forward(qg[:, h:h + 1], one(kg), one(vg), {"layer_idx": 0, "attn_forward_config": {
+            "best_pattern": [{"0": [ty, a, b, 1.0]}]}}).float()
+        assert ((out[:, h:h + 1] - got).abs() <= 2.0 ** -6 * mass[:, h:h + 1]).all(), (h, ty)
