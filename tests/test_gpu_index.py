@@ -219,18 +219,30 @@ def test_config3_shape_bit_exact(gpu):
 @pytest.mark.parametrize("n,batch", [(64, 1), (1000, 2), (4097, 3)])
 def test_counts_are_written_for_every_row_and_full_sequences_need_no_lengths(gpu, n, batch):
     """Payload-only builds into memory that holds other values: row blocks past a sequence get zero counts from
-    the kernel itself (both builders), and a build without sequence lengths equals one with full ones."""
+    the kernel itself (every builder), and a build without sequence lengths equals one with full ones."""
+    from minference_amd import _lib
     from minference_amd.index import _build, convert_vertical_slash_indexes
     v, s = gen.vs_index_inputs(2, n, min(n, 60), min(n, 90), seed=n, batch=batch)
     vg, sg = torch.from_numpy(v).to(gpu), torch.from_numpy(s.copy()).to(gpu)
     lens = torch.tensor([n, max(1, n // 2), 1][:batch], dtype=torch.int32, device=gpu)
     full = torch.full((batch,), n, dtype=torch.int32, device=gpu)
-    junk = torch.full((4, 1 << 16), 77, dtype=torch.int32, device=gpu)
-    del junk                                                   # (the caching allocator hands it out again)
+    lib = _lib.load()
+    H, V, S, rows = 2, vg.shape[2], sg.shape[2], (n + 63) // 64
+    ws_bytes = lib.minf_vs_index_workspace_bytes(batch, H, S, rows)
     for seqlens in (lens, full):
         want = convert_vertical_slash_indexes(seqlens, vg, sg, n)
-        for tables in (True, False):
-            got = convert_vertical_slash_indexes(seqlens, vg, sg, n, zero_fill=False, use_tables=tables)
-            assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2]), tables
+        for builder in ("minf_vs_index_build", "minf_vs_index_build_ws", "minf_vs_index_build_full_ws"):
+            if builder == "minf_vs_index_build_full_ws" and seqlens is lens:
+                continue
+            got = [torch.full_like(t, 77) for t in want]
+            ws = torch.full((max(ws_bytes, 4),), 77, dtype=torch.uint8, device=gpu)
+            args = [seqlens.data_ptr()] if builder != "minf_vs_index_build_full_ws" else []
+            args += [t.data_ptr() for t in (vg, sg, *got)] + [batch, H, rows, V, S, 0, None]
+            args += [ws.data_ptr(), ws_bytes] if builder != "minf_vs_index_build" else []
+            assert getattr(lib, builder)(*args, _lib.stream_ptr(gpu)) == 0
+            assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2]), builder
+            for count, payload, ref in ((got[0], got[1], want[1]), (got[2], got[3], want[3])):
+                live = torch.arange(payload.shape[-1], device=gpu) < count[..., None]
+                assert torch.equal(payload[live], ref[live]), builder
     got = _build(None, vg, sg, n, zero_fill=True)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
