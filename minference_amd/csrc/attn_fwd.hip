@@ -187,20 +187,6 @@ template <> __device__ __forceinline__ float pair_sum<_Float16>(const Frag &f, f
     for (int j = 0; j < 4; ++j) { f16x2_t pr = {f.h[2 * j], f.h[2 * j + 1]}; acc = __builtin_amdgcn_fdot2(pr, one, acc, false); }
     return acc;
 }
-// 16 bytes per lane from its own global address into LDS at a wave-uniform base (lane i -> base +
-// 16 i).  Written as assembly because the compiler counts the builtin's instruction as a "flat" access,
-// which may touch the LDS counter out of order: one of them on any path through the tile loop turned
-// every wait for a fragment read into a wait for ALL outstanding reads (lgkmcnt(0): the first PV MFMA
-// waited for the whole V tile, every second k-step for the reads issued just before it).  The copies
-// are counted by vmcnt alone, and the loop waits for vmcnt(0) before each barrier.  131072-token
-// vertical-slash layer 15.15 -> 15.0 ms, 16001 tokens 1.68 -> 1.66 ms; on all-zero operands 1.52 -> 1.50
-// (dense, 16384 tokens): little, because a SIMD's other wave filled most of those waits and the chip
-// holds a lower clock on live data whatever the schedule.
-__device__ __forceinline__ void copy16_to_lds(const char *src, char *dst) {
-    const int lds = (int)(unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)dst;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
-}
-
 // One tile of keys: either 64 consecutive tokens from `start`, or 64 gathered
 // token ids read from `gather` (entries >= nvalid are padding).
 struct Tile {

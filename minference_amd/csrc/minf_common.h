@@ -23,3 +23,17 @@ __device__ __forceinline__ uint64_t minf_lanemask_lt() {
 __device__ __forceinline__ int minf_readlane(int x, int src) {
     return __builtin_amdgcn_readlane(x, __builtin_amdgcn_readfirstlane(src));
 }
+
+// 16 bytes per lane from its own global address into LDS at a wave-uniform base (lane i -> base +
+// 16 i).  Written as assembly because the compiler counts the builtin's instruction as a "flat" access,
+// which may touch the LDS counter out of order: one of them on any path through a loop turns every wait
+// for a fragment read into a wait for ALL outstanding reads (lgkmcnt(0): in the attention walk the first PV
+// MFMA waited for the whole V tile, every second k-step for the reads issued just before it).  The copies
+// are counted by vmcnt alone, and the callers wait for vmcnt(0) before each barrier.  Attention: 16001-token
+// vertical-slash layer 1.68 -> 1.66 ms, dense 16384 tokens on all-zero operands 1.52 -> 1.50; nothing beyond noise
+// at 131072 tokens: a SIMD's other wave filled most of those waits, and the chip holds a lower clock on live
+// data whatever the schedule.
+__device__ __forceinline__ void copy16_to_lds(const char *src, char *dst) {
+    const int lds = (int)(unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)dst;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
+}

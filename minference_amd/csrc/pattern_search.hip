@@ -81,12 +81,6 @@ __device__ __forceinline__ unsigned load_u32_unaligned(const unsigned char *p) {
     return w;
 }
 
-// (see copy16_to_lds in attn_fwd.hip: assembly keeps the LDS read counter in order)
-__device__ __forceinline__ void copy16_to_lds(const char *src, char *dst) {
-    const int lds = (int)(unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)dst;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
-}
-
 // two values rounded to bf16 (nearest), and what the rounding left of each: one instruction per value
 __device__ __forceinline__ unsigned pack_bf16(float x, float y) {
     const f32x2_t v = {x, y};
