@@ -1,8 +1,10 @@
 // Top-k index selection over fp32 score rows for gfx950 (vertical / slash
 // candidates: k = 1000 / 6096 of up to ~10^6 entries per head).
 //
-// Rows longer than 4096 entries, one 1024-thread workgroup per row (shorter rows: one wavefront
-// per row, see topk_wave_kernel):
+// Three kernels (launch_topk): rows of 257 .. 4096 entries in launches of up to TK_FEW_ROWS rows, and all of
+// 4097 .. 16384, are selected from the registers of a workgroup (topk_regs_kernel); other rows of up to 4096
+// entries, and rows read to the diagonal only, by one wavefront each (topk_wave_kernel).  Longer rows, one 1024-thread
+// workgroup per row (topk_kernel):
 //   1. MSB-first radix select (4 x 8 bits, LDS histogram) finds the exact value
 //      T of the k-th largest entry and how many entries equal to T are needed;
 //   2. every wavefront counts, over its contiguous slice, entries > T and == T;

@@ -144,11 +144,10 @@ def test_ragged_topk_pads_with_noop_entries(gpu, n):
                                               # workgroup with waves past the last chunk
                                               (14, 2, 40001, torch.bfloat16, 64), (16, 8, 20481, torch.float16, 128)])
 def test_a_heads_scores_do_not_depend_on_the_heads_it_is_launched_with(gpu, hq, hk, n, dtype, d):
-    """Grouped-query launches score four (or two) heads per workgroup, one wave per head over a whole
-    2048-key chunk; a head on its own is scored by four waves of 512 keys.  Both sum a chunk as the same
-    four pieces in the same order, so the score vectors -- and with them the selected sets and the
-    attention output of the per-head dispatcher -- are identical bit for bit however the heads are
-    grouped into launches."""
+    """Grouped-query launches score four (or two) heads per workgroup, one wave per head over a whole chunk of
+    keys (128 .. 512 of them at these lengths); a head on its own is scored by four waves of a quarter each.  Both
+    sum a chunk as the same four pieces in the same order, so the score vectors -- and with them the selected
+    sets -- are identical bit for bit however the heads are grouped into launches."""
     from minference_amd.estimate import vertical_slash_scores
     q, k, _ = gen.qkv(1, hq, hk, n, d, seed=n + hq, scale=1.0)
     qg, kg = q.to(dtype).to(gpu), k.to(dtype).to(gpu)
