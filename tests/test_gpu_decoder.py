@@ -35,6 +35,18 @@ def test_add_rms_norm(gpu, dtype, rows, dim):
         assert torch.equal(h, want_h) and close(out, want, dtype)
 
 
+@pytest.mark.parametrize("dim", [1000, 3072, 4096, 16384])
+def test_rms_norm_of_fp32_rows_rounds_three_times(gpu, dim):
+    """Against fp64: the root, its product with the row and that with the weight are rounded once each, the sum is
+    not: a relative error of 2^-24 sqrt(3 / 3 * E[m^-2]) = 0.736 * 2^-24 over log-uniform significands m
+    (0.76 for the sample; a sum in fp32 gives 0.85 and more)."""
+    m = model(dim, torch.float32, gpu)
+    g = torch.Generator(device=gpu).manual_seed(dim)
+    x, w = torch.randn(4096, dim, device=gpu, generator=g), torch.randn(dim, device=gpu, generator=g)
+    want = x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + m.cfg.rms_eps) * w.double()
+    assert (m._rms(x, w).double() - want).norm() <= 0.76 * 2.0 ** -24 * want.norm()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("n,hq,hk,d", [(1, 1, 1, 128), (33, 5, 2, 128), (70, 2, 1, 96), (9, 3, 3, 20), (5, 1, 1, 6)])
 def test_rope_in_place(gpu, dtype, n, hq, hk, d):
