@@ -34,11 +34,14 @@ _NATIVE_D = (64, 128)         # head_dims every kernel is instantiated for; othe
 _NATIVE_D_STREAMING = (64, 128, 256)   # ... and the A-shape / tri-shape / dense kernels also for 256
 
 
+def _aligned_rows(t: torch.Tensor) -> bool:
+    """16-byte aligned rows with unit head_dim stride."""
+    return t.stride(-1) == 1 and not any(s % 8 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
+
+
 def _prep(t: torch.Tensor) -> torch.Tensor:
-    """16-byte aligned rows with unit head_dim stride (copies only if needed)."""
-    if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]) or t.data_ptr() % 16:
-        t = t.contiguous()
-    return t
+    """Rows the kernels take (copies only if needed)."""
+    return t if _aligned_rows(t) else t.contiguous()
 
 
 def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
@@ -134,7 +137,7 @@ class _Call:
         # twice and by the launches of other pattern types
         self.out = out
         if out is not None and tuple(out.shape) == (B, H, N, Dk) and out.dtype == self.q.dtype == self.out_dtype \
-                and out.device == q.device and out.stride(2) >= Dk and _prep(out) is out \
+                and out.device == q.device and out.stride(2) >= Dk and _aligned_rows(out) \
                 and not any(_overlap(out, t) for t in (self.q, self.k, self.v)):
             self.o = out
         else:

@@ -49,3 +49,18 @@ def test_which_views_share_memory():
     assert _overlap(x, x) and _overlap(x, x[1:, 2:, 9:, 7:]) and not _overlap(x[:1], x[1:]) and not _overlap(x[0, :, :4], x[1])
     assert _overlap(x[..., :4], x[..., 4:]) and not _overlap(x, torch.empty_like(x)) and not _overlap(x[:, :0], x)
     assert _overlap(x.transpose(1, 2)[:, 5:], x[0, 0, 9:]) and _overlap(x[:1, :1, :1].expand(2, 3, 10, 8), x[0, 0, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", sorted(OPS))
+def test_out_need_not_be_aligned(gpu, op):
+    """A contiguous ``out`` that starts an element past a 16-byte boundary, and one whose rows are not whole
+    16-byte vectors apart, take the bits of a call without."""
+    import minference_amd as M
+    n, H, d = 700, 2, 128
+    q, k, v = (t.bfloat16().to(gpu) for t in gen.qkv(1, H, H, n, d, seed=4, scale=1.0))
+    want = OPS[op](M, q, k, v, None)
+    shifted = torch.zeros(q.numel() + 8, dtype=q.dtype, device=gpu)[1:1 + q.numel()].view(q.shape)
+    padded = torch.zeros(1, H, n, d + 3, dtype=q.dtype, device=gpu)[..., :d]
+    for out in (shifted, padded):
+        assert OPS[op](M, q, k, v, out) is out and torch.equal(out, want)
