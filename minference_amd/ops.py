@@ -35,8 +35,9 @@ _NATIVE_D_STREAMING = (64, 128, 256)   # ... and the A-shape / tri-shape / dense
 
 
 def _aligned_rows(t: torch.Tensor) -> bool:
-    """16-byte aligned rows with unit head_dim stride."""
-    return t.stride(-1) == 1 and not any(s % 8 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
+    """16-byte aligned rows (of [B, H, N, D] tensors) with unit head_dim stride."""
+    s0, s1, s2, s3 = t.stride()
+    return s3 == 1 and not (s0 | s1 | s2) & 7 and not t.data_ptr() & 15
 
 
 def _prep(t: torch.Tensor) -> torch.Tensor:
@@ -92,6 +93,7 @@ def _check_qkv(q, k, v):
 class _Call:
     """Holds the (possibly cast/padded) tensors of one operator call and the
     filled ``minf_qkvo`` struct."""
+    _scratch = None
 
     def __init__(self, q, k, v, seqlens=None, need_out=True, native_dims=_NATIVE_D, sm_scale=None, out=None,
                  attention_only=False):
@@ -194,10 +196,11 @@ class _Call:
         """Give the next launch of ``op`` the scratch memory its split walks use (none for most).  List operators:
         n_init / n_local are the widths of the column / block lists."""
         nbytes = _lib.load().minf_attn_workspace_bytes(self.ref, op, int(n_init), int(n_local), int(n_last))
-        # (a block freed here is reused only by later work on the same stream)
-        self._scratch = torch.empty(nbytes, dtype=torch.uint8, device=self.q.device) if nbytes else None
-        self.struct.workspace = self._scratch.data_ptr() if nbytes else None
-        self.struct.workspace_bytes = nbytes
+        if nbytes or self._scratch is not None:
+            # (a block freed here is reused only by later work on the same stream)
+            self._scratch = torch.empty(nbytes, dtype=torch.uint8, device=self.q.device) if nbytes else None
+            self.struct.workspace = self._scratch.data_ptr() if nbytes else None
+            self.struct.workspace_bytes = nbytes
 
     def result(self):
         o = self.o

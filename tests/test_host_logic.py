@@ -163,3 +163,19 @@ def test_layer_plan_is_cached_per_table_object_and_checks_head_coverage():
         prefill._layer_plan(cfg([{"0": ["no_such_pattern", 1, 1, 0.5]}]), 0, 1)
     prefill.clear_plan_cache()
     assert prefill._layer_plan(config, 0, 3) is not a
+
+
+def test_which_rows_the_kernels_take():
+    """Unit head_dim stride, every other stride whole 16-byte vectors, start on one; against the rule stride by stride."""
+    from minference_amd.ops import _aligned_rows
+    buf = torch.zeros(1 << 14, dtype=torch.bfloat16)
+    base = buf[(-buf.data_ptr() // 2) % 8:]                    # starts on a 16-byte boundary
+    seen = set()
+    for offset in (0, 1, 4, 8):
+        for strides in ((2048, 512, 64, 1), (0, 0, 64, 1), (2048, 512, 68, 1), (2048, 516, 64, 1), (2052, 512, 64, 1),
+                        (2048, 64, 512, 1), (2048, 512, 64, 2), (1, 8, 16, 24), (0, 0, 0, 0), (0, 0, 0, 1)):
+            t = base[offset:].as_strided((2, 2, 4, 8), strides)
+            want = strides[3] == 1 and all(s % 8 == 0 for s in strides[:3]) and offset % 8 == 0
+            assert _aligned_rows(t) == want, (offset, strides)
+            seen.add(want)
+    assert seen == {True, False}
