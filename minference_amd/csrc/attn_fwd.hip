@@ -987,7 +987,6 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     {
         float l_tot = l_i + __shfl_xor(l_i, 32);
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-        // pitch: 8-byte lane writes spread over all banks (four waves only fit without the pad)
         constexpr int OP = ROW_BYTES;
         // a row sum at 2^100 or beyond (or infinite, or no number at all): some probability may have
         // overflowed.  Compared on the bit pattern: the library is compiled without NaN semantics, which
@@ -1019,6 +1018,10 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         }
         __syncthreads();                                  // K/V tiles no longer needed
         char *ot = (half ? lds_v : lds_k) + wave * 32 * OP;    // 32 rows per wave
+        // the 16-byte chunks of a row are permuted like those of a K tile: at a row's own pitch all 32 rows' writes of
+        // one instruction went to one pair of banks, and a workgroup's epilogue took 5.1 us of its 34 (A-shape, window
+        // 512, head_dim 128) where it takes 3.4 now: A-shape, 100000 tokens, window 3968, 32 / 8 heads 6486 -> 6430 us; 16
+        // heads of 64, 24000 tokens, window 512 138.5 -> 134.9; dense, 2 x 6144 tokens, 32 / 8 heads 594 -> 588
         const bool live = qrow < seqlen;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
@@ -1027,7 +1030,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
                 union { T e[4]; u32x2_t u; } out4;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) out4.e[e] = live ? (T)(oacc[db][rq * 4 + e] * inv) : (T)0.f;
-                *reinterpret_cast<u32x2_t *>(ot + l32 * OP + (32 * db + 8 * rq + 4 * g) * 2) = out4.u;
+                *reinterpret_cast<u32x2_t *>(ot + l32 * OP + (((4 * db + rq) ^ swz_k(l32)) << 4) + 8 * g) = out4.u;
             }
         __builtin_amdgcn_wave_barrier();
         // lane -> (row = RPI*i + lane/NCH, chunk = lane%NCH)
@@ -1035,7 +1038,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         for (int i = 0; i < 32 / RPI; ++i) {
             const int r = RPI * i + lane / NCH;
             const int grow = row0 + wave * 32 + r;
-            const u32x4_t val = *reinterpret_cast<const u32x4_t *>(ot + r * OP + (lane % NCH) * 16);
+            const u32x4_t val = *reinterpret_cast<const u32x4_t *>(ot + r * OP + (((lane % NCH) ^ swz_k(r)) << 4));
             if (grow < p.n && have_rows) *reinterpret_cast<u32x4_t *>(o_base + (long long)grow * p.os[2] * 2 + (lane % NCH) * 16) = val;
         }
     }
