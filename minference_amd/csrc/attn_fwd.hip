@@ -240,7 +240,8 @@ __device__ __forceinline__ bool tile_on_list(const AttnParams &p, int m, int sta
 template <int MODE, int HD> struct AttnLds {
     static constexpr bool VSP = MODE == MODE_VS || MODE == MODE_BS;      // walks of two block lists
     static constexpr int TILE_BYTES = BN * HD * 2;
-    static constexpr int NK = (VSP ? 2 : 1) * TILE_BYTES;
+    static constexpr int NK = 2 * TILE_BYTES;                            // (the epilogue's 128 rows of O, too)
+    static constexpr int NV = (VSP ? 2 : 1) * TILE_BYTES;
     static constexpr int NONLY = VSP ? 2 * VS_ONLY_MAX : 1;
 };
 
@@ -251,7 +252,7 @@ template <int MODE, int HD> struct AttnLds {
 // EVERY_MAX (the output it wrote is then overwritten).
 template <typename T, int MODE, int HD, bool EVERY_MAX, bool CUT>
 __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[AttnLds<MODE, HD>::NK],
-                                          char (&lds_v)[AttnLds<MODE, HD>::NK],
+                                          char (&lds_v)[AttnLds<MODE, HD>::NV],
                                           int (&vs_only)[AttnLds<MODE, HD>::NONLY], int (&vs_wsum)[4], int &vs_bad,
                                           int &lds_redo) {
     static_assert(HD == 256 || HD == 128 || HD == 64, "head_dim 64, 128 or 256");
@@ -988,22 +989,24 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         float l_tot = l_i + __shfl_xor(l_i, 32);
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
         constexpr int OP = ROW_BYTES;
-        // a row sum at 2^100 or beyond (or infinite, or no number at all): some probability may have
-        // overflowed.  Compared on the bit pattern: the library is compiled without NaN semantics, which
-        // lets the compiler turn !(l < x) into l >= x -- false for the NaN that inf * 0 leaves in a
-        // row sum when the maximum is raised after an overflow
-        // ... and an accumulator that is infinite or no number: O^T sums twice as many terms per tile
-        // as a lane's share of the row sum (and terms scaled by |v|), so it can overflow while the row
-        // sum still fits, and a later rescale then hides the size of the sum but not the inf / NaN
-        if constexpr (!every_max) {
-            unsigned obits = 0;
+        auto check_range = [&]() {
+            // a row sum at 2^100 or beyond (or infinite, or no number at all): some probability may have
+            // overflowed.  Compared on the bit pattern: the library is compiled without NaN semantics, which
+            // lets the compiler turn !(l < x) into l >= x -- false for the NaN that inf * 0 leaves in a
+            // row sum when the maximum is raised after an overflow
+            // ... and an accumulator that is infinite or no number: O^T sums twice as many terms per tile
+            // as a lane's share of the row sum (and terms scaled by |v|), so it can overflow while the row
+            // sum still fits, and a later rescale then hides the size of the sum but not the inf / NaN
+            if constexpr (!every_max) {
+                unsigned obits = 0;
 #pragma unroll
-            for (int i = 0; i < NDB; ++i)
+                for (int i = 0; i < NDB; ++i)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) obits = max(obits, __float_as_uint(oacc[i][r]) & 0x7fffffffu);
-            const bool suspect = (__float_as_uint(l_tot) & 0x7fffffffu) >= __float_as_uint(0x1p100f) || obits >= 0x7f800000u;
-            if (__any(suspect) && lane == 0) lds_redo = 1;
-        }
+                    for (int r = 0; r < 16; ++r) obits = max(obits, __float_as_uint(oacc[i][r]) & 0x7fffffffu);
+                const bool suspect = (__float_as_uint(l_tot) & 0x7fffffffu) >= __float_as_uint(0x1p100f) || obits >= 0x7f800000u;
+                if (__any(suspect) && lane == 0) lds_redo = 1;
+            }
+        };
         if (CUT && slot) {                               // a segment: the sums as they are (16 bytes per lane, contiguous)
             char *acc = slot + (wave_wg * NDB * 4 * 64 + lane) * 16;
 #pragma unroll
@@ -1013,11 +1016,14 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
                     *reinterpret_cast<float4 *>(acc + (db * 4 + rq) * 1024) =
                         make_float4(oacc[db][rq * 4], oacc[db][rq * 4 + 1], oacc[db][rq * 4 + 2], oacc[db][rq * 4 + 3]);
             *(reinterpret_cast<float2 *>(slot + SplitSlot<HD>::ACC) + tid) = make_float2(m_i, l_tot);
+            check_range();
             __syncthreads();
             return !every_max && lds_redo != 0;           // (workgroup-uniform)
         }
-        __syncthreads();                                  // K/V tiles no longer needed
-        char *ot = (half ? lds_v : lds_k) + wave * 32 * OP;    // 32 rows per wave
+        // 32 rows per wave, in the K tiles: everyone was done with those at the last step's second barrier, so a
+        // wave need not wait for the others' last softmax (tri-shape, 16 heads of 64, 24000 tokens 137.4 -> 135.8 us,
+        // dense, 2 x 6144 tokens, 32 / 8 heads 591 -> 587)
+        char *ot = lds_k + wave_wg * 32 * OP;
         // the 16-byte chunks of a row are permuted like those of a K tile: at a row's own pitch all 32 rows' writes of
         // one instruction went to one pair of banks, and a workgroup's epilogue took 5.1 us of its 34 (A-shape, window
         // 512, head_dim 128) where it takes 3.4 now: A-shape, 100000 tokens, window 3968, 32 / 8 heads 6486 -> 6430 us; 16
@@ -1029,7 +1035,8 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             for (int rq = 0; rq < 4; ++rq) {
                 union { T e[4]; u32x2_t u; } out4;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) out4.e[e] = live ? (T)(oacc[db][rq * 4 + e] * inv) : (T)0.f;
+                for (int e = 0; e < 4; ++e) out4.e[e] = (T)(oacc[db][rq * 4 + e] * inv);
+                if (!live) out4.u = u32x2_t{0u, 0u};
                 *reinterpret_cast<u32x2_t *>(ot + l32 * OP + (((4 * db + rq) ^ swz_k(l32)) << 4) + 8 * g) = out4.u;
             }
         __builtin_amdgcn_wave_barrier();
@@ -1041,8 +1048,10 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             const u32x4_t val = *reinterpret_cast<const u32x4_t *>(ot + r * OP + (((lane % NCH) ^ swz_k(r)) << 4));
             if (grow < p.n && have_rows) *reinterpret_cast<u32x4_t *>(o_base + (long long)grow * p.os[2] * 2 + (lane % NCH) * 16) = val;
         }
+        check_range();                                    // (while the stores are on their way)
     }
-    // (the flag was written before the barrier at the head of the epilogue)
+    if constexpr (every_max) return false;
+    __syncthreads();                                      // (the flag is known)
     return !every_max && lds_redo != 0;                   // (workgroup-uniform)
 }
 
@@ -1054,7 +1063,7 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
     typedef AttnLds<MODE, HD> L;
     if (p.select && *as_const(p.select) != dtype_code<T>()) return;
     __shared__ __attribute__((aligned(16))) char lds_k[L::NK];
-    __shared__ __attribute__((aligned(16))) char lds_v[L::NK];
+    __shared__ __attribute__((aligned(16))) char lds_v[L::NV];
     __shared__ int vs_only[L::NONLY];        // paired list walks: [row block][entries the other list lacks]
     __shared__ int vs_wsum[4];
     __shared__ int vs_bad;
