@@ -253,7 +253,7 @@ template <int MODE, int HD> struct AttnLds {
 template <typename T, int MODE, int HD, bool EVERY_MAX, bool CUT>
 __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[AttnLds<MODE, HD>::NK],
                                           char (&lds_v)[AttnLds<MODE, HD>::NV],
-                                          int (&vs_only)[AttnLds<MODE, HD>::NONLY], int (&vs_wsum)[4], int &vs_bad,
+                                          int (&vs_only)[AttnLds<MODE, HD>::NONLY], int (&vs_wsum)[4], int (&vs_bad)[2],
                                           int &lds_redo) {
     static_assert(HD == 256 || HD == 128 || HD == 64, "head_dim 64, 128 or 256");
     static_assert(HD <= 128 || !(MODE == MODE_VS || MODE == MODE_BS), "the list walks are built for head_dim <= 128");
@@ -376,10 +376,18 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     [[maybe_unused]] int vs_na = 0, vs_nb = 0, vs_cca = 0, vs_ccb = 0, vs_nc = 0;
     [[maybe_unused]] bool vs_merged = false;
     [[maybe_unused]] long long vs_ra = 0, vs_rb = 0;
+    [[maybe_unused]] const int *ga = nullptr, *gb = nullptr;
+    [[maybe_unused]] int vs_head_a = 0, vs_head_b = 0;
     if constexpr (VSP) {
         const bool b_exists = 2 * mslot + 1 < p.rows && (2 * mslot + 1) * BM < seqlen;
         vs_ra = ((long long)b * p.index_heads + hs) * list_rows + mA;
         vs_rb = b_exists ? vs_ra + 1 : vs_ra;
+        // the lists' first 256 entries are fetched beside their lengths, not after them (a list row has list_w
+        // entries whatever its length)
+        ga = list_base + vs_ra * list_w;
+        gb = list_base + vs_rb * list_w;
+        vs_head_a = ga[min(tid, list_w - 1)];
+        vs_head_b = gb[min(tid, list_w - 1)];
         if constexpr (MODE == MODE_BS) {
             // row block m visits the first min(m + 1, max_blocks) entries of its row; no columns
             vs_na = min(mA + 1, p.max_blocks);
@@ -437,7 +445,11 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // loop: both lists are staged in LDS, every entry looks itself up in the other list by binary
     // search, and a workgroup prefix sum over the hits places it either in the list of COMMON
     // entries (tiles that both row blocks visit: copied once by four waves, one LDS word per step)
-    // or in its row block's list of entries the other one lacks (run ends).  The walk is then
+    // or in its row block's list of entries the other one lacks (run ends).  Each pair of waves looks up one
+    // list, both at once; with a pass per list and a check before them a workgroup took 6.5 us to its first tile
+    // copy (block-sparse, top-100; 2.9 of them chains of LDS reads and six barriers) where it takes 3.4 now:
+    // vertical-slash, 16001 tokens, 32 / 8 heads 1531 -> 1519 us, block-sparse, 32768 tokens 2909 -> 2892.
+    // The walk is then
     //   common tiles, both halves computing;
     //   split steps: every half visits its own leftover tiles -- the entries the other list lacks,
     //   then its gathered column tiles -- with the K/V buffers of its own half,
@@ -449,58 +461,51 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         if (vs_na <= VS_PAIR_MAX && vs_nb <= VS_PAIR_MAX && vs_na > 0 && vs_nb > 0) {
             int *rawA = reinterpret_cast<int *>(lds_k1), *rawB = rawA + VS_PAIR_MAX;
             int *common = reinterpret_cast<int *>(lds_v1);
-            const int *ga = list_base + vs_ra * list_w, *gb = list_base + vs_rb * list_w;
-            if (tid == 0) vs_bad = 0;
-            for (int i = tid; i < vs_na; i += NT) rawA[i] = ga[i] * LIST_SCALE;
-            for (int i = tid; i < vs_nb; i += NT) rawB[i] = gb[i] * LIST_SCALE;
+            if (tid < 2) vs_bad[tid] = 0;
+            if (tid < vs_na) rawA[tid] = vs_head_a * LIST_SCALE;
+            if (tid < vs_nb) rawB[tid] = vs_head_b * LIST_SCALE;
+            for (int i = tid + NT; i < vs_na; i += NT) rawA[i] = ga[i] * LIST_SCALE;
+            for (int i = tid + NT; i < vs_nb; i += NT) rawB[i] = gb[i] * LIST_SCALE;
             __syncthreads();
-            bool bad = false;                              // the look-ups need strictly ascending lists
-            for (int i = tid; i + 1 < vs_na; i += NT) bad |= rawA[i + 1] <= rawA[i];
-            for (int i = tid; i + 1 < vs_nb; i += NT) bad |= rawB[i + 1] <= rawB[i];
-            if (__any(bad) && lane == 0) vs_bad = 1;
-            __syncthreads();
-            if (!vs_bad) {                                 // (workgroup-uniform)
-                const unsigned long long lt = (1ull << lane) - 1ull;
-                // entry i of `mine` goes to common[#hits before i] when `other` holds it too (first
-                // pass only), else to only[i - #hits before i]; -> number of hits
-                auto pass = [&](const int *mine, int nmine, const int *other, int nother, int *only, bool write_common) {
-                    int carry = 0;
-                    for (int base = 0; base < nmine; base += NT) {        // uniform trip count
-                        const int i = base + tid;
-                        const bool valid = i < nmine;
-                        const int x = valid ? mine[i] : 0;
-                        int lo = 0, hi = nother;                           // first entry of `other` >= x
-                        while (lo < hi) {
-                            const int mid = (lo + hi) >> 1;
-                            if (other[mid] < x) lo = mid + 1; else hi = mid;
-                        }
-                        const bool eq = valid && lo < nother && other[lo] == x;
-                        const unsigned long long bal = __ballot(eq);
-                        if (lane == 0) vs_wsum[wave_wg] = __builtin_popcountll(bal);
-                        __syncthreads();
-                        int pre = carry, tot = 0;
-#pragma unroll
-                        for (int w = 0; w < 4; ++w) {
-                            const int c = vs_wsum[w];
-                            pre += w < wave_wg ? c : 0;
-                            tot += c;
-                        }
-                        pre += __builtin_popcountll(bal & lt);
-                        if (valid) {
-                            if (eq) { if (write_common) common[pre] = x; }
-                            else if (i - pre < VS_ONLY_MAX) only[i - pre] = x;
-                        }
-                        carry += tot;
-                        __syncthreads();
-                    }
-                    return carry;
-                };
-                vs_nc = pass(rawA, vs_na, rawB, vs_nb, vs_only, true);
-                pass(rawB, vs_nb, rawA, vs_na, vs_only + VS_ONLY_MAX, false);
-                // (the last barrier of the passes also orders these LDS lists before their readers)
-                vs_merged = vs_nc > 0 && vs_na - vs_nc <= VS_ONLY_MAX && vs_nb - vs_nc <= VS_ONLY_MAX;
-                if (!vs_merged) vs_nc = 0;
+            // waves 0 and 1 look up list A in list B, waves 2 and 3 list B in list A.  Entry i of `mine` goes to
+            // common[#hits before i] when `other` holds it too (written once, by the first pair), else to
+            // only[i - #hits before i].  The look-ups need strictly ascending lists, which is checked along the way:
+            // in other lists they find something or other, inside the list's bounds, and nothing of it is used
+            const int *mine = half ? rawB : rawA, *other = half ? rawA : rawB;
+            const int nmine = half ? vs_nb : vs_na, nother = half ? vs_na : vs_nb;
+            int *only = vs_only + half * VS_ONLY_MAX;
+            const unsigned long long lt = (1ull << lane) - 1ull;
+            bool bad = false;
+            int carry = 0;
+            for (int base = 0; base < max(vs_na, vs_nb); base += NTHREADS) {      // uniform trip count
+                const int i = base + (tid & (NTHREADS - 1));
+                const bool valid = i < nmine;
+                const int x = valid ? mine[i] : 0;
+                bad |= valid && i > 0 && mine[max(i - 1, 0)] >= x;
+                int lo = 0, hi = nother;                           // first entry of `other` >= x
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (other[mid] < x) lo = mid + 1; else hi = mid;
+                }
+                const bool eq = valid && lo < nother && other[lo] == x;
+                const unsigned long long bal = __ballot(eq);
+                if (lane == 0) vs_wsum[wave_wg] = __builtin_popcountll(bal);
+                __syncthreads();
+                const int first = vs_wsum[2 * half], second = vs_wsum[2 * half + 1];
+                const int pre = carry + (wave ? first : 0) + __builtin_popcountll(bal & lt);
+                if (valid) {
+                    if (eq) { if (!half) common[pre] = x; }
+                    else if (i - pre < VS_ONLY_MAX) only[i - pre] = x;
+                }
+                carry += first + second;
+                if (base + NTHREADS >= max(vs_na, vs_nb) && __any(bad) && lane == 0) vs_bad[0] = 1;
+                if (base + NTHREADS >= max(vs_na, vs_nb) && tid == 0) vs_bad[1] = carry;
+                __syncthreads();
             }
+            // (the last barrier also orders these LDS lists before their readers)
+            vs_nc = __builtin_amdgcn_readfirstlane(vs_bad[1]);
+            vs_merged = !__builtin_amdgcn_readfirstlane(vs_bad[0]) && vs_nc > 0 && vs_na - vs_nc <= VS_ONLY_MAX && vs_nb - vs_nc <= VS_ONLY_MAX;
+            if (!vs_merged) vs_nc = 0;
         }
     }
     // paired vertical-slash: vs_nc common steps, then the split steps: per half its leftover block
@@ -1066,7 +1071,7 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
     __shared__ __attribute__((aligned(16))) char lds_v[L::NV];
     __shared__ int vs_only[L::NONLY];        // paired list walks: [row block][entries the other list lacks]
     __shared__ int vs_wsum[4];
-    __shared__ int vs_bad;
+    __shared__ int vs_bad[2];                // paired list walks: a list is not ascending, number of common entries
     __shared__ int lds_redo;
     if (threadIdx.x == 0) lds_redo = 0;      // (ordered before its readers by the barriers of the walk)
     if constexpr (std::is_same<T, __bf16>::value) {
