@@ -216,6 +216,33 @@ def test_block_sparse_lists_that_differ_between_neighbouring_row_blocks(gpu, n, 
     check(out, ref, "bs-lists")
 
 
+@pytest.mark.parametrize("order", ["ascending", "one pair swapped"])
+@pytest.mark.parametrize("entries", [1, 127, 128, 129, 255, 256, 257, 300])
+def test_block_list_lengths_around_the_split_chunks(gpu, entries, order):
+    """Lists are split 128 entries at a time, the first 256 of them from registers: lengths around both, for the two
+    row blocks of the last pair (two thirds of the entries in common); a list out of order is walked as it is."""
+    from minference_amd import block_sparse_attention_from_index
+    rows, n = 320, 320 * 64
+    print(f"case block lists of {entries} entries, {order}", flush=True)
+    q, k, v = make(1, 1, 1, n, 23, torch.bfloat16)
+    rng = np.random.default_rng(entries)
+    common = rng.permutation(rows - 2)
+    lists = np.zeros((rows, entries), dtype=np.int64)
+    for j, m in enumerate((rows - 2, rows - 1)):
+        kept = 2 * entries // 3
+        own = common[entries + j * (entries - kept):][:entries - kept] if 2 * entries <= rows - 2 \
+            else rng.choice(common[kept:], entries - kept, replace=False)
+        lists[m] = np.sort(np.concatenate([common[:kept], own]))
+    if order != "ascending" and entries > 1:
+        lists[rows - 1, entries - 2:] = lists[rows - 1, entries - 2:][::-1].copy()
+    out = block_sparse_attention_from_index(q.to(gpu), k.to(gpu), v.to(gpu),
+                                            torch.from_numpy(lists.astype(np.int32))[None, None].to(gpu))
+    for m in (rows - 2, rows - 1):
+        keys = (torch.from_numpy(lists[m])[:, None] * 64 + torch.arange(64)).reshape(-1)
+        s = q[0, 0, m * 64:m * 64 + 64].float() @ k[0, 0, keys].float().T * 128 ** -0.5
+        check(out[0, 0, m * 64:m * 64 + 64], torch.softmax(s, -1) @ v[0, 0, keys].float(), f"row block {m}")
+
+
 def test_block_sparse_op_topk_covers_everything_equals_sdpa(gpu):
     from minference_amd import block_sparse_attention
     n = 900
