@@ -91,6 +91,21 @@ constexpr int VALU_PER_MFMA = 6;
 #endif
 constexpr int VALU_MASK = 0x402;             // sched_group_barrier classes: VALU | transcendental
 
+// n / d for n < 2^31 by a multiplication and a shift (round-up method: m = ceil(2^(31+bits) / d) fits 32 bits, its
+// excess times n stays below 2^(31+bits) / d).  A 32-bit division takes some forty dependent instructions here, and
+// every workgroup made five of them before it could ask for its first byte: 1.2 -> 0.7 us; A-shape, 16 heads, 49152
+// tokens, window 128: head_dim 64 125.3 -> 122.4 us, 128 218.7 -> 216.9; nothing beyond noise on walks of 50 steps.
+struct FastDiv {
+    unsigned d, m, shift;
+};
+inline FastDiv fast_div(unsigned d) {
+    unsigned bits = 0;
+    while ((1ull << bits) < d) ++bits;
+    if (bits == 0) return FastDiv{1u, 0x80000000u, 31u};
+    return FastDiv{d, (unsigned)(((1ull << (31 + bits)) + d - 1) / d), 31u + bits};
+}
+__device__ __forceinline__ unsigned fast_quot(unsigned n, const FastDiv &f) { return (unsigned)(((unsigned long long)n * f.m) >> f.shift); }
+
 struct AttnParams {
     const char *q, *k, *v;
     char *o;
@@ -110,7 +125,8 @@ struct AttnParams {
     int n_init, n_local, dense_from;
     long long total_wg;
     int descending;          // row blocks are handed out from the last one down
-    int stripes;             // the row-block pairs of a kv group are dealt to this many XCD ranges (see launch_hd)
+    int stripes_log2;        // the row-block pairs of a kv group are dealt to this many XCD ranges (see launch_hd)
+    FastDiv by_group, by_stripe, by_heads;   // hq / hk; workgroups of a stripe per head; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
     // every head is processed and index_heads = hq
@@ -292,9 +308,10 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     const unsigned per_xcd = (total_wg + 7u) >> 3;
     const unsigned logical = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
     if (logical >= total_wg) return false;
-    const int group = p.hq / p.hk;
+    const int group = (int)p.by_group.d;
     unsigned rest = logical;
-    const int hin = (int)(rest % (unsigned)group); rest /= (unsigned)group;
+    auto next_digit = [&](const FastDiv &f) { const unsigned q = fast_quot(rest, f), r = rest - q * f.d; rest = q; return r; };
+    const int hin = (int)next_digit(p.by_group);
     // Dense causal work grows with the row block, so the heavy (late) blocks go first.  The sparse
     // modes have near-constant work per row block once the context is long and then measure 1 %
     // faster in ascending order; up to 64K tokens their early row blocks are still growing and the
@@ -302,9 +319,9 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     const int rows_wg = (p.rows + 1) >> 1;                           // row-block pairs per (batch, head)
     const int split_units = (rows_wg - p.split_first) * p.nseg;      // (no split: split_first == rows_wg)
     const unsigned units = (unsigned)(p.split_first + split_units);
-    const unsigned per_stripe = (units + (unsigned)p.stripes - 1u) / (unsigned)p.stripes;
-    const unsigned in_stripe = rest % per_stripe; rest /= per_stripe;
-    const int mi = (int)(in_stripe * (unsigned)p.stripes + rest % (unsigned)p.stripes); rest /= (unsigned)p.stripes;
+    const unsigned in_stripe = next_digit(p.by_stripe);
+    const int mi = (int)((in_stripe << p.stripes_log2) + (rest & ((1u << p.stripes_log2) - 1u)));
+    rest >>= p.stripes_log2;
     if (mi >= (int)units) return false;              // padding of the last round (workgroup-uniform)
     int mslot, seg = -1;                             // row-block pair, segment of its walk (-1: the whole walk)
     if (CUT && mi < split_units) {                    // the split pairs, longest walks first
@@ -322,16 +339,15 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     if (p.head_list) {
         // the selected heads in chunks of `group` consecutive list entries take the place of the kv
         // groups: neighbours in the (ascending) list mostly share a kv head
-        const int nch = (p.index_heads + group - 1) / group;
-        const int ch = (int)(rest % (unsigned)nch);
-        b = (int)(rest / (unsigned)nch);
+        const int ch = (int)next_digit(p.by_heads);
+        b = (int)rest;
         hs = ch * group + hin;
         if (hs >= p.index_heads) return false;       // padding of the last chunk (workgroup-uniform)
         h = as_const(p.head_list)[hs];
-        hkv = h / group;
+        hkv = (int)fast_quot((unsigned)h, p.by_group);
     } else {
-        hkv = (int)(rest % (unsigned)p.hk);
-        b = (int)(rest / (unsigned)p.hk);
+        hkv = (int)next_digit(p.by_heads);
+        b = (int)rest;
         h = hkv * group + hin;
         hs = h;
     }
@@ -1216,7 +1232,8 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.head_list = t->head_list;
     p.index_heads = t->head_list ? t->index_heads : t->heads_q;
     p.total_wg = 0;          // set by the launcher
-    p.stripes = 1;
+    p.stripes_log2 = 0;
+    p.by_group = p.by_stripe = p.by_heads = fast_div(1);      // set by the launcher
     p.descending = 0;
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
     p.dtype = t->dtype;
@@ -1336,10 +1353,11 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
                      MODE == MODE_ASHAPE ? (int)(((long long)p.n_local + p.n_init) / BN) + 2 : p.rows;    // steps of a full walk (lists: unknown)
     const bool grows = MODE == MODE_DENSE || split_pairs > 0 ||
                        (p.rows <= 1024 && p.rows <= 14ll * most && groups * group >= 8 && groups * group * units >= 1024);
-    p.stripes = 1;
+    p.stripes_log2 = 0;
     if (grows)
-        while (p.stripes < 8 && groups * p.stripes % 8) p.stripes *= 2;
-    p.total_wg = groups * group * p.stripes * ((units + p.stripes - 1) / p.stripes);
+        while (p.stripes_log2 < 3 && (groups << p.stripes_log2) % 8) ++p.stripes_log2;
+    const long long per_stripe = (units + (1 << p.stripes_log2) - 1) >> p.stripes_log2;
+    p.total_wg = (groups * group * per_stripe) << p.stripes_log2;
     // Longest walks first wherever they grow with the row block over much of the sequence.  A-shape and
     // block-sparse, 32 / 8 heads: 3000 tokens 107 -> 91 and 118 -> 92 us, 6000 tokens 336 -> 315 (6824) and
     // 333 -> 308, 12000 tokens 702 -> 677 and 921 -> 897, 24000 tokens 1508 -> 1487 and (32768) 2947 -> 2920;
@@ -1350,6 +1368,9 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
     const long long per_xcd = (p.total_wg + 7) >> 3;
     const long long grid = per_xcd * 8;
     if (grid > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
+    p.by_group = fast_div((unsigned)group);
+    p.by_stripe = fast_div((unsigned)per_stripe);
+    p.by_heads = fast_div((unsigned)(grid_heads / group));
     const dim3 block(2 * NTHREADS);
     hipStream_t st = (hipStream_t)stream;
 #define MINF_LAUNCH_ATTN(T)                                                                                      \
