@@ -244,7 +244,7 @@ __global__ __launch_bounds__(IDX_WAVES *MINF_WAVE) void vs_index_kernel(
 //   run_a[r], run_e[r]   [start, end) of range r
 //   cgaps[i]  the number of entries j <= i with t_j > t_{j-1} + 64 ("gap entries": the only entries
 //             at which a range can start, for any row block -- skipping and clipping only shrink gaps)
-//   glist[j]  the gap entries, ascending, j < ngaps (compacted from cgaps by the bitmap pass): the
+//   glist[j]  the gap entries, ascending, j < ngaps: the
 //             first gap entry at or after entry x is glist[cgaps[x - 1]]
 // all in the virtual row's coordinates (real position = virtual + end_m - V).
 // vs_index_fast_kernel then handles a row block as follows: entries from the first valid one are
@@ -267,79 +267,94 @@ __host__ __device__ __forceinline__ long long idx_tab_ints(int nnz_s, int rows) 
     return IDX_TAB_HDR + 7ll * nnz_s + idx_bm_words(rows);
 }
 
-// The walk of chunks [c_begin, c_end) of one head's list by one wavefront, starting from the state
-// (cur_a, carried_e, carried_t) that the entries before chunk c_begin leave behind and from the
-// counts (nb, nr, ng) of blocks, ranges and gap entries before it.  WRITE = false only counts.
-struct PrepState { int cur_a, carried_e, carried_t; };
-template <bool WRITE>
-__device__ __forceinline__ void prep_walk(const int32_t *__restrict__ sl, int32_t *__restrict__ hdr, int nnz_s, int V,
-                                          int c_begin, int c_end, PrepState &st, int &nb, int &nr, int &ng) {
-    const int lane = minf_lane();
-    int32_t *cpos = hdr + IDX_TAB_HDR, *cpre = cpos + nnz_s, *crun = cpre + nnz_s;
-    int32_t *run_a = crun + nnz_s, *run_e = run_a + nnz_s, *cgaps = run_e + nnz_s;
-    int carried_e = st.carried_e, carried_t = st.carried_t, cur_a = st.cur_a;
-    // the walk is one chain of chunks; the list entries of the next two chunks are fetched ahead so
-    // that no chunk waits for a load
-    int o_next = sl[min(c_begin * MINF_WAVE + lane, nnz_s - 1)], o_next2 = sl[min((c_begin + 1) * MINF_WAVE + lane, nnz_s - 1)];
-    for (int c = c_begin; c < c_end; ++c) {
-        const int base = c * MINF_WAVE;
-        const int cnt = min(MINF_WAVE, nnz_s - base);
-        const bool valid = lane < cnt;
-        const int o_cur = o_next;
-        o_next = o_next2;
-        o_next2 = sl[min(base + 2 * MINF_WAVE + lane, nnz_s - 1)];
-        int t = valid ? max(V - o_cur, 64) : 0;
-        const int tlast = minf_readlane(t, cnt - 1);
-        if (!valid) t = tlast;
-        if (c == 0) {
-            const int t0 = minf_readlane(t, 0);
-            cur_a = t0 - 64;
-            carried_e = t0 - 64;
-            carried_t = t0;
-        }
-        uint64_t starts, gm;
-        const int a = chunk_ranges(t, lane, cur_a, carried_e, carried_t, starts, &gm);
-        if (WRITE && valid) cgaps[base + lane] = ng + __builtin_popcountll(gm & (minf_lanemask_lt() | (1ull << lane)));
-        ng += __builtin_popcountll(gm);             // (padding lanes repeat the last entry: never a gap)
-        const bool is_start = valid && (((starts >> lane) & 1ull) || (c == 0 && lane == 0));
-        const int e = a + ((((t - a) + 63) >> 6) << 6);
-        int eprev = lane_above(e);
-        if (lane == 0) eprev = carried_e;
-        const bool changed = valid && (e != eprev);
-        const uint64_t cm = __ballot(changed), sm = __ballot(is_start);
-        if (WRITE) {
-            const uint64_t lt = minf_lanemask_lt();
-            const int kpos = nb + __builtin_popcountll(cm & lt);
-            if (changed) cpos[kpos] = e - 64;
-            if (valid) {
-                const int r = nr + __builtin_popcountll(sm & lt);
-                cpre[base + lane] = is_start ? kpos : -1;
-                crun[base + lane] = is_start ? r : -1;
-                if (is_start) {
-                    run_a[r] = a;
-                    if (r > 0) run_e[r - 1] = eprev;
-                }
-            }
-        }
-        nb += __builtin_popcountll(cm);
-        nr += __builtin_popcountll(sm);
-        carried_e = minf_readlane(e, cnt - 1);
-        carried_t = tlast;
-        cur_a = minf_readlane(a, cnt - 1);
-    }
-    st.cur_a = cur_a; st.carried_e = carried_e; st.carried_t = carried_t;
+// Coverage bitmap of a head's virtual row: bit p is set iff position p lies inside one of the tabulated ranges.  A
+// range is the union of its blocks (its end moves by 64 at a time), so every block sets its 64 bits; what lies past the
+// bitmap (up to 63 positions behind the last entry) is never looked up.
+__device__ __forceinline__ void mark_block(uint32_t *bm, int words, int p) {
+    const unsigned w = (unsigned)(p >> 5), sh = (unsigned)p & 31u;
+    if (w < (unsigned)words) atomicOr(&bm[w], ~0u << sh);
+    if (w + 1 < (unsigned)words) atomicOr(&bm[w + 1], ~0u);
+    if (sh && w + 2 < (unsigned)words) atomicOr(&bm[w + 2], (1u << sh) - 1u);
 }
 
-__device__ __forceinline__ void prep_header(int32_t *hdr, int nnz_s, int rows, int V, const PrepState &st, int nb, int nr, int ng) {
+// The walk of a head's list over chunks of 64 entries by one wavefront: (cur_a, carried_e, carried_t) is what the
+// entries before a chunk leave behind, (nb, nr, ng) the number of blocks, ranges and gap entries before it.
+struct PrepState { int cur_a, carried_e, carried_t; };
+struct PrepCount { int nb, nr, ng; };
+struct PrepChunk {                                   // one chunk, taken through the range logic
+    int t, a, eprev0;                                // this lane's entry and its range start; range end before the chunk
+    uint64_t starts, gaps;
+    int base, cnt;
+};
+__device__ __forceinline__ void prep_chunk(PrepChunk &k, PrepState &st, PrepCount &n) {
+    const int lane = minf_lane();
+    if (k.base == 0) {
+        const int t0 = minf_readlane(k.t, 0);
+        st.cur_a = st.carried_e = t0 - 64;
+        st.carried_t = t0;
+    }
+    k.a = chunk_ranges(k.t, lane, st.cur_a, st.carried_e, st.carried_t, k.starts, &k.gaps);
+    const uint64_t valid = k.cnt == MINF_WAVE ? ~0ull : (1ull << k.cnt) - 1ull;
+    if (k.base == 0) k.starts |= 1ull;
+    k.starts &= valid;
+    k.eprev0 = st.carried_e;
+    const int e = k.a + ((((k.t - k.a) + 63) >> 6) << 6);
+    int eprev = lane_above(e);
+    if (lane == 0) eprev = st.carried_e;
+    n.nb += __builtin_popcountll(__ballot(lane < k.cnt && e != eprev));
+    n.nr += __builtin_popcountll(k.starts);
+    n.ng += __builtin_popcountll(k.gaps);            // (padding lanes repeat the last entry: never a gap)
+    st.carried_e = minf_readlane(e, k.cnt - 1);
+    st.carried_t = minf_readlane(k.t, k.cnt - 1);
+    st.cur_a = minf_readlane(k.a, k.cnt - 1);
+}
+// writes a chunk's entries of the tables; n: the counts before the chunk
+__device__ __forceinline__ void prep_write(const PrepChunk &k, const PrepCount &n, int32_t *hdr, int nnz_s, uint32_t *bm, int bm_words) {
+    const int lane = minf_lane();
+    int32_t *cpos = hdr + IDX_TAB_HDR, *cpre = cpos + nnz_s, *crun = cpre + nnz_s;
+    int32_t *run_a = crun + nnz_s, *run_e = run_a + nnz_s, *cgaps = run_e + nnz_s, *glist = cgaps + nnz_s;
+    const uint64_t lt = minf_lanemask_lt();
+    const bool valid = lane < k.cnt, is_start = (k.starts >> lane) & 1ull;
+    const int e = k.a + ((((k.t - k.a) + 63) >> 6) << 6);
+    int eprev = lane_above(e);
+    if (lane == 0) eprev = k.eprev0;
+    const bool changed = valid && e != eprev;
+    const int kpos = n.nb + __builtin_popcountll(__ballot(changed) & lt);
+    if (changed) {
+        cpos[kpos] = e - 64;
+        if (bm) mark_block(bm, bm_words, e - 64);
+    }
+    if (valid) {
+        const int r = n.nr + __builtin_popcountll(k.starts & lt), gapno = n.ng + __builtin_popcountll(k.gaps & lt);
+        const bool gap = (k.gaps >> lane) & 1ull;
+        cgaps[k.base + lane] = gapno + (gap ? 1 : 0);
+        if (gap) glist[gapno] = k.base + lane;
+        cpre[k.base + lane] = is_start ? kpos : -1;
+        crun[k.base + lane] = is_start ? r : -1;
+        if (is_start) {
+            run_a[r] = k.a;
+            if (r > 0) run_e[r - 1] = eprev;
+        }
+    }
+}
+__device__ __forceinline__ PrepChunk prep_load(const int32_t *__restrict__ sl, int nnz_s, int V, int c) {
+    PrepChunk k;
+    k.base = c * MINF_WAVE;
+    k.cnt = min(MINF_WAVE, nnz_s - k.base);
+    k.t = max(V - sl[min(k.base + minf_lane(), nnz_s - 1)], 64);     // (padding lanes repeat the last entry)
+    return k;
+}
+
+__device__ __forceinline__ void prep_header(int32_t *hdr, int nnz_s, int rows, int V, const PrepState &st, const PrepCount &n) {
     int32_t *run_e = hdr + IDX_TAB_HDR + 4ll * nnz_s;
-    run_e[nr - 1] = st.carried_e;
-    hdr[0] = nb;
-    hdr[1] = nr;
+    run_e[n.nr - 1] = st.carried_e;
+    hdr[0] = n.nb;
+    hdr[1] = n.nr;
     hdr[2] = V;
     // the bitmap covers positions [0, 32 * bm_words); a list whose largest offset lies far
     // outside the context does not fit and the row blocks fall back to searching the ranges
     hdr[3] = (long long)V <= 32 * (idx_bm_words(rows) - 1) ? 1 : 0;
-    hdr[4] = ng;
+    hdr[4] = n.ng;
 }
 
 // The table pass: one workgroup of PREP_WAVES wavefronts per head.  The walk over the list is a chain
@@ -349,15 +364,23 @@ __device__ __forceinline__ void prep_header(int32_t *hdr, int nnz_s, int rows, i
 // wavefront takes a contiguous share of the chunks; all of them first mark the sure and maybe entries
 // of their chunks (independent work); a wavefront then finds the state at the head of its share by
 // going back to the last sure start before it and replaying only the maybe entries in between (none
-// inside a dense run, a handful when the offsets are scattered); it walks its share once to count its
-// blocks, ranges and gap entries, the counts are summed over the wavefronts before it, and it walks
-// the share again to write the tables.  Lists of at most two chunks, or of more chunks than the mark
-// arrays hold, are walked by one wavefront alone.
+// inside a dense run, a handful when the offsets are scattered); it takes its share through the range logic,
+// the counts of blocks, ranges and gap entries are summed over the wavefronts before it, and it writes the tables.
+// A share of at most PREP_KEEP chunks stays in registers from the marks to the tables (one round of loads in flight
+// together); longer ones are loaded and walked once to count and again to write.  Lists of at most two
+// chunks, or of more chunks than the mark arrays hold, are walked by one wavefront alone.
+// The coverage bitmap is built in LDS beside the tables (where it fits: `bm_words` > 0) and copied out at the end.
+// Latency-bound, one workgroup per head.  With a bitmap kernel behind it that searched the ranges, and a share's state
+// found by reading the marks one chunk at a time, the two took (us, now in one kernel): 6096 slashes, clustered, 16001
+// tokens 29 + 5 -> 16, 131072 tokens 25 + 5 -> 15; uniform, 262144 tokens 39 + 7 -> 28; 2048 slashes, 8192 tokens,
+// 4 heads 12 + 5 -> 9.
 #define PREP_WAVES 16
 #define PREP_MAX_CHUNKS 2048
+#define PREP_KEEP 8
+#define PREP_BITMAP_MAX_BYTES 98304
 __global__ __launch_bounds__(PREP_WAVES *MINF_WAVE) void vs_index_prep_kernel(const int32_t *__restrict__ slash,
-                                                                              int32_t *__restrict__ tables, int nnz_s, int rows) {
-    __shared__ uint64_t sure_m[PREP_MAX_CHUNKS], maybe_m[PREP_MAX_CHUNKS];
+                                                                              int32_t *__restrict__ tables, int nnz_s, int rows, int bm_words) {
+    extern __shared__ uint64_t prep_lds[];           // sure and maybe marks of every chunk, later the bitmap
     __shared__ int cnt_b[PREP_WAVES], cnt_r[PREP_WAVES], cnt_g[PREP_WAVES];
     const int lane = minf_lane();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -366,92 +389,154 @@ __global__ __launch_bounds__(PREP_WAVES *MINF_WAVE) void vs_index_prep_kernel(co
     int32_t *hdr = tables + bh * idx_tab_ints(nnz_s, rows);
     const int V = sl[0] + 64;
     const int nchunks = (nnz_s + MINF_WAVE - 1) / MINF_WAVE;
+    uint32_t *bm = bm_words > 0 ? reinterpret_cast<uint32_t *>(prep_lds) : nullptr;
+    auto clear_bitmap = [&]() {
+        for (int i = (int)threadIdx.x; i < bm_words; i += PREP_WAVES * MINF_WAVE) bm[i] = 0u;
+        __syncthreads();
+    };
 
     if (nchunks <= 2 || nchunks > PREP_MAX_CHUNKS) {        // (workgroup-uniform)
+        clear_bitmap();
         if (wave == 0) {
             PrepState st{0, 0, 0};
-            int nb = 0, nr = 0, ng = 0;
-            prep_walk<true>(sl, hdr, nnz_s, V, 0, nchunks, st, nb, nr, ng);
-            if (lane == 0) prep_header(hdr, nnz_s, rows, V, st, nb, nr, ng);
+            PrepCount n{0, 0, 0};
+            for (int c = 0; c < nchunks; ++c) {
+                PrepChunk k = prep_load(sl, nnz_s, V, c);
+                const PrepCount before = n;
+                prep_chunk(k, st, n);
+                prep_write(k, before, hdr, nnz_s, bm, bm_words);
+            }
+            if (lane == 0) prep_header(hdr, nnz_s, rows, V, st, n);
         }
-        return;
-    }
-    const int per = (nchunks + PREP_WAVES - 1) / PREP_WAVES;
-    const int c0 = wave * per, c1 = min(c0 + per, nchunks);
-    // ---- marks: entry i is a sure start when t_i > t_{i-1} + 127, a maybe when t_i > t_{i-1} + 64
-    // (entry 0 starts the first range)
-    for (int c = c0; c < c1; ++c) {
-        const int i = c * MINF_WAVE + lane;
-        const bool valid = i < nnz_s;
-        const int t = max(V - sl[min(i, nnz_s - 1)], 64);
-        const int tp = max(V - sl[min(max(i - 1, 0), nnz_s - 1)], 64);
-        const bool sure = valid && (i == 0 || t > tp + 127);
-        const bool maybe = valid && !sure && t > tp + 64;
-        const uint64_t sm = __ballot(sure), mm = __ballot(maybe);
-        if (lane == 0) { sure_m[c] = sm; maybe_m[c] = mm; }
-    }
-    __syncthreads();
-    // ---- the state at the head of this wavefront's share (wave-uniform scalar work)
-    PrepState st{0, 0, 0};
-    if (c0 > 0 && c0 < nchunks) {
-        int cs = c0 - 1;
-        while (cs > 0 && sure_m[cs] == 0) --cs;              // (chunk 0 holds entry 0, a sure start)
-        const uint64_t smask = sure_m[cs];
-        const int js = cs * MINF_WAVE + (63 - __builtin_clzll(smask));     // the last sure start before the share
-        int a = max(V - sl[js], 64) - 64;
-        for (int c = cs; c < c0; ++c) {
-            uint64_t mm = maybe_m[c];
-            if (c == cs) mm &= ~((2ull << (js - cs * MINF_WAVE)) - 1ull);    // maybes above the sure start only
-            while (mm) {
-                const int j = c * MINF_WAVE + __builtin_ctzll(mm);
-                mm &= mm - 1;
-                const int tj = max(V - sl[j], 64), tp = max(V - sl[j - 1], 64);
-                const int ep = a + ((((tp - a) + 63) >> 6) << 6);
-                if (tj > ep + 64) a = tj - 64;
+    } else {
+        uint64_t *sure_m = prep_lds, *maybe_m = prep_lds + nchunks;
+        const int per = (nchunks + PREP_WAVES - 1) / PREP_WAVES;
+        const int c0 = min(wave * per, nchunks), c1 = min(c0 + per, nchunks);
+        const bool keep = per <= PREP_KEEP;
+        PrepChunk held[PREP_KEEP];
+        // ---- marks: entry i is a sure start when t_i > t_{i-1} + 127, a maybe when t_i > t_{i-1} + 64
+        // (entry 0 starts the first range)
+        auto mark = [&](const PrepChunk &k, int before) {
+            const int i = k.base + lane;
+            int tp = lane_above(k.t);
+            if (lane == 0) tp = before;
+            const bool valid = lane < k.cnt;
+            const bool sure = valid && (i == 0 || k.t > tp + 127);
+            const bool maybe = valid && !sure && k.t > tp + 64;
+            const uint64_t sm = __ballot(sure), mm = __ballot(maybe);
+            if (lane == 0) { sure_m[k.base / MINF_WAVE] = sm; maybe_m[k.base / MINF_WAVE] = mm; }
+        };
+        const int t_before = c0 > 0 ? max(V - sl[c0 * MINF_WAVE - 1], 64) : 0;      // the entry before the share
+        if (keep) {
+#pragma unroll
+            for (int j = 0; j < PREP_KEEP; ++j)
+                if (c0 + j < c1) held[j] = prep_load(sl, nnz_s, V, c0 + j);
+#pragma unroll
+            for (int j = 0; j < PREP_KEEP; ++j)
+                if (c0 + j < c1) mark(held[j], j ? minf_readlane(held[j ? j - 1 : 0].t, 63) : t_before);
+        } else {
+            for (int c = c0; c < c1; ++c)
+                mark(prep_load(sl, nnz_s, V, c), c > 0 ? max(V - sl[c * MINF_WAVE - 1], 64) : 0);
+        }
+        __syncthreads();
+        // ---- the state at the head of this wavefront's share (wave-uniform scalar work)
+        PrepState st{0, 0, 0};
+        if (c0 > 0 && c0 < nchunks) {
+            // (64 chunks' marks per step, one a lane: a dense run has none over a hundred chunks)
+            int cs = c0 - 1;
+            uint64_t smask = 0, some;
+            for (;;) {                                           // (chunk 0 holds entry 0, a sure start)
+                const uint64_t mine = sure_m[max(cs - lane, 0)];
+                some = __ballot(mine != 0 && lane <= cs);
+                if (some) break;
+                cs -= 64;
+            }
+            cs -= __builtin_ctzll(some);
+            smask = sure_m[cs];
+            const int js = cs * MINF_WAVE + (63 - __builtin_clzll(smask));     // the last sure start before the share
+            int a = max(V - sl[js], 64) - 64;
+            for (int cb = cs; cb < c0; cb += 64) {
+                uint64_t mine = cb + lane < c0 ? maybe_m[cb + lane] : 0;
+                if (cb + lane == cs) mine &= ~((2ull << (js - cs * MINF_WAVE)) - 1ull);      // maybes above the sure start only
+                for (uint64_t left = __ballot(mine != 0); left; left &= left - 1) {
+                    const int c = __builtin_ctzll(left);
+                    uint64_t mm = ((uint64_t)(unsigned)minf_readlane((int)(mine >> 32), c) << 32) | (unsigned)minf_readlane((int)mine, c);
+                    while (mm) {
+                        const int j = (cb + c) * MINF_WAVE + __builtin_ctzll(mm);
+                        mm &= mm - 1;
+                        const int tj = max(V - sl[j], 64), tp = max(V - sl[j - 1], 64);
+                        const int ep = a + ((((tp - a) + 63) >> 6) << 6);
+                        if (tj > ep + 64) a = tj - 64;
+                    }
+                }
+            }
+            st.cur_a = a;
+            st.carried_t = t_before;
+            st.carried_e = a + ((((t_before - a) + 63) >> 6) << 6);
+        }
+        // ---- count, sum over the wavefronts before this one, write
+        const PrepState head = st;
+        PrepCount n{0, 0, 0};
+        if (keep) {
+#pragma unroll
+            for (int j = 0; j < PREP_KEEP; ++j)
+                if (c0 + j < c1) prep_chunk(held[j], st, n);
+        } else {
+            for (int c = c0; c < c1; ++c) {
+                PrepChunk k = prep_load(sl, nnz_s, V, c);
+                prep_chunk(k, st, n);
             }
         }
-        st.cur_a = a;
-        st.carried_t = max(V - sl[c0 * MINF_WAVE - 1], 64);
-        st.carried_e = a + ((((st.carried_t - a) + 63) >> 6) << 6);
-    }
-    // ---- count, sum over the wavefronts before this one, write
-    int nb = 0, nr = 0, ng = 0;
-    if (c0 < nchunks) {
-        PrepState probe = st;
-        prep_walk<false>(sl, hdr, nnz_s, V, c0, c1, probe, nb, nr, ng);
-    }
-    if (lane == 0) { cnt_b[wave] = nb; cnt_r[wave] = nr; cnt_g[wave] = ng; }
-    __syncthreads();
-    int ob = 0, orr = 0, og = 0, tb = 0, tr = 0, tg = 0;
+        if (lane == 0) { cnt_b[wave] = n.nb; cnt_r[wave] = n.nr; cnt_g[wave] = n.ng; }
+        __syncthreads();
+        PrepCount at{0, 0, 0}, all{0, 0, 0};
 #pragma unroll
-    for (int w = 0; w < PREP_WAVES; ++w) {
-        const int b = cnt_b[w], r = cnt_r[w], g = cnt_g[w];
-        if (w < wave) { ob += b; orr += r; og += g; }
-        tb += b; tr += r; tg += g;
+        for (int w = 0; w < PREP_WAVES; ++w) {
+            const int b = cnt_b[w], r = cnt_r[w], g = cnt_g[w];
+            if (w < wave) { at.nb += b; at.nr += r; at.ng += g; }
+            all.nb += b; all.nr += r; all.ng += g;
+        }
+        clear_bitmap();                                          // (everyone is done with the marks)
+        if (keep) {
+#pragma unroll
+            for (int j = 0; j < PREP_KEEP; ++j)
+                if (c0 + j < c1) {
+                    prep_write(held[j], at, hdr, nnz_s, bm, bm_words);
+                    const PrepChunk &k = held[j];
+                    const int e = k.a + ((((k.t - k.a) + 63) >> 6) << 6);
+                    int eprev = lane_above(e);
+                    if (lane == 0) eprev = k.eprev0;
+                    at.nb += __builtin_popcountll(__ballot(lane < k.cnt && e != eprev));
+                    at.nr += __builtin_popcountll(k.starts);
+                    at.ng += __builtin_popcountll(k.gaps);
+                }
+        } else {
+            st = head;
+            for (int c = c0; c < c1; ++c) {
+                PrepChunk k = prep_load(sl, nnz_s, V, c);
+                const PrepCount before = at;
+                prep_chunk(k, st, at);
+                prep_write(k, before, hdr, nnz_s, bm, bm_words);
+            }
+        }
+        if (c0 < nchunks && c1 == nchunks && lane == 0) prep_header(hdr, nnz_s, rows, V, st, all);
     }
-    if (c0 < nchunks) {
-        nb = ob; nr = orr; ng = og;
-        prep_walk<true>(sl, hdr, nnz_s, V, c0, c1, st, nb, nr, ng);
-        if (c1 == nchunks && lane == 0) prep_header(hdr, nnz_s, rows, V, st, tb, tr, tg);
+    if (bm) {
+        __syncthreads();                                         // every block is marked
+        uint32_t *dst = reinterpret_cast<uint32_t *>(hdr + IDX_TAB_HDR + 7ll * nnz_s);
+        for (int i = (int)threadIdx.x; i < bm_words; i += PREP_WAVES * MINF_WAVE) dst[i] = bm[i];
     }
 }
 
-// Coverage bitmap of a head's virtual row: bit p of the bitmap is set iff position p lies inside one
-// of the tabulated ranges [run_a[r], run_e[r]).  One thread per 32-bit word: a binary search finds
-// the first range that ends after the word's first position; ranges are at least 64 long, so at
-// most two of them touch a word.
+// The coverage bitmap of contexts for which it does not fit the table pass's LDS (beyond 786000 tokens).  One thread
+// per 32-bit word: a binary search finds the first range that ends after the word's first position; ranges are at
+// least 64 long, so at most two of them touch a word.
 __global__ __launch_bounds__(256) void vs_index_bitmap_kernel(int32_t *__restrict__ tables, int nnz_s, int rows) {
     const long long bh = blockIdx.y;
     int32_t *hdr = tables + bh * idx_tab_ints(nnz_s, rows);
     const int32_t *run_a = hdr + IDX_TAB_HDR + 3ll * nnz_s, *run_e = run_a + nnz_s;
     uint32_t *bm = reinterpret_cast<uint32_t *>(hdr + IDX_TAB_HDR + 7ll * nnz_s);
     const long long w = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w < nnz_s) {                           // (thread w also serves list entry w: the gap list)
-        const int32_t *cgaps = hdr + IDX_TAB_HDR + 5ll * nnz_s;
-        int32_t *glist = hdr + IDX_TAB_HDR + 6ll * nnz_s;
-        const int c = cgaps[w], cprev = w ? cgaps[w - 1] : 0;
-        if (c != cprev) glist[c - 1] = (int)w;
-    }
     if (w >= idx_bm_words(rows) || !hdr[3]) return;
     const int nr = hdr[1];
     const long long p0 = 32 * w, p1 = p0 + 32;
@@ -754,15 +839,21 @@ static int index_build_tables(const int32_t *seqlens, const int32_t *vertical_id
                               hipStream_t stream) {
     const long long nblk = (total + IDX_WAVES - 1) / IDX_WAVES;
     if (nblk > 0x7fffffffLL || (long long)batch * heads > 65535) return MINF_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(vs_index_prep_kernel, dim3((unsigned)(batch * heads)), dim3(PREP_WAVES * MINF_WAVE), 0,
-                       stream, slash_idx, workspace, nnz_s, rows);
+    const int nchunks = (nnz_s + MINF_WAVE - 1) / MINF_WAVE;
+    const long long bm_words = idx_bm_words(rows);
+    const bool bm_in_lds = bm_words * 4 <= PREP_BITMAP_MAX_BYTES;
+    size_t lds = nchunks <= PREP_MAX_CHUNKS ? 16 * (size_t)nchunks : 0;
+    if (bm_in_lds && (size_t)bm_words * 4 > lds) lds = (size_t)bm_words * 4;
+    hipLaunchKernelGGL(vs_index_prep_kernel, dim3((unsigned)(batch * heads)), dim3(PREP_WAVES * MINF_WAVE), lds,
+                       stream, slash_idx, workspace, nnz_s, rows, bm_in_lds ? (int)bm_words : 0);
     int status = minf_launch_status();
     if (status != MINF_OK) return status;
-    const long long bm_threads = idx_bm_words(rows) > nnz_s ? idx_bm_words(rows) : (long long)nnz_s;   // words and list entries
-    hipLaunchKernelGGL(vs_index_bitmap_kernel, dim3((unsigned)((bm_threads + 255) / 256), (unsigned)(batch * heads)),
-                       dim3(256), 0, stream, workspace, nnz_s, rows);
-    status = minf_launch_status();
-    if (status != MINF_OK) return status;
+    if (!bm_in_lds) {
+        hipLaunchKernelGGL(vs_index_bitmap_kernel, dim3((unsigned)((bm_words + 255) / 256), (unsigned)(batch * heads)),
+                           dim3(256), 0, stream, workspace, nnz_s, rows);
+        status = minf_launch_status();
+        if (status != MINF_OK) return status;
+    }
     // With zero-filled outputs the row-block pass is bound by its stores, and 24 resident waves per CU
     // write faster than 32 (6-9 % at 128K-512K tokens: fewer rows in flight, better DRAM locality); the
     // payload-only form is bound by its chains of dependent loads and wants every wave it can get.

@@ -142,6 +142,14 @@ def test_table_pass_shares_of_the_list(gpu, kind):
         assert_same(run_gpu([n], v, s, n, gpu), ref)
 
 
+@pytest.mark.parametrize("n,nv,ns", [(40000, 300, 8191), (40000, 300, 8192), (40000, 300, 8193),   # shares kept in registers up to 8192
+                                     (524288, 200, 300), (786000, 100, 130), (787000, 100, 130)])   # bitmap in LDS up to 786368
+def test_limits_of_the_table_pass(gpu, n, nv, ns):
+    print(f"case table pass limits n={n} nv={nv} ns={ns}", flush=True)
+    v, s = gen.vs_index_inputs(1, n, nv, ns, seed=9, force_v=4, force_s=64)
+    assert_same(run_gpu([n], v, s, n, gpu), O.vs_index_build([n], v, s, n))
+
+
 def test_hand_kat(gpu):
     V = np.array([[[0, 1, 2, 3, 100, 130, 700]]], np.int32)
     S = np.array([[[500, 70, 64, 3, 0]]], np.int32)
