@@ -26,8 +26,7 @@ namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4_t;
 
@@ -35,6 +34,7 @@ constexpr int HD = 128;
 constexpr int NC = 8;            // candidates per sweep (bits of a flag byte)
 constexpr int TILE = 64;         // query rows per wave pair (two tiles per workgroup)
 constexpr int KB = 32;           // keys per block
+constexpr int DW = (2 * TILE + 2 * KB) / 4;   // words of diagonal flags that 128 rows and 64 keys touch
 
 union Frag {
     u32x4_t u;
@@ -75,28 +75,15 @@ __device__ __forceinline__ void load_frag(const char *base, long long tok_stride
     for (int ks = 0; ks < 8; ++ks) f[ks].u = *reinterpret_cast<const u32x4_t *>(rp + ks * 32);
 }
 
-__device__ __forceinline__ unsigned load_u32_unaligned(const unsigned char *p) {
-    unsigned w;
-    __builtin_memcpy(&w, p, 4);
-    return w;
-}
-
-// two values rounded to bf16 (nearest), and what the rounding left of each: one instruction per value
-__device__ __forceinline__ unsigned pack_bf16(float x, float y) {
-    const f32x2_t v = {x, y};
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2_t));
-}
-__device__ __forceinline__ float left_of(float x, unsigned rounded, unsigned minus_one) {
+// D[t][row] = A[t] . B[row] + C[t][row] for 16 groups of 4 lanes: a lane's B belongs to its own row, its A is row
+// t = lane % 4 of its group's A, its D are rows 0..3 of its own column
+__device__ __forceinline__ f32x4_t mma4(float a, float b, f32x4_t c) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, rounded), __builtin_bit_cast(bf16x2_t, minus_one), x, false);
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 #else
-    return x;
+    return c;
 #endif
 }
-// bf16 -1 in the low / high half, 0 in the other, in a register: as an inline constant of the instruction, the
-// compiler's form of the first, -1 stands in the high half
-__device__ __forceinline__ unsigned minus_one_lo() { unsigned x; asm("s_mov_b32 %0, 0x0000bf80" : "=s"(x)); return x; }
-__device__ __forceinline__ unsigned minus_one_hi() { unsigned x; asm("s_mov_b32 %0, 0xbf800000" : "=s"(x)); return x; }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -118,30 +105,35 @@ __device__ __forceinline__ void merge_into(RowState &a, float m, float z, const 
 // blocks) from the diagonal holds the offsets 32 d - 31 .. 32 d + 31.  Per aligned group of 32 offsets the
 // table holds the OR and the AND of its flag bytes, and the same without the group's first offset.
 constexpr int DIAG_GROUPS = 8192;            // (262144 tokens; farther blocks are treated as mixed)
+constexpr int DIAG_GROUPS_SMALL = 4096;      // (131072 tokens: three workgroups fit a CU's LDS)
 
-// The masked sums as matrix products.  Per 32-key block and row,  Z_t += sum_c mask_t(c) e(c)  with e the
-// block's exponentials in B-operand layout straight from the S^T accumulators and the masks as the A
-// operand: row t of A is candidate t (t < 8), row 8 is all ones (the row sum itself).  That covers the
-// columns, and -- by setting a candidate's whole row -- the blocks and those blocks all of whose diagonals
-// a candidate keeps (most of a window, of a run of slashes).  Only candidates with SOME of a block's
-// diagonals are added element by element (their columns left out: those are in the product already).  The
-// exponentials enter as the sum of three bf16 terms, which is exact (8 + 8 + 8 bits) and has the exponents of
-// fp32: what lies far below a row's maximum -- every other key, where a head has a sink -- keeps its 24 bits for
-// the candidates that leave the maximum out.  (Two f16 terms, of 24 bits near the maximum only, had lost 4e-4 of
-// such a candidate's score under a sink 22 nats above the rest, and all of it under one of 26.)  The sums are fp32.
-// Relative error of the scores against fp64 sums, 4096 .. 16384 tokens: up to 7.6e-8; 6000 tokens under a sink of
-// 14 .. 30 nats up to 1.3e-6, of 80 nats 1.9e-6 (fp32 sums element by element: 1.2e-7, 4.8e-6, 1.9e-6).
-// Bound by its vector instructions: about 140 per 32 x 32 block (fma and exp 32, conversions 56, maximum 14,
-// masks) and 40 per candidate with mixed diagonals, beside 14 MFMAs, where testing a bit per element and
-// candidate took about 550.  32 / 8 heads, 16384 tokens, the six candidates of the reference: 7.00 ms (bits)
-// -> 2.86; with two f16 terms, which this replaces, 2.46.  K shared through LDS instead of fragments from global
-// memory is worth 0.35 ms of it; the score products alone take 0.44 ms at the nominal rate.
-template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_kernel(const RecallParams p) {
-    __shared__ unsigned dtab[DIAG_GROUPS];             // bytes: OR, AND, OR without the first, AND without the first
-    __shared__ float lds[4][TILE][NC + 2];
+// The masked sums as matrix products.  Per 32-key block and row,  Z_t = sum_c mask_t(c) e(c)  over the columns that
+// candidate t keeps, e the block's exponentials in fp32 straight from the S^T accumulators: v_mfma_f32_4x4x1 takes one
+// e per lane as its own row's B, its A is one key's flags of four candidates, so the products are exact and the sums
+// stay with the lane that owns the row.  A block that a candidate keeps as a whole (a block of its list, one all of
+// whose diagonals it keeps: most of a window, of a run of slashes) adds the block's row sum instead.  Only
+// candidates with SOME of a block's diagonals are added element by element (without the columns, which are in the
+// product already).  A block's sums start from zero and are added once to the running ones.
+// Relative error of the scores against fp64 sums, 4096 .. 16384 tokens, bf16 and fp16: up to 6.8e-8 (three bf16 terms per
+// exponential on 32x32x16 products, which this replaces: 6.8e-8), under a sink of 14 nats 3.3e-8 (1.8e-7); shares of
+// candidates without a sink of 14 .. 80 nats 1.9e-6 at most (6.5e-6; 3.1e-7 against 2.2e-7 at 14): there the rounding of
+// the scale in fp32 bounds it.
+// Bound by its vector instructions, 147 per 32 x 32 block (fma and exp 32, of which the exp take four times as long; maximum,
+// row sum, and 40 per candidate with mixed diagonals) beside 10 MFMAs.  32 / 8 heads, 16384 tokens, the six candidates of the
+// reference: 2.83 -> 2.19 ms against the bf16 terms (56 conversions per block; masks built in registers by every
+// wave, where one of a workgroup's threads now writes them to LDS once; two waves per SIMD, now three, since neither accumulators
+// with nine used rows of 32 nor masks occupy registers).  Beyond 131072 tokens the table of diagonals leaves LDS for two.
+template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS_SMALL ? 2 : 3) void pattern_recall_kernel(const RecallParams p) {
+    __shared__ unsigned dtab[DG];                       // bytes: OR, AND, OR without the first, AND without the first
     // two steps of two 32-key blocks each (one per key parity), 256-byte rows whose 16-byte chunks are
     // XOR-permuted (chunk ^ row % 16) so that the fragment reads of 32 rows hit distinct banks
     __shared__ __attribute__((aligned(16))) char kt[2][2 * KB * HD * 2];
+    // ... and their column flags: as fp32 ones and zeros by candidate and key (chunks of four keys permuted: chunk ^
+    // 2 (candidate % 4)), and as they are; and the flags of the diagonals a step touches, the farthest first
+    __shared__ __attribute__((aligned(16))) float cmask[2][NC][2 * KB];
+    __shared__ __attribute__((aligned(16))) unsigned cbytes[2][2 * KB / 4], dbytes[2][DW];
+    float (*const lds)[TILE][NC + 2] = reinterpret_cast<float (*)[TILE][NC + 2]>(&kt[0][0]);   // after the sweep
+    static_assert(sizeof(float) * 4 * TILE * (NC + 2) <= sizeof(kt), "the waves' shares take the place of K");
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
@@ -171,7 +163,7 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
         return;
     }
 
-    const int groups = min(min(4 * tp + 4, brows), DIAG_GROUPS);
+    const int groups = min(min(4 * tp + 4, brows), DG);
     for (int i = tid; i < groups; i += 256) {
         const unsigned *w = reinterpret_cast<const unsigned *>(diag + 32ll * i);
         unsigned o = 0u, an = 0xffffffffu, w0 = w[0];
@@ -195,21 +187,13 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
                 qf[1][ks].u[i] ^= p.q_flip;
             }
 
-    const unsigned neg_lo = minus_one_lo(), neg_hi = minus_one_hi();
     constexpr float LAZY = 6.f;                        // exponentials reach 2^-1 .. 2^LAZY
     float m[2] = {-INFINITY, -INFINITY};               // running maximum of the lane's row (same in both lane halves)
-    f32x16_t zacc[2];                                  // rows t = 8 (r / 4) + 4 g + r % 4: r 0..3 candidates 4 g + r, r 4 (g 0) the sum
-    float zx[2][NC];                                   // this lane's share of the element-wise sums
+    float zs[2] = {0.f, 0.f}, zc[2][NC];               // this lane's share (its keys) of the row sum and the masked sums
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
+    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) zacc[nb][r] = 0.f;
-#pragma unroll
-        for (int t = 0; t < NC; ++t) zx[nb][t] = 0.f;
-    }
-    // A operand: lane l holds row t = l % 32, contraction index 8 g + e <-> key 16 s + 8 (e / 4) + 4 g + e % 4
-    const unsigned a_and = l32 < NC ? 0x01010101u : 0u, a_or = l32 == NC ? 0x01010101u : 0u;
-    const int a_shift = l32 & 7;
+        for (int t = 0; t < NC; ++t) zc[nb][t] = 0.f;
 
     const bool counts = rt < p.tiles && (rt + 1) * TILE > p.row_begin;
     const int last_kb = counts ? min(2 * rt + 1, brows - 1) : -1;  // last key block any row of the tile sees
@@ -218,9 +202,7 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
     // the sequence read a valid row instead: no row of a head sees those keys)
     const int cp_r = lane >> 4, cp_c = lane & 15;
     const int row_bytes = (int)p.ks[2] * 2;
-    int cp_off[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) cp_off[j] = cp_r * row_bytes + ((cp_c ^ (4 * j + cp_r)) << 4);
+    const int cp_row = cp_r * row_bytes, cp_chunk = (cp_c ^ cp_r) << 4;
     auto copy_k = [&](int kb0, int buf) {
 #if defined(__HIP_DEVICE_COMPILE__)      // (the builtins do not exist in the host pass)
         if ((kb0 + 2) * KB <= p.n && p.ks[2] >= 0 && p.ks[2] <= (1 << 22)) {       // (the copies' offsets are 32-bit and unsigned)
@@ -229,54 +211,67 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
             const int extent = (2 * KB - 1) * row_bytes + HD * 2;
             const __amdgpu_buffer_rsrc_t srd = __builtin_amdgcn_make_buffer_rsrc((void *)(kbase + (long long)kb0 * KB * row_bytes), 0, extent, 0x00020000);
             const int lds0 = (int)(unsigned)(unsigned long long)(__attribute__((address_space(3))) char *)kt[buf] + 16 * wave * HD * 2;
+            int chunk = cp_chunk;
+            asm volatile("" : "+v"(chunk));            // (one instruction per copy rather than a register)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(srd, (__attribute__((address_space(3))) void *)(unsigned long long)(unsigned)(lds0 + 4 * j * HD * 2),
-                                                         16, cp_off[j], (16 * wave + 4 * j) * row_bytes, 0, 0);
+                                                         16, (chunk ^ (64 * j)) + cp_row, (16 * wave + 4 * j) * row_bytes, 0, 0);
             return;
         }
 #endif
+        int ln = lane;
+        asm volatile("" : "+v"(ln));                   // (or the addresses of this rare form occupy registers throughout the sweep)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int r = 16 * wave + 4 * j + cp_r;
-            const char *src = kbase + (long long)min(kb0 * KB + r, p.n - 1) * p.ks[2] * 2 + ((cp_c ^ (r & 15)) << 4);
+            const int r = 16 * wave + 4 * j + (ln >> 4);
+            const char *src = kbase + (long long)min(kb0 * KB + r, p.n - 1) * p.ks[2] * 2 + (((ln & 15) ^ (r & 15)) << 4);
             copy16_to_lds(src, kt[buf] + (16 * wave + 4 * j) * HD * 2);
         }
     };
-    // flags of this wave's key block: column words of the lane's 16 keys (keys n0 + 8j + 4g + i, one aligned
-    // word per j) and the block bytes of its two row blocks; fetched a step ahead
-    unsigned cw[4], bb[2] = {0u, 0u}, cw_next[4], bb_next[2] = {0u, 0u};
-    auto fetch_flags = [&](int kb, unsigned (&c)[4], unsigned (&bk)[2]) {
-        const int at = min(kb, brows - 1);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) c[j] = *reinterpret_cast<const unsigned *>(col + at * KB + 8 * j + 4 * g);
+    // what the next step needs beside K, fetched a step ahead: the flags of key kb0 * 32 + lane, four diagonal flags
+    // per thread (word w of a step holds offsets top - 4 w - 3 .. top - 4 w, top = 128 tp + 127 - 32 kb0; offsets below 0
+    // lie above the diagonal), the block bytes of this wave's two row blocks
+    unsigned cb_next = 0u, dw_next = 0u, bb_next[2] = {0u, 0u};
+    auto fetch_flags = [&](int kb0) {
+        cb_next = col[min(kb0 * KB + lane, brows * KB - 1)];
+        if (tid < DW) {
+            const int at = 2 * TILE * tp + 2 * TILE - 4 - KB * kb0 - 4 * tid;
+            dw_next = at >= 0 && at + 4 <= (int)p.flag_pitch ? *reinterpret_cast<const unsigned *>(diag + at) : 0u;
+        }
         if (blk)
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) bk[nb] = blk[(long long)min(2 * rt + nb, brows - 1) * p.blk_pitch + at];
+            for (int nb = 0; nb < 2; ++nb) bb_next[nb] = blk[(long long)min(2 * rt + nb, brows - 1) * p.blk_pitch + min(kb0 + kpar, brows - 1)];
     };
     copy_k(0, 0);
-    fetch_flags(kpar, cw_next, bb_next);
+    fetch_flags(0);
     for (int kb0 = 0; kb0 <= last_any; kb0 += 2) {
         const int buf = (kb0 >> 1) & 1, kb = kb0 + kpar, n0 = kb * KB;
+        const unsigned cb = cb_next, bb[2] = {bb_next[0], bb_next[1]};
+        // (nobody reads these buffers: their last readers were done before the last barrier)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) cw[j] = cw_next[j];
-        bb[0] = bb_next[0]; bb[1] = bb_next[1];
+        for (int t = 0; t < NC; t += 4)
+            cmask[buf][t + wave][(((lane >> 2) ^ (2 * wave)) << 2) | (lane & 3)] = (float)((cb >> (t + wave)) & 1u);
+        if (wave == 3) reinterpret_cast<unsigned char *>(cbytes[buf])[lane] = (unsigned char)cb;
+        if (tid < DW) dbytes[buf][tid] = __builtin_bswap32(dw_next);
+        const unsigned long long kept_lo = __ballot((cb & 0x0fu) != 0u), kept_hi = __ballot((cb & 0xf0u) != 0u);
+        const bool cols[2] = {(unsigned)(kept_lo >> (32 * kpar)) != 0u, (unsigned)(kept_hi >> (32 * kpar)) != 0u};   // candidates 0..3, 4..7
         __builtin_amdgcn_s_waitcnt(0x0f70);            // vmcnt(0): this wave's share of the step is in LDS
         __syncthreads();                               // ... and everybody's; everyone is done with the step before
         if (kb0 + 2 <= last_any) {
             copy_k(kb0 + 2, buf ^ 1);
-            fetch_flags(kb + 2, cw_next, bb_next);
+            fetch_flags(kb0 + 2);
         }
         if (kb > last_kb) continue;                    // (wave-uniform; no barrier below)
         unsigned full[2], mixed[2];                    // candidates that keep all / some of a block, by its row block
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
             const int rb = min(2 * rt + nb, brows - 1), d = max(rb - kb, 0);
-            const unsigned here = __builtin_amdgcn_readfirstlane(dtab[min(d, DIAG_GROUPS - 1)]);
-            unsigned before = __builtin_amdgcn_readfirstlane(dtab[min(max(d - 1, 0), DIAG_GROUPS - 1)]) >> 16;
+            const unsigned here = __builtin_amdgcn_readfirstlane(dtab[min(d, DG - 1)]);
+            unsigned before = __builtin_amdgcn_readfirstlane(dtab[min(max(d - 1, 0), DG - 1)]) >> 16;
             if (d == 0) before = 0xff00u;              // (nothing before the main diagonal)
             unsigned any = (here | before) & 0xffu, all = (here & before) >> 8;
-            if (d >= DIAG_GROUPS) { any = 0xffu; all = 0u; }
+            if (d >= DG) { any = 0xffu; all = 0u; }
             full[nb] = __builtin_amdgcn_readfirstlane(bb[nb]) | (all & 0xffu);
             mixed[nb] = any & ~full[nb];
         }
@@ -291,16 +286,6 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
             acc[0] = mma<T>(kf, qf[0][ks], acc[0]);
             acc[1] = mma<T>(kf, qf[1][ks], acc[1]);
         }
-
-        Frag am[2];                                    // the columns' masks, shared by both row blocks
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj) {
-                const unsigned x = ((cw[2 * s + jj] >> a_shift) & a_and) | a_or;
-                am[s].u[2 * jj] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c010c00u), 0x3f80u);
-                am[s].u[2 * jj + 1] = __umul24(__builtin_amdgcn_perm(0u, x, 0x0c030c02u), 0x3f80u);
-            }
 
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
@@ -324,57 +309,37 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
                 // and what is summed under the next are in proportion to the last bit)
                 const float up = ceilf(cand), alpha = grow ? fast_exp2(m[nb] - up) : 1.0f;
                 m[nb] = grow ? up : m[nb];
+                zs[nb] *= alpha;
 #pragma unroll
-                for (int r = 0; r < 5; ++r) zacc[nb][r] *= alpha;
-#pragma unroll
-                for (int t = 0; t < NC; ++t) zx[nb][t] *= alpha;
+                for (int t = 0; t < NC; ++t) zc[nb][t] *= alpha;
             }
             float e[16];
             const float off = m[nb] == -INFINITY ? 0.f : -m[nb];           // (no key yet whose score is above -inf)
 #pragma unroll
             for (int r = 0; r < 16; ++r) e[r] = fast_exp2(fmaf(acc[nb][r], p.scale_log2, off));
-            Frag a0 = am[0], a1 = am[1];
-            if (full[nb]) {                                            // candidates that keep the whole block
-                const bool mine = (full[nb] >> a_shift) & a_and & 1u;
+            // the block's sums from zero: row sum, columns of each candidate
+            f32x4_t zb[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    a0.u[i] = mine ? 0x3f803f80u : a0.u[i];
-                    a1.u[i] = mine ? 0x3f803f80u : a1.u[i];
-                }
-            }
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                Frag hi, mid, lo;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float x = e[8 * s + 2 * i], y = e[8 * s + 2 * i + 1];
-                    hi.u[i] = pack_bf16(x, y);
-                    const float x1 = left_of(x, hi.u[i], neg_lo), y1 = left_of(y, hi.u[i], neg_hi);
-                    mid.u[i] = pack_bf16(x1, y1);
-                    lo.u[i] = pack_bf16(left_of(x1, mid.u[i], neg_lo), left_of(y1, mid.u[i], neg_hi));
-                }
-                zacc[nb] = mma<__bf16>(s ? a1 : a0, hi, zacc[nb]);
-                zacc[nb] = mma<__bf16>(s ? a1 : a0, mid, zacc[nb]);
-                zacc[nb] = mma<__bf16>(s ? a1 : a0, lo, zacc[nb]);
-            }
-            if (mixed[nb]) {
-                // diagonal flags: key i of group j has offset o0 - i, o0 = row - (n0 + 8j + 4g); the word
-                // read at o0-3 holds it in byte 3-i
-                unsigned pm[4];
-                const int first = row - n0 - 4 * g - 3;
-                if (kb != rb) {                                    // every offset is positive
-                    const unsigned char *dp = diag + first;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) pm[j] = __builtin_bswap32(load_u32_unaligned(dp - 8 * j)) & ~cw[j];
-                } else {
-                    // on the main diagonal o0-3 may be negative: read at 0 and shift the bytes up (offsets < 0
-                    // are above the diagonal, their exponentials are 0 anyway)
+            for (int c = 0; c < 2; ++c)
+                if (cols[c])
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const int at = first - 8 * j, base = max(at, 0), up = base - at;
-                        const unsigned w = load_u32_unaligned(diag + base);
-                        pm[j] = __builtin_bswap32(up >= 4 ? 0u : (w << (8 * up))) & ~cw[j];
+                        const f32x4_t a = *reinterpret_cast<const f32x4_t *>(&cmask[buf][4 * c + (lane & 3)][((8 * kpar + 2 * j + g) ^ (2 * (lane & 3))) << 2]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) zb[c] = mma4(a[i], e[4 * j + i], zb[c]);
                     }
+            const float sum = (((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7])))
+                + (((e[8] + e[9]) + (e[10] + e[11])) + ((e[12] + e[13]) + (e[14] + e[15])));
+            zs[nb] += sum;
+            if (mixed[nb]) {
+                // diagonal flags of keys n0 + 8j + 4g + 0..3, without the kept columns
+                unsigned pm[4];
+                const unsigned char *const dp = reinterpret_cast<const unsigned char *>(dbytes[buf]) + (2 * TILE * tp + 2 * TILE - 1 - KB * kb0) - (row - n0 - 4 * g);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    unsigned w;
+                    __builtin_memcpy(&w, dp + 8 * j, 4);
+                    pm[j] = w & ~cbytes[buf][8 * kpar + 2 * j + g];
                 }
 #pragma unroll
                 for (int t = 0; t < NC; ++t)
@@ -382,29 +347,33 @@ template <typename T> __global__ __launch_bounds__(256, 2) void pattern_recall_k
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             const unsigned x = (pm[j] >> t) & 0x01010101u;
-                            float z = zx[nb][t];
+                            float z = zb[t >> 2][t & 3];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) z = fmaf((float)((x >> (8 * i)) & 0xffu), e[4 * j + i], z);
-                            zx[nb][t] = z;
+                            zb[t >> 2][t & 3] = z;
                         }
                     }
             }
+#pragma unroll
+            for (int t = 0; t < NC; ++t) zc[nb][t] += (full[nb] >> t) & 1u ? sum : zb[t >> 2][t & 3];
         }
     }
 
-    // merge the two lanes of a row and the element-wise sums, then the two waves
+    // merge the two lanes of a row, then the two waves
+    __syncthreads();
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
         float *dst = lds[wave][nb * 32 + l32];
+        const float total = zs[nb] + __shfl_xor(zs[nb], 32);
         if (g == 0) {
             dst[0] = m[nb];
-            dst[1] = zacc[nb][4];
+            dst[1] = total;
         }
         float own[NC];
 #pragma unroll
-        for (int t = 0; t < NC; ++t) own[t] = zx[nb][t] + __shfl_xor(zx[nb][t], 32);
+        for (int t = 0; t < NC; ++t) own[t] = zc[nb][t] + __shfl_xor(zc[nb][t], 32);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) dst[2 + 4 * g + r] = zacc[nb][r] + (g ? own[4 + r] : own[r]);
+        for (int r = 0; r < 4; ++r) dst[2 + 4 * g + r] = g ? own[4 + r] : own[r];
     }
     __syncthreads();
     if (kpar == 0 && rt < p.tiles) {
@@ -527,10 +496,15 @@ extern "C" int minf_pattern_recall(const void *q, const void *k, const int64_t *
     if (wgs > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
     p.total_wg = (unsigned)wgs;
     const dim3 grid((unsigned)wgs);
-    if (dtype == MINF_BF16)
-        hipLaunchKernelGGL(pattern_recall_kernel<__bf16>, grid, dim3(256), 0, st, p);
+    const bool small = (n + KB - 1) / KB <= DIAG_GROUPS_SMALL;
+    if (dtype == MINF_BF16 && small)
+        hipLaunchKernelGGL((pattern_recall_kernel<__bf16, DIAG_GROUPS_SMALL>), grid, dim3(256), 0, st, p);
+    else if (dtype == MINF_BF16)
+        hipLaunchKernelGGL((pattern_recall_kernel<__bf16, DIAG_GROUPS>), grid, dim3(256), 0, st, p);
+    else if (small)
+        hipLaunchKernelGGL((pattern_recall_kernel<_Float16, DIAG_GROUPS_SMALL>), grid, dim3(256), 0, st, p);
     else
-        hipLaunchKernelGGL(pattern_recall_kernel<_Float16>, grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((pattern_recall_kernel<_Float16, DIAG_GROUPS>), grid, dim3(256), 0, st, p);
     int status = minf_launch_status();
     if (status != MINF_OK) return status;
     hipLaunchKernelGGL(pattern_recall_finalize, dim3(batch * heads_q), dim3(64), 0, st, p.partial, tiles, n,

@@ -210,6 +210,42 @@ def _recall_of(q, k_ptr, k_strides, hk, n, cands, sm_scale=128.0 ** -0.5, flags=
     return recall[:, :len(cands)] if flags is None else recall
 
 
+@pytest.mark.parametrize("n", [131072, 131073, 131199, 262144 + 33])
+def test_recall_where_the_table_of_diagonals_grows_and_ends(gpu, n):
+    """The two table sizes (131072 and 262144 tokens) and distances past the table, for the last rows: random columns and
+    diagonals, windows that end inside a block, a candidate without columns, one with all.  Both sums of a row are fp32
+    sums of about n / 64 block sums, each with a rounding of at most 2^-24."""
+    g = torch.Generator(device=gpu).manual_seed(n)
+    q = torch.randn(1, 1, n, 128, device=gpu, generator=g).bfloat16()
+    k = torch.randn(1, 1, n, 128, device=gpu, generator=g).bfloat16()
+    begin, pitch = n - 70, (n + 63) // 64 * 64
+    col = torch.randint(0, 256, (1, pitch), device=gpu, generator=g, dtype=torch.uint8) & 0x5d
+    col |= 0x80
+    diag = torch.randint(0, 256, (1, pitch), device=gpu, generator=g, dtype=torch.uint8) & 0x16
+    diag[:, :1000] |= 0x08
+    diag[:, 999:n // 2 + 5] |= 0x20
+    got = _recall_begin(q, k, col, diag, begin)
+    r, c = torch.arange(begin, n, device=gpu)[:, None], torch.arange(n, device=gpu)[None]
+    s = q[0, 0, begin:].double() @ k[0, 0].double().t().contiguous() * 128 ** -0.5
+    p = torch.softmax(s.masked_fill(c > r, float("-inf")), -1)
+    flags = col[0, :n][None] | diag[0][(r - c).clamp(min=0)]
+    for t in range(8):
+        want = float((p * ((flags >> t) & 1)).sum() / (n - begin))
+        assert abs(float(got[0, t]) - want) <= 2 * (n / 64 + 64) * 2.0 ** -24 * want, t
+
+
+def _recall_begin(q, k, col, diag, begin):
+    from minference_amd import _lib
+    lib, n, i64x3 = _lib.load(), q.shape[2], _lib.c_i64 * 3
+    recall = torch.empty(1, 8, dtype=torch.float32, device=q.device)
+    nbytes = lib.minf_pattern_recall_workspace_bytes(1, 1, n)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+    _lib.check(lib.minf_pattern_recall(q.data_ptr(), k.data_ptr(), i64x3(*q.stride()[:3]), i64x3(*k.stride()[:3]), 1, 1, 1, n, 128,
+                                       _lib.MINF_BF16, 128 ** -0.5, col.data_ptr(), diag.data_ptr(), col.shape[1], None, 0, begin,
+                                       recall.data_ptr(), ws.data_ptr(), nbytes, _lib.stream_ptr(q.device)), "minf_pattern_recall")
+    return recall
+
+
 @pytest.mark.parametrize("n", [64, 300, 1025])
 @pytest.mark.parametrize("stride", [0, 8, 64, 136])
 def test_recall_reads_every_row_of_k_whatever_its_token_stride(gpu, n, stride):
