@@ -118,11 +118,14 @@ constexpr int DIAG_GROUPS_SMALL = 4096;      // (131072 tokens: three workgroups
 // exponential on 32x32x16 products, which this replaces: 6.8e-8), under a sink of 14 nats 3.3e-8 (1.8e-7); shares of
 // candidates without a sink of 14 .. 80 nats 1.9e-6 at most (6.5e-6; 3.1e-7 against 2.2e-7 at 14): there the rounding of
 // the scale in fp32 bounds it.
-// Bound by its vector instructions, 147 per 32 x 32 block (fma and exp 32, of which the exp take four times as long; maximum,
-// row sum, and 40 per candidate with mixed diagonals) beside 10 MFMAs.  32 / 8 heads, 16384 tokens, the six candidates of the
-// reference: 2.83 -> 2.19 ms against the bf16 terms (56 conversions per block; masks built in registers by every
-// wave, where one of a workgroup's threads now writes them to LDS once; two waves per SIMD, now three, since neither accumulators
-// with nine used rows of 32 nor masks occupy registers).  Beyond 131072 tokens the table of diagonals leaves LDS for two.
+// Bound by its vector instructions, 131 per 32 x 32 block (fma and exp 32, of which the exp take four times as long; maximum,
+// row sum, and 40 per candidate with mixed diagonals: 630 of 894 cycles) and its matrix products (270 cycles), which overlap
+// little.  32 / 8 heads, 16384 tokens, the six candidates of the reference: 2.81 -> 2.00 ms against the bf16 terms (56
+// conversions per block; masks built in registers by every wave, where one of a workgroup's threads now writes them to LDS
+// once; two waves per SIMD, now three, since neither accumulators with nine used rows of 32 nor masks occupy
+// registers).  0.18 ms of it: no value that a step fetches for the next is touched before the next barrier (a wait for a
+// flag byte was a wait for the K rows before it), one LDS read for the four distances of a step, fragment addresses by XOR from
+// one register.  Beyond 131072 tokens the table of diagonals leaves LDS for two.
 template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS_SMALL ? 2 : 3) void pattern_recall_kernel(const RecallParams p) {
     __shared__ unsigned dtab[DG];                       // bytes: OR, AND, OR without the first, AND without the first
     // two steps of two 32-key blocks each (one per key parity), 256-byte rows whose 16-byte chunks are
@@ -229,12 +232,12 @@ template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS
             copy16_to_lds(src, kt[buf] + (16 * wave + 4 * j) * HD * 2);
         }
     };
-    // what the next step needs beside K, fetched a step ahead: the flags of key kb0 * 32 + lane, four diagonal flags
+    // what the next step needs beside K, fetched a step ahead: the flags of four keys around kb0 * 32 + lane, four diagonal flags
     // per thread (word w of a step holds offsets top - 4 w - 3 .. top - 4 w, top = 128 tp + 127 - 32 kb0; offsets below 0
     // lie above the diagonal), the block bytes of this wave's two row blocks
     unsigned cb_next = 0u, dw_next = 0u, bb_next[2] = {0u, 0u};
     auto fetch_flags = [&](int kb0) {
-        cb_next = col[min(kb0 * KB + lane, brows * KB - 1)];
+        cb_next = *reinterpret_cast<const unsigned *>(col + min(kb0 * KB + (lane & ~3), brows * KB - 4));   // (its byte is taken when it is used: no wait here)
         if (tid < DW) {
             const int at = 2 * TILE * tp + 2 * TILE - 4 - KB * kb0 - 4 * tid;
             dw_next = at >= 0 && at + 4 <= (int)p.flag_pitch ? *reinterpret_cast<const unsigned *>(diag + at) : 0u;
@@ -247,7 +250,7 @@ template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS
     fetch_flags(0);
     for (int kb0 = 0; kb0 <= last_any; kb0 += 2) {
         const int buf = (kb0 >> 1) & 1, kb = kb0 + kpar, n0 = kb * KB;
-        const unsigned cb = cb_next, bb[2] = {bb_next[0], bb_next[1]};
+        const unsigned cb = (cb_next >> (8 * (lane & 3))) & 0xffu, bb[2] = {bb_next[0], bb_next[1]};
         // (nobody reads these buffers: their last readers were done before the last barrier)
 #pragma unroll
         for (int t = 0; t < NC; t += 4)
@@ -264,12 +267,15 @@ template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS
         }
         if (kb > last_kb) continue;                    // (wave-uniform; no barrier below)
         unsigned full[2], mixed[2];                    // candidates that keep all / some of a block, by its row block
+        // (one read for the two distances and the ones before them: lane 2 nb + 1 - x holds distance d(nb) - x)
+        const int d0 = 2 * rt - kb;
+        const unsigned near_ = dtab[min(max(d0 - 1 + (lane & 1) + ((lane >> 1) & 1), 0), DG - 1)];
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
-            const int rb = min(2 * rt + nb, brows - 1), d = max(rb - kb, 0);
-            const unsigned here = __builtin_amdgcn_readfirstlane(dtab[min(d, DG - 1)]);
-            unsigned before = __builtin_amdgcn_readfirstlane(dtab[min(max(d - 1, 0), DG - 1)]) >> 16;
-            if (d == 0) before = 0xff00u;              // (nothing before the main diagonal)
+            const int d = d0 + nb;
+            const unsigned here = __builtin_amdgcn_readlane(near_, 2 * nb + 1);
+            unsigned before = __builtin_amdgcn_readlane(near_, 2 * nb) >> 16;
+            if (d <= 0) before = 0xff00u;              // (nothing before the main diagonal)
             unsigned any = (here | before) & 0xffu, all = (here & before) >> 8;
             if (d >= DG) { any = 0xffu; all = 0u; }
             full[nb] = __builtin_amdgcn_readfirstlane(bb[nb]) | (all & 0xffu);
@@ -278,11 +284,11 @@ template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS
         f32x16_t acc[2];
 #pragma unroll
         for (int r = 0; r < 16; ++r) { acc[0][r] = 0.f; acc[1][r] = 0.f; }
-        const char *krow = kt[buf] + (kpar * KB + l32) * HD * 2;
+        const int kat = ((buf * 2 + kpar) * KB + l32) * HD * 2 + ((g ^ (l32 & 15)) << 4);
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
             Frag kf;
-            kf.u = *reinterpret_cast<const u32x4_t *>(krow + (((2 * ks + g) ^ (l32 & 15)) << 4));
+            kf.u = *reinterpret_cast<const u32x4_t *>(&kt[0][0] + (kat ^ (32 * ks)));
             acc[0] = mma<T>(kf, qf[0][ks], acc[0]);
             acc[1] = mma<T>(kf, qf[1][ks], acc[1]);
         }
@@ -346,7 +352,8 @@ template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS
                     if ((mixed[nb] >> t) & 1u) {
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
-                            const unsigned x = (pm[j] >> t) & 0x01010101u;
+                            unsigned x = (pm[j] >> t) & 0x01010101u;
+                            asm("" : "+v"(x));         // (four conversions of its bytes, not a bit field and a conversion for each)
                             float z = zb[t >> 2][t & 3];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) z = fmaf((float)((x >> (8 * i)) & 0xffu), e[4 * j + i], z);
@@ -355,7 +362,10 @@ template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS
                     }
             }
 #pragma unroll
-            for (int t = 0; t < NC; ++t) zc[nb][t] += (full[nb] >> t) & 1u ? sum : zb[t >> 2][t & 3];
+            for (int c = 0; c < 2; ++c)
+                if (cols[c] || (((full[nb] | mixed[nb]) >> (4 * c)) & 0xfu))
+#pragma unroll
+                    for (int t = 4 * c; t < 4 * c + 4; ++t) zc[nb][t] += (full[nb] >> t) & 1u ? sum : zb[c][t & 3];
         }
     }
 
