@@ -7,13 +7,17 @@
 // of its workgroups, every workgroup of the second one folds those, converts its share and one of them
 // leaves the dtype code that the attention launches and the widening kernel read
 // (minf_qkvo.dtype_select).  Bound by bytes: q, k and v are read twice (the second time mostly from the
-// Infinity Cache) and written once at half the size.  With the choice read back by the host (three
+// Infinity Cache) and written once at half the size.  The first
+// kernel has four vectors of a thread under way and reads a tensor that fills one stretch of memory by its vectors' numbers
+// alone: with one load at a time, placed by three divisions, it took 13.4 us for 3 x 16.8 MB (8192 tokens, 4 heads of
+// 128), now 9.0 = 5.6 TB/s; the second one 13.4 = 5.7 TB/s with one step or four under way.  With the choice read back by the host (three
 // reductions, a synchronisation, three conversions) the GPU idled about 60 us per call.
 #include "minf_common.h"
 
 namespace {
 
 constexpr int NARROW_THREADS = 256;
+constexpr int UNDER_WAY = 4;     // vectors a thread of the first kernel has under way
 constexpr int NARROW_PARTIALS = MINF_NARROW_WORKSPACE_INTS - 1;      // amax workgroups, a third per tensor
 constexpr int NARROW_WGS = NARROW_PARTIALS / 3;
 static_assert(NARROW_WGS * 3 == NARROW_PARTIALS, "the same number of workgroups for each tensor");
@@ -24,17 +28,25 @@ struct NarrowTensor {
     long long stride[3];         // elements: batch, head, token
     long long rows;              // batch * heads * n
     int heads;
+    int dense;                   // the tensor fills one stretch of memory
+    FastDiv by_n, by_heads;
 };
 struct NarrowParams {
     NarrowTensor t[3];
-    int n, dim, dim_out;
+    int dim;
+    FastDiv by_dim, by_dim_out;  // vectors per row, in / out
     int *ws;                     // [0]: the dtype code, then the partial maxima (bit patterns)
 };
 
-// (I: 32-bit numbers of vectors wherever they fit; 64-bit divisions cost more than the loads they place)
-template <typename I> __device__ __forceinline__ const float *row_ptr(const NarrowTensor &t, int n, I row) {
-    const unsigned bh = (unsigned)(row / (I)n), at = (unsigned)(row - (I)bh * (I)n);
-    return t.in + (long long)(bh / (unsigned)t.heads) * t.stride[0] + (long long)(bh % (unsigned)t.heads) * t.stride[1] + (long long)at * t.stride[2];
+// (I: 32-bit numbers of vectors wherever they fit, placed by multiplications; else 64-bit ones, placed by divisions)
+__device__ __forceinline__ unsigned quot(unsigned x, const FastDiv &f) { return fast_quot(x, f); }
+__device__ __forceinline__ unsigned long long quot(unsigned long long x, const FastDiv &f) { return x / f.d; }
+
+// where vector i of a row-wise walk of a tensor lies, `width` elements per vector
+template <typename I> __device__ __forceinline__ const float *vector_ptr(const NarrowTensor &t, const FastDiv &per_row, int width, I i, int &d) {
+    const I row = quot(i, per_row), bh = quot(row, t.by_n), b = quot(bh, t.by_heads);
+    d = width * (int)(i - row * per_row.d);
+    return t.in + (long long)b * t.stride[0] + (long long)(bh - b * t.by_heads.d) * t.stride[1] + (long long)(row - bh * t.by_n.d) * t.stride[2] + d;
 }
 
 // largest bit pattern of |x| (NaN above infinity above every number) over the workgroup, in thread 0 .. 255
@@ -51,13 +63,19 @@ __device__ __forceinline__ unsigned wg_max(unsigned m, unsigned (&part)[NARROW_T
 template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_amax_kernel(const NarrowParams p) {
     __shared__ unsigned part[NARROW_THREADS / 64];
     const NarrowTensor t = p.t[blockIdx.y];
-    const unsigned per_row = (unsigned)p.dim / 4u;
-    const I total = (I)(t.rows * per_row);
+    const I total = (I)t.rows * p.by_dim.d, step = (I)NARROW_WGS * NARROW_THREADS;
     unsigned m = 0;
-    for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += (I)NARROW_WGS * NARROW_THREADS) {
-        const I row = i / per_row;
-        const uint4 x = *reinterpret_cast<const uint4 *>(row_ptr<I>(t, p.n, row) + 4 * (int)(i - row * per_row));
-        m = max(max(max(m, x.x & 0x7fffffffu), x.y & 0x7fffffffu), max(x.z & 0x7fffffffu, x.w & 0x7fffffffu));
+    for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += UNDER_WAY * step) {
+        uint4 x[UNDER_WAY];
+#pragma unroll
+        for (int u = 0; u < UNDER_WAY; ++u) {
+            const I at = min(i + u * step, total - 1);     // (the last vector again, past the end)
+            int d;
+            x[u] = *reinterpret_cast<const uint4 *>(t.dense ? t.in + 4 * (long long)at : vector_ptr<I>(t, p.by_dim, 4, at, d));
+        }
+#pragma unroll
+        for (int u = 0; u < UNDER_WAY; ++u)
+            m = max(max(max(m, x[u].x & 0x7fffffffu), x[u].y & 0x7fffffffu), max(x[u].z & 0x7fffffffu, x[u].w & 0x7fffffffu));
     }
     m = wg_max(m, part);
     if (threadIdx.x == 0) p.ws[1 + blockIdx.y * NARROW_WGS + blockIdx.x] = (int)m;
@@ -71,12 +89,10 @@ template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_k
     const bool f16 = m >= __float_as_uint(0x1p-10f) && m <= __float_as_uint(32768.0f);
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.ws[0] = f16 ? MINF_F16 : MINF_BF16;
     const NarrowTensor t = p.t[blockIdx.y];
-    const unsigned per_row = (unsigned)p.dim_out / 8u;                   // 8 output elements per thread and step
-    const I total = (I)(t.rows * per_row);
+    const I total = (I)t.rows * p.by_dim_out.d;                          // 8 output elements per thread and step
     for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += (I)gridDim.x * NARROW_THREADS) {
-        const I row = i / per_row;
-        const int d = 8 * (int)(i - row * per_row);
-        const float *src = row_ptr<I>(t, p.n, row) + d;
+        int d;
+        const float *src = vector_ptr<I>(t, p.by_dim_out, 8, i, d);
         float4 x[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) x[h] = d + 4 * h < p.dim ? *reinterpret_cast<const float4 *>(src + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -110,6 +126,22 @@ __global__ __launch_bounds__(NARROW_THREADS) void widen_kernel(const char *__res
     }
 }
 
+// does the tensor fill one stretch of memory, whatever the order of its dimensions?
+bool fills_memory(const NarrowTensor &t, int batch, int n, int dim) {
+    const long long size[3] = {batch, t.heads, n};
+    bool done[3] = {false, false, false};
+    long long extent = dim;
+    for (int round = 0; round < 3; ++round) {
+        int next = -1;
+        for (int i = 0; i < 3; ++i)
+            if (!done[i] && (size[i] == 1 || t.stride[i] == extent)) next = i;
+        if (next < 0) return false;
+        done[next] = true;
+        extent *= size[next];
+    }
+    return true;
+}
+
 unsigned narrow_grid(long long vectors) {
     const long long wgs = (vectors + 4 * NARROW_THREADS - 1) / (4 * NARROW_THREADS);
     return (unsigned)(wgs < 1 ? 1 : (wgs > 2048 ? 2048 : wgs));
@@ -136,18 +168,24 @@ extern "C" int minf_narrow_qkv(const minf_qkvo *t, int dim_in, void *q16, void *
         p.t[i].out = (char *)out[i];
         p.t[i].heads = i == 0 ? t->heads_q : t->heads_kv;
         p.t[i].rows = (long long)t->batch * p.t[i].heads * t->n;
+        p.t[i].by_n = fast_div((unsigned)t->n);
+        p.t[i].by_heads = fast_div((unsigned)p.t[i].heads);
+        p.t[i].dense = fills_memory(p.t[i], t->batch, t->n, dim_in);
     }
-    p.n = t->n; p.dim = dim_in; p.dim_out = t->head_dim;
+    p.dim = dim_in;
+    p.by_dim = fast_div((unsigned)dim_in / 4u);
+    p.by_dim_out = fast_div((unsigned)t->head_dim / 8u);
     p.ws = workspace;
     hipStream_t st = (hipStream_t)stream;
-    // (a margin below 2^32 for the last step past the end)
+    // (multiplications place numbers below 2^31)
     const long long most = p.t[0].rows > p.t[1].rows ? p.t[0].rows : p.t[1].rows;
-    const bool small = most * (dim_in / 4 > p.dim_out / 8 ? dim_in / 4 : p.dim_out / 8) < 0xf0000000LL;
+    const long long widest = p.by_dim.d > p.by_dim_out.d ? p.by_dim.d : p.by_dim_out.d;
+    const bool small = most * widest < 0x7fffffffLL;
     if (small) hipLaunchKernelGGL(narrow_amax_kernel<unsigned>, dim3(NARROW_WGS, 3), dim3(NARROW_THREADS), 0, st, p);
     else hipLaunchKernelGGL(narrow_amax_kernel<unsigned long long>, dim3(NARROW_WGS, 3), dim3(NARROW_THREADS), 0, st, p);
     const int status = minf_launch_status();
     if (status != MINF_OK) return status;
-    const dim3 grid(narrow_grid(p.t[0].rows * (p.dim_out / 8)), 3);
+    const dim3 grid(narrow_grid(p.t[0].rows * p.by_dim_out.d), 3);
     if (small) hipLaunchKernelGGL(narrow_kernel<unsigned>, grid, dim3(NARROW_THREADS), 0, st, p);
     else hipLaunchKernelGGL(narrow_kernel<unsigned long long>, grid, dim3(NARROW_THREADS), 0, st, p);
     return minf_launch_status();

@@ -46,6 +46,34 @@ def test_strided_unaligned_and_caller_owned_tensors(gpu):
                        M.dense_causal_attention(q.half(), k[:, :1].expand(2, 2, 400, 128).half(), v.half()).float())
 
 
+@pytest.mark.parametrize("n", [1024, 1025, 3071, 4096, 4097])
+@pytest.mark.parametrize("layout", ["rows", "tokens first", "gaps", "one row for all heads"])
+def test_the_largest_value_is_found_wherever_it_lies(gpu, n, layout):
+    """2 heads of 128 around the 65536 vectors that all threads read in one step and the 262144 of four; tensors that fill
+    one stretch of memory and ones that do not; the one value that asks for bf16 first, last and in between."""
+    import minference_amd as M
+    g = torch.Generator(device=gpu).manual_seed(n)
+    q, k, x = (torch.randn(1, 2, n, 128, device=gpu, generator=g) for _ in range(3))
+    if layout == "tokens first":
+        v = x.transpose(1, 2).contiguous().transpose(1, 2)
+    elif layout == "gaps":
+        v = torch.full((1, 2, n, 132), 1e9, device=gpu)[..., :128]      # (what lies in the gaps must not count)
+        v.copy_(x)
+    elif layout == "rows":
+        v = x
+    else:
+        v = x[:, :1].expand(1, 2, n, 128)
+    f = lambda: M.streaming_forward(q, k, v, 16, 100)
+    want = lambda dtype: M.streaming_forward(q.to(dtype), k.to(dtype), v.to(dtype), 16, 100).float()
+    assert torch.equal(f(), want(torch.float16))
+    last = 0 if layout.startswith("one") else 1
+    for h, t, d in ((0, 0, 0), (last, n - 1, 127), (last, n // 2, 64)):
+        old = float(v[0, h, t, d])
+        v[0, h, t, d] = 40000.0
+        assert torch.equal(f(), want(torch.bfloat16)), (h, t, d)
+        v[0, h, t, d] = old
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_values_that_are_no_numbers_choose_bf16(gpu, bad):
     import minference_amd as M
