@@ -8,9 +8,11 @@
 // read and written in all): each wavefront owns a contiguous stretch of the row in registers and ranks it
 // 64 values at a time -- eight ballots find the lanes with the same digit, one LDS word per digit and
 // wavefront counts them -- so that nothing is contended and the order of equal digits is kept.
-// Rows of 1000 + 2048 int64 values, 4 heads: 10.7 us, where the conversions, the two sorts and the copies
-// around them were ten launches and 50 us of GPU time; the operator on them, fp32 tensors of 8192 tokens,
-// 309 -> 265 us, on rows of 100 + 750 values, 2 x 16 heads of 597 tokens 119 -> 78 us.
+// A pass has three barriers; the scan reads a digit's counts of all wavefronts before it stores any (load behind
+// store was a round trip to LDS each).  Pairs of 500 + 700 int64 values, one row: 7.5 -> 4.9 us, 1000 + 6096, 32 rows
+// 17.2 -> 13.7.  Before this kernel the conversions, the two sorts and
+// the copies around them were ten launches and 50 us of GPU time (1000 + 2048 values, 4 heads); the operator on them, fp32 tensors of 8192 tokens,
+// took 309 instead of 265 us, on rows of 100 + 750 values, 2 x 16 heads of 597 tokens 119 -> 78 us.
 #include "minf_common.h"
 
 namespace {
@@ -31,8 +33,8 @@ template <int E>
 __global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProblem pa, const SortProblem pb, int rows) {
     __shared__ unsigned keys[E * SORT_THREADS];
     __shared__ unsigned hist[SORT_WAVES][SORT_DIGITS];     // values of a digit in the wavefronts before (after the scan)
-    __shared__ unsigned first[SORT_DIGITS];                // place of a digit's first value
-    __shared__ unsigned wsum[SORT_WAVES], differ;
+    __shared__ unsigned first[SORT_DIGITS];                // place of a digit's first value behind those of its 64 digits
+    __shared__ unsigned wsum[SORT_DIGITS / MINF_WAVE], differ;     // values of 64 digits; bytes in which values differ
     const bool second = (int)blockIdx.x >= rows;           // (workgroup-uniform)
     const SortProblem p = second ? pb : pa;
     const long long row = (long long)blockIdx.x - (second ? rows : 0);
@@ -48,9 +50,16 @@ __global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProb
         const long long at = row * p.n + i;
         return (unsigned)(p.is64 ? (int32_t)reinterpret_cast<const int64_t *>(p.in)[at] : reinterpret_cast<const int32_t *>(p.in)[at]) ^ p.flip;
     };
-    const unsigned key0 = load(0);
+    // (each wavefront alone uses its row of hist between the scans: no barrier around the zeros)
+    auto clear_own = [&]() {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < SORT_DIGITS; i += MINF_WAVE) hist[wave][i + lane] = 0;
+    };
+    clear_own();
     if (tid == 0) differ = 0;
     __syncthreads();
+    const unsigned key0 = load(0);
     unsigned diff = 0;
 #pragma unroll
     for (int r = 0; r < E; ++r) {
@@ -61,7 +70,11 @@ __global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProb
             diff |= key[r] ^ key0;
         }
     }
-    if (diff) atomicOr(&differ, diff);
+    unsigned bytes = 0;                                    // bit b: values of this wavefront differ in byte b
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+        if (__ballot(((diff >> (8 * b)) & 0xffu) != 0)) bytes |= 1u << b;
+    if (lane == 0 && bytes) atomicOr(&differ, bytes);
 #pragma unroll
     for (int r = 0; r < E; ++r)
         if (r < groups) keys[base + r * MINF_WAVE] = key[r];
@@ -69,9 +82,7 @@ __global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProb
     const unsigned differing = differ;
 
     for (int shift = 0; shift < 32; shift += 8) {
-        if (((differing >> shift) & 0xffu) == 0) continue;                // (uniform)
-        for (int i = tid; i < SORT_WAVES * SORT_DIGITS; i += SORT_THREADS) (&hist[0][0])[i] = 0;
-        __syncthreads();
+        if (((differing >> (shift / 8)) & 1u) == 0) continue;             // (uniform)
         unsigned rank[E];
 #pragma unroll
         for (int r = 0; r < E; ++r) {
@@ -92,35 +103,34 @@ __global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProb
             __builtin_amdgcn_wave_barrier();
         }
         __syncthreads();
-        unsigned total = 0, incl = 0;
         if (tid < SORT_DIGITS) {
+            unsigned c[SORT_WAVES], total = 0;                            // (read at once, not each behind a store)
+#pragma unroll
+            for (int w = 0; w < SORT_WAVES; ++w) c[w] = hist[w][tid];
 #pragma unroll
             for (int w = 0; w < SORT_WAVES; ++w) {
-                const unsigned c = hist[w][tid];
                 hist[w][tid] = total;
-                total += c;
+                total += c[w];
             }
-            incl = total;
+            unsigned incl = total;
 #pragma unroll
             for (int s = 1; s < MINF_WAVE; s <<= 1) {
                 const unsigned up = __shfl_up(incl, s);
                 if (lane >= s) incl += up;
             }
             if (lane == MINF_WAVE - 1) wsum[wave] = incl;
+            first[tid] = incl - total;
         }
         __syncthreads();
-        if (tid < SORT_DIGITS) {
-            unsigned below = 0;
-            for (int w = 0; w < wave; ++w) below += wsum[w];
-            first[tid] = below + incl - total;
-        }
-        __syncthreads();
+        const unsigned below1 = wsum[0], below2 = below1 + wsum[1], below3 = below2 + wsum[2];
 #pragma unroll
         for (int r = 0; r < E; ++r)
             if (r < groups) {
                 const unsigned d = (key[r] >> shift) & 0xffu;
-                keys[first[d] + hist[wave][d] + rank[r]] = key[r];
+                const unsigned below = d < 128 ? (d < 64 ? 0 : below1) : (d < 192 ? below2 : below3);
+                keys[below + first[d] + hist[wave][d] + rank[r]] = key[r];
             }
+        clear_own();
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < E; ++r)
