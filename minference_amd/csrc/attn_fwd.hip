@@ -1101,7 +1101,9 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
 // fp32 range whatever a segment's (lazily raised) maximum was.  A segment is left out only where its row sum
 // is the zero of an unused or fully masked one, by bit pattern: a NaN among the keys makes the row sum NaN,
 // and the row is to be NaN, as a whole walk leaves it.  Latency-bound and small: it reads what the
-// segments wrote (66 KB each at head_dim 128, from L2) and writes the rows once.
+// segments wrote (66 KB each at head_dim 128, from L2) and writes the rows once.  The statistics of eight segments
+// and the sums of four are loaded together: one segment after the other, each was two round trips to L2.  Tri-shape,
+// head_dim 64: one bf16 head of 5086 tokens, whole call 26.1 -> 23.2 us; 16 fp16 heads of 24000 131.5 -> 129.5.
 template <int HD>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     constexpr int NDB = HD / 32, ROW_BYTES = HD * 2, NCH = ROW_BYTES / 16;
@@ -1125,10 +1127,15 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     const int nseg = (p.split_first + pair) * 2 * BM < seqlen ? p.nseg : 0;
     auto stat = [&](int s) { return *(reinterpret_cast<const float2 *>(slots + (long long)s * SplitSlot<HD>::BYTES + SplitSlot<HD>::ACC) + part * 64 + lane); };
     float top = -INFINITY;
-    for (int s = 0; s < nseg; ++s) {
-        const float2 ml = stat(s);
-        const bool number = (__float_as_uint(ml.y) & 0x7fffffffu) <= 0x7f800000u;
-        if (__float_as_uint(ml.y) != 0 && number) top = fmaxf(top, ml.x + __builtin_amdgcn_logf(ml.y));
+    for (int s0 = 0; s0 < nseg; s0 += 8) {
+        float2 ml[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) ml[u] = stat(min(s0 + u, nseg - 1));
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const bool number = (__float_as_uint(ml[u].y) & 0x7fffffffu) <= 0x7f800000u;
+            if (__float_as_uint(ml[u].y) != 0 && number) top = fmaxf(top, ml[u].x + __builtin_amdgcn_logf(ml[u].y));
+        }
     }
     const bool live = row0 + l32 < seqlen;
     float l_tot = 0.f;
@@ -1137,24 +1144,46 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     for (int i = 0; i < (NDB > 4 ? 2 : 1); ++i)
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) acc[i][rq] = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s = 0; s < nseg; ++s) {
-        const float2 ml = stat(s);
-        const bool used = __float_as_uint(ml.y) != 0;
-        const float w = used ? __builtin_amdgcn_exp2f(ml.x - top) : 0.f;
-        if (!__any(used)) continue;                                     // an unused slot holds nothing
-        l_tot += w * ml.y;
+    constexpr int UP = NDB > 4 ? 2 : 4, NI = NDB > 4 ? 2 : 1;
+    for (int s0 = 0; s0 < nseg; s0 += UP) {
+        float2 ml[UP];
+        bool any[UP];
 #pragma unroll
-        for (int i = 0; i < (NDB > 4 ? 2 : 1); ++i) {
-            const int db = wave + 4 * i;
-            if (db < NDB) {
-                const char *src = slots + (long long)s * SplitSlot<HD>::BYTES + ((part * NDB + db) * 4 * 64 + lane) * 16;
+        for (int u = 0; u < UP; ++u) ml[u] = stat(min(s0 + u, nseg - 1));
+        bool some = false;
 #pragma unroll
-                for (int rq = 0; rq < 4; ++rq) {
-                    const float4 x = *reinterpret_cast<const float4 *>(src + rq * 1024);
-                    acc[i][rq].x = fmaf(w, x.x, acc[i][rq].x); acc[i][rq].y = fmaf(w, x.y, acc[i][rq].y);
-                    acc[i][rq].z = fmaf(w, x.z, acc[i][rq].z); acc[i][rq].w = fmaf(w, x.w, acc[i][rq].w);
+        for (int u = 0; u < UP; ++u) some |= any[u] = s0 + u < nseg && __any(__float_as_uint(ml[u].y) != 0);
+        if (!some) continue;
+        // an unused slot holds nothing: in its place the one before is read again, for no use
+        float4 x[UP][NI][4];
+        int from = s0;
+#pragma unroll
+        for (int u = 0; u < UP; ++u) {
+            if (any[u]) from = s0 + u;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const int db = wave + 4 * i;
+                if (db < NDB) {
+                    const char *src = slots + (long long)from * SplitSlot<HD>::BYTES + ((part * NDB + db) * 4 * 64 + lane) * 16;
+#pragma unroll
+                    for (int rq = 0; rq < 4; ++rq) x[u][i][rq] = *reinterpret_cast<const float4 *>(src + rq * 1024);
                 }
             }
+        }
+#pragma unroll
+        for (int u = 0; u < UP; ++u) {
+            const float w = any[u] && __float_as_uint(ml[u].y) != 0 ? __builtin_amdgcn_exp2f(ml[u].x - top) : 0.f;
+            l_tot = any[u] ? fmaf(w, ml[u].y, l_tot) : l_tot;
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                if (wave + 4 * i < NDB)
+#pragma unroll
+                    for (int rq = 0; rq < 4; ++rq) {
+                        float4 &o = acc[i][rq];
+                        const float4 v = x[u][i][rq];
+                        o.x = any[u] ? fmaf(w, v.x, o.x) : o.x; o.y = any[u] ? fmaf(w, v.y, o.y) : o.y;
+                        o.z = any[u] ? fmaf(w, v.z, o.z) : o.z; o.w = any[u] ? fmaf(w, v.w, o.w) : o.w;
+                    }
         }
     }
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
