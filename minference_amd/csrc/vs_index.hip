@@ -244,8 +244,7 @@ __global__ __launch_bounds__(IDX_WAVES *MINF_WAVE) void vs_index_kernel(
 //   run_a[r], run_e[r]   [start, end) of range r
 //   cgaps[i]  the number of entries j <= i with t_j > t_{j-1} + 64 ("gap entries": the only entries
 //             at which a range can start, for any row block -- skipping and clipping only shrink gaps)
-//   glist[j]  the gap entries, ascending, j < ngaps: the
-//             first gap entry at or after entry x is glist[cgaps[x - 1]]
+//   glist[j]  the gap entries, ascending, j < ngaps: the first gap entry at or after entry x is glist[cgaps[x - 1]]
 // all in the virtual row's coordinates (real position = virtual + end_m - V).
 // vs_index_fast_kernel then handles a row block as follows: entries from the first valid one are
 // processed exactly like vs_index_kernel until a range starts at an entry that also starts a range
@@ -282,11 +281,11 @@ __device__ __forceinline__ void mark_block(uint32_t *bm, int words, int p) {
 struct PrepState { int cur_a, carried_e, carried_t; };
 struct PrepCount { int nb, nr, ng; };
 struct PrepChunk {                                   // one chunk, taken through the range logic
-    int t, a, eprev0;                                // this lane's entry and its range start; range end before the chunk
-    uint64_t starts, gaps;
+    int t, a, e, eprev;                              // this lane's entry, its range's start and end, the end one entry before
+    uint64_t starts, gaps, changed;                  // entries that start a range, that follow a gap, that end a new block
     int base, cnt;
 };
-__device__ __forceinline__ void prep_chunk(PrepChunk &k, PrepState &st, PrepCount &n) {
+__device__ __forceinline__ void prep_chunk(PrepChunk &k, PrepState &st) {
     const int lane = minf_lane();
     if (k.base == 0) {
         const int t0 = minf_readlane(k.t, 0);
@@ -297,16 +296,19 @@ __device__ __forceinline__ void prep_chunk(PrepChunk &k, PrepState &st, PrepCoun
     const uint64_t valid = k.cnt == MINF_WAVE ? ~0ull : (1ull << k.cnt) - 1ull;
     if (k.base == 0) k.starts |= 1ull;
     k.starts &= valid;
-    k.eprev0 = st.carried_e;
-    const int e = k.a + ((((k.t - k.a) + 63) >> 6) << 6);
-    int eprev = lane_above(e);
-    if (lane == 0) eprev = st.carried_e;
-    n.nb += __builtin_popcountll(__ballot(lane < k.cnt && e != eprev));
-    n.nr += __builtin_popcountll(k.starts);
-    n.ng += __builtin_popcountll(k.gaps);            // (padding lanes repeat the last entry: never a gap)
-    st.carried_e = minf_readlane(e, k.cnt - 1);
+    k.e = k.a + ((((k.t - k.a) + 63) >> 6) << 6);
+    k.eprev = lane_above(k.e);
+    if (lane == 0) k.eprev = st.carried_e;
+    k.changed = __ballot(lane < k.cnt && k.e != k.eprev);
+    st.carried_e = minf_readlane(k.e, k.cnt - 1);
     st.carried_t = minf_readlane(k.t, k.cnt - 1);
     st.cur_a = minf_readlane(k.a, k.cnt - 1);
+}
+// the counts behind a chunk
+__device__ __forceinline__ void prep_count(const PrepChunk &k, PrepCount &n) {
+    n.nb += __builtin_popcountll(k.changed);
+    n.nr += __builtin_popcountll(k.starts);
+    n.ng += __builtin_popcountll(k.gaps);            // (padding lanes repeat the last entry: never a gap)
 }
 // writes a chunk's entries of the tables; n: the counts before the chunk
 __device__ __forceinline__ void prep_write(const PrepChunk &k, const PrepCount &n, int32_t *hdr, int nnz_s, uint32_t *bm, int bm_words) {
@@ -315,14 +317,10 @@ __device__ __forceinline__ void prep_write(const PrepChunk &k, const PrepCount &
     int32_t *run_a = crun + nnz_s, *run_e = run_a + nnz_s, *cgaps = run_e + nnz_s, *glist = cgaps + nnz_s;
     const uint64_t lt = minf_lanemask_lt();
     const bool valid = lane < k.cnt, is_start = (k.starts >> lane) & 1ull;
-    const int e = k.a + ((((k.t - k.a) + 63) >> 6) << 6);
-    int eprev = lane_above(e);
-    if (lane == 0) eprev = k.eprev0;
-    const bool changed = valid && e != eprev;
-    const int kpos = n.nb + __builtin_popcountll(__ballot(changed) & lt);
-    if (changed) {
-        cpos[kpos] = e - 64;
-        if (bm) mark_block(bm, bm_words, e - 64);
+    const int kpos = n.nb + __builtin_popcountll(k.changed & lt);
+    if ((k.changed >> lane) & 1ull) {
+        cpos[kpos] = k.e - 64;
+        if (bm) mark_block(bm, bm_words, k.e - 64);
     }
     if (valid) {
         const int r = n.nr + __builtin_popcountll(k.starts & lt), gapno = n.ng + __builtin_popcountll(k.gaps & lt);
@@ -333,16 +331,34 @@ __device__ __forceinline__ void prep_write(const PrepChunk &k, const PrepCount &
         crun[k.base + lane] = is_start ? r : -1;
         if (is_start) {
             run_a[r] = k.a;
-            if (r > 0) run_e[r - 1] = eprev;
+            if (r > 0) run_e[r - 1] = k.eprev;
         }
     }
 }
-__device__ __forceinline__ PrepChunk prep_load(const int32_t *__restrict__ sl, int nnz_s, int V, int c) {
+__device__ __forceinline__ int prep_entry(const int32_t *__restrict__ sl, int nnz_s, int c) {      // this lane's entry of chunk c
+    return sl[min(c * MINF_WAVE + minf_lane(), nnz_s - 1)];          // (padding lanes repeat the last entry)
+}
+__device__ __forceinline__ PrepChunk prep_place(int entry, int nnz_s, int V, int c) {
     PrepChunk k;
     k.base = c * MINF_WAVE;
     k.cnt = min(MINF_WAVE, nnz_s - k.base);
-    k.t = max(V - sl[min(k.base + minf_lane(), nnz_s - 1)], 64);     // (padding lanes repeat the last entry)
+    k.t = max(V - entry, 64);
     return k;
+}
+__device__ __forceinline__ PrepChunk prep_load(const int32_t *__restrict__ sl, int nnz_s, int V, int c) {
+    return prep_place(prep_entry(sl, nnz_s, c), nnz_s, V, c);
+}
+// f(chunk) for chunks [c0, c1) in turn.  What f does is one chain over the chunks, so the entries of the next two are
+// on their way meanwhile (60000 slashes, 8 heads, builder with payload only: 174 -> 170 us against each chunk loaded
+// where it is used; in the walk of one wavefront 140000 slashes 1443 -> 1116).
+template <typename F> __device__ __forceinline__ void prep_each(const int32_t *__restrict__ sl, int nnz_s, int V, int c0, int c1, F f) {
+    int next = prep_entry(sl, nnz_s, c0), next2 = prep_entry(sl, nnz_s, c0 + 1);
+    for (int c = c0; c < c1; ++c) {
+        PrepChunk k = prep_place(next, nnz_s, V, c);
+        next = next2;
+        next2 = prep_entry(sl, nnz_s, c + 2);
+        f(k);
+    }
 }
 
 __device__ __forceinline__ void prep_header(int32_t *hdr, int nnz_s, int rows, int V, const PrepState &st, const PrepCount &n) {
@@ -367,17 +383,18 @@ __device__ __forceinline__ void prep_header(int32_t *hdr, int nnz_s, int rows, i
 // inside a dense run, a handful when the offsets are scattered); it takes its share through the range logic,
 // the counts of blocks, ranges and gap entries are summed over the wavefronts before it, and it writes the tables.
 // A share of at most PREP_KEEP chunks stays in registers from the marks to the tables (one round of loads in flight
-// together); longer ones are loaded and walked once to count and again to write.  Lists of at most two
-// chunks, or of more chunks than the mark arrays hold, are walked by one wavefront alone.
+// together); longer ones are loaded and walked once to count and again to write.  Lists of at most two chunks, or of
+// more chunks than LDS holds marks for, are walked by one wavefront alone: 500000 slashes, one head, take 3365 us (no
+// bitmap atomics in that chain; with them 4895), 393216, the most that are shared, 625 (a limit of 131072: 3652).
 // The coverage bitmap is built in LDS beside the tables (where it fits: `bm_words` > 0) and copied out at the end.
 // Latency-bound, one workgroup per head.  With a bitmap kernel behind it that searched the ranges, and a share's state
 // found by reading the marks one chunk at a time, the two took (us, now in one kernel): 6096 slashes, clustered, 16001
 // tokens 29 + 5 -> 16, 131072 tokens 25 + 5 -> 15; uniform, 262144 tokens 39 + 7 -> 28; 2048 slashes, 8192 tokens,
 // 4 heads 12 + 5 -> 9.
 #define PREP_WAVES 16
-#define PREP_MAX_CHUNKS 2048
 #define PREP_KEEP 8
-#define PREP_BITMAP_MAX_BYTES 98304
+#define PREP_LDS_MAX_BYTES 98304
+#define PREP_MAX_CHUNKS (PREP_LDS_MAX_BYTES / 16)          // 393216 entries
 __global__ __launch_bounds__(PREP_WAVES *MINF_WAVE) void vs_index_prep_kernel(const int32_t *__restrict__ slash,
                                                                               int32_t *__restrict__ tables, int nnz_s, int rows, int bm_words) {
     extern __shared__ uint64_t prep_lds[];           // sure and maybe marks of every chunk, later the bitmap
@@ -400,12 +417,11 @@ __global__ __launch_bounds__(PREP_WAVES *MINF_WAVE) void vs_index_prep_kernel(co
         if (wave == 0) {
             PrepState st{0, 0, 0};
             PrepCount n{0, 0, 0};
-            for (int c = 0; c < nchunks; ++c) {
-                PrepChunk k = prep_load(sl, nnz_s, V, c);
-                const PrepCount before = n;
-                prep_chunk(k, st, n);
-                prep_write(k, before, hdr, nnz_s, bm, bm_words);
-            }
+            prep_each(sl, nnz_s, V, 0, nchunks, [&](PrepChunk &k) {
+                prep_chunk(k, st);
+                prep_write(k, n, hdr, nnz_s, bm, bm_words);
+                prep_count(k, n);
+            });
             if (lane == 0) prep_header(hdr, nnz_s, rows, V, st, n);
         }
     } else {
@@ -480,12 +496,15 @@ __global__ __launch_bounds__(PREP_WAVES *MINF_WAVE) void vs_index_prep_kernel(co
         if (keep) {
 #pragma unroll
             for (int j = 0; j < PREP_KEEP; ++j)
-                if (c0 + j < c1) prep_chunk(held[j], st, n);
+                if (c0 + j < c1) {
+                    prep_chunk(held[j], st);
+                    prep_count(held[j], n);
+                }
         } else {
-            for (int c = c0; c < c1; ++c) {
-                PrepChunk k = prep_load(sl, nnz_s, V, c);
-                prep_chunk(k, st, n);
-            }
+            prep_each(sl, nnz_s, V, c0, c1, [&](PrepChunk &k) {
+                prep_chunk(k, st);
+                prep_count(k, n);
+            });
         }
         if (lane == 0) { cnt_b[wave] = n.nb; cnt_r[wave] = n.nr; cnt_g[wave] = n.ng; }
         __syncthreads();
@@ -502,22 +521,15 @@ __global__ __launch_bounds__(PREP_WAVES *MINF_WAVE) void vs_index_prep_kernel(co
             for (int j = 0; j < PREP_KEEP; ++j)
                 if (c0 + j < c1) {
                     prep_write(held[j], at, hdr, nnz_s, bm, bm_words);
-                    const PrepChunk &k = held[j];
-                    const int e = k.a + ((((k.t - k.a) + 63) >> 6) << 6);
-                    int eprev = lane_above(e);
-                    if (lane == 0) eprev = k.eprev0;
-                    at.nb += __builtin_popcountll(__ballot(lane < k.cnt && e != eprev));
-                    at.nr += __builtin_popcountll(k.starts);
-                    at.ng += __builtin_popcountll(k.gaps);
+                    prep_count(held[j], at);
                 }
         } else {
             st = head;
-            for (int c = c0; c < c1; ++c) {
-                PrepChunk k = prep_load(sl, nnz_s, V, c);
-                const PrepCount before = at;
-                prep_chunk(k, st, at);
-                prep_write(k, before, hdr, nnz_s, bm, bm_words);
-            }
+            prep_each(sl, nnz_s, V, c0, c1, [&](PrepChunk &k) {
+                prep_chunk(k, st);
+                prep_write(k, at, hdr, nnz_s, bm, bm_words);
+                prep_count(k, at);
+            });
         }
         if (c0 < nchunks && c1 == nchunks && lane == 0) prep_header(hdr, nnz_s, rows, V, st, all);
     }
@@ -528,9 +540,10 @@ __global__ __launch_bounds__(PREP_WAVES *MINF_WAVE) void vs_index_prep_kernel(co
     }
 }
 
-// The coverage bitmap of contexts for which it does not fit the table pass's LDS (beyond 786000 tokens).  One thread
-// per 32-bit word: a binary search finds the first range that ends after the word's first position; ranges are at
-// least 64 long, so at most two of them touch a word.
+// The coverage bitmap where the table pass leaves it out: contexts whose bitmap does not fit its LDS (beyond 786304
+// tokens), lists that one wavefront walks for being longer than the mark arrays (its atomics would lengthen that chain).
+// One thread per 32-bit word: a binary search finds the first range that ends after the word's first position; ranges
+// are at least 64 long, so at most two of them touch a word.
 __global__ __launch_bounds__(256) void vs_index_bitmap_kernel(int32_t *__restrict__ tables, int nnz_s, int rows) {
     const long long bh = blockIdx.y;
     int32_t *hdr = tables + bh * idx_tab_ints(nnz_s, rows);
@@ -841,7 +854,7 @@ static int index_build_tables(const int32_t *seqlens, const int32_t *vertical_id
     if (nblk > 0x7fffffffLL || (long long)batch * heads > 65535) return MINF_ERR_UNSUPPORTED;
     const int nchunks = (nnz_s + MINF_WAVE - 1) / MINF_WAVE;
     const long long bm_words = idx_bm_words(rows);
-    const bool bm_in_lds = bm_words * 4 <= PREP_BITMAP_MAX_BYTES;
+    const bool bm_in_lds = bm_words * 4 <= PREP_LDS_MAX_BYTES && nchunks <= PREP_MAX_CHUNKS;
     size_t lds = nchunks <= PREP_MAX_CHUNKS ? 16 * (size_t)nchunks : 0;
     if (bm_in_lds && (size_t)bm_words * 4 > lds) lds = (size_t)bm_words * 4;
     hipLaunchKernelGGL(vs_index_prep_kernel, dim3((unsigned)(batch * heads)), dim3(PREP_WAVES * MINF_WAVE), lds,

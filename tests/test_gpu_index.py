@@ -102,15 +102,14 @@ def test_structured_lists_all_rows(gpu, mode):
         assert_same(run_gpu([seqlen], v, s, n, gpu), ref)
 
 
-@pytest.mark.parametrize("kind", ["maybe chains", "two or three chunks", "more chunks than the marks hold"])
+@pytest.mark.parametrize("kind", ["maybe chains", "two or three chunks", "hundreds of chunks to the share"])
 def test_table_pass_shares_of_the_list(gpu, kind):
     """The table pass cuts a head's list into shares for 16 wavefronts; a wavefront finds the state at
     the head of its share by replaying the "maybe" entries (65..127 above their predecessor) since
     the last "sure" start (more than 127 above).  Lists built to stress that: hundreds of entries in
     a row whose gaps are all 65..127 (no sure start for whole shares, so the replay crosses several
-    of them), lists of two chunks (walked by one wavefront) and three (shared), and a list of more
-    chunks than the mark arrays hold (walked by one wavefront).  Bit-exact against the C oracle and
-    against the plain wave-per-row builder."""
+    of them), lists of two chunks (walked by one wavefront) and three (shared), and a list of 2049
+    chunks.  Bit-exact against the C oracle and against the plain wave-per-row builder."""
     rng = np.random.default_rng(len(kind))
     cases = []
     if kind == "maybe chains":
@@ -143,10 +142,24 @@ def test_table_pass_shares_of_the_list(gpu, kind):
 
 
 @pytest.mark.parametrize("n,nv,ns", [(40000, 300, 8191), (40000, 300, 8192), (40000, 300, 8193),   # shares kept in registers up to 8192
-                                     (524288, 200, 300), (786000, 100, 130), (787000, 100, 130)])   # bitmap in LDS up to 786368
+                                     (524288, 200, 300), (786000, 100, 130), (786304, 100, 130),     # bitmap in LDS up to 786304
+                                     (786305, 100, 130), (787000, 100, 130)])
 def test_limits_of_the_table_pass(gpu, n, nv, ns):
     print(f"case table pass limits n={n} nv={nv} ns={ns}", flush=True)
     v, s = gen.vs_index_inputs(1, n, nv, ns, seed=9, force_v=4, force_s=64)
+    assert_same(run_gpu([n], v, s, n, gpu), O.vs_index_build([n], v, s, n))
+
+
+@pytest.mark.parametrize("ns", [131072, 131073, 393215, 393216, 393217])
+def test_lists_around_the_most_that_are_shared(gpu, ns):
+    """393216 entries are as many as the table pass holds marks for; a longer list is walked by one wavefront and its
+    bitmap made by a kernel of its own.  32 row blocks, most of the offsets beyond the context; gaps of all kinds."""
+    print(f"case list of {ns} slashes", flush=True)
+    rng = np.random.default_rng(ns)
+    n, V = 2000, 90
+    steps = rng.choice([1, 1, 1, 64, 65, 100, 127, 128, 300], size=ns - 1, p=[0.3, 0.2, 0.2, 0.1, 0.1, 0.04, 0.02, 0.02, 0.02])
+    s = np.ascontiguousarray(np.concatenate([[0], np.cumsum(steps)])[::-1][None, None].astype(np.int32))
+    v = np.sort(rng.choice(n, size=V, replace=False))[None, None].astype(np.int32)
     assert_same(run_gpu([n], v, s, n, gpu), O.vs_index_build([n], v, s, n))
 
 
