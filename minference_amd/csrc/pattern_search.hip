@@ -120,7 +120,7 @@ constexpr int DIAG_GROUPS_SMALL = 4096;      // (131072 tokens: three workgroups
 // the scale in fp32 bounds it.
 // Bound by its vector instructions, 131 per 32 x 32 block (fma and exp 32, of which the exp take four times as long; maximum,
 // row sum, and 40 per candidate with mixed diagonals: 630 of 894 cycles) and its matrix products (270 cycles), which overlap
-// little.  32 / 8 heads, 16384 tokens, the six candidates of the reference: 2.81 -> 2.00 ms against the bf16 terms (56
+// little.  32 / 8 heads, 16384 tokens, the six candidates of the reference: 2.73 -> 1.79 ms against the bf16 terms (56
 // conversions per block; masks built in registers by every wave, where one of a workgroup's threads now writes them to LDS
 // once; two waves per SIMD, now three, since neither accumulators with nine used rows of 32 nor masks occupy
 // registers).  0.18 ms of it: no value that a step fetches for the next is touched before the next barrier (a wait for a
@@ -338,15 +338,15 @@ template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS
                 + (((e[8] + e[9]) + (e[10] + e[11])) + ((e[12] + e[13]) + (e[14] + e[15])));
             zs[nb] += sum;
             if (mixed[nb]) {
-                // diagonal flags of keys n0 + 8j + 4g + 0..3, without the kept columns
+                // diagonal flags of keys n0 + 8j + 4g + 0..3, without the kept columns.  They begin at any byte: two words
+                // and a byte shift, since an LDS read off its alignment took about a hundred cycles (32 / 8 heads, 4096
+                // tokens: 325 -> 300 us, 16384 1890 -> 1795; one head, 6000 tokens 324 -> 308)
                 unsigned pm[4];
-                const unsigned char *const dp = reinterpret_cast<const unsigned char *>(dbytes[buf]) + (2 * TILE * tp + 2 * TILE - 1 - KB * kb0) - (row - n0 - 4 * g);
+                const int at = (2 * TILE * tp + 2 * TILE - 1 - KB * kb0) - (row - n0 - 4 * g);      // (in bytes; 0 .. 4 DW - 32 + 7)
+                const unsigned *const dp = dbytes[buf] + (at >> 2);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    unsigned w;
-                    __builtin_memcpy(&w, dp + 8 * j, 4);
-                    pm[j] = w & ~cbytes[buf][8 * kpar + 2 * j + g];
-                }
+                for (int j = 0; j < 4; ++j)
+                    pm[j] = __builtin_amdgcn_alignbyte(dp[2 * j + 1], dp[2 * j], at & 3) & ~cbytes[buf][8 * kpar + 2 * j + g];
 #pragma unroll
                 for (int t = 0; t < NC; ++t)
                     if ((mixed[nb] >> t) & 1u) {

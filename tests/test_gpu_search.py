@@ -234,6 +234,24 @@ def test_recall_where_the_table_of_diagonals_grows_and_ends(gpu, n):
         assert abs(float(got[0, t]) - want) <= 2 * (n / 64 + 64) * 2.0 ** -24 * want, t
 
 
+@pytest.mark.parametrize("n", [33, 127, 130, 260, 515])
+def test_diagonals_of_every_row_and_byte(gpu, n):
+    """Random flags of all eight candidates on every diagonal, all rows counted: a lane's flags begin at each byte of a
+    word, at the first and the last one of a step.  Both sums of a row are fp32 sums of at most 64 + n / 64 terms in a chain."""
+    g = torch.Generator(device=gpu).manual_seed(n)
+    q, k = (torch.randn(1, 1, n, 128, device=gpu, generator=g).bfloat16() for _ in range(2))
+    pitch = (n + 63) // 64 * 64
+    col, diag = (torch.randint(0, 256, (1, pitch), device=gpu, generator=g, dtype=torch.uint8) for _ in range(2))
+    got = _recall_begin(q, k, col & 0x0f & torch.roll(col, 7), diag, 0)
+    r, c = torch.arange(n, device=gpu)[:, None], torch.arange(n, device=gpu)[None]
+    s = q[0, 0].double() @ k[0, 0].double().t().contiguous() * 128 ** -0.5
+    p = torch.softmax(s.masked_fill(c > r, float("-inf")), -1)
+    flags = (col & 0x0f & torch.roll(col, 7))[0, :n][None] | diag[0][(r - c).clamp(min=0)]
+    for t in range(8):
+        want = float((p * ((flags >> t) & 1)).sum() / n)
+        assert abs(float(got[0, t]) - want) <= 2 * (n / 64 + 64) * 2.0 ** -24 * want, t
+
+
 def _recall_begin(q, k, col, diag, begin):
     from minference_amd import _lib
     lib, n, i64x3 = _lib.load(), q.shape[2], _lib.c_i64 * 3
