@@ -705,7 +705,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // ---- mask, V^T fragment reads, online softmax, O^T += V^T . P^T
     auto sm_pv_block = [&](const Tile &cur, const char *vbuf, f32x16_t &s0, f32x16_t &s1) {
         // (head_dim 256: the 64 registers of a whole tile's V^T fragments do not fit next to O^T and Q;
-        // that form reads the fragments of one key group at a time, right before their MFMAs)
+        // that form reads a fragment two MFMAs ahead of its own)
         constexpr bool VF_AHEAD = HD <= 128;
         Frag vf[VF_AHEAD ? 4 : 1][NDB];
         // element (blk, r) of this lane is tile-local key tk = tkc + 4*g with the compile-time
@@ -870,6 +870,17 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
 #pragma unroll
                 for (int db = 0; db < NDB; ++db)
                     oacc[db] = Mma<T>::mfma(frag_as<T>(vf[0][db]), frag_as<T>(pfr[s]), oacc[db]);
+            }
+            // one MFMA, the reads of the fragment two MFMAs ahead, softmax instructions of the next key groups.  Left to
+            // the compiler the order turned with every change elsewhere in the kernel (1 wave per SIMD: nothing hides a
+            // wait): dense, 16 heads of 20000 tokens, bf16 3640 us, 3715 after one to the epilogue, 3518 in this order;
+            // fp16 3834, 3808, 3739; A-shape, window 1000, bf16 588, 561, 538
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+            for (int i = 0; i < 4 * NDB; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (i < 4 * NDB - 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                if (i < 3 * NDB) __builtin_amdgcn_sched_group_barrier(VALU_MASK, VALU_PER_MFMA * 4 / NDB, 0);
             }
             }
         }
