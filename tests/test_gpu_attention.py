@@ -216,11 +216,13 @@ def test_block_sparse_lists_that_differ_between_neighbouring_row_blocks(gpu, n, 
     check(out, ref, "bs-lists")
 
 
-@pytest.mark.parametrize("order", ["ascending", "one pair swapped"])
-@pytest.mark.parametrize("entries", [1, 127, 128, 129, 255, 256, 257, 300])
+@pytest.mark.parametrize("entries,order", [(1, "ascending")] + [(e, o) for e in (127, 128, 129, 255, 256, 257, 300) for o in (
+    "ascending", "one pair swapped", "first list rotated", "second list rotated")])
 def test_block_list_lengths_around_the_split_chunks(gpu, entries, order):
     """Lists are split 128 entries at a time, the first 256 of them from registers: lengths around both, for the two
-    row blocks of the last pair (two thirds of the entries in common); a list out of order is walked as it is."""
+    row blocks of the last pair (two thirds of the entries in common); a list out of order is walked as it is.  Each
+    list's order is checked by its own waves: either list alone is out of order in one place, in long ones between the
+    chunks, where the larger entries end and the smaller ones begin (most look-ups of the other list's entries miss)."""
     from minference_amd import block_sparse_attention_from_index
     rows, n = 320, 320 * 64
     print(f"case block lists of {entries} entries, {order}", flush=True)
@@ -233,8 +235,11 @@ def test_block_list_lengths_around_the_split_chunks(gpu, entries, order):
         own = common[entries + j * (entries - kept):][:entries - kept] if 2 * entries <= rows - 2 \
             else rng.choice(common[kept:], entries - kept, replace=False)
         lists[m] = np.sort(np.concatenate([common[:kept], own]))
-    if order != "ascending" and entries > 1:
+    if order == "one pair swapped":
         lists[rows - 1, entries - 2:] = lists[rows - 1, entries - 2:][::-1].copy()
+    elif order != "ascending":
+        m = rows - 2 if order.startswith("first") else rows - 1
+        lists[m] = np.roll(lists[m], entries // 2 if entries <= 128 else 128 if entries < 300 else 256)
     out = block_sparse_attention_from_index(q.to(gpu), k.to(gpu), v.to(gpu),
                                             torch.from_numpy(lists.astype(np.int32))[None, None].to(gpu))
     for m in (rows - 2, rows - 1):
