@@ -26,16 +26,18 @@
 // the probabilities of a lane are exactly the B operand of the second MFMA once
 // the contraction (token) index is permuted the same way on the V side.
 //
-// LDS: one K and one V tile per workgroup (two of each for vertical-slash lists: the second pair
-// serves row block B in split steps), [64 tokens][128] 16-bit, 256-byte rows whose 16-byte
+// LDS: one K and one V tile per workgroup (two of each for the list walks: the second pair serves
+// row block B in split steps; a second K tile's room in every form: the epilogue's 128 output rows
+// lie there), [64 tokens][128] 16-bit, 256-byte rows whose 16-byte
 // chunks are XOR-permuted (K: chunk ^ row%16, V: chunk ^ 4*(row%4)) so that the ds_read_b128 of 32
 // K rows and the 4-row transpose reads of V hit distinct banks.  Tiles are copied global -> LDS
 // directly (no staging registers, no LDS store instructions); the permutation is applied on the
 // global-address side.  Contiguous tiles use buffer_load_dwordx4 ... lds with a scalar descriptor of
 // the 64 tile rows, a scalar row offset and one of five loop-invariant per-lane offsets: no vector
 // instruction per copy and 8 cycles less issue time per copy than the 64-bit-address form, which
-// remains for gathered and clamped rows (global_load_lds_dwordx4).  32-68 KB of LDS and <= 256 registers
-// keep two waves per SIMD resident (two 4-wave workgroups per CU).
+// remains for gathered and clamped rows (global_load_lds_dwordx4).  At head_dim 128 48 KB of LDS (68 for
+// lists, which also hold the split ones) and <= 256 registers keep two waves per SIMD resident (two
+// 4-wave workgroups per CU); at 64 24 (36) KB and three of them, at 256 96 KB and one.
 //
 // One iteration of a wave (two workgroup barriers per tile, single buffers):
 //   wait own K(it) copies; barrier (all of K(it) visible, everyone done with V(it-1))
@@ -449,7 +451,8 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // or in its row block's list of entries the other one lacks (run ends).  Each pair of waves looks up one
     // list, both at once; with a pass per list and a check before them a workgroup took 6.5 us to its first tile
     // copy (block-sparse, top-100; 2.9 of them chains of LDS reads and six barriers) where it takes 3.4 now:
-    // vertical-slash, 16001 tokens, 32 / 8 heads 1531 -> 1519 us, block-sparse, 32768 tokens 2909 -> 2892.
+    // vertical-slash, 16001 tokens, 32 / 8 heads 1531 -> 1519 us (runs of one side 0.5 % apart); on longer
+    // walks nothing beyond noise.
     // The walk is then
     //   common tiles, both halves computing;
     //   split steps: every half visits its own leftover tiles -- the entries the other list lacks,
@@ -1052,8 +1055,8 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         char *ot = lds_k + wave_wg * 32 * OP;
         // the 16-byte chunks of a row are permuted like those of a K tile: at a row's own pitch all 32 rows' writes of
         // one instruction went to one pair of banks, and a workgroup's epilogue took 5.1 us of its 34 (A-shape, window
-        // 512, head_dim 128) where it takes 3.4 now: A-shape, 100000 tokens, window 3968, 32 / 8 heads 6486 -> 6430 us; 16
-        // heads of 64, 24000 tokens, window 512 138.5 -> 134.9; dense, 2 x 6144 tokens, 32 / 8 heads 594 -> 588
+        // 512, head_dim 128) where it takes 3.4 now: 16 heads of 64, 24000 tokens, window 512 138.5 -> 134.9 us; dense,
+        // 2 x 6144 tokens, 32 / 8 heads 594 -> 588; A-shape, 100000 tokens, window 3968 6486 -> 6430 (hardly beyond noise)
         const bool live = qrow < seqlen;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)

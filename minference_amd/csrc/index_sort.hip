@@ -8,11 +8,12 @@
 // read and written in all): each wavefront owns a contiguous stretch of the row in registers and ranks it
 // 64 values at a time -- eight ballots find the lanes with the same digit, one LDS word per digit and
 // wavefront counts them -- so that nothing is contended and the order of equal digits is kept.
-// A pass has three barriers; the scan reads a digit's counts of all wavefronts before it stores any (load behind
-// store was a round trip to LDS each).  Pairs of 500 + 700 int64 values, one row: 7.5 -> 4.9 us, 1000 + 6096, 32 rows
-// 17.2 -> 13.7.  Before this kernel the conversions, the two sorts and
-// the copies around them were ten launches and 50 us of GPU time (1000 + 2048 values, 4 heads); the operator on them, fp32 tensors of 8192 tokens,
-// took 309 instead of 265 us, on rows of 100 + 750 values, 2 x 16 heads of 597 tokens 119 -> 78 us.
+// A pass has three barriers; the scan reads a digit's counts of all wavefronts before it stores any (a load behind
+// each store was a round trip to LDS each).  Pairs of 500 + 700 int64 values, one row: 7.5 -> 4.9 us; 1000 + 6096,
+// 32 rows: 17.2 -> 13.7.
+// Before this kernel the conversions, the two sorts and the copies around them were ten launches and 50 us of GPU
+// time (1000 + 2048 values, 4 heads).  The operator on such indices: fp32 tensors of 8192 tokens 309 -> 265 us, rows of
+// 100 + 750 values, 2 x 16 heads of 597 tokens 119 -> 78.
 #include "minf_common.h"
 
 namespace {

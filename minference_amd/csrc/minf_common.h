@@ -40,8 +40,9 @@ __device__ __forceinline__ void copy16_to_lds(const char *src, char *dst) {
 
 // n / d for n < 2^31 by a multiplication and a shift (round-up method: m = ceil(2^(31+bits) / d) fits 32 bits, its
 // excess times n stays below 2^(31+bits) / d).  A 32-bit division takes some forty dependent instructions here, and
-// every workgroup of the attention kernels made five of them before it could ask for its first byte: 1.2 -> 0.7 us; A-shape, 16 heads, 49152
-// tokens, window 128: head_dim 64 125.3 -> 122.4 us, 128 218.7 -> 216.9; nothing beyond noise on walks of 50 steps.
+// every workgroup of the attention kernels made five of them before it could ask for its first byte: 1.2 -> 0.7 us;
+// A-shape, 16 heads of 64, 49152 tokens, window 128 125.3 -> 122.4 us, of 128 218.7 -> 216.9; nothing beyond noise
+// on walks of 50 steps.
 struct FastDiv {
     unsigned d, m, shift;
 };

@@ -7,11 +7,11 @@
 // of its workgroups, every workgroup of the second one folds those, converts its share and one of them
 // leaves the dtype code that the attention launches and the widening kernel read
 // (minf_qkvo.dtype_select).  Bound by bytes: q, k and v are read twice (the second time mostly from the
-// Infinity Cache) and written once at half the size.  The first
-// kernel has four vectors of a thread under way and reads a tensor that fills one stretch of memory by its vectors' numbers
-// alone: with one load at a time, placed by three divisions, it took 13.4 us for 3 x 16.8 MB (8192 tokens, 4 heads of
-// 128), now 9.0 = 5.6 TB/s; the second one 13.4 = 5.7 TB/s with one step or four under way.  With the choice read back by the host (three
-// reductions, a synchronisation, three conversions) the GPU idled about 60 us per call.
+// Infinity Cache) and written once at half the size.  The first kernel has four vectors of a thread under way
+// and reads a tensor that fills one stretch of memory by its vectors' numbers alone: with one load at a time,
+// placed by three divisions, it took 13.4 us for 3 x 16.8 MB (8192 tokens, 4 heads of 128), now 9.0 = 5.6 TB/s;
+// the second one 13.4 = 5.7 TB/s with one step or four under way.  With the choice read back by the host
+// (three reductions, a synchronisation, three conversions) the GPU idled about 60 us per call.
 #include "minf_common.h"
 
 namespace {

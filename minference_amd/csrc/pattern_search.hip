@@ -118,14 +118,14 @@ constexpr int DIAG_GROUPS_SMALL = 4096;      // (131072 tokens: three workgroups
 // exponential on 32x32x16 products, which this replaces: 6.8e-8), under a sink of 14 nats 3.3e-8 (1.8e-7); shares of
 // candidates without a sink of 14 .. 80 nats 1.9e-6 at most (6.5e-6; 3.1e-7 against 2.2e-7 at 14): there the rounding of
 // the scale in fp32 bounds it.
-// Bound by its vector instructions, 131 per 32 x 32 block (fma and exp 32, of which the exp take four times as long; maximum,
-// row sum, and 40 per candidate with mixed diagonals: 630 of 894 cycles) and its matrix products (270 cycles), which overlap
-// little.  32 / 8 heads, 16384 tokens, the six candidates of the reference: 2.73 -> 1.79 ms against the bf16 terms (56
-// conversions per block; masks built in registers by every wave, where one of a workgroup's threads now writes them to LDS
-// once; two waves per SIMD, now three, since neither accumulators with nine used rows of 32 nor masks occupy
-// registers).  0.18 ms of it: no value that a step fetches for the next is touched before the next barrier (a wait for a
-// flag byte was a wait for the K rows before it), one LDS read for the four distances of a step, fragment addresses by XOR from
-// one register.  Beyond 131072 tokens the table of diagonals leaves LDS for two.
+// Bound by its vector instructions, 131 per 32 x 32 block (fma and exp 32, of which the exp take four times as long;
+// maximum, row sum) and 40 per candidate with mixed diagonals, and by its matrix products, which overlap little with them.
+// 32 / 8 heads, 16384 tokens, the six candidates of the reference: 2.73 -> 1.79 ms against the bf16 terms (56 conversions
+// per block; masks built in registers by every wave, where one of a workgroup's threads now writes them to LDS once; two
+// waves per SIMD, now three, since neither accumulators with nine used rows of 32 nor masks occupy registers).  0.18 ms
+// of it: no value that a step fetches for the next is touched before the next barrier (a wait for a flag byte was a wait
+// for the K rows before it), one LDS read for the four distances of a step, fragment addresses by XOR from one register.
+// Beyond 131072 tokens the table of diagonals leaves LDS for two waves per SIMD.
 template <typename T, int DG> __global__ __launch_bounds__(256, DG > DIAG_GROUPS_SMALL ? 2 : 3) void pattern_recall_kernel(const RecallParams p) {
     __shared__ unsigned dtab[DG];                       // bytes: OR, AND, OR without the first, AND without the first
     // two steps of two 32-key blocks each (one per key parity), 256-byte rows whose 16-byte chunks are
