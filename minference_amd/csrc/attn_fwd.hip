@@ -110,10 +110,9 @@ struct AttnParams {
     int max_blocks, bidx_rows;
     // a-shape; query rows >= dense_from attend to every earlier key (tri-shape), INT_MAX = none
     int n_init, n_local, dense_from;
-    long long total_wg;
     int descending;          // row blocks are handed out from the last one down
-    int stripes_log2;        // the row-block pairs of a kv group are dealt to this many XCD ranges (see launch_hd)
-    FastDiv by_group, by_stripe, by_heads;   // hq / hk; workgroups of a stripe per head; kv heads, or chunks of the head list
+    int chunk, turn;         // units per deal, whether an XCD takes another place in every round of deals (see launch_hd)
+    FastDiv by_deal, by_group, by_groups, by_heads;   // workgroups of a deal; hq / hk; batch x kv groups; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
     // every head is processed and index_heads = hq
@@ -285,19 +284,18 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     char *const lds_v1 = lds_v + (VSP ? TILE_BYTES : 0);
 
     // ---- which (batch, head, row block): XCD-aware remap --------------------
-    // Consecutive workgroup ids are dealt round-robin to the 8 XCDs; give each
-    // XCD one contiguous range of the logical order (batch, kv head, row block,
-    // query head inside the GQA group) so that the row blocks and the query
-    // heads that share K/V also share an L2.
+    // Consecutive workgroup ids go round-robin to the 8 XCDs.  Deal number 8 r + x of the launch, the workgroups
+    // that share K/V and so an L2 (some neighbouring row-block pairs of the query heads of a kv group), is worked
+    // through by one of them, consecutive deals by different ones (see launch_hd).
     // (32-bit arithmetic: the launcher refuses grids beyond 2^31 workgroups, and 64-bit divisions of
     // wave-uniform values cost a thousand scalar instructions per workgroup here)
-    const unsigned total_wg = (unsigned)p.total_wg;
-    const unsigned per_xcd = (total_wg + 7u) >> 3;
-    const unsigned logical = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
-    if (logical >= total_wg) return false;
     const int group = (int)p.by_group.d;
-    unsigned rest = logical;
+    unsigned rest = blockIdx.x >> 3;
     auto next_digit = [&](const FastDiv &f) { const unsigned q = fast_quot(rest, f), r = rest - q * f.d; rest = q; return r; };
+    const unsigned in_deal = next_digit(p.by_deal);
+    rest = 8u * rest + ((blockIdx.x + rest * (unsigned)p.turn) & 7u);
+    const unsigned gi = next_digit(p.by_groups), first_unit = rest * (unsigned)p.chunk;
+    rest = in_deal;
     const int hin = (int)next_digit(p.by_group);
     // Dense causal work grows with the row block, so the heavy (late) blocks go first.  The sparse
     // modes have near-constant work per row block once the context is long and then measure 1 %
@@ -306,10 +304,9 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     const int rows_wg = (p.rows + 1) >> 1;                           // row-block pairs per (batch, head)
     const int split_units = (rows_wg - p.split_first) * p.nseg;      // (no split: split_first == rows_wg)
     const unsigned units = (unsigned)(p.split_first + split_units);
-    const unsigned in_stripe = next_digit(p.by_stripe);
-    const int mi = (int)((in_stripe << p.stripes_log2) + (rest & ((1u << p.stripes_log2) - 1u)));
-    rest >>= p.stripes_log2;
-    if (mi >= (int)units) return false;              // padding of the last round (workgroup-uniform)
+    const int mi = (int)(first_unit + rest);
+    rest = gi;
+    if (mi >= (int)units) return false;              // padding of the last deal (workgroup-uniform)
     int mslot, seg = -1;                             // row-block pair, segment of its walk (-1: the whole walk)
     if (CUT && mi < split_units) {                    // the split pairs, longest walks first
         // first segments of all of them, then second segments, ...: a walk's own segments side by side, of
@@ -1268,9 +1265,8 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.n_init = p.n_local = 0; p.dense_from = 0x7fffffff;
     p.head_list = t->head_list;
     p.index_heads = t->head_list ? t->index_heads : t->heads_q;
-    p.total_wg = 0;          // set by the launcher
-    p.stripes_log2 = 0;
-    p.by_group = p.by_stripe = p.by_heads = fast_div(1);      // set by the launcher
+    p.chunk = 1; p.turn = 0;      // set by the launcher
+    p.by_deal = p.by_group = p.by_groups = p.by_heads = fast_div(1);      // set by the launcher
     p.descending = 0;
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
     p.dtype = t->dtype;
@@ -1373,40 +1369,54 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
     const long long grid_heads = p.head_list ? (long long)((p.index_heads + group - 1) / group) * group : p.hq;
     const int split_pairs = (p.rows + 1) / 2 - p.split_first;
     const long long units = p.split_first + (long long)split_pairs * p.nseg;
-    // Every XCD works through one contiguous eighth of the logical order.  When the kv groups do not
-    // divide evenly among the XCDs, an eighth is a stretch of one group's row blocks, and where the work
-    // grows with the row block the XCD with the last ones is left working alone.  The row blocks are then
-    // dealt to the XCDs in turn, as many stripes per group as make the count divisible by eight: dense,
-    // 16384 tokens, 8 / 2 heads 750 -> 480 us, 28 / 4 heads 2.11 -> 1.69 ms.  The list walks and A-shape
-    // grow only at the start of the sequence and share tiles with their neighbours, which the stripes
-    // part: vertical-slash 28 / 4 heads 16384 tokens 1.63 -> 1.39 ms, 60000 tokens 6.27 -> 5.85, 8 / 2
-    // heads 16384 tokens 698 -> 645 us; but 4 / 4 heads 32768 tokens 546 -> 577 us, one head 65536 tokens
-    // 366 -> 381, A-shape 4 / 4 heads 16384 tokens 129 -> 134: so from eight heads and two rounds of
-    // workgroups on, up to 64K tokens.
+    // The launch is a sequence of deals, `chunk` units (row-block pairs, or segments) of one kv group each: the first
+    // units of every group, then the next ones, ...  Consecutive deals go to the 8 XCDs in turn, so every XCD gets an
+    // equal part of every stretch of the sequence, and where it matters (`turn`) of every group: where each worked
+    // through an eighth of the launch (or of a few groups), the one with the longest walks or the densest heads was left
+    // working alone.  32 / 8 heads with a table of unlike patterns, 50000 tokens 5.54 -> 4.60 ms (28 / 4 heads 4.70 ->
+    // 3.79), 20000 tokens 2.22 -> 1.86 (1.78 -> 1.40); vertical-slash, 32 / 8 heads, 131072 tokens 14.86 -> 13.96 ms, 500
+    // columns and 700 slashes 4.41 -> 4.04 (28 / 4 heads 120000 tokens 3.87 -> 3.08); 9000 tokens, 8 / 2 heads,
+    // vertical-slash 359 -> 214 us, block-sparse 318 -> 202, A-shape 224 -> 142.  A launch that fits the chip at
+    // once gains little and may lose (vertical-slash, 4 heads 13000 tokens 214 -> 193 us, 15000 223 -> 220, 16384 212 -> 233).
+    // A deal's workgroups share K/V through an L2, but it has to be small beside what an XCD gets in all:
+    //  * 32 workgroups for whole layers of vertical-slash lists: 32 / 8 heads, 65000 tokens, 500 columns and 700 slashes, deals
+    //    of 16, 32, 64, 128: 2016, 1996, 1991, 1996 us; 16 heads 30000 tokens, of 1, 2, 4, 8, 16: 1710, 1574, 1543, 1523,
+    //    1520; 12 / 3 heads 9000 tokens, of 4, 8, 16, 32: 240, 239, 241, 271;
+    //  * 16 for heads of a list (32 / 8 heads, 50000 tokens, of 4, 8, 16, 32, 64: 4788, 4625, 4582, 4645, 4739 us) and
+    //    block-sparse or A-shape walks in ascending order;
+    //  * 8 in launches of up to two rounds of workgroups (block-sparse, 7 heads 9000 tokens, of 8, 16: 177 and 201 us;
+    //    A-shape, 4 heads 18000 tokens, 164 and 206);
+    //  * 4 where the longest walks go first, so that the last ones stay short: A-shape, 16 heads 10000 tokens, of 1, 4,
+    //    16: 269, 273, 290 us; 28 / 4 heads 9000 tokens, of 7, 28, 56: 407, 417, 433;
+    //  * one unit in dense and split walks.  Dense, 8 / 2 heads 16384 tokens, of 1, 2, 4, 8 units 492, 499, 512, 553 us;
+    //  * one head of up to 131072 tokens: an eighth (vertical-slash, 65536 tokens 204 us, in deals of 16 225; 100000
+    //    tokens 366 : 394).
+    // turn: an XCD takes another place in every round of deals, so that with 2, 4 or 8 groups it meets all of them.
+    // Heads of a list are unlike, and so are the slashes of a layer's heads: 32 / 8 heads, 65000 tokens, 500 columns, 700
+    // slashes 2.13 -> 1.93 ms.  Equal heads keep an XCD to its groups (A-shape, 70000 tokens 4.44 : 4.58 ms).
     const long long groups = (long long)p.batch * (grid_heads / group);
-    // (block-sparse, 50000 tokens, 28 / 4 heads: top-100 4.19 -> 4.00 ms, top-50 2.12 -> 2.16: where the walks
-    // grow over less than a fourteenth of the rows the stripes do not pay)
     const int most = MODE == MODE_BS ? p.max_blocks :
                      MODE == MODE_ASHAPE ? (int)(((long long)p.n_local + p.n_init) / BN) + 2 : p.rows;    // steps of a full walk (lists: unknown)
-    const bool grows = MODE == MODE_DENSE || split_pairs > 0 ||
-                       (p.rows <= 1024 && p.rows <= 14ll * most && groups * group >= 8 && groups * group * units >= 1024);
-    p.stripes_log2 = 0;
-    if (grows)
-        while (p.stripes_log2 < 3 && (groups << p.stripes_log2) % 8) ++p.stripes_log2;
-    const long long per_stripe = (units + (1 << p.stripes_log2) - 1) >> p.stripes_log2;
-    p.total_wg = (groups * group * per_stripe) << p.stripes_log2;
+    const long long wgs = groups * group * units;
     // Longest walks first wherever they grow with the row block over much of the sequence.  A-shape and
     // block-sparse, 32 / 8 heads: 3000 tokens 107 -> 91 and 118 -> 92 us, 6000 tokens 336 -> 315 (6824) and
     // 333 -> 308, 12000 tokens 702 -> 677 and 921 -> 897, 24000 tokens 1508 -> 1487 and (32768) 2947 -> 2920;
     // neither order wins past 60000 tokens, and with fewer than two rounds of workgroups and walks that are
     // full-length early the first rows finish last (A-shape, 8 / 2 heads, 12000 tokens 227 -> 234 us).
     p.descending = MODE == MODE_DENSE || (MODE == MODE_VS ? p.rows <= 1024 :
-                   p.rows <= most || (p.rows <= 8ll * most && groups * group * units >= 1024));
-    const long long per_xcd = (p.total_wg + 7) >> 3;
-    const long long grid = per_xcd * 8;
+                   p.rows <= most || (p.rows <= 8ll * most && wgs >= 1024));
+    const int share = MODE != MODE_VS && p.descending ? 4 : (wgs <= 1024 ? 8 : (MODE == MODE_VS && !p.head_list ? 32 : 16));
+    long long chunk = MODE == MODE_DENSE || split_pairs > 0 || group >= share ? 1 : share / group;
+    if (MODE != MODE_DENSE && split_pairs == 0 && groups * group == 1 && units <= 1024) chunk = (units + 7) / 8;
+    if (chunk > units) chunk = units;
+    p.chunk = (int)chunk;
+    p.turn = p.head_list || MODE == MODE_VS;
+    const long long deal = chunk * group, deals = (units + chunk - 1) / chunk * groups;
+    const long long grid = (deals + 7) / 8 * 8 * deal;
     if (grid > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
     p.by_group = fast_div((unsigned)group);
-    p.by_stripe = fast_div((unsigned)per_stripe);
+    p.by_deal = fast_div((unsigned)deal);
+    p.by_groups = fast_div((unsigned)groups);
     p.by_heads = fast_div((unsigned)(grid_heads / group));
     const dim3 block(2 * NTHREADS);
     hipStream_t st = (hipStream_t)stream;

@@ -152,6 +152,32 @@ def test_striped_row_blocks_cover_every_row(gpu, hq, hk, n, b):
         assert (out.float() - 1).abs().max().item() <= 2.0 ** -8
 
 
+@pytest.mark.parametrize("hq,hk,n,b", [(20, 1, 8300, 1), (6, 3, 8300, 2), (3, 3, 8300, 1), (9, 9, 8500, 1), (1, 1, 66000, 1),
+                                       (2, 1, 66000, 1)])
+def test_heads_do_not_depend_on_how_a_launch_is_dealt(gpu, hq, hk, n, b):
+    """Every head of a launch against the head on its own, bit for bit (lengths that are not split): more
+    query heads than a deal has workgroups, batches, deals of an eighth of the launch and of a few pairs, both
+    sides of 512 and 1024 workgroups; the output is full of NaN before, so that no row can be left out."""
+    import minference_amd as M
+    q, k, v = (t.to(gpu) for t in make(b, hq, hk, n, 7, torch.bfloat16, 64))
+    group = hq // hk
+    bi = M.ops._build_block_index(q, k, 4)
+    vi, si = M.estimate_vertical_slash(q, k, 40, 60)
+    ix = M.index._build(None, vi, si, n, zero_fill=False)
+    out = torch.empty_like(q)
+    for name, f in (("a-shape", lambda q, k, v, i, o: M.streaming_forward(q, k, v, 64, 100, o)),
+                    ("block-sparse", lambda q, k, v, i, o: M.ops.block_sparse_attention_from_index(q, k, v, bi[i].contiguous(), o)),
+                    ("vertical-slash", lambda q, k, v, i, o: M.ops.vertical_slash_attention_from_index(
+                        q, k, v, *(t[i].contiguous() for t in ix), out=o))):
+        out.fill_(float("nan"))
+        f(q, k, v, (slice(None), slice(None)), out)
+        for bb in range(b):
+            for h in range(hq):
+                i = (slice(bb, bb + 1), slice(h, h + 1))
+                j = (slice(bb, bb + 1), slice(h // group, h // group + 1))
+                assert torch.equal(f(q[i], k[j], v[j], i, None), out[i]), (name, bb, h)
+
+
 @pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16)])
 def test_a_nan_key_reaches_every_row_that_attends_to_it(gpu, d, dtype):
     """The row sum of a segment with a NaN score is NaN: the fold keeps it, as a whole walk's rows are NaN,
