@@ -456,6 +456,20 @@ int minf_flags_set_range(int begin, int end, int rows, int bit, uint8_t *flags, 
                          void *stream);
 
 /*
+ * The column and diagonal flags of up to 8 candidates in one launch, from the score rows of minf_vs_estimate:
+ * vertical, slash [rows, n] fp32 with row_stride elements between rows; candidates: HOST array of `count` x
+ * {columns, diagonals, first_columns, first_diagonals} -- candidate t keeps the `columns` best entries of vertical (all
+ * from n on; ties: lowest index), the diagonals n-1-j of the `diagonals` best entries j of slash, and every position
+ * below first_columns / first_diagonals.  col_flags, diag_flags [rows, flag_pitch] uint8 (flag_pitch >= n) are written
+ * whole, padding with zeros.  A score row may be NULL where no candidate selects from it.  n up to
+ * MINF_SEARCH_FLAGS_MAX (a row is held in registers), else MINF_ERR_UNSUPPORTED.
+ */
+#define MINF_SEARCH_FLAGS_MAX 32768
+int minf_search_flags(const float *vertical, const float *slash, int rows, int n, int64_t row_stride,
+                      const int32_t *candidates, int count, uint8_t *col_flags, uint8_t *diag_flags,
+                      int64_t flag_pitch, void *stream);
+
+/*
  * Block index of the block_sparse candidate of the pattern search (reference
  * minference_forward.py:175-186): like minf_bs_block_index with 32-token blocks,
  * rows = ceil(n/32) (zero padding only up to the next multiple of 32) and no forced blocks.

@@ -525,12 +525,47 @@ __device__ __forceinline__ void topk_rank(unsigned *list, int m, TopkShared &sh,
     need = sh.need;
 }
 
+// The k-th largest of a row held in registers (see topk_regs_kernel): T its key, need the number of entries equal to T
+// that are taken.  8-bit radix passes from the top digit only until the bucket is small enough to be ranked at once.
+// first_digit: the histogram of the top digit where it is there already, else null.
+template <int ITEMS, int COPIES>
+__device__ __forceinline__ void topk_threshold(const unsigned (&key)[ITEMS], int n, int k, int begin, unsigned *hist,
+                                               const unsigned *first_digit, unsigned *list, TopkShared &sh, unsigned &T, unsigned &need) {
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    unsigned prefix = 0;
+    need = (unsigned)k;
+    int shift = 32;
+    do {
+        const unsigned above = shift == 32 ? 0u : prefix >> shift;
+        const int top = shift;
+        shift -= 8;
+        if (top < 32 || !first_digit) {
+#pragma unroll
+            for (int i = 0; i < 256 * COPIES / TK_THREADS; ++i) hist[i * TK_THREADS + tid] = 0;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < ITEMS; ++j)
+                if (top == 32 || key[j] >> top == above)
+                    atomicAdd(&hist[((key[j] >> shift) & 255u) * COPIES + (lane & (COPIES - 1))], 1u);
+            __syncthreads();
+        }
+        topk_digit<COPIES>(top == 32 && first_digit ? first_digit : hist, sh, prefix, need, shift);
+    } while (shift > 0 && sh.count > TK_LIST);
+    T = prefix;
+    if (shift > 0) {                                          // (workgroup-uniform) the bucket fits the list
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j)
+            if (key[j] >> shift == prefix >> shift && begin + 64 * j + lane < n) list[atomicAdd(&sh.listed, 1u)] = key[j];
+        __syncthreads();
+        topk_rank(list, (int)sh.listed, sh, T, need);        // (the bucket's count may hold padding)
+    }
+}
+
 // Rows of up to 16384 entries (from the number of rows on at which one wavefront per row fills the chip:
 // only rows longer than topk_wave_kernel takes): one 1024-thread workgroup per row that holds the row's
 // keys in registers (ITEMS per thread; wave w owns the contiguous slice of 64 * ITEMS entries from
 // 64 * ITEMS * w on, item j of a lane is entry 64 j + lane of it), so that the row is read once where
-// topk_kernel sweeps it six times, and every pass after the load is LDS and register work.  Same selection,
-// with 8-bit radix passes from the top digit only until the bucket is small enough to be ranked at once.
+// topk_kernel sweeps it six times, and every pass after the load is LDS and register work.  Same selection.
 // Two selections in a launch, 32 rows each, us, before (wave kernel up to 4096 entries, else topk_kernel) and
 // now: 2048 entries 18.3 / 6.4, 4096 31.5 / 7.0, 5000 11.9 / 9.2, 8192 13.2 / 10.4, 16001 26.3 / 13.8; 32768
 // in 32 registers per thread 25.6 / 26.0 (and 64 spill), so longer rows are swept.  Rows of 2048 entries:
@@ -559,30 +594,8 @@ __global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem
         const int i = begin + 64 * j + lane;
         key[j] = i < n ? order_key(x[i]) : 0u;               // padding sorts below every score
     }
-    unsigned prefix = 0, need = (unsigned)k;
-    int shift = 32;
-    do {
-        const unsigned above = shift == 32 ? 0u : prefix >> shift;
-        const int top = shift;
-        shift -= 8;
-#pragma unroll
-        for (int i = 0; i < 256 * COPIES / TK_THREADS; ++i) hist[i * TK_THREADS + tid] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j)
-            if (top == 32 || key[j] >> top == above)
-                atomicAdd(&hist[((key[j] >> shift) & 255u) * COPIES + (lane & (COPIES - 1))], 1u);
-        __syncthreads();
-        topk_digit<COPIES>(hist, sh, prefix, need, shift);
-    } while (shift > 0 && sh.count > TK_LIST);
-    unsigned T = prefix;
-    if (shift > 0) {                                          // (workgroup-uniform) the bucket fits the list
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j)
-            if (key[j] >> shift == prefix >> shift && begin + 64 * j + lane < n) list[atomicAdd(&sh.listed, 1u)] = key[j];
-        __syncthreads();
-        topk_rank(list, (int)sh.listed, sh, T, need);        // (the bucket's count may hold padding)
-    }
+    unsigned T, need;
+    topk_threshold<ITEMS, COPIES>(key, n, k, begin, hist, nullptr, list, sh, T, need);
     const int r = (int)need;                                  // entries equal to T that are taken
     int cgt = 0, ceq = 0;
 #pragma unroll
@@ -617,6 +630,90 @@ __global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem
         const int pad = pr.pad_mode == 2 ? sh.last : pr.pad_value;
         for (int i = k + tid; i < kmax; i += TK_THREADS) o[i] = pad;
     }
+}
+
+// The flag bytes of the pattern search's candidates (bit t of a byte: candidate t keeps the position): the k[t] best
+// entries of a score row and the first first[t] positions.  One workgroup per row and array, the row in registers as in
+// topk_regs_kernel, one selection per candidate (the histogram of the top digit is made once), every byte written once.
+// Bound by the selections' barriers and LDS atomics.  A selection, two scatters into zeroed flags per
+// candidate and the zeros before them were fifteen launches: 32 heads, 16384 tokens, the reference's six candidates,
+// 116 -> 39 us, whole search 1885 -> 1810.
+constexpr int FLAG_CANDS = 8;
+struct FlagsProblem {
+    const float *scores;         // may be null when every k is zero
+    int k[FLAG_CANDS], first[FLAG_CANDS];
+    unsigned char *flags;
+    int reverse;                 // entry i of a row is position n - 1 - i
+};
+template <int ITEMS>
+__global__ __launch_bounds__(TK_THREADS) void topk_flags_kernel(const FlagsProblem p0, const FlagsProblem p1, int n, long long row_stride,
+                                                                int count, long long pitch) {
+    const FlagsProblem &pr = blockIdx.y == 0 ? p0 : p1;
+    constexpr int COPIES = ITEMS > 4 ? 32 : 8;
+    __shared__ unsigned first_digit[256 * COPIES], hist[256 * COPIES];
+    __shared__ __attribute__((aligned(16))) unsigned list[TK_LIST + 4];
+    __shared__ TopkShared sh;
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int begin = wave * 64 * ITEMS;
+    unsigned char *out = pr.flags + (long long)blockIdx.x * pitch;
+    bool select = false;
+    for (int t = 0; t < count; ++t) select |= pr.k[t] > 0 && pr.k[t] < n;
+    unsigned key[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) key[j] = 0u;
+    if (select) {                                             // (workgroup-uniform)
+        const float *x = pr.scores + (long long)blockIdx.x * row_stride;
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const int i = begin + 64 * j + lane;
+            key[j] = i < n ? order_key(x[i]) : 0u;            // padding sorts below every score
+        }
+#pragma unroll
+        for (int i = 0; i < 256 * COPIES / TK_THREADS; ++i) first_digit[i * TK_THREADS + tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) atomicAdd(&first_digit[(key[j] >> 24) * COPIES + (lane & (COPIES - 1))], 1u);
+        __syncthreads();
+    }
+    unsigned bits[ITEMS / 4];                                 // four entries' flag bytes a word
+#pragma unroll
+    for (int j = 0; j < ITEMS / 4; ++j) bits[j] = 0u;
+    const uint64_t lt = minf_lanemask_lt();
+    for (int t = 0; t < count; ++t) {
+        const int k = pr.k[t], first = pr.first[t];
+        unsigned T = 0u, need = 0u;
+        const bool all = k >= n;
+        int gt_all = 0, eq_before = 0;
+        if (k > 0 && !all) {                                  // (workgroup-uniform)
+            topk_threshold<ITEMS, COPIES>(key, n, k, begin, hist, first_digit, list, sh, T, need);
+            int ceq = 0;
+#pragma unroll
+            for (int j = 0; j < ITEMS; ++j) ceq += __builtin_popcountll(__ballot(key[j] == T && begin + 64 * j + lane < n));
+            if (lane == 0) sh.wave_eq[wave] = ceq;
+            __syncthreads();
+            for (int wv = 0; wv < wave; ++wv) eq_before += sh.wave_eq[wv];
+            gt_all = 1;
+        }
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const int i = begin + 64 * j + lane, at = pr.reverse ? n - 1 - i : i;
+            bool take = all || at < first;
+            if (gt_all) {
+                const bool eq = key[j] == T && i < n;         // (of equal entries the lowest indexes are taken)
+                const uint64_t me = __ballot(eq);
+                take |= key[j] > T || (eq && eq_before + __builtin_popcountll(me & lt) < (int)need);
+                eq_before += __builtin_popcountll(me);
+            }
+            bits[j >> 2] |= (take ? 1u << t : 0u) << (8 * (j & 3));
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const int i = begin + 64 * j + lane;
+        if (i < n) out[pr.reverse ? n - 1 - i : i] = (unsigned char)(bits[j >> 2] >> (8 * (j & 3)));
+    }
+    for (long long i = n + tid; i < pitch; i += TK_THREADS) out[i] = 0;
 }
 
 void launch_topk(const TopkProblem &pa, const TopkProblem &pb, int problems, int rows, int n, hipStream_t st) {
@@ -693,5 +790,30 @@ extern "C" int minf_topk_indices_pair_ragged(const float *scores_a, const int32_
     TopkProblem pa{scores_a, (long long)row_stride, k_max_a, out_a, (long long)out_stride_a, reverse_base_a, 0, k_rows_a, pad_mode_a, pad_value_a};
     TopkProblem pb{scores_b, (long long)row_stride, k_max_b, out_b, (long long)out_stride_b, reverse_base_b, 0, k_rows_b, pad_mode_b, pad_value_b};
     launch_topk(pa, pb, 2, rows, n, (hipStream_t)stream);
+    return minf_launch_status();
+}
+
+extern "C" int minf_search_flags(const float *vertical, const float *slash, int rows, int n, int64_t row_stride,
+                                 const int32_t *candidates, int count, uint8_t *col_flags, uint8_t *diag_flags,
+                                 int64_t flag_pitch, void *stream) {
+    if (!candidates || !col_flags || !diag_flags || rows < 0 || n <= 0 || count < 0 || count > FLAG_CANDS) return MINF_ERR_INVALID_ARG;
+    if (flag_pitch < n) return MINF_ERR_INVALID_ARG;
+    FlagsProblem p[2] = {{vertical, {0}, {0}, col_flags, 0}, {slash, {0}, {0}, diag_flags, 1}};
+    for (int t = 0; t < count; ++t)
+        for (int i = 0; i < 2; ++i) {
+            const int k = candidates[4 * t + i], first = candidates[4 * t + 2 + i];
+            if (k < 0 || first < 0) return MINF_ERR_INVALID_ARG;
+            if (k > 0 && k < n && (!p[i].scores || row_stride < n)) return MINF_ERR_INVALID_ARG;
+            p[i].k[t] = k;
+            p[i].first[t] = first;
+        }
+    if (n > MINF_SEARCH_FLAGS_MAX) return MINF_ERR_UNSUPPORTED;
+    if (rows == 0) return MINF_OK;
+    const dim3 grid((unsigned)rows, 2), block(TK_THREADS);
+    hipStream_t st = (hipStream_t)stream;
+    if (n <= 4 * TK_THREADS) hipLaunchKernelGGL(topk_flags_kernel<4>, grid, block, 0, st, p[0], p[1], n, (long long)row_stride, count, (long long)flag_pitch);
+    else if (n <= 8 * TK_THREADS) hipLaunchKernelGGL(topk_flags_kernel<8>, grid, block, 0, st, p[0], p[1], n, (long long)row_stride, count, (long long)flag_pitch);
+    else if (n <= 16 * TK_THREADS) hipLaunchKernelGGL(topk_flags_kernel<16>, grid, block, 0, st, p[0], p[1], n, (long long)row_stride, count, (long long)flag_pitch);
+    else hipLaunchKernelGGL(topk_flags_kernel<32>, grid, block, 0, st, p[0], p[1], n, (long long)row_stride, count, (long long)flag_pitch);
     return minf_launch_status();
 }

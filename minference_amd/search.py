@@ -11,6 +11,8 @@ not fit anywhere.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -53,6 +55,42 @@ def _search_block_index(q16, k16, keep):
     return out
 
 
+def _position_flags(candidates, scores, rows, N, pitch, dev):
+    """The candidates' flag bytes per key column and per diagonal, [rows, pitch] uint8 each."""
+    vertical, slash = scores
+    lib = _lib.load()
+    stream = _lib.stream_ptr(dev)
+    sizes = []                                         # columns, diagonals selected; columns, diagonals from the first one on
+    for ty, a, b in candidates:
+        if ty not in ("stream_llm", "vertical_and_slash", "block_sparse"):
+            raise ValueError(f"unknown pattern type {ty!r}")
+        a, b = min(int(a), N), int(b)
+        if ty == "vertical_and_slash" and min(a, b) < 1:
+            raise _lib.MinfError(f"a vertical_and_slash candidate selects at least one entry of each kind, got {a}, {b}")
+        sizes.append((0, 0, max(a, 0), max(min(b + 1, N), 0)) if ty == "stream_llm" else
+                     (a, min(b, N), 0, 0) if ty == "vertical_and_slash" else (0, 0, 0, 0))
+    if N <= _lib.MINF_SEARCH_FLAGS_MAX:
+        col, diag = (torch.empty((rows, pitch), dtype=torch.uint8, device=dev) for _ in range(2))
+        cand = (ctypes.c_int32 * (4 * len(sizes)))(*(x for c in sizes for x in c))
+        with torch.cuda.device(dev):
+            st = lib.minf_search_flags(vertical.data_ptr() if vertical is not None else None,
+                                       slash.data_ptr() if slash is not None else None, rows, N, N, cand, len(sizes),
+                                       col.data_ptr(), diag.data_ptr(), pitch, stream)
+        _lib.check(st, "minf_search_flags")
+        return col, diag
+    col, diag = (torch.zeros((rows, pitch), dtype=torch.uint8, device=dev) for _ in range(2))
+    with torch.cuda.device(dev):
+        for bit, (kv, ks, first_col, first_diag) in enumerate(sizes):
+            for first, flags in ((first_col, col), (first_diag, diag)):
+                _lib.check(lib.minf_flags_set_range(0, first, rows, bit, flags.data_ptr(), pitch, stream), "minf_flags_set_range")
+            if candidates[bit][0] == "vertical_and_slash":
+                for idx, flags in zip(topk_vertical_slash(vertical, slash, kv, ks), (col, diag)):
+                    kk = idx.shape[-1]
+                    _lib.check(lib.minf_flags_set_indices(idx.data_ptr(), rows, kk, kk, bit, flags.data_ptr(), pitch, N, stream),
+                               "minf_flags_set_indices")
+    return col, diag
+
+
 def pattern_recall(q, k, candidates=CANDIDATES, row_begin=ROW_BEGIN):
     """-> [B, H, len(candidates)] fp32: for every head and candidate ``(type, a, b)`` the mean over
     query rows >= row_begin of the exact causal softmax mass inside the candidate's mask, with the
@@ -81,38 +119,23 @@ def pattern_recall(q, k, candidates=CANDIDATES, row_begin=ROW_BEGIN):
     pitch = (N + 63) // 64 * 64
     rows32 = (N + 31) // 32
     bpitch = (rows32 + 3) // 4 * 4
-    col = torch.zeros((B * H, pitch), dtype=torch.uint8, device=dev)
-    diag = torch.zeros((B * H, pitch), dtype=torch.uint8, device=dev)
     blk = None
-    scores = None
+    select = any(ty == "vertical_and_slash" for ty, _, _ in candidates)
+    scores = vertical_slash_scores(q, k, 64, SEARCH_FORCE, SEARCH_FORCE, reference_rounding=False) if select else (None, None)
+    col, diag = _position_flags(candidates, scores, B * H, N, pitch, dev)
     with torch.cuda.device(dev):
         for bit, (ty, a, b) in enumerate(candidates):
-            a, b = int(a), int(b)
-            if ty == "stream_llm":
-                _lib.check(lib.minf_flags_set_range(0, min(a, N), B * H, bit, col.data_ptr(), pitch, stream),
-                           "minf_flags_set_range")
-                _lib.check(lib.minf_flags_set_range(0, min(b + 1, N), B * H, bit, diag.data_ptr(), pitch, stream),
-                           "minf_flags_set_range")
-            elif ty == "vertical_and_slash":
-                if scores is None:
-                    scores = vertical_slash_scores(q, k, 64, SEARCH_FORCE, SEARCH_FORCE, reference_rounding=False)
-                v_idx, s_idx = topk_vertical_slash(scores[0], scores[1], a, b)
-                for idx, flags in ((v_idx, col), (s_idx, diag)):
-                    kk = idx.shape[-1]
-                    _lib.check(lib.minf_flags_set_indices(idx.data_ptr(), B * H, kk, kk, bit, flags.data_ptr(),
-                                                          pitch, N, stream), "minf_flags_set_indices")
-            elif ty == "block_sparse":
-                keep = rows32 // a
-                if blk is None:
-                    blk = torch.zeros((B * H * rows32, bpitch), dtype=torch.uint8, device=dev)
-                if keep > 0:
-                    bi = _search_block_index(q16, k16, keep)
-                    kk = bi.shape[-1]
-                    _lib.check(lib.minf_flags_set_indices(bi.data_ptr(), B * H * rows32, kk, kk, bit,
-                                                          blk.data_ptr(), bpitch, rows32, stream),
-                               "minf_flags_set_indices")
-            else:
-                raise ValueError(f"unknown pattern type {ty!r}")
+            if ty != "block_sparse":
+                continue
+            keep = rows32 // int(a)
+            if blk is None:
+                blk = torch.zeros((B * H * rows32, bpitch), dtype=torch.uint8, device=dev)
+            if keep > 0:
+                bi = _search_block_index(q16, k16, keep)
+                kk = bi.shape[-1]
+                _lib.check(lib.minf_flags_set_indices(bi.data_ptr(), B * H * rows32, kk, kk, bit,
+                                                      blk.data_ptr(), bpitch, rows32, stream),
+                           "minf_flags_set_indices")
         recall = torch.empty((B * H, MAX_CANDIDATES), dtype=torch.float32, device=dev)
         ws_bytes = lib.minf_pattern_recall_workspace_bytes(B, H, N)
         ws = torch.empty((ws_bytes + 15) // 16 * 16, dtype=torch.uint8, device=dev)

@@ -120,6 +120,12 @@ def test_argument_validation_of_the_index_estimate_and_search_entry_points(lib):
     assert lib.minf_flags_set_indices(P, 4, 10, 10, 0, P, 190, 130, None) == -1           # pitch % 4
     assert lib.minf_flags_set_range(0, 200, 4, 0, P, 192, None) == -1                     # end > pitch
     assert lib.minf_flags_set_range(10, 10, 4, 0, P, 192, None) == 0                      # empty range: nothing to do
+    cand = (ctypes.c_int32 * 4)(10, 10, 0, 0)
+    assert lib.minf_search_flags(P, P, 4, 130, 130, cand, 9, P, P, 192, None) == -1       # more than 8 candidates
+    assert lib.minf_search_flags(P, P, 4, 130, 130, cand, 1, P, P, 129, None) == -1       # pitch < n
+    assert lib.minf_search_flags(P, None, 4, 130, 130, cand, 1, P, P, 192, None) == -1    # selects from nothing
+    assert lib.minf_search_flags(P, P, 4, 40000, 40000, cand, 1, P, P, 40000, None) == -2 # longer rows than a workgroup holds
+    assert lib.minf_search_flags(P, P, 0, 130, 130, cand, 1, P, P, 192, None) == 0
 
 
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):

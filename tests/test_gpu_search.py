@@ -346,3 +346,35 @@ def test_candidates_without_the_sink_keep_their_accuracy(gpu, nats):
     for t in range(5):
         want = (p * ((keep >> t) & 1)).sum() / n
         assert abs(got[t] - want) <= 2.0 ** -23 * (nats * 1.4427 + 10 + 32) * want, (t, got[t].item(), want.item())
+
+
+@pytest.mark.parametrize("n", [1, 63, 257, 4096, 4097, 8192, 8193, 16384, 16385, 32768])
+def test_flags_of_all_candidates_in_one_launch(gpu, n):
+    """minf_search_flags against a stable sort: sizes around what a thread holds, scores that tie in thousands, infinities,
+    selections of one entry, of nearly all and of all, candidates that select nothing, first positions beside
+    selections; the arrays hold other bytes before and rows lie apart.  (No negative zeros: they rank below zero.)"""
+    import ctypes
+    from minference_amd import _lib
+    rows, stride, pitch = 3, n + 5, (n + 63) // 64 * 64 + 64
+    g = np.random.default_rng(n)
+    sc = [g.standard_normal((rows, stride)).astype(np.float32), np.round(4 * g.standard_normal((rows, stride))).astype(np.float32) + 0.0]
+    sc[1][1, :n // 2] = -np.inf
+    sc[0][2, :n // 3] = np.inf
+    sc[1][2] = 0.0
+    cand = [(1, 1, 0, 0), (0, 0, min(n, 100), min(n, 7)), (min(n, 500), min(n, 700), 0, 0), (max(n - 1, 1), max(n - 1, 1), 0, 0),
+            (n, n, 0, 0), (0, 0, 0, 0), ((n + 1) // 2, (n + 3) // 4, 3, 1), (min(n, 129), min(n, 128), 0, n)]
+    flags = [torch.full((rows, pitch), 255, dtype=torch.uint8, device=gpu) for _ in range(2)]
+    dev = [torch.from_numpy(x).to(gpu) for x in sc]
+    arr = (ctypes.c_int32 * 32)(*(x for c in cand for x in c))
+    st = _lib.load().minf_search_flags(dev[0].data_ptr(), dev[1].data_ptr(), rows, n, stride, arr, 8, flags[0].data_ptr(),
+                                       flags[1].data_ptr(), pitch, _lib.stream_ptr(gpu))
+    assert st == 0
+    for i in range(2):
+        want = np.zeros((rows, pitch), np.uint8)
+        for r in range(rows):
+            order = np.argsort(-sc[i][r, :n].astype(np.float64), kind="stable")
+            for t, c in enumerate(cand):
+                at = order[:c[i]]
+                want[r, n - 1 - at if i else at] |= 1 << t
+                want[r, :min(c[2 + i], n)] |= 1 << t
+        assert np.array_equal(flags[i].cpu().numpy(), want), i
