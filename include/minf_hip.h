@@ -482,6 +482,18 @@ int minf_search_block_index(const void *q, const void *k, const int64_t *q_strid
                             void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * The same selection as flags: bit `bit` of block_flags[row, c] (see minf_pattern_recall; rows of flag_pitch >= ceil(n/32)
+ * bytes) for the top_k blocks c of every row, ORed into what is there, or with `clear` in place of it (zero elsewhere,
+ * padding included).  ceil(n/32) up to 4096, else MINF_ERR_UNSUPPORTED.
+ * minf_topk_flags_block_causal: the selection alone, of rows as in minf_topk_indices_block_causal.
+ */
+int minf_search_block_flags(const void *q, const void *k, const int64_t *q_stride, const int64_t *k_stride, int batch,
+                            int heads_q, int heads_kv, int n, int head_dim, int dtype, int top_k, int bit, int clear,
+                            uint8_t *block_flags, int64_t flag_pitch, void *workspace, size_t workspace_bytes, void *stream);
+int minf_topk_flags_block_causal(const float *scores, int rows, int n, int64_t row_stride, int k, int rows_per_head,
+                                 int bit, int clear, uint8_t *flags, int64_t flag_pitch, void *stream);
+
+/*
  * The element-wise passes of a decoder layer around the attention path (reference
  * minference/patch.py:500-558, :688-693, as chains of torch ops); dtype MINF_BF16, MINF_F16 or
  * MINF_F32, contiguous tensors (minf_rope, minf_silu_mul: 16-byte aligned).  Values are rounded to

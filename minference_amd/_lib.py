@@ -57,6 +57,8 @@ SIGNATURES = {
     "minf_flags_set_indices": (c_int, [c_ptr, c_int, c_int, c_i64, c_int, c_ptr, c_i64, c_int, c_ptr]),
     "minf_flags_set_range": (c_int, [c_int, c_int, c_int, c_int, c_ptr, c_i64, c_ptr]),
     "minf_search_flags": (c_int, [c_ptr, c_ptr, c_int, c_int, c_i64, c_ptr, c_int, c_ptr, c_ptr, c_i64, c_ptr]),
+    "minf_search_block_flags": (c_int, [c_ptr, c_ptr, c_ptr, c_ptr] + [c_int] * 9 + [c_ptr, c_i64, c_ptr, ctypes.c_size_t, c_ptr]),
+    "minf_topk_flags_block_causal": (c_int, [c_ptr, c_int, c_int, c_i64] + [c_int] * 4 + [c_ptr, c_i64, c_ptr]),
     "minf_rms_norm": (c_int, [c_ptr] * 4 + [c_i64, c_int, c_f32, c_int, c_ptr]),
     "minf_rope": (c_int, [c_ptr] * 4 + [c_i64] + [c_int] * 4 + [c_ptr]),
     "minf_silu_mul": (c_int, [c_ptr, c_ptr, c_i64, c_int, c_ptr]),
@@ -86,7 +88,7 @@ MINF_BF16, MINF_F16, MINF_F32, MINF_16BIT_SELECT = 0, 1, 2, 3
 MINF_NARROW_WORKSPACE_INTS = 769
 MINF_OP_VERTICAL_SLASH, MINF_OP_BLOCK_SPARSE, MINF_OP_ASHAPE, MINF_OP_DENSE = 0, 1, 2, 3
 MINF_INDEX_SORT_MAX = 16384
-MINF_SEARCH_FLAGS_MAX = 32768
+MINF_SEARCH_FLAGS_MAX, MINF_SEARCH_BLOCK_FLAGS_MAX = 32768, 4096
 MINF_ROUND_NONE, MINF_ROUND_INPUT_DTYPE = 0, 1
 MINF_BS_FORCE_DIAG_FIRST, MINF_BS_ROUND_INPUT_DTYPE = 1, 2
 

@@ -240,8 +240,9 @@ namespace {
 int block_index_impl(const void *q, const void *k, const int64_t *q_stride, const int64_t *k_stride, int batch,
                      int heads_q, int heads_kv, int n, int head_dim, int dtype, int blk, int rows, int top_k,
                      int flags, int32_t *block_index, void *workspace, size_t workspace_bytes,
-                     void *stream, const int32_t *head_list = nullptr, int index_heads = 0) {
-    if (!q || !k || !q_stride || !k_stride || !block_index) return MINF_ERR_INVALID_ARG;
+                     void *stream, const int32_t *head_list = nullptr, int index_heads = 0,
+                     uint8_t *block_flags = nullptr, int64_t flag_pitch = 0, int bit = 0, int clear = 0) {
+    if (!q || !k || !q_stride || !k_stride || !(block_index || block_flags)) return MINF_ERR_INVALID_ARG;
     if (head_list && index_heads <= 0) return MINF_ERR_INVALID_ARG;
     if (!head_list) index_heads = heads_q;
     if (batch < 0 || heads_q <= 0 || heads_kv <= 0 || n <= 0 || top_k <= 0) return MINF_ERR_INVALID_ARG;
@@ -291,6 +292,8 @@ int block_index_impl(const void *q, const void *k, const int64_t *q_stride, cons
     if (status != MINF_OK) return status;
 
     const int kk = top_k < rows ? top_k : rows;
+    if (block_flags)
+        return minf_topk_flags_block_causal(scores, batch * index_heads * rows, rows, pitch, kk, rows, bit, clear, block_flags, flag_pitch, stream);
     if (causal_topk)
         return minf_topk_indices_block_causal(scores, batch * index_heads * rows, rows, pitch, kk, block_index, kk, rows, stream);
     return minf_topk_indices(scores, batch * index_heads * rows, rows, pitch, kk, block_index, kk, -1, stream);
@@ -335,4 +338,14 @@ extern "C" int minf_search_block_index(const void *q, const void *k, const int64
                                        void *workspace, size_t workspace_bytes, void *stream) {
     return block_index_impl(q, k, q_stride, k_stride, batch, heads_q, heads_kv, n, head_dim, dtype, 32,
                             n > 0 ? (n + 31) / 32 : 0, top_k, 0, block_index, workspace, workspace_bytes, stream);
+}
+
+extern "C" int minf_search_block_flags(const void *q, const void *k, const int64_t *q_stride, const int64_t *k_stride, int batch,
+                                       int heads_q, int heads_kv, int n, int head_dim, int dtype, int top_k, int bit, int clear,
+                                       uint8_t *block_flags, int64_t flag_pitch, void *workspace, size_t workspace_bytes, void *stream) {
+    const int rows = n > 0 ? (n + 31) / 32 : 0;
+    if (!block_flags || bit < 0 || bit > 7 || flag_pitch < rows) return MINF_ERR_INVALID_ARG;
+    if (rows > 64 * 64) return MINF_ERR_UNSUPPORTED;
+    return block_index_impl(q, k, q_stride, k_stride, batch, heads_q, heads_kv, n, head_dim, dtype, 32, rows, top_k, 0, nullptr,
+                            workspace, workspace_bytes, stream, nullptr, 0, block_flags, flag_pitch, bit, clear);
 }

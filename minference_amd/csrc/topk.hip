@@ -48,6 +48,11 @@ struct TopkProblem {
     // k_rows == nullptr: every row keeps k entries.
     const int *k_rows;
     int pad_mode, pad_value;
+    // flag rows instead of index lists (wave kernel, FLAGS): flags[row][i] gets `flag` where entry i is selected, ORed
+    // into what is there, or with `clear` in place of it (zero where it is not selected, and up to flag_pitch)
+    unsigned char *flags;
+    long long flag_pitch;
+    int flag, clear;
 };
 
 // blockIdx.y selects one of two problems over rows of the same length n (vertical and slash
@@ -290,7 +295,9 @@ __global__ __launch_bounds__(TK_THREADS) void topk_kernel(const TopkProblem p0, 
 constexpr int TKW_WAVES = 4;
 // (the second launch bound is the number of resident waves per SIMD the register budget must allow:
 // the kernel is latency bound, and left alone the 64-item variant took 141 registers = 3 waves)
-template <int ITEMS>
+// FLAGS: the pattern search's block flags, one byte per entry (see TopkProblem).  As index lists that a kernel scattered
+// into zeroed flags, 32 heads, 512 rows of 512 blocks, 64 kept, took 80 us in three launches; 41 now.
+template <int ITEMS, bool FLAGS = false>
 __global__ __launch_bounds__(TKW_WAVES * 64, ITEMS >= 64 ? 3 : (ITEMS >= 40 ? 5 : 8)) void topk_wave_kernel(const TopkProblem p0, const TopkProblem p1,
                                                                    int n, int rows) {
     const TopkProblem &pr = blockIdx.y == 0 ? p0 : p1;
@@ -301,8 +308,19 @@ __global__ __launch_bounds__(TKW_WAVES * 64, ITEMS >= 64 ? 3 : (ITEMS >= 40 ? 5 
     int32_t *__restrict__ o = pr.out + (long long)row * pr.out_stride;
     const int kcap = pr.k, reverse_base = pr.reverse_base;
     const int k = pr.k_rows ? max(1, min(pr.k_rows[row], kcap)) : kcap;
+    [[maybe_unused]] unsigned char *const flags = FLAGS ? pr.flags + (long long)row * pr.flag_pitch : nullptr;
+    [[maybe_unused]] auto set_flag = [&](int i, bool take) {
+        if (pr.clear) flags[i] = (unsigned char)(take ? pr.flag : 0);
+        else if (take) flags[i] |= (unsigned char)pr.flag;
+    };
+    if constexpr (FLAGS)
+        for (long long i = n + lane; pr.clear && i < pr.flag_pitch; i += 64) flags[i] = 0;
     if (k >= n) {
-        for (int i = lane; i < n; i += 64) o[i] = reverse_base >= 0 ? reverse_base - i : i;
+        if constexpr (FLAGS) {
+            for (int i = lane; i < n; i += 64) set_flag(i, true);
+        } else {
+            for (int i = lane; i < n; i += 64) o[i] = reverse_base >= 0 ? reverse_base - i : i;
+        }
         return;
     }
     constexpr unsigned KEY_FLOOR = 0x007fffffu;          // order_key(-inf)
@@ -426,6 +444,17 @@ __global__ __launch_bounds__(TKW_WAVES * 64, ITEMS >= 64 ? 3 : (ITEMS >= 40 ? 5 
     int lastv = 0;
     bool has_last = false;
     const uint64_t lt = minf_lanemask_lt();
+    if constexpr (FLAGS) {
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            const int i = j * 64 + lane;
+            const bool eq = key[j] == T;
+            const uint64_t me = __ballot(eq);
+            if (i < n) set_flag(i, key[j] > T || (eq && eq_before + __builtin_popcountll(me & lt) < r));
+            eq_before += __builtin_popcountll(me);
+        }
+        return;
+    }
 #pragma unroll
     for (int jb = 0; jb < ITEMS; jb += GROUP) {
         if (jb < jmax) {
@@ -744,7 +773,7 @@ extern "C" int minf_topk_indices(const float *scores, int rows, int n, int64_t r
     if (!scores || !out || rows < 0 || n <= 0 || k <= 0) return MINF_ERR_INVALID_ARG;
     if (row_stride < n || out_stride < (k < n ? k : n)) return MINF_ERR_INVALID_ARG;
     if (rows == 0) return MINF_OK;
-    TopkProblem p{scores, (long long)row_stride, k, out, (long long)out_stride, reverse_base, 0, nullptr, 0, 0};
+    TopkProblem p{scores, (long long)row_stride, k, out, (long long)out_stride, reverse_base, 0, nullptr, 0, 0, nullptr, 0, 0, 0};
     launch_topk(p, p, 1, rows, n, (hipStream_t)stream);
     return minf_launch_status();
 }
@@ -755,7 +784,7 @@ extern "C" int minf_topk_indices_block_causal(const float *scores, int rows, int
     if (row_stride < n || out_stride < (k < n ? k : n)) return MINF_ERR_INVALID_ARG;
     if (n > 64 * 64) return MINF_ERR_UNSUPPORTED;      // only the one-wave-per-row kernel knows about stored prefixes
     if (rows == 0) return MINF_OK;
-    TopkProblem p{scores, (long long)row_stride, k, out, (long long)out_stride, -1, rows_per_head, nullptr, 0, 0};
+    TopkProblem p{scores, (long long)row_stride, k, out, (long long)out_stride, -1, rows_per_head, nullptr, 0, 0, nullptr, 0, 0, 0};
     launch_topk(p, p, 1, rows, n, (hipStream_t)stream);
     return minf_launch_status();
 }
@@ -769,8 +798,8 @@ extern "C" int minf_topk_indices_pair(const float *scores_a, int k_a, int32_t *o
     if (row_stride < n || out_stride_a < (k_a < n ? k_a : n) || out_stride_b < (k_b < n ? k_b : n))
         return MINF_ERR_INVALID_ARG;
     if (rows == 0) return MINF_OK;
-    TopkProblem pa{scores_a, (long long)row_stride, k_a, out_a, (long long)out_stride_a, reverse_base_a, 0, nullptr, 0, 0};
-    TopkProblem pb{scores_b, (long long)row_stride, k_b, out_b, (long long)out_stride_b, reverse_base_b, 0, nullptr, 0, 0};
+    TopkProblem pa{scores_a, (long long)row_stride, k_a, out_a, (long long)out_stride_a, reverse_base_a, 0, nullptr, 0, 0, nullptr, 0, 0, 0};
+    TopkProblem pb{scores_b, (long long)row_stride, k_b, out_b, (long long)out_stride_b, reverse_base_b, 0, nullptr, 0, 0, nullptr, 0, 0, 0};
     launch_topk(pa, pb, 2, rows, n, (hipStream_t)stream);
     return minf_launch_status();
 }
@@ -787,8 +816,8 @@ extern "C" int minf_topk_indices_pair_ragged(const float *scores_a, const int32_
     if (k_max_b > n) k_max_b = n;
     if (row_stride < n || out_stride_a < k_max_a || out_stride_b < k_max_b) return MINF_ERR_INVALID_ARG;
     if (rows == 0) return MINF_OK;
-    TopkProblem pa{scores_a, (long long)row_stride, k_max_a, out_a, (long long)out_stride_a, reverse_base_a, 0, k_rows_a, pad_mode_a, pad_value_a};
-    TopkProblem pb{scores_b, (long long)row_stride, k_max_b, out_b, (long long)out_stride_b, reverse_base_b, 0, k_rows_b, pad_mode_b, pad_value_b};
+    TopkProblem pa{scores_a, (long long)row_stride, k_max_a, out_a, (long long)out_stride_a, reverse_base_a, 0, k_rows_a, pad_mode_a, pad_value_a, nullptr, 0, 0, 0};
+    TopkProblem pb{scores_b, (long long)row_stride, k_max_b, out_b, (long long)out_stride_b, reverse_base_b, 0, k_rows_b, pad_mode_b, pad_value_b, nullptr, 0, 0, 0};
     launch_topk(pa, pb, 2, rows, n, (hipStream_t)stream);
     return minf_launch_status();
 }
@@ -815,5 +844,21 @@ extern "C" int minf_search_flags(const float *vertical, const float *slash, int 
     else if (n <= 8 * TK_THREADS) hipLaunchKernelGGL(topk_flags_kernel<8>, grid, block, 0, st, p[0], p[1], n, (long long)row_stride, count, (long long)flag_pitch);
     else if (n <= 16 * TK_THREADS) hipLaunchKernelGGL(topk_flags_kernel<16>, grid, block, 0, st, p[0], p[1], n, (long long)row_stride, count, (long long)flag_pitch);
     else hipLaunchKernelGGL(topk_flags_kernel<32>, grid, block, 0, st, p[0], p[1], n, (long long)row_stride, count, (long long)flag_pitch);
+    return minf_launch_status();
+}
+
+extern "C" int minf_topk_flags_block_causal(const float *scores, int rows, int n, int64_t row_stride, int k, int rows_per_head,
+                                            int bit, int clear, uint8_t *flags, int64_t flag_pitch, void *stream) {
+    if (!scores || !flags || rows < 0 || n <= 0 || k <= 0 || rows_per_head <= 0 || bit < 0 || bit >= FLAG_CANDS) return MINF_ERR_INVALID_ARG;
+    if (row_stride < n || flag_pitch < n) return MINF_ERR_INVALID_ARG;
+    if (n > 64 * 64) return MINF_ERR_UNSUPPORTED;
+    if (rows == 0) return MINF_OK;
+    const TopkProblem p{scores, (long long)row_stride, k, nullptr, 0, -1, rows_per_head, nullptr, 0, 0, flags, (long long)flag_pitch, 1 << bit, clear};
+    const dim3 grid((unsigned)((rows + TKW_WAVES - 1) / TKW_WAVES)), block(TKW_WAVES * 64);
+    hipStream_t st = (hipStream_t)stream;
+    if (n <= 64 * 4) hipLaunchKernelGGL((topk_wave_kernel<4, true>), grid, block, 0, st, p, p, n, rows);
+    else if (n <= 64 * 16) hipLaunchKernelGGL((topk_wave_kernel<16, true>), grid, block, 0, st, p, p, n, rows);
+    else if (n <= 64 * 40) hipLaunchKernelGGL((topk_wave_kernel<40, true>), grid, block, 0, st, p, p, n, rows);
+    else hipLaunchKernelGGL((topk_wave_kernel<64, true>), grid, block, 0, st, p, p, n, rows);
     return minf_launch_status();
 }

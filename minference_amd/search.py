@@ -34,25 +34,33 @@ def _dtype_code(t):
     return _lib.MINF_BF16 if t.dtype == torch.bfloat16 else _lib.MINF_F16
 
 
-def _search_block_index(q16, k16, keep):
-    """Top ``keep`` key blocks (32 tokens) per query block of the pooled scores, :175-186."""
+def _add_block_flags(q16, k16, keep, bit, blk, bpitch, clear):
+    """Bit ``bit`` of the flags of the top ``keep`` key blocks (32 tokens) per query block of the pooled scores, :175-186.
+    ``clear``: the flags hold nothing yet."""
     B, H, N, _ = q16.shape
     Hk = k16.shape[1]
     rows = (N + 31) // 32
     keep = min(keep, rows)
     lib = _lib.load()
     dev = q16.device
-    out = torch.empty((B, H, rows, keep), dtype=torch.int32, device=dev)
     ws_bytes = lib.minf_search_block_index_workspace_bytes(B, H, Hk, N)
     ws = torch.empty((ws_bytes + 15) // 16 * 16, dtype=torch.uint8, device=dev)
     i64x3 = _lib.c_i64 * 3
+    args = (q16.data_ptr(), k16.data_ptr(), i64x3(*q16.stride()[:3]), i64x3(*k16.stride()[:3]),
+            B, H, Hk, N, 128, _dtype_code(q16), keep)
     with torch.cuda.device(dev):
-        st = lib.minf_search_block_index(
-            q16.data_ptr(), k16.data_ptr(), i64x3(*q16.stride()[:3]), i64x3(*k16.stride()[:3]),
-            B, H, Hk, N, 128, _dtype_code(q16), keep, out.data_ptr(), ws.data_ptr(), ws_bytes,
-            _lib.stream_ptr(dev))
-    _lib.check(st, "minf_search_block_index")
-    return out
+        stream = _lib.stream_ptr(dev)
+        if rows <= _lib.MINF_SEARCH_BLOCK_FLAGS_MAX:
+            st = lib.minf_search_block_flags(*args, bit, clear, blk.data_ptr(), bpitch, ws.data_ptr(), ws_bytes, stream)
+            _lib.check(st, "minf_search_block_flags")
+            return
+        if clear:
+            blk.zero_()
+        out = torch.empty((B, H, rows, keep), dtype=torch.int32, device=dev)
+        st = lib.minf_search_block_index(*args, out.data_ptr(), ws.data_ptr(), ws_bytes, stream)
+        _lib.check(st, "minf_search_block_index")
+        st = lib.minf_flags_set_indices(out.data_ptr(), B * H * rows, keep, keep, bit, blk.data_ptr(), bpitch, rows, stream)
+        _lib.check(st, "minf_flags_set_indices")
 
 
 def _position_flags(candidates, scores, rows, N, pitch, dev):
@@ -123,19 +131,14 @@ def pattern_recall(q, k, candidates=CANDIDATES, row_begin=ROW_BEGIN):
     select = any(ty == "vertical_and_slash" for ty, _, _ in candidates)
     scores = vertical_slash_scores(q, k, 64, SEARCH_FORCE, SEARCH_FORCE, reference_rounding=False) if select else (None, None)
     col, diag = _position_flags(candidates, scores, B * H, N, pitch, dev)
-    with torch.cuda.device(dev):
-        for bit, (ty, a, b) in enumerate(candidates):
-            if ty != "block_sparse":
-                continue
-            keep = rows32 // int(a)
+    for bit, (ty, a, _) in enumerate(candidates):
+        if ty == "block_sparse" and rows32 // int(a) > 0:
             if blk is None:
-                blk = torch.zeros((B * H * rows32, bpitch), dtype=torch.uint8, device=dev)
-            if keep > 0:
-                bi = _search_block_index(q16, k16, keep)
-                kk = bi.shape[-1]
-                _lib.check(lib.minf_flags_set_indices(bi.data_ptr(), B * H * rows32, kk, kk, bit,
-                                                      blk.data_ptr(), bpitch, rows32, stream),
-                           "minf_flags_set_indices")
+                blk = torch.empty((B * H * rows32, bpitch), dtype=torch.uint8, device=dev)
+                _add_block_flags(q16, k16, rows32 // int(a), bit, blk, bpitch, True)
+            else:
+                _add_block_flags(q16, k16, rows32 // int(a), bit, blk, bpitch, False)
+    with torch.cuda.device(dev):
         recall = torch.empty((B * H, MAX_CANDIDATES), dtype=torch.float32, device=dev)
         ws_bytes = lib.minf_pattern_recall_workspace_bytes(B, H, N)
         ws = torch.empty((ws_bytes + 15) // 16 * 16, dtype=torch.uint8, device=dev)

@@ -126,6 +126,9 @@ def test_argument_validation_of_the_index_estimate_and_search_entry_points(lib):
     assert lib.minf_search_flags(P, None, 4, 130, 130, cand, 1, P, P, 192, None) == -1    # selects from nothing
     assert lib.minf_search_flags(P, P, 4, 40000, 40000, cand, 1, P, P, 40000, None) == -2 # longer rows than a workgroup holds
     assert lib.minf_search_flags(P, P, 0, 130, 130, cand, 1, P, P, 192, None) == 0
+    assert lib.minf_search_block_flags(P, P, i3, i3, 1, 4, 4, 130, 128, 0, 2, 8, 1, P, 8, P, 1 << 30, None) == -1     # bit 8
+    assert lib.minf_search_block_flags(P, P, i3, i3, 1, 4, 4, 130, 128, 0, 2, 0, 1, P, 4, P, 1 << 30, None) == -1     # pitch < 5
+    assert lib.minf_search_block_flags(P, P, i3, i3, 1, 4, 4, 131073, 128, 0, 2, 0, 1, P, 4100, P, 1 << 40, None) == -2
 
 
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):

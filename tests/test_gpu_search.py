@@ -378,3 +378,24 @@ def test_flags_of_all_candidates_in_one_launch(gpu, n):
                 want[r, n - 1 - at if i else at] |= 1 << t
                 want[r, :min(c[2 + i], n)] |= 1 << t
         assert np.array_equal(flags[i].cpu().numpy(), want), i
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (4, 3), (256, 31), (257, 257), (1000, 125), (1025, 1), (2560, 320), (2561, 320), (4096, 512)])
+def test_block_flags_are_the_indices_of_the_same_selection(gpu, n, k):
+    """Block-causal rows (some with fewer entries above -inf than are kept, scores that tie), first in place of what the
+    flags hold, then a second candidate's ORed in; against the index lists of the same kernel."""
+    from minference_amd import _lib
+    lib, per_head, pitch, s = _lib.load(), n, (n + 3) // 4 * 4 + 4, _lib.stream_ptr(gpu)
+    rows = 2 * per_head if n < 300 else 300
+    g = torch.Generator().manual_seed(n)
+    sc = (8 * torch.randn(rows, n, generator=g)).round() + 0.0
+    sc[torch.arange(n)[None] > (torch.arange(rows) % per_head)[:, None]] = float("-inf")
+    sc = sc.to(gpu)
+    flags = torch.full((rows, pitch), 255, dtype=torch.uint8, device=gpu)
+    want = torch.zeros((rows, pitch), dtype=torch.uint8)
+    for bit, kk, clear in ((3, k, 1), (5, max(k // 2, 1), 0)):
+        idx = torch.empty((rows, kk), dtype=torch.int32, device=gpu)
+        assert lib.minf_topk_indices_block_causal(sc.data_ptr(), rows, n, n, kk, idx.data_ptr(), kk, per_head, s) == 0
+        assert lib.minf_topk_flags_block_causal(sc.data_ptr(), rows, n, n, kk, per_head, bit, clear, flags.data_ptr(), pitch, s) == 0
+        want.scatter_(1, idx.cpu().long(), want.gather(1, idx.cpu().long()) | (1 << bit))
+        assert torch.equal(flags.cpu(), want), bit
