@@ -591,11 +591,11 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // rows_c: tile rows copied by one wave (16: the four waves of a pair share the tile, 32: the
     // two waves of a row block copy it); wsel: which part of the tile this wave copies
     auto copy_rows = [&](const Tile &t, const char *base, long long rowstride, auto is_v_c, int idv,
-                         char *ldsbuf, auto rows_c, const int wsel) {
+                         char *ldsbuf, auto rows_c, const int wsel, auto whole_c) {
         constexpr bool is_v = decltype(is_v_c)::value;
         constexpr int CROWS = decltype(rows_c)::value;
         const bool gathered = MODE == MODE_VS && t.gathered;
-        if (!gathered && t.start >= 0 && t.start + BN <= seqlen) {
+        if (decltype(whole_c)::value || (!gathered && t.start >= 0 && t.start + BN <= seqlen)) {
             // buffer form: descriptor of the 64 tile rows (scalar), one of five per-lane offsets (the V
             // swizzle does not depend on j, the K swizzle only on j % 4) and a scalar row offset
             const char *tb = base + (long long)t.start * rowstride;      // wave-uniform
@@ -642,11 +642,11 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     auto copy_tile = [&](const Tile &t, const char *base, long long rowstride, auto is_v_c, int idv, char *ldsbuf) {
         if constexpr (VSP) {
             if (t.split) {
-                if (t.on_a) copy_rows(t, base, rowstride, is_v_c, idv, ldsbuf + half * TILE_BYTES, std::integral_constant<int, 32>{}, wave);
+                if (t.on_a) copy_rows(t, base, rowstride, is_v_c, idv, ldsbuf + half * TILE_BYTES, std::integral_constant<int, 32>{}, wave, std::false_type{});
                 return;
             }
         }
-        copy_rows(t, base, rowstride, is_v_c, idv, ldsbuf, std::integral_constant<int, CROWS>{}, wave_wg);
+        copy_rows(t, base, rowstride, is_v_c, idv, ldsbuf, std::integral_constant<int, CROWS>{}, wave_wg, std::false_type{});
     };
 
     // ---- accumulators -------------------------------------------------------
@@ -703,17 +703,20 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     };
 
     // ---- mask, V^T fragment reads, online softmax, O^T += V^T . P^T
-    auto sm_pv_block = [&](const Tile &cur, const char *vbuf, f32x16_t &s0, f32x16_t &s1) {
+    // (PLAIN: a tile none of whose keys is masked, right after another such tile)
+    auto sm_pv_block = [&](const Tile &cur, const char *vbuf, f32x16_t &s0, f32x16_t &s1, auto plain_c) {
+        constexpr bool PLAIN = decltype(plain_c)::value;
         // (head_dim 256: the 64 registers of a whole tile's V^T fragments do not fit next to O^T and Q;
         // that form reads a fragment two MFMAs ahead of its own)
         constexpr bool VF_AHEAD = HD <= 128;
         Frag vf[VF_AHEAD ? 4 : 1][NDB];
         // element (blk, r) of this lane is tile-local key tk = tkc + 4*g with the compile-time
         // part tkc = 32*blk + 8*(r/4) + r%4.  keep <=> tk <= hi && (tk > wlo || tk < slim).
-        bool need_mask;
+        bool need_mask = false;
         const int wrow_lo = row0 + wave * 32, wrow_hi = wrow_lo + 31;
-        int hi, wlo = -1, slim = 0;      // per-lane bounds on tkc (4*g already subtracted)
-        if (MODE == MODE_VS && cur.gathered) {
+        int hi = 0, wlo = -1, slim = 0;  // per-lane bounds on tkc (4*g already subtracted)
+        if (PLAIN) {
+        } else if (MODE == MODE_VS && cur.gathered) {
             need_mask = cur.nvalid < BN;
             hi = cur.nvalid - 1 - 4 * g;
         } else {
@@ -787,7 +790,8 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         // but may differ by any amount across a jump.  A tile after a masked one counts as a jump too:
         // a row that saw none of the masked tile's keys (the window starts a tile later for the last
         // rows of a row block) still carries the maximum from before the jump.
-        const bool jump = (MODE == MODE_VS && cur.gathered) || cur.start != sm_prev_start + BN || sm_prev_masked;
+        const bool jump = PLAIN ? VSP && cur.start != sm_prev_start + BN :
+                          (MODE == MODE_VS && cur.gathered) || cur.start != sm_prev_start + BN || sm_prev_masked;
         sm_prev_start = cur.start;
         sm_prev_masked = need_mask;
         if (every_max || ((sm_steps++ & (MAX_PERIOD - 1)) == 0) || jump || __any(m_i == -INFINITY)) {
@@ -916,7 +920,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     [[maybe_unused]] int sp_entry = 0;
     auto step = [&](const int it, auto kind_c) {
         constexpr int KIND = decltype(kind_c)::value;
-        constexpr bool COMMON = KIND == 1, SPLIT = KIND == 2;
+        constexpr bool COMMON = KIND == 1 || (VSP && KIND == 3), SPLIT = KIND == 2, PLAIN = KIND == 3;
         __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wave's part of K(it) is in LDS
         __syncthreads();
         bool have_nxt;
@@ -927,7 +931,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             nxt.start = vs_entry;
             gt_nxt = 0;
             cur.gathered = 0; cur.nvalid = BN; cur.on_a = cur.on_b = 1; cur.split = 0;
-            copy_rows(cur, v_base, v_row, std::true_type{}, 0, lds_v, std::integral_constant<int, CROWS>{}, wave_wg);
+            copy_rows(cur, v_base, v_row, std::true_type{}, 0, lds_v, std::integral_constant<int, CROWS>{}, wave_wg, std::integral_constant<bool, PLAIN>{});
         } else if constexpr (SPLIT) {
             const int j = it - vs_nc;                      // this step's position in the leftover lists
             if (vs_merged) vs_pref = vs_only[half * VS_ONLY_MAX + min(j + 2, VS_ONLY_MAX - 1)];
@@ -937,7 +941,14 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             nxt.start = sp_entry;
             gt_nxt = 0;
             cur.gathered = 0; cur.nvalid = BN; cur.on_a = cur.on_b = 1; cur.split = 1;
-            copy_rows(cur, v_base, v_row, std::true_type{}, 0, lds_v + half * TILE_BYTES, std::integral_constant<int, 32>{}, wave);
+            copy_rows(cur, v_base, v_row, std::true_type{}, 0, lds_v + half * TILE_BYTES, std::integral_constant<int, 32>{}, wave, std::false_type{});
+        } else if constexpr (PLAIN) {
+            have_nxt = true;
+            cur.gathered = 0; cur.nvalid = BN; cur.on_a = cur.on_b = 1; cur.split = 0;
+            nxt = cur;
+            nxt.start = cur.start + BN;
+            gt_nxt = 0;
+            copy_rows(cur, v_base, v_row, std::true_type{}, 0, lds_v, std::integral_constant<int, CROWS>{}, wave_wg, std::true_type{});
         } else if constexpr (VSP) {
             // the merged list shares an LDS object with the V tiles: its entry is read while no copy
             // is in flight, so that the read never waits for one
@@ -964,17 +975,18 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
 
         // is this tile on the list of this wave's row block ?
         bool active = true;
-        if constexpr (COMMON || SPLIT) active = have_rows;
+        if constexpr (COMMON || SPLIT || PLAIN) active = have_rows;
         else if constexpr (VSP) active = have_rows && (half ? cur.on_b : cur.on_a);   // (split steps: on_a == on_b == own flag)
         else active = have_rows && tile_on_list<MODE>(p, m, cur.start);
         f32x16_t s0, s1;
         if (active) qk_block(lds_k, s0, s1);
         __builtin_amdgcn_s_waitcnt(0x0f70);          // vmcnt(0): this wave's part of V(it) is in LDS
         __syncthreads();
-        if constexpr (COMMON) copy_rows(nxt, k_base, k_row, std::false_type{}, 0, lds_k, std::integral_constant<int, CROWS>{}, wave_wg);
-        else if constexpr (SPLIT) copy_rows(nxt, k_base, k_row, std::false_type{}, 0, lds_k + half * TILE_BYTES, std::integral_constant<int, 32>{}, wave);
+        if constexpr (COMMON) copy_rows(nxt, k_base, k_row, std::false_type{}, 0, lds_k, std::integral_constant<int, CROWS>{}, wave_wg, std::integral_constant<bool, PLAIN>{});
+        else if constexpr (SPLIT) copy_rows(nxt, k_base, k_row, std::false_type{}, 0, lds_k + half * TILE_BYTES, std::integral_constant<int, 32>{}, wave, std::false_type{});
+        else if constexpr (PLAIN) copy_rows(nxt, k_base, k_row, std::false_type{}, 0, lds_k, std::integral_constant<int, CROWS>{}, wave_wg, std::true_type{});
         else if (have_nxt) copy_tile(nxt, k_base, k_row, std::false_type{}, gt_nxt, lds_k);
-        if (active) sm_pv_block(cur, lds_v, s0, s1);
+        if (active) sm_pv_block(cur, lds_v, s0, s1, std::integral_constant<bool, PLAIN>{});
         if constexpr (SPLIT) sp_entry = __builtin_amdgcn_readfirstlane(vs_pref);
         else if constexpr (VSP) vs_entry = __builtin_amdgcn_readfirstlane(vs_pref);
         cur = nxt;
@@ -985,6 +997,14 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     if constexpr (VSP) {
         // (a first step exists whenever there is a common entry; steps 0 .. vs_nc-2 have a common successor)
         const int common_end = min(vs_nc, it_end);
+        // the common entries ascend: all but the last few are tiles of which both row blocks see every key
+        if (vs_nc > 1) {
+            const int back = vs_nc - 1 - lane;
+            const unsigned long long late = __ballot(back >= 0 && vs_list(max(back, 0)) > mA * BM - BN);
+            const int nlate = __builtin_popcountll(late);
+            const int plain_end = nlate < 64 && __builtin_amdgcn_readfirstlane(vs_list(0)) >= 0 ? min(vs_nc - nlate, it_end) : 0;
+            for (; it + 1 < plain_end; ++it) step(it, std::integral_constant<int, 3>{});
+        }
         for (; it + 1 < common_end; ++it) step(it, std::integral_constant<int, 1>{});
         // block entries of their own that both row blocks still have (leftovers of the split, or the
         // whole lists when they were not split): these steps run in the SPLIT form
@@ -1005,6 +1025,23 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             const int j1 = it - vs_nc + 1;
             sp_entry = vs_merged ? __builtin_amdgcn_readfirstlane(vs_only[half * VS_ONLY_MAX + j1]) : sp_list[j1] * LIST_SCALE;
             for (; it + 1 < split_end; ++it) step(it, std::integral_constant<int, 2>{});
+        }
+    }
+    if constexpr (!VSP && HD <= 128) {
+        // tiles of which both row blocks see every key, after another such tile and before one that both visit or mask
+        const bool causal = MODE == MODE_DENSE || mA * BM >= p.dense_from;
+        const bool windowed = MODE == MODE_ASHAPE && mB * BM + BM - 1 < p.dense_from;
+        if (causal || windowed) {
+            int first = 1, shift = 0;                      // tile number of the first such tile; tile number - step
+            if (windowed) {
+                shift = pair_tile_start<MODE>(p, mA, mB, nblk, nblk) / BN - nblk;
+                first = max((mB * BM + BM - p.n_local + BN - 1) >> 6, shift + nblk) + 1;
+            }
+            const int lo = max(first - shift, it_begin + 1), hi = min(mA - 1 - shift, it_end - 1);
+            if (hi - lo >= (HD == 64 ? 8 : 1)) {
+                for (; it < lo; ++it) step(it, std::integral_constant<int, 0>{});
+                for (; it < hi; ++it) step(it, std::integral_constant<int, 3>{});
+            }
         }
     }
     for (; have_cur; ++it) step(it, std::integral_constant<int, 0>{});
