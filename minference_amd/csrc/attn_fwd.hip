@@ -82,9 +82,9 @@ constexpr int BN = 64;        // keys per tile
 // head_dim (template parameter HD of the kernel): 64, 128 or, for dense / A-shape / tri-shape only, 256
 constexpr int NTHREADS = 128; // 2 wavefronts per 64-row block, two row blocks per workgroup
 // Scheduling constants (measured on MI355X): K fragments are read QK_AHEAD k-steps ahead of their
-// MFMAs; VALU_PER_MFMA softmax instructions are placed behind each of the first twelve PV MFMAs.
+// MFMAs; VALU_PER_MFMA softmax instructions (five, or six with the row sums among them) are placed behind each of the first
+// twelve PV MFMAs.
 constexpr int QK_AHEAD = 2;
-constexpr int VALU_PER_MFMA = 6;
 #ifndef MAX_PERIOD
 #define MAX_PERIOD 8      // (a power of two) the row maximum is recomputed at least every MAX_PERIOD tiles
 #endif
@@ -709,6 +709,8 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
         // (head_dim 256: the 64 registers of a whole tile's V^T fragments do not fit next to O^T and Q;
         // that form reads a fragment two MFMAs ahead of its own)
         constexpr bool VF_AHEAD = HD <= 128;
+        constexpr bool SUM_LAST = HD == 128 || (HD == 64 && PLAIN);      // (see the row sums below)
+        constexpr int VALU_PER_MFMA = SUM_LAST ? 5 : 6;
         Frag vf[VF_AHEAD ? 4 : 1][NDB];
         // element (blk, r) of this lane is tile-local key tk = tkc + 4*g with the compile-time
         // part tkc = 32*blk + 8*(r/4) + r%4.  keep <=> tk <= hi && (tk > wlo || tk < slim).
@@ -833,7 +835,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
 #pragma unroll
             for (int r = 0; r < 8; ++r) pv[r] = __builtin_amdgcn_exp2f(fmaf(sx[8 * (q & 1) + r], sc_l2, -m_use));
             cvt8<T>(&pv[0], pfr[q]);
-            psum = pair_sum<T>(pfr[q], psum);
+            if constexpr (!SUM_LAST) psum = pair_sum<T>(pfr[q], psum);
         };
         probs(0);
         if (__any(alpha != 1.0f)) {
@@ -849,7 +851,6 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             probs(1);
             probs(2);
             probs(3);
-            l_i = (l_i * alpha) * alpha + psum;
             if constexpr (VF_AHEAD) {
 #pragma unroll
             for (int s = 0; s < 4; ++s)
@@ -888,6 +889,17 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             }
             }
         }
+        // The row sums of the whole tile in one go behind the last product: a v_dot2 between two MFMAs takes about 11
+        // cycles of the matrix pipe's (a product with the tile's share of fma, exp and cvt behind it 35 cycles, with half
+        // a v_dot2 as well 41; four in a row 12 in all).  A batch behind each key group's products took, dense, 16384
+        // tokens, 32 / 8 heads 1882 us against 1832 (on zeros 1365 : 1315); plain adds of the unpacked halves 2000.
+        // (Not at head_dim 256, 7 % slower, whose one wave has nothing else to run meanwhile, and not in the general form
+        // at 64: A-shape, window 512, 1 to 2 % slower.)
+        if constexpr (SUM_LAST) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) psum = pair_sum<T>(pfr[q], psum);
+        }
+        l_i = (l_i * alpha) * alpha + psum;
         __builtin_amdgcn_s_setprio(0);
     };
 
@@ -1027,7 +1039,8 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
             for (; it + 1 < split_end; ++it) step(it, std::integral_constant<int, 2>{});
         }
     }
-    if constexpr (!VSP && HD <= 128) {
+    // (not in the segments of 64-wide heads: tri-shape, 24000 tokens, 128 dense rows, 117 -> 119 us)
+    if constexpr (!VSP && (HD == 128 || (HD == 64 && !CUT))) {
         // tiles of which both row blocks see every key, after another such tile and before one that both visit or mask
         const bool causal = MODE == MODE_DENSE || mA * BM >= p.dense_from;
         const bool windowed = MODE == MODE_ASHAPE && mB * BM + BM - 1 < p.dense_from;
