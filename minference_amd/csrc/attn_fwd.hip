@@ -1162,10 +1162,14 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
 // fp32 range whatever a segment's (lazily raised) maximum was.  A segment is left out only where its row sum
 // is the zero of an unused or fully masked one, by bit pattern: a NaN among the keys makes the row sum NaN,
 // and the row is to be NaN, as a whole walk leaves it.  Latency-bound and small: it reads what the
-// segments wrote (66 KB each at head_dim 128, from L2) and writes the rows once.  The statistics of eight segments
-// and the sums of four are loaded together: one segment after the other, each was two round trips to L2.  Tri-shape,
-// head_dim 64: one bf16 head of 5086 tokens, whole call 26.1 -> 23.2 us; 16 fp16 heads of 24000 131.5 -> 129.5.
-template <int HD>
+// segments wrote (66 KB each at head_dim 128, from L2) and writes the rows once.  The statistics of all segments (up
+// to 16) are loaded together and kept, then the sums of UP of them: two round trips to L2 up to UP segments, where
+// statistics by eight, then statistics again and sums by four took eight for nine segments.  Vertical-slash, one head
+// of 4096 tokens, 500 columns and 700 slashes, fp16, index given 27.2 -> 25.5 us; dense, one head 8000 tokens
+// 35.6 -> 34.3.  Up to four segments, where the folds of many pairs fill the chip, they take the registers of four
+// (with those of eight, 8 / 2 heads 8000 tokens, dense 149 -> 150).
+constexpr int MERGE_FEW = 4, MERGE_HELD = 16;
+template <int HD, bool FEW>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     constexpr int NDB = HD / 32, ROW_BYTES = HD * 2, NCH = ROW_BYTES / 16;
     __shared__ __attribute__((aligned(16))) char lds_o[32 * ROW_BYTES];
@@ -1187,15 +1191,24 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     // (a pair that starts past the sequence was not walked at all)
     const int nseg = (p.split_first + pair) * 2 * BM < seqlen ? p.nseg : 0;
     auto stat = [&](int s) { return *(reinterpret_cast<const float2 *>(slots + (long long)s * SplitSlot<HD>::BYTES + SplitSlot<HD>::ACC) + part * 64 + lane); };
+    constexpr int HELD = FEW ? MERGE_FEW : MERGE_HELD;
+    float2 held[HELD];
     float top = -INFINITY;
-    for (int s0 = 0; s0 < nseg; s0 += 8) {
-        float2 ml[8];
+    auto look = [&](const float2 &ml) {
+        const bool number = (__float_as_uint(ml.y) & 0x7fffffffu) <= 0x7f800000u;
+        if (__float_as_uint(ml.y) != 0 && number) top = fmaxf(top, ml.x + __builtin_amdgcn_logf(ml.y));
+    };
+    if (nseg <= HELD) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) ml[u] = stat(min(s0 + u, nseg - 1));
+        for (int u = 0; u < HELD; ++u) held[u] = u < nseg ? stat(u) : make_float2(-INFINITY, 0.f);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const bool number = (__float_as_uint(ml[u].y) & 0x7fffffffu) <= 0x7f800000u;
-            if (__float_as_uint(ml[u].y) != 0 && number) top = fmaxf(top, ml[u].x + __builtin_amdgcn_logf(ml[u].y));
+        for (int u = 0; u < HELD; ++u) look(held[u]);
+    } else {
+        for (int s0 = 0; s0 < nseg; s0 += HELD) {
+#pragma unroll
+            for (int u = 0; u < HELD; ++u) held[u] = stat(min(s0 + u, nseg - 1));
+#pragma unroll
+            for (int u = 0; u < HELD; ++u) look(held[u]);
         }
     }
     const bool live = row0 + l32 < seqlen;
@@ -1205,36 +1218,32 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
     for (int i = 0; i < (NDB > 4 ? 2 : 1); ++i)
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) acc[i][rq] = make_float4(0.f, 0.f, 0.f, 0.f);
-    constexpr int UP = NDB > 4 ? 2 : 4, NI = NDB > 4 ? 2 : 1;
-    for (int s0 = 0; s0 < nseg; s0 += UP) {
-        float2 ml[UP];
+    constexpr int UP = (FEW ? 4 : 8) / (NDB > 4 ? 2 : 1), NI = NDB > 4 ? 2 : 1;
+    auto fold = [&](const float2 (&ml)[UP], int s0) {
         bool any[UP];
-#pragma unroll
-        for (int u = 0; u < UP; ++u) ml[u] = stat(min(s0 + u, nseg - 1));
         bool some = false;
 #pragma unroll
         for (int u = 0; u < UP; ++u) some |= any[u] = s0 + u < nseg && __any(__float_as_uint(ml[u].y) != 0);
-        if (!some) continue;
-        // an unused slot holds nothing: in its place the one before is read again, for no use
+        if (!some) return;
+        // (an unused slot holds nothing and is not read)
         float4 x[UP][NI][4];
-        int from = s0;
 #pragma unroll
-        for (int u = 0; u < UP; ++u) {
-            if (any[u]) from = s0 + u;
+        for (int u = 0; u < UP; ++u)
+            if (any[u])
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int db = wave + 4 * i;
-                if (db < NDB) {
-                    const char *src = slots + (long long)from * SplitSlot<HD>::BYTES + ((part * NDB + db) * 4 * 64 + lane) * 16;
+                for (int i = 0; i < NI; ++i) {
+                    const int db = wave + 4 * i;
+                    if (db < NDB) {
+                        const char *src = slots + (long long)(s0 + u) * SplitSlot<HD>::BYTES + ((part * NDB + db) * 4 * 64 + lane) * 16;
 #pragma unroll
-                    for (int rq = 0; rq < 4; ++rq) x[u][i][rq] = *reinterpret_cast<const float4 *>(src + rq * 1024);
+                        for (int rq = 0; rq < 4; ++rq) x[u][i][rq] = *reinterpret_cast<const float4 *>(src + rq * 1024);
+                    }
                 }
-            }
-        }
 #pragma unroll
         for (int u = 0; u < UP; ++u) {
-            const float w = any[u] && __float_as_uint(ml[u].y) != 0 ? __builtin_amdgcn_exp2f(ml[u].x - top) : 0.f;
-            l_tot = any[u] ? fmaf(w, ml[u].y, l_tot) : l_tot;
+            if (!any[u]) continue;
+            const float w = __float_as_uint(ml[u].y) != 0 ? __builtin_amdgcn_exp2f(ml[u].x - top) : 0.f;
+            l_tot = fmaf(w, ml[u].y, l_tot);
 #pragma unroll
             for (int i = 0; i < NI; ++i)
                 if (wave + 4 * i < NDB)
@@ -1242,9 +1251,24 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnParams p) {
                     for (int rq = 0; rq < 4; ++rq) {
                         float4 &o = acc[i][rq];
                         const float4 v = x[u][i][rq];
-                        o.x = any[u] ? fmaf(w, v.x, o.x) : o.x; o.y = any[u] ? fmaf(w, v.y, o.y) : o.y;
-                        o.z = any[u] ? fmaf(w, v.z, o.z) : o.z; o.w = any[u] ? fmaf(w, v.w, o.w) : o.w;
+                        o.x = fmaf(w, v.x, o.x); o.y = fmaf(w, v.y, o.y); o.z = fmaf(w, v.z, o.z); o.w = fmaf(w, v.w, o.w);
                     }
+        }
+    };
+    if (nseg <= HELD) {
+#pragma unroll
+        for (int s0 = 0; s0 < HELD; s0 += UP) {
+            float2 ml[UP];
+#pragma unroll
+            for (int u = 0; u < UP; ++u) ml[u] = held[s0 + u];
+            if (s0 < nseg) fold(ml, s0);
+        }
+    } else {
+        for (int s0 = 0; s0 < nseg; s0 += UP) {
+            float2 ml[UP];
+#pragma unroll
+            for (int u = 0; u < UP; ++u) ml[u] = stat(min(s0 + u, nseg - 1));
+            fold(ml, s0);
         }
     }
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
@@ -1481,7 +1505,8 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
     const int status = minf_launch_status();
     if (status != MINF_OK || p.nseg == 1) return status;
     const unsigned merge_wgs = (unsigned)(4ll * split_pairs * p.batch * (p.head_list ? p.index_heads : p.hq));
-    hipLaunchKernelGGL((attn_merge_kernel<HD>), dim3(merge_wgs), dim3(256), 0, st, p);
+    if (p.nseg <= MERGE_FEW) hipLaunchKernelGGL((attn_merge_kernel<HD, true>), dim3(merge_wgs), dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((attn_merge_kernel<HD, false>), dim3(merge_wgs), dim3(256), 0, st, p);
     return minf_launch_status();
 }
 

@@ -30,6 +30,29 @@ def test_split_walks_match_the_oracle(gpu, n, hq, hk, b, d, dtype):
               O.vertical_slash_sparse_attention(q, ke, ve, v_idx.cpu(), s_idx.cpu()), "vertical-slash")
 
 
+@pytest.mark.parametrize("op,n,segments", [("ashape", 1024, 2), ("ashape", 2048, 4), ("ashape", 2100, 5), ("ashape", 4000, 8),
+                                           ("ashape", 4200, 9), ("ashape", 8192, 16), ("dense", 16000, 6), ("tri", 9000, 18)])
+def test_folds_of_every_number_of_segments(gpu, op, n, segments):
+    """One head, walks of every earlier key (tri-shape: those of the last 128 rows): the fold takes the registers of four
+    segments, holds the statistics of up to sixteen, adds eight at once.  Every such row against fp32."""
+    import minference_amd as M
+    from minference_amd import _lib
+    q, k, v = (t.to(gpu) for t in make(1, 1, 1, n, n, torch.bfloat16))
+    last = 128 if op == "tri" else 0
+    sizes = {"ashape": (_lib.MINF_OP_ASHAPE, 0, n, 0), "dense": (_lib.MINF_OP_DENSE, 0, 0, 0), "tri": (_lib.MINF_OP_ASHAPE, 64, 128, last)}[op]
+    nbytes = _lib.load().minf_attn_workspace_bytes(M.ops._Call(q, k, v).ref, *sizes)
+    pairs = (n + 127) // 128 - ((n - last) // 128 if last else 0)
+    assert nbytes == pairs * segments * (4 * 128 * 32 * 4 + 4 * 64 * 8)
+    out = M.tri_shape_forward(q, k, v, 64, 128, last) if last else M.dense_causal_attention(q, k, v) if op == "dense" else \
+        M.streaming_forward(q, k, v, 0, n)
+    qf, kf, vf = (t[0, 0].float() for t in (q, k, v))
+    for r0 in range(n - last if last else 0, n, 1000):
+        rows = torch.arange(r0, min(r0 + 1000, n), device=gpu)
+        p = (qf[rows] @ kf.T) * 128 ** -0.5
+        p.masked_fill_(torch.arange(n, device=gpu)[None] > rows[:, None], float("-inf"))
+        check(out[0, 0, rows], (torch.softmax(p, -1) @ vf).cpu(), f"{n} rows {r0}")
+
+
 @pytest.mark.parametrize("n,hq,hk,b", [(2111, 12, 3, 1), (4033, 4, 4, 2)])
 def test_half_full_launches_are_split_by_their_share(gpu, n, hq, hk, b):
     """More than 64 row-block pairs, too few to fill the chip: segments of 1.4 shares (lone last row block,
