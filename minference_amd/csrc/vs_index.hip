@@ -568,11 +568,16 @@ __global__ __launch_bounds__(256) void vs_index_bitmap_kernel(int32_t *__restric
     bm[w] = bits;
 }
 
-// (Two instantiations: the zero-filled form is bound by its stores and measures 3 % faster at 512K
-// tokens when the compiler is held to 64 registers; the payload-only form is bound by its chains of
-// dependent loads and loses more to the few spills that limit costs than it gains.)
-template <bool ZERO_FILL>
-__global__ __launch_bounds__(IDX_WAVES *MINF_WAVE, ZERO_FILL ? 8 : 1) void vs_index_fast_kernel(
+// Zero-filled rows of more than IDX_SHORT_ROW slashes (LONG) are bound by their stores: six workgroups per CU (see
+// index_build_tables), held to 64 registers, which measures 3 % faster at 512K tokens.  Shorter ones are bound by
+// their chains of dependent loads like the payload alone: every wave that 72 registers allow, no spills.  Us, as
+// the long rows run and so: 32 heads, 262144 tokens, 30 columns and 800 slashes 187 -> 156, 500 and 700 275 -> 226, 3500
+// and 100 637 -> 548; 131072 tokens, 1000 and 3000 295 -> 254; 4 heads 100000 tokens, 100 and 750 27.2 -> 23.5.
+// The line: 32 heads, 131072 tokens, 1000 columns and, uniform, 4000 slashes 322 -> 293, 4500 338 -> 339, 5000 357 ->
+// 363, 6096 411 -> 436; clustered ones as fast or faster up to 5600, 6096 410 -> 422.
+constexpr int IDX_SHORT_ROW = 4096;
+template <bool ZERO_FILL, bool LONG>
+__global__ __launch_bounds__(IDX_WAVES *MINF_WAVE, ZERO_FILL ? (LONG ? 8 : 7) : 1) void vs_index_fast_kernel(
     const int32_t *__restrict__ seqlens, const int32_t *__restrict__ vertical,
     const int32_t *__restrict__ slash, const int32_t *__restrict__ tables,
     int32_t *__restrict__ block_count, int32_t *__restrict__ block_offset,
@@ -867,21 +872,15 @@ static int index_build_tables(const int32_t *seqlens, const int32_t *vertical_id
         status = minf_launch_status();
         if (status != MINF_OK) return status;
     }
-    // With zero-filled outputs the row-block pass is bound by its stores, and 24 resident waves per CU
-    // write faster than 32 (6-9 % at 128K-512K tokens: fewer rows in flight, better DRAM locality); the
-    // payload-only form is bound by its chains of dependent loads and wants every wave it can get.
-    // Unused dynamic LDS is the occupancy limiter: 3 KB static + 24000 B -> 6 workgroups per CU.
-    const unsigned occupancy_lds = zero_fill ? 24000u : 0u;
-    if (zero_fill)
-        hipLaunchKernelGGL(vs_index_fast_kernel<true>, dim3((unsigned)nblk), dim3(IDX_WAVES * MINF_WAVE), occupancy_lds,
-                           stream, seqlens, vertical_idx, slash_idx, (const int32_t *)workspace,
-                           block_count, block_offset, column_count, column_index, heads, rows, nnz_v, nnz_s,
-                           error_flag, total);
-    else
-        hipLaunchKernelGGL(vs_index_fast_kernel<false>, dim3((unsigned)nblk), dim3(IDX_WAVES * MINF_WAVE), occupancy_lds,
-                           stream, seqlens, vertical_idx, slash_idx, (const int32_t *)workspace,
-                           block_count, block_offset, column_count, column_index, heads, rows, nnz_v, nnz_s,
-                           error_flag, total);
+    // Long zero-filled rows: 24 resident waves per CU write faster than 32 (6-9 % at 128K-512K tokens: fewer rows in
+    // flight, better DRAM locality).  Unused dynamic LDS is the occupancy limiter: 3 KB static + 24000 B -> 6
+    // workgroups per CU.
+    const bool long_rows = zero_fill && nnz_s > IDX_SHORT_ROW;
+    const unsigned occupancy_lds = long_rows ? 24000u : 0u;
+    auto *const kernel = long_rows ? vs_index_fast_kernel<true, true> : zero_fill ? vs_index_fast_kernel<true, false> : vs_index_fast_kernel<false, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(IDX_WAVES * MINF_WAVE), occupancy_lds, stream, seqlens, vertical_idx,
+                       slash_idx, (const int32_t *)workspace, block_count, block_offset, column_count, column_index, heads,
+                       rows, nnz_v, nnz_s, error_flag, total);
     return minf_launch_status();
 }
 

@@ -163,6 +163,13 @@ def test_lists_around_the_most_that_are_shared(gpu, ns):
     assert_same(run_gpu([n], v, s, n, gpu), O.vs_index_build([n], v, s, n))
 
 
+@pytest.mark.parametrize("ns", [4095, 4096, 4097])
+def test_zero_filled_rows_around_the_length_that_limits_the_waves(gpu, ns):
+    print(f"case zero-filled rows of {ns} slashes", flush=True)
+    v, s = gen.vs_index_inputs(3, 20001, 333, ns, seed=ns, force_v=4, force_s=64)
+    assert_same(run_gpu([20001], v, s, 20001, gpu), O.vs_index_build([20001], v, s, 20001))
+
+
 def test_hand_kat(gpu):
     V = np.array([[[0, 1, 2, 3, 100, 130, 700]]], np.int32)
     S = np.array([[[500, 70, 64, 3, 0]]], np.int32)
