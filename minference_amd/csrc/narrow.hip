@@ -3,22 +3,22 @@
 // The attention kernels compute on 16-bit operands with fp32 accumulation (the reference picks fp16 operands for
 // every input that is not bf16, pit_sparse_flash_attention_v2.py:175).  fp32 q/k/v become fp16 when the
 // largest |value| of the three lies in [2^-10, 32768], else bf16 (fp16 would overflow, or flush most of
-// the tensor).  The choice is made here, on the device: a first kernel leaves the largest |value| of each
-// of its workgroups, every workgroup of the second one folds those, converts its share and one of them
-// leaves the dtype code that the attention launches and the widening kernel read
-// (minf_qkvo.dtype_select).  Bound by bytes: q, k and v are read twice (the second time mostly from the
-// Infinity Cache) and written once at half the size.  The first kernel has four vectors of a thread under way
-// and reads a tensor that fills one stretch of memory by its vectors' numbers alone: with one load at a time,
-// placed by three divisions, it took 13.4 us for 3 x 16.8 MB (8192 tokens, 4 heads of 128), now 9.0 = 5.6 TB/s;
-// the second one 13.4 = 5.7 TB/s with one step or four under way.  With the choice read back by the host
-// (three reductions, a synchronisation, three conversions) the GPU idled about 60 us per call.
+// the tensor).  The choice is made here, on the device: a first kernel converts to fp16 and leaves the largest |value|
+// of each of its workgroups, every workgroup of the second one folds those, one of them leaves the dtype code
+// that the attention launches and the widening kernel read (minf_qkvo.dtype_select), and where the code is bf16 they
+// convert once more, over what the first kernel wrote.  Bound by bytes: q, k and v are read and written once.
+// With a pass for the largest |value| alone before the conversion (8192 tokens, 4 heads of 128, 3 x 16.8 MB)
+// the two took 9.0 + 13.4 us, now 13.6 + 3.7; 32768 tokens, 16 heads 365 -> 223, 65536 tokens, 32 / 8 heads 744 -> 446,
+// 5.4 TB/s.  Tensors that do need bf16 pay for the second conversion: 366 -> 450 and 743 -> 1008.
+// With the choice read back by the host (three reductions, a synchronisation, three conversions) the GPU
+// idled about 60 us per call.
 #include "minf_common.h"
 
 namespace {
 
 constexpr int NARROW_THREADS = 256;
-constexpr int UNDER_WAY = 4;     // vectors a thread of the first kernel has under way
-constexpr int NARROW_PARTIALS = MINF_NARROW_WORKSPACE_INTS - 1;      // amax workgroups, a third per tensor
+constexpr int UNDER_WAY = 2;     // steps of 8 elements a thread has under way
+constexpr int NARROW_PARTIALS = MINF_NARROW_WORKSPACE_INTS - 1;      // workgroups of a launch, a third per tensor
 constexpr int NARROW_WGS = NARROW_PARTIALS / 3;
 static_assert(NARROW_WGS * 3 == NARROW_PARTIALS, "the same number of workgroups for each tensor");
 
@@ -28,13 +28,12 @@ struct NarrowTensor {
     long long stride[3];         // elements: batch, head, token
     long long rows;              // batch * heads * n
     int heads;
-    int dense;                   // the tensor fills one stretch of memory
     FastDiv by_n, by_heads;
 };
 struct NarrowParams {
     NarrowTensor t[3];
     int dim;
-    FastDiv by_dim, by_dim_out;  // vectors per row, in / out
+    FastDiv by_dim_out;          // vectors of 8 elements per output row
     int *ws;                     // [0]: the dtype code, then the partial maxima (bit patterns)
 };
 
@@ -60,53 +59,51 @@ __device__ __forceinline__ unsigned wg_max(unsigned m, unsigned (&part)[NARROW_T
     return m;
 }
 
-template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_amax_kernel(const NarrowParams p) {
-    __shared__ unsigned part[NARROW_THREADS / 64];
-    const NarrowTensor t = p.t[blockIdx.y];
-    const I total = (I)t.rows * p.by_dim.d, step = (I)NARROW_WGS * NARROW_THREADS;
+// One pass over a workgroup's share of a tensor, 8 output elements per thread and step, converted to T and written;
+// the largest bit pattern of |x| read.
+template <typename T, typename I> __device__ __forceinline__ unsigned convert_share(const NarrowParams &p, const NarrowTensor &t) {
+    const I total = (I)t.rows * p.by_dim_out.d, step = (I)NARROW_WGS * NARROW_THREADS;
     unsigned m = 0;
     for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += UNDER_WAY * step) {
-        uint4 x[UNDER_WAY];
+        float4 x[UNDER_WAY][2];
+        I at[UNDER_WAY];
 #pragma unroll
         for (int u = 0; u < UNDER_WAY; ++u) {
-            const I at = min(i + u * step, total - 1);     // (the last vector again, past the end)
+            at[u] = min(i + u * step, total - 1);      // (the last vector again, past the end)
             int d;
-            x[u] = *reinterpret_cast<const uint4 *>(t.dense ? t.in + 4 * (long long)at : vector_ptr<I>(t, p.by_dim, 4, at, d));
+            const float *src = vector_ptr<I>(t, p.by_dim_out, 8, at[u], d);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) x[u][h] = d + 4 * h < p.dim ? *reinterpret_cast<const float4 *>(src + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
-        for (int u = 0; u < UNDER_WAY; ++u)
-            m = max(max(max(m, x[u].x & 0x7fffffffu), x[u].y & 0x7fffffffu), max(x[u].z & 0x7fffffffu, x[u].w & 0x7fffffffu));
+        for (int u = 0; u < UNDER_WAY; ++u) {
+            const float v[8] = {x[u][0].x, x[u][0].y, x[u][0].z, x[u][0].w, x[u][1].x, x[u][1].y, x[u][1].z, x[u][1].w};
+            union { T e[8]; uint4 u4; } o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                o.e[e] = (T)v[e];
+                m = max(m, __float_as_uint(v[e]) & 0x7fffffffu);
+            }
+            *reinterpret_cast<uint4 *>(t.out + (long long)at[u] * 16) = o.u4;
+        }
     }
-    m = wg_max(m, part);
-    if (threadIdx.x == 0) p.ws[1 + blockIdx.y * NARROW_WGS + blockIdx.x] = (int)m;
+    return m;
 }
 
 template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_kernel(const NarrowParams p) {
+    __shared__ unsigned part[NARROW_THREADS / 64];
+    const unsigned m = wg_max(convert_share<_Float16, I>(p, p.t[blockIdx.y]), part);
+    if (threadIdx.x == 0) p.ws[1 + blockIdx.y * NARROW_WGS + blockIdx.x] = (int)m;
+}
+
+template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_choose_kernel(const NarrowParams p) {
     __shared__ unsigned part[NARROW_THREADS / 64];
     unsigned m = 0;
     for (int i = (int)threadIdx.x; i < NARROW_PARTIALS; i += NARROW_THREADS) m = max(m, (unsigned)p.ws[1 + i]);
     m = wg_max(m, part);
     const bool f16 = m >= __float_as_uint(0x1p-10f) && m <= __float_as_uint(32768.0f);
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.ws[0] = f16 ? MINF_F16 : MINF_BF16;
-    const NarrowTensor t = p.t[blockIdx.y];
-    const I total = (I)t.rows * p.by_dim_out.d;                          // 8 output elements per thread and step
-    for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += (I)gridDim.x * NARROW_THREADS) {
-        int d;
-        const float *src = vector_ptr<I>(t, p.by_dim_out, 8, i, d);
-        float4 x[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) x[h] = d + 4 * h < p.dim ? *reinterpret_cast<const float4 *>(src + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float v[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
-        union { _Float16 h[8]; __bf16 b[8]; uint4 u; } o;
-        if (f16) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o.h[e] = (_Float16)v[e];
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o.b[e] = (__bf16)v[e];
-        }
-        *reinterpret_cast<uint4 *>(t.out + (long long)i * 16) = o.u;
-    }
+    if (!f16) convert_share<__bf16, I>(p, p.t[blockIdx.y]);
 }
 
 __global__ __launch_bounds__(NARROW_THREADS) void widen_kernel(const char *__restrict__ in, float *__restrict__ out, long long rows,
@@ -124,22 +121,6 @@ __global__ __launch_bounds__(NARROW_THREADS) void widen_kernel(const char *__res
         else o = make_float4((float)x.b[0], (float)x.b[1], (float)x.b[2], (float)x.b[3]);
         *reinterpret_cast<float4 *>(out + i * 4) = o;
     }
-}
-
-// does the tensor fill one stretch of memory, whatever the order of its dimensions?
-bool fills_memory(const NarrowTensor &t, int batch, int n, int dim) {
-    const long long size[3] = {batch, t.heads, n};
-    bool done[3] = {false, false, false};
-    long long extent = dim;
-    for (int round = 0; round < 3; ++round) {
-        int next = -1;
-        for (int i = 0; i < 3; ++i)
-            if (!done[i] && (size[i] == 1 || t.stride[i] == extent)) next = i;
-        if (next < 0) return false;
-        done[next] = true;
-        extent *= size[next];
-    }
-    return true;
 }
 
 unsigned narrow_grid(long long vectors) {
@@ -170,24 +151,21 @@ extern "C" int minf_narrow_qkv(const minf_qkvo *t, int dim_in, void *q16, void *
         p.t[i].rows = (long long)t->batch * p.t[i].heads * t->n;
         p.t[i].by_n = fast_div((unsigned)t->n);
         p.t[i].by_heads = fast_div((unsigned)p.t[i].heads);
-        p.t[i].dense = fills_memory(p.t[i], t->batch, t->n, dim_in);
     }
     p.dim = dim_in;
-    p.by_dim = fast_div((unsigned)dim_in / 4u);
     p.by_dim_out = fast_div((unsigned)t->head_dim / 8u);
     p.ws = workspace;
     hipStream_t st = (hipStream_t)stream;
-    // (multiplications place numbers below 2^31)
+    // (multiplications place numbers below 2^31, and so must the steps past the end be)
     const long long most = p.t[0].rows > p.t[1].rows ? p.t[0].rows : p.t[1].rows;
-    const long long widest = p.by_dim.d > p.by_dim_out.d ? p.by_dim.d : p.by_dim_out.d;
-    const bool small = most * widest < 0x7fffffffLL;
-    if (small) hipLaunchKernelGGL(narrow_amax_kernel<unsigned>, dim3(NARROW_WGS, 3), dim3(NARROW_THREADS), 0, st, p);
-    else hipLaunchKernelGGL(narrow_amax_kernel<unsigned long long>, dim3(NARROW_WGS, 3), dim3(NARROW_THREADS), 0, st, p);
+    const bool small = most * p.by_dim_out.d < 0x7fffffffLL - 2ll * UNDER_WAY * NARROW_WGS * NARROW_THREADS;
+    const dim3 grid(NARROW_WGS, 3), block(NARROW_THREADS);
+    if (small) hipLaunchKernelGGL(narrow_kernel<unsigned>, grid, block, 0, st, p);
+    else hipLaunchKernelGGL(narrow_kernel<unsigned long long>, grid, block, 0, st, p);
     const int status = minf_launch_status();
     if (status != MINF_OK) return status;
-    const dim3 grid(narrow_grid(p.t[0].rows * p.by_dim_out.d), 3);
-    if (small) hipLaunchKernelGGL(narrow_kernel<unsigned>, grid, dim3(NARROW_THREADS), 0, st, p);
-    else hipLaunchKernelGGL(narrow_kernel<unsigned long long>, grid, dim3(NARROW_THREADS), 0, st, p);
+    if (small) hipLaunchKernelGGL(narrow_choose_kernel<unsigned>, grid, block, 0, st, p);
+    else hipLaunchKernelGGL(narrow_choose_kernel<unsigned long long>, grid, block, 0, st, p);
     return minf_launch_status();
 }
 

@@ -46,10 +46,10 @@ def test_strided_unaligned_and_caller_owned_tensors(gpu):
                        M.dense_causal_attention(q.half(), k[:, :1].expand(2, 2, 400, 128).half(), v.half()).float())
 
 
-@pytest.mark.parametrize("n", [1024, 1025, 3071, 4096, 4097])
+@pytest.mark.parametrize("n", [1024, 1025, 2048, 2049, 3071, 4096, 4097])
 @pytest.mark.parametrize("layout", ["rows", "tokens first", "gaps", "one row for all heads"])
 def test_the_largest_value_is_found_wherever_it_lies(gpu, n, layout):
-    """2 heads of 128 around the 65536 vectors that all threads read in one step and the 262144 of four; tensors that fill
+    """2 heads of 128 around the 65536 vectors of 8 that all threads read in one step and the 131072 of two; tensors that fill
     one stretch of memory and ones that do not; the one value that asks for bf16 first, last and in between."""
     import minference_amd as M
     g = torch.Generator(device=gpu).manual_seed(n)
