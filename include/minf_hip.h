@@ -320,6 +320,17 @@ int minf_vs_estimate_heads(const void *q, const void *k, const int64_t *q_stride
                            size_t workspace_bytes, void *stream);
 
 /*
+ * The whole vertical_and_slash layer (minference/modules/minference_forward.py:599-614) in one call: minf_vs_estimate,
+ * minf_topk_indices_pair, minf_vs_index_build_full_ws and minf_vs_attn_fwd, in this order on `stream`.  nnz_v, nnz_s:
+ * sizes of the selections, 1 .. n; the other arguments as in minf_vs_estimate.  t->seqlens and t->head_list null, dtype
+ * bf16 or fp16, t->workspace unused.  workspace: minf_vs_prefill_workspace_bytes() bytes, 16-byte aligned (0 for
+ * arguments the call refuses).
+ */
+size_t minf_vs_prefill_workspace_bytes(const minf_qkvo *t, int nnz_v, int nnz_s);
+int minf_vs_prefill(const minf_qkvo *t, int nnz_v, int nnz_s, int last_q, int force_vertical, int force_slash,
+                    int rounding, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Indices of the k largest entries of each fp32 row, written in ASCENDING
  * INDEX order (ties at the k-th value: lowest index first).  Replaces
  * torch.topk(...).indices followed by the sort in the op wrapper (reference

@@ -41,6 +41,8 @@ SIGNATURES = {
                          + [c_ptr, c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
     "minf_vs_estimate_heads": (c_int, [c_ptr, c_ptr, c_ptr, c_ptr] + [c_int] * 6 + [c_f32] + [c_int] * 4 + [c_ptr, c_int]
                                + [c_ptr, c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
+    "minf_vs_prefill_workspace_bytes": (ctypes.c_size_t, [c_ptr, c_int, c_int]),
+    "minf_vs_prefill": (c_int, [c_ptr] + [c_int] * 6 + [c_ptr, ctypes.c_size_t, c_ptr]),
     "minf_topk_indices_pair_ragged": (c_int, [c_ptr, c_ptr, c_int, c_ptr, c_i64, c_int, c_int, c_int] * 2
                                       + [c_int, c_int, c_i64, c_ptr]),
     "minf_bs_block_index_heads": (c_int, [c_ptr, c_ptr, c_ptr, c_ptr] + [c_int] * 8 + [c_ptr, c_int]

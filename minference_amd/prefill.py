@@ -18,10 +18,11 @@ from collections import OrderedDict
 
 import torch
 
-from .estimate import estimate_vertical_slash
+from . import _lib
+from .estimate import FORCE_SLASH, FORCE_VERTICAL, LAST_Q, estimate_vertical_slash
 from .index import _build as _build_index
 from .index import convert_vertical_slash_indexes
-from .ops import (block_sparse_attention, dense_causal_attention, streaming_forward, tri_shape_forward,
+from .ops import (_Call, block_sparse_attention, dense_causal_attention, streaming_forward, tri_shape_forward,
                   vertical_slash_attention_from_index, vertical_slash_sparse_attention)
 
 DEFAULT_PATTERN = ("vertical_and_slash", 1000, 6096, 1)   # minference_forward.py:621
@@ -31,6 +32,19 @@ def vertical_slash_prefill(q, k, v, vertical_size=1000, slash_size=6096, out=Non
     """estimate -> top-k -> index build -> mixed sparse attention for all heads of ``q``
     (``vertical_and_slash_kernel``, minference_forward.py:599-614)."""
     N = q.shape[2]
+    if q.dtype in (torch.bfloat16, torch.float16) and q.numel() and k.numel():
+        # one call and one workspace for all four stages
+        c = _Call(q, k, v, out=out)
+        dev = c.q.device
+        nv, ns = min(N, max(int(vertical_size), 30)), min(N, max(int(slash_size), 50))       # (:600)
+        lib = _lib.load()
+        nbytes = lib.minf_vs_prefill_workspace_bytes(c.ref, nv, ns)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        with torch.cuda.device(dev):
+            st = lib.minf_vs_prefill(c.ref, nv, ns, LAST_Q, FORCE_VERTICAL, FORCE_SLASH, _lib.MINF_ROUND_INPUT_DTYPE,
+                                     ws.data_ptr(), nbytes, _lib.stream_ptr(dev))
+        _lib.check(st, "minf_vs_prefill")
+        return c.result()
     v_idx, s_idx = estimate_vertical_slash(q, k, vertical_size, slash_size)
     bc, bo, cc, ci = _build_index(None, v_idx, s_idx, N, zero_fill=False)
     return vertical_slash_attention_from_index(q, k, v, bc, bo, cc, ci, out=out)
@@ -153,9 +167,8 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
     * stream_llm heads: one launch per distinct (n_init, n_local).
 
     The reference runs one operator call per head here (minference_forward.py:657-667)."""
-    from . import _lib
-    from .estimate import FORCE_SLASH, FORCE_VERTICAL, LAST_Q, reference_rounding_for
-    from .ops import _Call, _streaming_scale
+    from .estimate import reference_rounding_for
+    from .ops import _streaming_scale
     B, H, N, D = query_states.shape
     rounded = reference_rounding_for(query_states.dtype)     # the reference's rounding points on 16-bit inputs
     dev = query_states.device

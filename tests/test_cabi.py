@@ -78,6 +78,19 @@ def test_argument_validation_needs_no_gpu(lib):
     t.q_stride[2] = 100
     assert lib.minf_dense_attn_fwd(ctypes.byref(t), None) == -3          # row pitch not 16-byte aligned
     assert lib.minf_vs_estimate_workspace_bytes(1, 32, 131072) > 0
+    t.q_stride[2] = 128
+    ref = ctypes.byref(t)                                                # 4 / 2 heads, 64 tokens
+    need = lib.minf_vs_prefill_workspace_bytes(ref, 30, 50)
+    assert need > 0 and lib.minf_vs_prefill_workspace_bytes(ref, 65, 50) == 0
+    assert lib.minf_vs_prefill(ref, 65, 50, 64, 30, 100, 1, 256, 1 << 30, None) == -1       # more columns than tokens
+    assert lib.minf_vs_prefill(ref, 30, 50, 64, 30, 100, 1, 256, need - 1, None) == -4
+    assert lib.minf_vs_prefill(ref, 30, 50, 64, 30, 100, 1, 8, need, None) == -3
+    t.seqlens = 16
+    assert lib.minf_vs_prefill(ref, 30, 50, 64, 30, 100, 1, 256, need, None) == -1
+    t.seqlens = None
+    t.dtype = _lib.MINF_16BIT_SELECT
+    assert lib.minf_vs_prefill(ref, 30, 50, 64, 30, 100, 1, 256, need, None) == -2
+    t.dtype = 0
     assert lib.minf_vs_estimate_workspace_bytes(0, 32, 131072) == 0
 
 
