@@ -19,6 +19,8 @@
 // negative zeros: they are sums of probabilities).  With reverse_base >= 0 the value written is reverse_base - index
 // (slash: diagonal offset = N-1-j, so ascending j gives descending offsets).
 #include "minf_common.h"
+#include "vs_index_tables.h"
+#include "vs_stages.h"
 #include <type_traits>
 
 namespace {
@@ -493,7 +495,6 @@ struct TopkShared {
     unsigned bins[4];                        // bin counts of waves 0..3
     unsigned prefix, need, count;            // the threshold's digits so far, rank inside the bucket, its size
     unsigned listed;
-    int last;
     int wave_gt[TK_WAVES], wave_eq[TK_WAVES];
 };
 template <int COPIES>
@@ -599,21 +600,17 @@ __device__ __forceinline__ void topk_threshold(const unsigned (&key)[ITEMS], int
 // now: 2048 entries 18.3 / 6.4, 4096 31.5 / 7.0, 5000 11.9 / 9.2, 8192 13.2 / 10.4, 16001 26.3 / 13.8; 32768
 // in 32 registers per thread 25.6 / 26.0 (and 64 spill), so longer rows are swept.  Rows of 2048 entries:
 // 512 of them 18.7 / 8.1, 1024 18.8 / 13.9, 2048 21.4 / 37 -- hence TK_FEW_ROWS.
-template <int ITEMS>
-__global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem p0, const TopkProblem p1, int n) {
-    const TopkProblem &pr = blockIdx.y == 0 ? p0 : p1;
-    const int kmax = pr.k, reverse_base = pr.reverse_base;
-    const int k = pr.k_rows ? max(1, min(pr.k_rows[blockIdx.x], kmax)) : kmax;
+// load(i): entry i of the row; emit(place, i): entry i is selected, as number `place` in ascending index order.
+template <int ITEMS, typename Load, typename Emit>
+__device__ __forceinline__ void topk_regs_select(int n, int k, Load load, Emit emit) {
     constexpr int COPIES = ITEMS > 4 ? 32 : 8;       // copies of the histogram: the fewer keys, the fewer collisions
     __shared__ unsigned hist[256 * COPIES];
     __shared__ __attribute__((aligned(16))) unsigned list[TK_LIST + 4];
     __shared__ TopkShared sh;
-    const float *__restrict__ x = pr.scores + (long long)blockIdx.x * pr.row_stride;
-    int32_t *__restrict__ o = pr.out + (long long)blockIdx.x * pr.out_stride;
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (k >= n) {                    // everything is selected
-        for (int i = tid; i < n; i += TK_THREADS) o[i] = reverse_base >= 0 ? reverse_base - i : i;
+        for (int i = tid; i < n; i += TK_THREADS) emit(i, i);
         return;
     }
     const int begin = wave * 64 * ITEMS;
@@ -621,7 +618,7 @@ __global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
         const int i = begin + 64 * j + lane;
-        key[j] = i < n ? order_key(x[i]) : 0u;               // padding sorts below every score
+        key[j] = i < n ? order_key(load(i)) : 0u;            // padding sorts below every score
     }
     unsigned T, need;
     topk_threshold<ITEMS, COPIES>(key, n, k, begin, hist, nullptr, list, sh, T, need);
@@ -644,21 +641,58 @@ __global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem
         const uint64_t mg = __ballot(gt), me = __ballot(eq);
         if (mg | me) {                                        // (wave-uniform)
             const int e_here = eq_before + __builtin_popcountll(me & lt);
-            if (gt || (eq && e_here < r)) {
-                const int pos = gt_before + __builtin_popcountll(mg & lt) + min(e_here, r);
-                const int val = reverse_base >= 0 ? reverse_base - i : i;
-                o[pos] = val;
-                if (pos == k - 1) sh.last = val;
-            }
+            if (gt || (eq && e_here < r)) emit(gt_before + __builtin_popcountll(mg & lt) + min(e_here, r), i);
             gt_before += __builtin_popcountll(mg);
             eq_before += __builtin_popcountll(me);
         }
     }
-    if (k < kmax && pr.pad_mode) {                            // (workgroup-uniform)
+}
+
+template <int ITEMS>
+__global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem p0, const TopkProblem p1, int n) {
+    const TopkProblem &pr = blockIdx.y == 0 ? p0 : p1;
+    __shared__ int last;
+    const int kmax = pr.k, reverse_base = pr.reverse_base;
+    const int k = pr.k_rows ? max(1, min(pr.k_rows[blockIdx.x], kmax)) : kmax;
+    const float *__restrict__ x = pr.scores + (long long)blockIdx.x * pr.row_stride;
+    int32_t *__restrict__ o = pr.out + (long long)blockIdx.x * pr.out_stride;
+    topk_regs_select<ITEMS>(n, k, [&](int i) { return x[i]; }, [&](int place, int i) {
+        const int val = reverse_base >= 0 ? reverse_base - i : i;
+        o[place] = val;
+        if (place == k - 1) last = val;
+    });
+    if (k < n && k < kmax && pr.pad_mode) {                   // (workgroup-uniform)
         __syncthreads();
-        const int pad = pr.pad_mode == 2 ? sh.last : pr.pad_value;
-        for (int i = k + tid; i < kmax; i += TK_THREADS) o[i] = pad;
+        const int pad = pr.pad_mode == 2 ? last : pr.pad_value;
+        for (int i = k + (int)threadIdx.x; i < kmax; i += TK_THREADS) o[i] = pad;
     }
+}
+
+// The vertical-slash layer's selections, straight from the estimation's sums, and behind a head's slashes, kept in LDS,
+// the index builder's tables of that head: three launches of 3 to 8 us each, chains of latency on one or two workgroups
+// a head, that read what the one before wrote.
+// The three and now, without the gaps between them: one head of 4096 tokens, 500 columns and 700 slashes 2.9 + 7.5 + 5.7 ->
+// 11.7 us, whole layer 68.1 -> 63.9, 1000 and 6096 (all diagonals) 73.3 -> 60.2; 32 heads, 16001 tokens, 1000 and 6096
+// 5.1 + 17.7 + 15.4 -> 31.5.
+template <int ITEMS>
+__global__ __launch_bounds__(TK_THREADS) void vs_select_kernel(const EstWindows e, int n, int nnz_v, int32_t *__restrict__ v_idx, int nnz_s,
+                                                               int32_t *__restrict__ s_idx, int32_t *__restrict__ tables, int rows, int bm_words) {
+    __shared__ int32_t slashes[ITEMS * TK_THREADS];
+    // marks of the list's chunks, then the bitmap of n + 64 positions
+    __shared__ uint64_t prep_lds[2 * ITEMS * TK_THREADS / MINF_WAVE + 2];
+    const long long bh = blockIdx.x;
+    if (blockIdx.y == 0) {
+        const float *__restrict__ x = e.vertical + bh * n;
+        int32_t *__restrict__ o = v_idx + bh * nnz_v;
+        topk_regs_select<ITEMS>(n, nnz_v, [&](int i) { return i < e.force_v ? INFINITY : x[i]; }, [&](int place, int i) { o[place] = i; });
+        return;
+    }
+    const float *__restrict__ windows = e.windows + bh * e.nchunks * ((1 << e.kc_log2) + EST_WINDOW_TAIL);
+    int32_t *__restrict__ o = s_idx + bh * nnz_s;
+    topk_regs_select<ITEMS>(n, nnz_s, [&](int i) { const float v = est_slash(windows, e.kc_log2, i); return e.force_s > 0 && i >= n - e.force_s ? INFINITY : v; },
+                            [&](int place, int i) { o[place] = slashes[place] = n - 1 - i; });
+    __syncthreads();
+    prep_tables(slashes, tables + bh * idx_tab_ints(nnz_s, rows), nnz_s, rows, bm_words, prep_lds);
 }
 
 // The flag bytes of the pattern search's candidates (bit t of a byte: candidate t keeps the position): the k[t] best
@@ -745,9 +779,12 @@ __global__ __launch_bounds__(TK_THREADS) void topk_flags_kernel(const FlagsProbl
     for (long long i = n + tid; i < pitch; i += TK_THREADS) out[i] = 0;
 }
 
+// whether a workgroup per row, the row in its registers, selects from rows of n entries
+bool rows_in_registers(long long rows, int n) { return n > 256 && n <= 16 * TK_THREADS && (n > 64 * 64 || rows <= TK_FEW_ROWS); }
+
 void launch_topk(const TopkProblem &pa, const TopkProblem &pb, int problems, int rows, int n, hipStream_t st) {
     const dim3 grid((unsigned)rows, (unsigned)problems);
-    if (pa.causal_rows == 0 && n > 256 && n <= 16 * TK_THREADS && (n > 64 * 64 || (long long)rows * problems <= TK_FEW_ROWS)) {
+    if (pa.causal_rows == 0 && rows_in_registers((long long)rows * problems, n)) {
         if (n <= 4 * TK_THREADS) hipLaunchKernelGGL(topk_regs_kernel<4>, grid, dim3(TK_THREADS), 0, st, pa, pb, n);
         else if (n <= 8 * TK_THREADS) hipLaunchKernelGGL(topk_regs_kernel<8>, grid, dim3(TK_THREADS), 0, st, pa, pb, n);
         else hipLaunchKernelGGL(topk_regs_kernel<16>, grid, dim3(TK_THREADS), 0, st, pa, pb, n);
@@ -767,6 +804,17 @@ void launch_topk(const TopkProblem &pa, const TopkProblem &pb, int problems, int
 }
 
 }  // namespace
+
+bool vs_select_takes(int heads, int n) { return rows_in_registers(2ll * heads, n); }
+
+int vs_select(const EstWindows &e, int heads, int n, int nnz_v, int32_t *v_idx, int nnz_s, int32_t *s_idx, int32_t *tables, hipStream_t st) {
+    const dim3 grid((unsigned)heads, 2), block(TK_THREADS);
+    const int rows = (n + 63) / 64, bm_words = (int)idx_bm_words(rows);
+    if (n <= 4 * TK_THREADS) hipLaunchKernelGGL(vs_select_kernel<4>, grid, block, 0, st, e, n, nnz_v, v_idx, nnz_s, s_idx, tables, rows, bm_words);
+    else if (n <= 8 * TK_THREADS) hipLaunchKernelGGL(vs_select_kernel<8>, grid, block, 0, st, e, n, nnz_v, v_idx, nnz_s, s_idx, tables, rows, bm_words);
+    else hipLaunchKernelGGL(vs_select_kernel<16>, grid, block, 0, st, e, n, nnz_v, v_idx, nnz_s, s_idx, tables, rows, bm_words);
+    return minf_launch_status();
+}
 
 extern "C" int minf_topk_indices(const float *scores, int rows, int n, int64_t row_stride, int k,
                                  int32_t *out, int64_t out_stride, int reverse_base, void *stream) {

@@ -33,6 +33,7 @@
 // dtype (the einsum's result), then the product with sm_scale to the input dtype again (the division
 // by sqrt(head_dim)), before the fp32 softmax (minference_forward.py:602-604).
 #include "minf_common.h"
+#include "vs_stages.h"
 #include <math.h>
 #include <type_traits>
 
@@ -612,13 +613,7 @@ __global__ __launch_bounds__(256) void est_finalize_kernel(const EstParams p) {
     const long long bh = blockIdx.y;
     const int j = (int)(blockIdx.x * 256 + threadIdx.x);
     if (j >= p.n) return;
-    const int KC = p.kc, WIN = KC + LQ;
-    const int c = j / KC, off = j - c * KC;
-    const float *wbase = p.win + bh * p.nchunks * WIN;
-    // diagonal j lives at window position `off` of chunk c and, when off < LQ, also at
-    // position KC + off of chunk c-1 (keys of the previous chunk seen by later rows)
-    float v = wbase[(long long)c * WIN + off];
-    if (c > 0 && off < LQ) v = wbase[(long long)(c - 1) * WIN + KC + off] + v;
+    float v = est_slash(p.win + bh * p.nchunks * (p.kc + LQ), __builtin_ctz(p.kc), j);
     if (p.force_s > 0 && j >= p.n - p.force_s) v = INFINITY;
     p.slash[bh * p.n + j] = v;
     if (j < p.force_v) p.vertical[bh * p.n + j] = INFINITY;
@@ -686,7 +681,7 @@ static int estimate_launch(const void *q, const void *k, const int64_t *q_stride
                            int batch, int heads_q, int heads_kv, int n, int head_dim, int dtype, float sm_scale,
                            int last_q, int force_vertical, int force_slash, float *vertical, float *slash,
                            void *workspace, size_t workspace_bytes, const int32_t *head_list, int index_heads,
-                           int rounding, void *stream) {
+                           int rounding, void *stream, EstWindows *windows = nullptr) {
     EstParams p;
     if (rounding != MINF_ROUND_NONE && rounding != MINF_ROUND_INPUT_DTYPE) return MINF_ERR_INVALID_ARG;
     if (batch == 0) return MINF_OK;
@@ -719,10 +714,19 @@ static int estimate_launch(const void *q, const void *k, const int64_t *q_stride
     } while (0)
     EST_LAUNCH(est_stats_kernel);
     EST_LAUNCH(est_scores_kernel);
-    hipLaunchKernelGGL(est_finalize_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)bh), dim3(256), 0, s, p);
+    if (windows) *windows = EstWindows{p.vertical, p.win, __builtin_ctz(p.kc), p.nchunks, p.force_v, p.force_s};
+    else hipLaunchKernelGGL(est_finalize_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)bh), dim3(256), 0, s, p);
 #undef EST_LAUNCH
 #undef EST_LAUNCH_RR
     return minf_launch_status();
+}
+
+static_assert(LQ == EST_WINDOW_TAIL, "a chunk's window reaches as far as there are rows");
+int vs_estimate_windows(const minf_qkvo *t, int last_q, int force_vertical, int force_slash, int rounding, float *vertical,
+                        void *workspace, size_t workspace_bytes, EstWindows *out, void *stream) {
+    return estimate_launch(t->q, t->k, t->q_stride, t->k_stride, t->batch, t->heads_q, t->heads_kv, t->n, t->head_dim, t->dtype,
+                           t->sm_scale, last_q, force_vertical, force_slash, vertical, vertical, workspace, workspace_bytes,
+                           nullptr, 0, rounding, stream, out);
 }
 
 extern "C" int minf_vs_estimate(const void *q, const void *k, const int64_t *q_stride,

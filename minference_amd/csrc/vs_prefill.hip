@@ -3,6 +3,7 @@
 // stages and a call from Python for each stage, enqueueing a layer took longer than its kernels.  One head, 1000 to 4096
 // tokens 80 -> 58 .. 68 us, a first pass on new tensors 165 -> 121; where the kernels take longer, as before.
 #include "minf_common.h"
+#include "vs_stages.h"
 
 namespace {
 
@@ -11,7 +12,7 @@ constexpr size_t PART_ALIGN = 256;
 // the parts of the workspace, in bytes from its start
 struct PrefillParts {
     size_t v_idx, s_idx, block_count, block_offset, column_count, column_index, shared;   // what lives on until the attention is done
-    size_t slash, estimate;                      // inside `shared`, while scores are made and selected (the vertical scores first)
+    size_t slash, estimate, tables;              // inside `shared`, until the index is built (the vertical scores first)
     size_t estimate_bytes, table_bytes, split_bytes, total;
 };
 
@@ -30,8 +31,8 @@ PrefillParts prefill_parts(const minf_qkvo *t, int nnz_v, int nnz_s) {
     w.block_offset = take(4 * heads * rows * nnz_s);
     w.column_count = take(4 * heads * rows);
     w.column_index = take(4 * heads * rows * nnz_v);
-    // one stretch for what the stages need for themselves, one after another: scores and their partial sums, the index
-    // builder's tables, the split walks' sums
+    // one stretch for what the stages need for themselves: scores, their partial sums and the index builder's tables, then
+    // the split walks' sums
     w.shared = at;
     w.estimate_bytes = minf_vs_estimate_workspace_bytes(t->batch, t->heads_q, t->n);
     w.table_bytes = minf_vs_index_workspace_bytes(t->batch, t->heads_q, nnz_s, (int)rows);
@@ -39,10 +40,11 @@ PrefillParts prefill_parts(const minf_qkvo *t, int nnz_v, int nnz_s) {
     take(4 * heads * t->n);
     w.slash = take(4 * heads * t->n);
     w.estimate = take(w.estimate_bytes);
-    const size_t scores_end = at;
+    w.tables = take(w.table_bytes);              // (tables are made while other heads' scores are still selected)
+    const size_t tables_end = at;
     at = w.shared;
-    take(w.table_bytes > w.split_bytes ? w.table_bytes : w.split_bytes);
-    w.total = at > scores_end ? at : scores_end;
+    take(w.split_bytes);
+    w.total = at > tables_end ? at : tables_end;
     return w;
 }
 
@@ -71,16 +73,26 @@ extern "C" int minf_vs_prefill(const minf_qkvo *t, int nnz_v, int nnz_s, int las
     auto ints = [&](size_t at) { return (int32_t *)(ws + at); };
     float *const vertical = (float *)shared, *const slash = (float *)(ws + w.slash);
     const int heads = t->batch * t->heads_q, rows = (t->n + 63) / 64;
-    st = minf_vs_estimate(t->q, t->k, t->q_stride, t->k_stride, t->batch, t->heads_q, t->heads_kv, t->n, t->head_dim, t->dtype,
-                          t->sm_scale, last_q, force_vertical, force_slash, rounding, vertical, slash, ws + w.estimate,
-                          w.estimate_bytes, stream);
-    if (st != MINF_OK) return st;
-    st = minf_topk_indices_pair(vertical, nnz_v, ints(w.v_idx), nnz_v, -1, slash, nnz_s, ints(w.s_idx), nnz_s, t->n - 1, heads,
-                                t->n, t->n, stream);
-    if (st != MINF_OK) return st;
-    st = minf_vs_index_build_full_ws(ints(w.v_idx), ints(w.s_idx), ints(w.block_count), ints(w.block_offset), ints(w.column_count),
-                                     ints(w.column_index), t->batch, t->heads_q, rows, nnz_v, nnz_s, 0, nullptr, shared,
-                                     w.table_bytes, stream);
+    if (vs_select_takes(heads, t->n)) {
+        EstWindows e;
+        st = vs_estimate_windows(t, last_q, force_vertical, force_slash, rounding, vertical, ws + w.estimate, w.estimate_bytes, &e, stream);
+        if (st != MINF_OK) return st;
+        st = vs_select(e, heads, t->n, nnz_v, ints(w.v_idx), nnz_s, ints(w.s_idx), ints(w.tables), (hipStream_t)stream);
+        if (st != MINF_OK) return st;
+        st = vs_index_rows(ints(w.v_idx), ints(w.s_idx), ints(w.block_count), ints(w.block_offset), ints(w.column_count),
+                           ints(w.column_index), t->batch, t->heads_q, rows, nnz_v, nnz_s, ints(w.tables), (hipStream_t)stream);
+    } else {
+        st = minf_vs_estimate(t->q, t->k, t->q_stride, t->k_stride, t->batch, t->heads_q, t->heads_kv, t->n, t->head_dim, t->dtype,
+                              t->sm_scale, last_q, force_vertical, force_slash, rounding, vertical, slash, ws + w.estimate,
+                              w.estimate_bytes, stream);
+        if (st != MINF_OK) return st;
+        st = minf_topk_indices_pair(vertical, nnz_v, ints(w.v_idx), nnz_v, -1, slash, nnz_s, ints(w.s_idx), nnz_s, t->n - 1, heads,
+                                    t->n, t->n, stream);
+        if (st != MINF_OK) return st;
+        st = minf_vs_index_build_full_ws(ints(w.v_idx), ints(w.s_idx), ints(w.block_count), ints(w.block_offset), ints(w.column_count),
+                                         ints(w.column_index), t->batch, t->heads_q, rows, nnz_v, nnz_s, 0, nullptr,
+                                         ints(w.tables), w.table_bytes, stream);
+    }
     if (st != MINF_OK) return st;
     minf_qkvo a = *t;
     a.workspace = w.split_bytes ? shared : nullptr;

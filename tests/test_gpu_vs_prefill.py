@@ -20,6 +20,9 @@ def stages(q, k, v, nv, ns):
 @pytest.mark.parametrize("batch,hq,hk,n,d,dtype,nv,ns", [
     (1, 1, 1, 1, 128, torch.bfloat16, 1000, 6096), (1, 1, 1, 33, 64, torch.float16, 30, 800), (2, 4, 2, 65, 128, torch.bfloat16, 1, 1),
     (1, 4, 4, 700, 96, torch.bfloat16, 100, 750), (2, 2, 1, 2049, 64, torch.bfloat16, 500, 700), (1, 1, 1, 4097, 128, torch.float16, 500, 700),
+    (1, 2, 1, 256, 128, torch.bfloat16, 100, 200), (1, 2, 1, 257, 128, torch.bfloat16, 257, 257), (1, 3, 3, 4096, 128, torch.bfloat16, 4096, 4096),
+    (1, 2, 2, 8192, 64, torch.bfloat16, 3500, 100), (1, 2, 2, 8193, 128, torch.bfloat16, 1000, 6096), (2, 260, 4, 300, 64, torch.bfloat16, 30, 60),
+    (1, 257, 1, 600, 64, torch.float16, 30, 128), (1, 256, 1, 4097, 64, torch.bfloat16, 30, 129), (1, 1, 1, 16384, 64, torch.bfloat16, 30, 16384),
     (1, 8, 2, 16384, 128, torch.bfloat16, 1000, 6096), (1, 4, 1, 16385, 128, torch.bfloat16, 3500, 100)])
 def test_same_bits_as_the_stages(gpu, batch, hq, hk, n, d, dtype, nv, ns):
     import minference_amd as M
