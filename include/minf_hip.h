@@ -258,6 +258,17 @@ int minf_bs_attn_fwd(const minf_qkvo *t, const int32_t *block_index, int rows,
 int minf_ashape_attn_fwd(const minf_qkvo *t, int n_init, int n_local, void *stream);
 
 /*
+ * minf_vs_attn_fwd, minf_bs_attn_fwd and minf_ashape_attn_fwd for a layer whose heads have different patterns
+ * (minference/modules/minference_forward.py:657-667), in one launch where none of them is split, else one after another:
+ * each part has its own minf_qkvo (head_list, sm_scale, workspace; a workspace may be the same for all), null where no
+ * head has that pattern.  No head may be in two parts.
+ */
+int minf_mixed_attn_fwd(const minf_qkvo *vs, const int32_t *block_count, const int32_t *block_offset,
+                        const int32_t *column_count, const int32_t *column_index, int rows, int nnz_s, int nnz_v,
+                        const minf_qkvo *bs, const int32_t *block_index, int block_rows, int max_blocks,
+                        const minf_qkvo *ashape, int n_init, int n_local, void *stream);
+
+/*
  * Tri-shape: A-shape for the first n - n_last query rows, dense causal attention for the last
  * n_last rows, in one launch of the same kernel.  Replaces tri_shape_kernel (reference
  * minference/ops/streaming_kernel.py:820-833 and minference/modules/minference_forward.py:444-455),

@@ -253,7 +253,7 @@ template <int MODE, int HD> struct AttnLds {
 // workgroup -- when a row sum left the safe range, i.e. when the walk has to be run again with
 // EVERY_MAX (the output it wrote is then overwritten).
 template <typename T, int MODE, int HD, bool EVERY_MAX, bool CUT>
-__device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[AttnLds<MODE, HD>::NK],
+__device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg, char (&lds_k)[AttnLds<MODE, HD>::NK],
                                           char (&lds_v)[AttnLds<MODE, HD>::NV],
                                           int (&vs_only)[AttnLds<MODE, HD>::NONLY], int (&vs_wsum)[4], int (&vs_bad)[2],
                                           int &lds_redo) {
@@ -290,10 +290,10 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
     // (32-bit arithmetic: the launcher refuses grids beyond 2^31 workgroups, and 64-bit divisions of
     // wave-uniform values cost a thousand scalar instructions per workgroup here)
     const int group = (int)p.by_group.d;
-    unsigned rest = blockIdx.x >> 3;
+    unsigned rest = wg >> 3;
     auto next_digit = [&](const FastDiv &f) { const unsigned q = fast_quot(rest, f), r = rest - q * f.d; rest = q; return r; };
     const unsigned in_deal = next_digit(p.by_deal);
-    rest = 8u * rest + ((blockIdx.x + rest * (unsigned)p.turn) & 7u);
+    rest = 8u * rest + ((wg + rest * (unsigned)p.turn) & 7u);
     const unsigned gi = next_digit(p.by_groups), first_unit = rest * (unsigned)p.chunk;
     rest = in_deal;
     const int hin = (int)next_digit(p.by_group);
@@ -1134,6 +1134,25 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, char (&lds_k)[Att
 // (head_dim 256: O^T, Q and the V^T fragments of a wave need more than 256 registers, so that form
 // runs one wave per SIMD with the accumulators in the second half of the register file)
 template <typename T> constexpr int dtype_code() { return std::is_same<T, __bf16>::value ? MINF_BF16 : MINF_F16; }
+// workgroup `wg` of a launch
+template <typename T, int MODE, int HD, bool CUT>
+__device__ __forceinline__ void attn_workgroup(const AttnParams &p, const unsigned wg, char (&lds_k)[AttnLds<MODE, HD>::NK],
+                                               char (&lds_v)[AttnLds<MODE, HD>::NV], int (&vs_only)[AttnLds<MODE, HD>::NONLY]) {
+    __shared__ int vs_wsum[4];
+    __shared__ int vs_bad[2];                // paired list walks: a list is not ascending, number of common entries
+    __shared__ int lds_redo;
+    if (threadIdx.x == 0) lds_redo = 0;      // (ordered before its readers by the barriers of the walk)
+    if constexpr (std::is_same<T, __bf16>::value) {
+        if (attn_walk<T, MODE, HD, false, CUT>(p, wg, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo)) {
+            __syncthreads();                 // everyone has read the flag and is done with LDS
+            attn_walk<T, MODE, HD, true, CUT>(p, wg, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
+        }
+    } else {
+        // f16 probabilities have no headroom above the lazy threshold: the maximum of every tile
+        attn_walk<T, MODE, HD, true, CUT>(p, wg, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
+    }
+}
+
 template <typename T, int MODE, int HD, bool CUT>
 __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kernel(const AttnParams p) {
     typedef AttnLds<MODE, HD> L;
@@ -1141,19 +1160,31 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
     __shared__ __attribute__((aligned(16))) char lds_k[L::NK];
     __shared__ __attribute__((aligned(16))) char lds_v[L::NV];
     __shared__ int vs_only[L::NONLY];        // paired list walks: [row block][entries the other list lacks]
-    __shared__ int vs_wsum[4];
-    __shared__ int vs_bad[2];                // paired list walks: a list is not ascending, number of common entries
-    __shared__ int lds_redo;
-    if (threadIdx.x == 0) lds_redo = 0;      // (ordered before its readers by the barriers of the walk)
-    if constexpr (std::is_same<T, __bf16>::value) {
-        if (attn_walk<T, MODE, HD, false, CUT>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo)) {
-            __syncthreads();                 // everyone has read the flag and is done with LDS
-            attn_walk<T, MODE, HD, true, CUT>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
-        }
-    } else {
-        // f16 probabilities have no headroom above the lazy threshold: the maximum of every tile
-        attn_walk<T, MODE, HD, true, CUT>(p, lds_k, lds_v, vs_only, vs_wsum, vs_bad, lds_redo);
-    }
+    attn_workgroup<T, MODE, HD, CUT>(p, blockIdx.x, lds_k, lds_v, vs_only);
+}
+
+// The pattern types of a layer in one launch: workgroups [0, first_bs) walk vertical-slash lists, [first_bs, first_as)
+// block-sparse lists, the rest A-shape windows (each part a multiple of 8 workgroups, see launch_hd).  As three launches
+// each waited for the last walks of the one before on a chip that was emptying.
+// Table of unlike patterns, 32 / 8 heads, whole layer, us: 9000 tokens 774 -> 692, 20000 fp16 1898 -> 1802, of 64 1059 ->
+// 995, 50000 4531 -> 4482, 100000 9316 -> 9243; 28 / 4 heads 20000 tokens 1390 -> 1352; 8 / 2 heads 12000 tokens 331 -> 328.
+// (bf16 at head_dim 128: 254 registers, the most of its three forms, no vector spills.)
+struct MixedParams {
+    AttnParams vs, bs, as;
+    unsigned first_bs, first_as;
+};
+template <typename T, int HD>
+__global__ __launch_bounds__(2 * NTHREADS, 2) void attn_mixed_kernel(const MixedParams p) {
+    typedef AttnLds<MODE_VS, HD> L;
+    typedef AttnLds<MODE_ASHAPE, HD> A;
+    static_assert(A::NK == L::NK && A::NV <= L::NV && A::NONLY <= L::NONLY, "an A-shape walk fits the LDS of a list walk");
+    __shared__ __attribute__((aligned(16))) char lds_k[L::NK];
+    __shared__ __attribute__((aligned(16))) char lds_v[L::NV];
+    __shared__ int vs_only[L::NONLY];
+    if (blockIdx.x < p.first_bs) attn_workgroup<T, MODE_VS, HD, false>(p.vs, blockIdx.x, lds_k, lds_v, vs_only);
+    else if (blockIdx.x < p.first_as) attn_workgroup<T, MODE_BS, HD, false>(p.bs, blockIdx.x - p.first_bs, lds_k, lds_v, vs_only);
+    else attn_workgroup<T, MODE_ASHAPE, HD, false>(p.as, blockIdx.x - p.first_as, lds_k, reinterpret_cast<char (&)[A::NV]>(lds_v),
+                                                   reinterpret_cast<int (&)[A::NONLY]>(vs_only));
 }
 
 // Folds the segments of a split pair: one workgroup per (batch, head position, pair, 32 query rows), a
@@ -1428,9 +1459,8 @@ size_t split_bytes(const SplitPlan &s, const AttnParams &p, int head_dim) {
     return pairs * s.nseg * slot;
 }
 
-template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void *stream) {
-    if (p.batch == 0 || p.rows == 0) return MINF_OK;
-    const int dtype = t->dtype;
+// Fills in how a launch is split and dealt out, -> its workgroups (beyond 2^31 - 1: it cannot be made)
+template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo *t) {
     if (t->workspace && ((uintptr_t)t->workspace & 15) == 0) {
         const SplitPlan s = plan_split(MODE, p, HD);
         if (s.nseg > 1 && split_bytes(s, p, HD) <= t->workspace_bytes) {
@@ -1486,12 +1516,19 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
     p.chunk = (int)chunk;
     p.turn = p.head_list || MODE == MODE_VS;
     const long long deal = chunk * group, deals = (units + chunk - 1) / chunk * groups;
-    const long long grid = (deals + 7) / 8 * 8 * deal;
-    if (grid > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
     p.by_group = fast_div((unsigned)group);
     p.by_deal = fast_div((unsigned)deal);
     p.by_groups = fast_div((unsigned)groups);
     p.by_heads = fast_div((unsigned)(grid_heads / group));
+    return (deals + 7) / 8 * 8 * deal;
+}
+
+template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void *stream) {
+    if (p.batch == 0 || p.rows == 0) return MINF_OK;
+    const int dtype = t->dtype;
+    const long long grid = plan_launch<MODE, HD>(p, t);
+    if (grid > 0x7fffffffLL) return MINF_ERR_UNSUPPORTED;
+    const int split_pairs = (p.rows + 1) / 2 - p.split_first;
     const dim3 block(2 * NTHREADS);
     hipStream_t st = (hipStream_t)stream;
 #define MINF_LAUNCH_ATTN(T)                                                                                      \
@@ -1519,43 +1556,118 @@ template <int MODE> int launch(const AttnParams &p, const minf_qkvo *t, void *st
 
 }  // namespace
 
-extern "C" int minf_vs_attn_fwd(const minf_qkvo *t, const int32_t *block_count,
-                                const int32_t *block_offset, const int32_t *column_count,
-                                const int32_t *column_index, int rows, int nnz_s, int nnz_v,
-                                void *stream) {
-    int st = check_tensors(t);
+// the arguments of the entry points, checked (`p` is filled in on MINF_OK)
+static int vs_params(AttnParams &p, const minf_qkvo *t, const int32_t *block_count, const int32_t *block_offset,
+                     const int32_t *column_count, const int32_t *column_index, int rows, int nnz_s, int nnz_v) {
+    const int st = check_tensors(t);
     if (st) return st;
     if (!block_count || !block_offset || !column_count || !column_index) return MINF_ERR_INVALID_ARG;
     if (nnz_s < 1 || nnz_v < 1) return MINF_ERR_INVALID_ARG;
-    AttnParams p;
     fill_params(p, t);
     if (rows != p.rows) return MINF_ERR_INVALID_ARG;
     p.bc = block_count; p.bo = block_offset; p.cc = column_count; p.ci = column_index;
     p.nnz_s = nnz_s; p.nnz_v = nnz_v;
-    return launch<MODE_VS>(p, t, stream);
+    return MINF_OK;
 }
 
-extern "C" int minf_bs_attn_fwd(const minf_qkvo *t, const int32_t *block_index, int rows,
-                                int max_blocks, void *stream) {
-    int st = check_tensors(t);
+static int bs_params(AttnParams &p, const minf_qkvo *t, const int32_t *block_index, int rows, int max_blocks) {
+    const int st = check_tensors(t);
     if (st) return st;
     if (!block_index || max_blocks < 1) return MINF_ERR_INVALID_ARG;
-    AttnParams p;
     fill_params(p, t);
     if (rows < p.rows) return MINF_ERR_INVALID_ARG;
     // block_index may have more rows than ceil(n/64) (the reference pads n first)
     p.bidx = block_index; p.max_blocks = max_blocks; p.bidx_rows = rows;
-    return launch<MODE_BS>(p, t, stream);
+    return MINF_OK;
+}
+
+static int ashape_params(AttnParams &p, const minf_qkvo *t, int n_init, int n_local) {
+    const int st = check_tensors(t, true);
+    if (st) return st;
+    if (n_init < 0 || n_local < 1) return MINF_ERR_INVALID_ARG;
+    fill_params(p, t);
+    p.n_init = n_init; p.n_local = n_local;
+    return MINF_OK;
+}
+
+extern "C" int minf_vs_attn_fwd(const minf_qkvo *t, const int32_t *block_count,
+                                const int32_t *block_offset, const int32_t *column_count,
+                                const int32_t *column_index, int rows, int nnz_s, int nnz_v,
+                                void *stream) {
+    AttnParams p;
+    const int st = vs_params(p, t, block_count, block_offset, column_count, column_index, rows, nnz_s, nnz_v);
+    return st ? st : launch<MODE_VS>(p, t, stream);
+}
+
+extern "C" int minf_bs_attn_fwd(const minf_qkvo *t, const int32_t *block_index, int rows,
+                                int max_blocks, void *stream) {
+    AttnParams p;
+    const int st = bs_params(p, t, block_index, rows, max_blocks);
+    return st ? st : launch<MODE_BS>(p, t, stream);
 }
 
 extern "C" int minf_ashape_attn_fwd(const minf_qkvo *t, int n_init, int n_local, void *stream) {
-    int st = check_tensors(t, true);
-    if (st) return st;
-    if (n_init < 0 || n_local < 1) return MINF_ERR_INVALID_ARG;
     AttnParams p;
-    fill_params(p, t);
-    p.n_init = n_init; p.n_local = n_local;
-    return launch<MODE_ASHAPE>(p, t, stream);
+    const int st = ashape_params(p, t, n_init, n_local);
+    return st ? st : launch<MODE_ASHAPE>(p, t, stream);
+}
+
+namespace {
+
+// The parts of a layer (null: absent) in one launch -> whether it was made: not where a walk is split, nothing is to be
+// done, or only one part is there
+template <typename T, int HD> bool launch_mixed(const AttnParams &vs, const minf_qkvo *vs_t, const AttnParams &bs, const minf_qkvo *bs_t,
+                                                const AttnParams &as, const minf_qkvo *as_t, void *stream) {
+    MixedParams m;
+    memset(&m, 0, sizeof(m));
+    long long vs_wgs = 0, bs_wgs = 0, as_wgs = 0;
+    if (vs_t) { m.vs = vs; vs_wgs = plan_launch<MODE_VS, HD>(m.vs, vs_t); }
+    if (bs_t) { m.bs = bs; bs_wgs = plan_launch<MODE_BS, HD>(m.bs, bs_t); }
+    if (as_t) { m.as = as; as_wgs = plan_launch<MODE_ASHAPE, HD>(m.as, as_t); }
+    if ((vs_t && m.vs.nseg > 1) || (bs_t && m.bs.nseg > 1) || (as_t && m.as.nseg > 1)) return false;
+    if (vs_wgs + bs_wgs + as_wgs > 0x7fffffffLL) return false;
+    m.first_bs = (unsigned)vs_wgs;
+    m.first_as = (unsigned)(vs_wgs + bs_wgs);
+    hipLaunchKernelGGL((attn_mixed_kernel<T, HD>), dim3((unsigned)(vs_wgs + bs_wgs + as_wgs)), dim3(2 * NTHREADS), 0, (hipStream_t)stream, m);
+    return true;
+}
+
+}  // namespace
+
+extern "C" int minf_mixed_attn_fwd(const minf_qkvo *vs, const int32_t *block_count, const int32_t *block_offset,
+                                   const int32_t *column_count, const int32_t *column_index, int rows, int nnz_s, int nnz_v,
+                                   const minf_qkvo *bs, const int32_t *block_index, int block_rows, int max_blocks,
+                                   const minf_qkvo *ashape, int n_init, int n_local, void *stream) {
+    AttnParams vs_p, bs_p, as_p;
+    int st = MINF_OK;
+    if (vs) st = vs_params(vs_p, vs, block_count, block_offset, column_count, column_index, rows, nnz_s, nnz_v);
+    if (st == MINF_OK && bs) st = bs_params(bs_p, bs, block_index, block_rows, max_blocks);
+    if (st == MINF_OK && ashape) st = ashape_params(as_p, ashape, n_init, n_local);
+    if (st != MINF_OK) return st;
+    const minf_qkvo *const parts[3] = {vs, bs, ashape};
+    const minf_qkvo *first = nullptr;
+    int count = 0;
+    bool alike = true;
+    for (const minf_qkvo *t : parts) {
+        if (!t) continue;
+        ++count;
+        if (!first) first = t;
+        alike = alike && t->head_dim == first->head_dim && t->dtype == first->dtype && t->batch > 0 && t->n > 0;
+    }
+    if (count > 1 && alike && first->head_dim <= 128 && first->dtype != MINF_16BIT_SELECT) {
+        bool made;
+        if (first->head_dim == 128)
+            made = first->dtype == MINF_BF16 ? launch_mixed<__bf16, 128>(vs_p, vs, bs_p, bs, as_p, ashape, stream)
+                                             : launch_mixed<_Float16, 128>(vs_p, vs, bs_p, bs, as_p, ashape, stream);
+        else
+            made = first->dtype == MINF_BF16 ? launch_mixed<__bf16, 64>(vs_p, vs, bs_p, bs, as_p, ashape, stream)
+                                             : launch_mixed<_Float16, 64>(vs_p, vs, bs_p, bs, as_p, ashape, stream);
+        if (made) return minf_launch_status();
+    }
+    if (vs) st = launch<MODE_VS>(vs_p, vs, stream);
+    if (st == MINF_OK && bs) st = launch<MODE_BS>(bs_p, bs, stream);
+    if (st == MINF_OK && ashape) st = launch<MODE_ASHAPE>(as_p, ashape, stream);
+    return st;
 }
 
 extern "C" int minf_trishape_attn_fwd(const minf_qkvo *t, int n_init, int n_local, int n_last,

@@ -12,6 +12,7 @@ reference's Python loop over heads.  K/V may have fewer heads than Q (no repeat_
 """
 from __future__ import annotations
 
+import ctypes
 import json
 import os
 from collections import OrderedDict
@@ -166,6 +167,9 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
     * block_sparse heads: one block index + one attention launch;
     * stream_llm heads: one launch per distinct (n_init, n_local).
 
+    With at most one distinct (n_init, n_local), and no launch that splits its walks (short prompts), the attention
+    launches are one.
+
     The reference runs one operator call per head here (minference_forward.py:657-667)."""
     from .estimate import reference_rounding_for
     from .ops import _streaming_scale
@@ -180,6 +184,18 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
     rows = (N + 63) // 64
     keep = []                                             # tensors the enqueued kernels still read
     dt = lp.device_tensors(B, N, dev)
+    vs_part = bs_part = None
+    vs_lists, bs_lists, windows = (None, None, None, None, rows, 0, 0), (None, 0, 0), []
+
+    def part(slot, op, n_init, n_local):
+        """A copy of the call's struct for the heads in `slot`, with scratch memory of its own."""
+        c.select_heads(slot)
+        c.scratch(op, n_init, n_local)
+        keep.append(c._scratch)
+        return _lib.QKVO.from_buffer_copy(c.struct)
+
+    def ref(struct):
+        return None if struct is None else ctypes.byref(struct)
 
     try:
         with torch.cuda.device(dev):
@@ -205,11 +221,8 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
                 _lib.check(st, "minf_topk_indices_pair_ragged")
                 seqlens = dt["seqlens"]
                 bc, bo, cc, ci = convert_vertical_slash_indexes(seqlens, v_idx, s_idx, N, 64, 64, zero_fill=False)
-                c.select_heads(slot)
-                c.scratch(_lib.MINF_OP_VERTICAL_SLASH, vmax, smax)
-                st = lib.minf_vs_attn_fwd(c.ref, bc.data_ptr(), bo.data_ptr(), cc.data_ptr(), ci.data_ptr(), rows,
-                                          smax, vmax, stream)
-                _lib.check(st, "minf_vs_attn_fwd")
+                vs_part = part(slot, _lib.MINF_OP_VERTICAL_SLASH, vmax, smax)
+                vs_lists = (bc.data_ptr(), bo.data_ptr(), cc.data_ptr(), ci.data_ptr(), rows, smax, vmax)
                 keep += [vertical, slash, ws, v_idx, s_idx, bc, bo, cc, ci]
             if lp.bs:
                 nh = len(lp.bs)
@@ -224,19 +237,28 @@ def _mixed_layer(query_states, key_states, value_states, lp, out=None):
                                                    slot.data_ptr(), nh, bi.data_ptr(),
                                                    ws.data_ptr(), ws_bytes, stream)
                 _lib.check(st, "minf_bs_block_index_heads")
-                c.select_heads(slot)
-                c.scratch(_lib.MINF_OP_BLOCK_SPARSE, 0, kk)
-                st = lib.minf_bs_attn_fwd(c.ref, bi.data_ptr(), brows, kk, stream)
-                _lib.check(st, "minf_bs_attn_fwd")
+                bs_part = part(slot, _lib.MINF_OP_BLOCK_SPARSE, 0, kk)
+                bs_lists = (bi.data_ptr(), brows, kk)
                 keep += [ws, bi]
             # (the reference's streaming operator scales by the power-of-two padded head_dim)
             c.struct.sm_scale = _streaming_scale(D)
             for (n_init, n_local), slot in dt["stream_heads"].items():
-                c.select_heads(slot)
                 if N > 0:
-                    c.scratch(_lib.MINF_OP_ASHAPE, n_init, n_local)
-                    st = lib.minf_ashape_attn_fwd(c.ref, int(n_init), int(n_local), stream)
-                    _lib.check(st, "minf_ashape_attn_fwd")
+                    windows.append((part(slot, _lib.MINF_OP_ASHAPE, n_init, n_local), int(n_init), int(n_local)))
+            if len(windows) <= 1:
+                # all of the layer's attention in one launch
+                window = windows[0] if windows else (None, 0, 0)
+                if vs_part or bs_part or window[0]:
+                    st = lib.minf_mixed_attn_fwd(ref(vs_part), *vs_lists, ref(bs_part), *bs_lists, ref(window[0]), *window[1:], stream)
+                    _lib.check(st, "minf_mixed_attn_fwd")
+            else:
+                # (windows of several sizes: a launch per type and size)
+                if vs_part:
+                    _lib.check(lib.minf_vs_attn_fwd(ref(vs_part), *vs_lists, stream), "minf_vs_attn_fwd")
+                if bs_part:
+                    _lib.check(lib.minf_bs_attn_fwd(ref(bs_part), *bs_lists, stream), "minf_bs_attn_fwd")
+                for as_part, n_init, n_local in windows:
+                    _lib.check(lib.minf_ashape_attn_fwd(ref(as_part), n_init, n_local, stream), "minf_ashape_attn_fwd")
     finally:
         c.struct.sm_scale = float(D) ** -0.5
         c.select_heads(None)
