@@ -147,6 +147,17 @@ int minf_index_sort_pair(const void *vertical, int vertical_is64, int nnz_v, int
                          void *stream);
 
 /*
+ * minf_index_sort_pair and minf_vs_index_build_full_ws (zero_fill 0) in one call: index tensors from lists in any order.
+ * vertical, slash [batch, heads, nnz] int32, or int64 where *_is64; vertical_out, slash_out: the sorted lists; both at
+ * most MINF_INDEX_SORT_MAX long; workspace as in minf_vs_index_build_ws.
+ */
+int minf_vs_index_from_lists(const void *vertical, int vertical_is64, int nnz_v, int32_t *vertical_out,
+                             const void *slash, int slash_is64, int nnz_s, int32_t *slash_out,
+                             int32_t *block_count, int32_t *block_offset, int32_t *column_count,
+                             int32_t *column_index, int batch, int heads, int rows, void *workspace,
+                             size_t workspace_bytes, void *stream);
+
+/*
  * Sparse flash-attention forward on one shared 64x64 bf16/f16 MFMA tile
  * engine.  Common arguments of the four entry points below:
  *

@@ -29,6 +29,7 @@ SIGNATURES = {
     "minf_vs_index_build_full_ws": (c_int, [c_ptr] * 6 + [c_int] * 6 + [c_ptr, c_ptr, ctypes.c_size_t, c_ptr]),
     "minf_vs_index_build_static": (c_int, [c_ptr] * 7 + [c_int] * 6 + [c_ptr, c_ptr]),
     "minf_index_sort_pair": (c_int, [c_ptr, c_int, c_int, c_ptr] * 2 + [c_int, c_ptr]),
+    "minf_vs_index_from_lists": (c_int, [c_ptr, c_int, c_int, c_ptr] * 2 + [c_ptr] * 4 + [c_int] * 3 + [c_ptr, ctypes.c_size_t, c_ptr]),
     "minf_narrow_qkv": (c_int, [c_ptr, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),
     "minf_widen_out": (c_int, [c_ptr, c_ptr, c_i64, c_int, c_int, c_ptr, c_ptr]),
     "minf_vs_attn_fwd": (c_int, [c_ptr] * 5 + [c_int] * 3 + [c_ptr]),

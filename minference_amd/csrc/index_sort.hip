@@ -15,6 +15,8 @@
 // time (1000 + 2048 values, 4 heads).  The operator on such indices: fp32 tensors of 8192 tokens 309 -> 265 us, rows of
 // 100 + 750 values, 2 x 16 heads of 597 tokens 119 -> 78.
 #include "minf_common.h"
+#include "vs_index_tables.h"
+#include "vs_stages.h"
 
 namespace {
 
@@ -29,16 +31,13 @@ struct SortProblem {
     unsigned flip;      // key = value ^ flip: ascending 0x80000000, descending 0x7fffffff
 };
 
-// E: 64-value groups per wavefront (rows of up to 1024 E values)
+// E: 64-value groups per wavefront (rows of up to 1024 E values).  Row `row` of p, sorted to p.out and, as values, to
+// keys[0 .. n) (each thread its own i % SORT_THREADS: no barrier behind).
 template <int E>
-__global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProblem pa, const SortProblem pb, int rows) {
-    __shared__ unsigned keys[E * SORT_THREADS];
+__device__ __forceinline__ void sort_row(const SortProblem &p, const long long row, unsigned (&keys)[E * SORT_THREADS]) {
     __shared__ unsigned hist[SORT_WAVES][SORT_DIGITS];     // values of a digit in the wavefronts before (after the scan)
     __shared__ unsigned first[SORT_DIGITS];                // place of a digit's first value behind those of its 64 digits
     __shared__ unsigned wsum[SORT_DIGITS / MINF_WAVE], differ;     // values of 64 digits; bytes in which values differ
-    const bool second = (int)blockIdx.x >= rows;           // (workgroup-uniform)
-    const SortProblem p = second ? pb : pa;
-    const long long row = (long long)blockIdx.x - (second ? rows : 0);
     const int tid = (int)threadIdx.x, lane = minf_lane();
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int groups = (p.n + SORT_THREADS - 1) / SORT_THREADS;          // <= E
@@ -137,8 +136,36 @@ __global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProb
         for (int r = 0; r < E; ++r)
             if (r < groups) key[r] = keys[base + r * MINF_WAVE];
     }
-    for (int i = tid; i < p.n; i += SORT_THREADS) p.out[row * p.n + i] = (int32_t)(keys[i] ^ p.flip);
+    for (int i = tid; i < p.n; i += SORT_THREADS) p.out[row * p.n + i] = (int32_t)(keys[i] ^= p.flip);
 }
+
+template <int E>
+__global__ __launch_bounds__(SORT_THREADS) void index_sort_kernel(const SortProblem pa, const SortProblem pb, int rows) {
+    __shared__ unsigned keys[E * SORT_THREADS];
+    const bool second = (int)blockIdx.x >= rows;           // (workgroup-uniform)
+    sort_row<E>(second ? pb : pa, (long long)blockIdx.x - (second ? rows : 0), keys);
+}
+
+// Both lists sorted as above (the slashes are pa's), and behind a head's slashes, where they lie in LDS, the index builder's tables.
+// As two launches, each a chain of latency on a workgroup or two per head, 4 heads, 1000 and 2048 int64 values 7.4 + 8.2 us, now
+// 13.5 and a gap less.  Operator on unsorted lists, us: 4 heads 600 tokens 56.8 -> 49.4, one head 4096 tokens 61.3 -> 53.5
+// (paced by the host, one call and one launch less), 4 heads 8192 tokens 130.1 -> 126.7, fp32 157.8 -> 156.5.
+template <int E>
+__global__ __launch_bounds__(SORT_THREADS) void index_sort_tables_kernel(const SortProblem pa, const SortProblem pb, int rows,
+                                                                         int32_t *__restrict__ tables, int blocks, int bm_words) {
+    __shared__ unsigned keys[E * SORT_THREADS];
+    extern __shared__ uint64_t prep_lds[];                 // (see prep_tables)
+    if ((int)blockIdx.x >= rows) {                         // (workgroup-uniform)
+        sort_row<E>(pb, (long long)blockIdx.x - rows, keys);
+        return;
+    }
+    sort_row<E>(pa, (long long)blockIdx.x, keys);
+    __syncthreads();
+    prep_tables(reinterpret_cast<const int32_t *>(keys), tables + (long long)blockIdx.x * idx_tab_ints(pa.n, blocks), pa.n, blocks, bm_words, prep_lds);
+}
+
+// the bitmap of the longest context that fits LDS beside 16384 slashes
+constexpr long long SORT_BITMAP_BYTES = 65536;
 
 }  // namespace
 
@@ -162,4 +189,40 @@ extern "C" int minf_index_sort_pair(const void *vertical, int vertical_is64, int
     else if (a.n <= 8192) hipLaunchKernelGGL((index_sort_kernel<8>), grid, block, 0, st, a, b, rows);
     else hipLaunchKernelGGL((index_sort_kernel<16>), grid, block, 0, st, a, b, rows);
     return minf_launch_status();
+}
+
+extern "C" int minf_vs_index_from_lists(const void *vertical, int vertical_is64, int nnz_v, int32_t *vertical_out,
+                                        const void *slash, int slash_is64, int nnz_s, int32_t *slash_out,
+                                        int32_t *block_count, int32_t *block_offset, int32_t *column_count,
+                                        int32_t *column_index, int batch, int heads, int rows, void *workspace,
+                                        size_t workspace_bytes, void *stream) {
+    if (!vertical || !vertical_out || !slash || !slash_out || !block_count || !block_offset || !column_count || !column_index)
+        return MINF_ERR_INVALID_ARG;
+    if (batch < 0 || heads < 0 || rows < 0 || nnz_v < 1 || nnz_s < 1) return MINF_ERR_INVALID_ARG;
+    const long long lists = (long long)batch * heads;
+    if (lists * rows == 0) return MINF_OK;
+    if (nnz_v > MINF_INDEX_SORT_MAX || nnz_s > MINF_INDEX_SORT_MAX || lists > 65535) return MINF_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < minf_vs_index_workspace_bytes(batch, heads, nnz_s, rows) || ((uintptr_t)workspace & 3))
+        return MINF_ERR_WORKSPACE;
+    const long long bm_words = idx_bm_words(rows);
+    if (bm_words * 4 > SORT_BITMAP_BYTES) {
+        const int st = minf_index_sort_pair(vertical, vertical_is64, nnz_v, vertical_out, slash, slash_is64, nnz_s, slash_out, (int)lists, stream);
+        return st ? st : minf_vs_index_build_full_ws(vertical_out, slash_out, block_count, block_offset, column_count, column_index,
+                                                     batch, heads, rows, nnz_v, nnz_s, 0, nullptr, workspace, workspace_bytes, stream);
+    }
+    const SortProblem v{vertical, vertical_out, nnz_v, vertical_is64 != 0, 0x80000000u};
+    const SortProblem s{slash, slash_out, nnz_s, slash_is64 != 0, 0x7fffffffu};
+    const int most = nnz_v > nnz_s ? nnz_v : nnz_s;
+    const size_t marks = 16 * (size_t)((nnz_s + MINF_WAVE - 1) / MINF_WAVE), bitmap = (size_t)bm_words * 4;
+    const size_t lds = marks > bitmap ? marks : bitmap;
+    const dim3 grid((unsigned)(2 * lists)), block(SORT_THREADS);
+    hipStream_t st = (hipStream_t)stream;
+    int32_t *const tables = (int32_t *)workspace;
+    auto *const kernel = most <= 1024 ? index_sort_tables_kernel<1> : most <= 2048 ? index_sort_tables_kernel<2> :
+                         most <= 4096 ? index_sort_tables_kernel<4> : most <= 8192 ? index_sort_tables_kernel<8> : index_sort_tables_kernel<16>;
+    hipLaunchKernelGGL(kernel, grid, block, lds, st, s, v, (int)lists, tables, rows, (int)bm_words);
+    const int status = minf_launch_status();
+    if (status != MINF_OK) return status;
+    return vs_index_rows(vertical_out, slash_out, block_count, block_offset, column_count, column_index, batch, heads, rows,
+                         nnz_v, nnz_s, tables, st);
 }

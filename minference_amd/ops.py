@@ -247,22 +247,50 @@ def vertical_slash_attention_from_index(query, key, value, block_count, block_of
     return c.result()
 
 
-def _sorted_indices(v_idx, s_idx, B, H):
-    """[B, H, nnz] int32: v_idx ascending, s_idx descending (one kernel; rows longer than its LDS are left
-    to torch)."""
+def _index_lists(v_idx, s_idx, B, H):
+    """[B, H, nnz] contiguous int32 or int64, and whether one kernel can sort both."""
     v = v_idx if v_idx.dtype in (torch.int32, torch.int64) else v_idx.to(torch.int32)
     s = s_idx if s_idx.dtype in (torch.int32, torch.int64) else s_idx.to(torch.int32)
     v, s = v.reshape((B, H, -1)).contiguous(), s.reshape((B, H, -1)).contiguous()
-    nv, ns = v.shape[-1], s.shape[-1]
-    if not (v.is_cuda and s.device == v.device) or max(nv, ns) > _lib.MINF_INDEX_SORT_MAX:
+    return v, s, v.is_cuda and s.device == v.device and max(v.shape[-1], s.shape[-1]) <= _lib.MINF_INDEX_SORT_MAX
+
+
+def _sorted_indices(v_idx, s_idx, B, H):
+    """[B, H, nnz] int32: v_idx ascending, s_idx descending (one kernel; rows longer than its LDS are left
+    to torch)."""
+    v, s, fits = _index_lists(v_idx, s_idx, B, H)
+    if not fits:
         return (v.to(torch.int32).sort(dim=-1, descending=False)[0], s.to(torch.int32).sort(dim=-1, descending=True)[0])
     vo, so = (torch.empty(t.shape, dtype=torch.int32, device=t.device) for t in (v, s))
     with torch.cuda.device(v.device):
-        st = _lib.load().minf_index_sort_pair(v.data_ptr(), v.dtype == torch.int64, nv, vo.data_ptr(),
-                                              s.data_ptr(), s.dtype == torch.int64, ns, so.data_ptr(), B * H,
+        st = _lib.load().minf_index_sort_pair(v.data_ptr(), v.dtype == torch.int64, v.shape[-1], vo.data_ptr(),
+                                              s.data_ptr(), s.dtype == torch.int64, s.shape[-1], so.data_ptr(), B * H,
                                               _lib.stream_ptr(v.device))
     _lib.check(st, "minf_index_sort_pair")
     return vo, so
+
+
+def _index_from_lists(v_idx, s_idx, B, H, N):
+    """The index tensors of v_idx and s_idx, in any order (payload only)."""
+    v, s, fits = _index_lists(v_idx, s_idx, B, H)
+    if not (fits and v.numel() and s.numel() and B * H <= 65535):
+        v, s = _sorted_indices(v, s, B, H)
+        if not v.is_cuda:
+            raise RuntimeError("vertical_slash_sparse_attention needs GPU tensors (no CPU path)")
+        return _build_index(None, v, s, N, zero_fill=False)
+    dev, rows, nv, ns = v.device, (N + 63) // 64, v.shape[-1], s.shape[-1]
+    lib = _lib.load()
+    empty = lambda *shape: torch.empty(shape, dtype=torch.int32, device=dev)
+    vo, so = empty(B, H, nv), empty(B, H, ns)
+    index = [empty(B, H, rows), empty(B, H, rows, ns), empty(B, H, rows), empty(B, H, rows, nv)]
+    nbytes = lib.minf_vs_index_workspace_bytes(B, H, ns, rows)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    with torch.cuda.device(dev):
+        st = lib.minf_vs_index_from_lists(v.data_ptr(), v.dtype == torch.int64, nv, vo.data_ptr(), s.data_ptr(), s.dtype == torch.int64,
+                                          ns, so.data_ptr(), *(t.data_ptr() for t in index), B, H, rows, ws.data_ptr(), nbytes,
+                                          _lib.stream_ptr(dev))
+    _lib.check(st, "minf_vs_index_from_lists")
+    return index
 
 
 def vertical_slash_sparse_attention(query, key, value, v_idx, s_idx, block_size_M: int = 64,
@@ -276,10 +304,7 @@ def vertical_slash_sparse_attention(query, key, value, v_idx, s_idx, block_size_
         raise ValueError("only 64x64 blocks are supported")
     _check_qkv(query, key, value)
     B, H, N, _ = query.shape
-    v_idx, s_idx = _sorted_indices(v_idx, s_idx, B, H)
-    if not v_idx.is_cuda:
-        raise RuntimeError("vertical_slash_sparse_attention needs GPU tensors (no CPU path)")
-    bc, bo, cc, ci = _build_index(None, v_idx, s_idx, N, zero_fill=False)
+    bc, bo, cc, ci = _index_from_lists(v_idx, s_idx, B, H, N)
     return vertical_slash_attention_from_index(query, key, value, bc, bo, cc, ci)
 
 

@@ -31,3 +31,24 @@ def test_index_forms_of_the_operator(gpu):
         vo, so = _sorted_indices(t, t, b, h)
         want = t.to(torch.int32).reshape(b, h, -1)
         assert torch.equal(vo, want.sort(-1)[0]) and torch.equal(so, want.sort(-1, descending=True)[0])
+
+
+@pytest.mark.parametrize("n,nv,ns", [(64, 1, 1), (700, 128, 128), (700, 30, 129), (5000, 1024, 1025), (9000, 2049, 2048), (20001, 500, 8192), (20001, 500, 8193),
+                                     (20001, 16384, 16384), (524160, 60, 300), (524224, 60, 300)])      # (the bitmap shares LDS with the lists up to 524160)
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_index_of_unsorted_lists(gpu, n, nv, ns, dtype):
+    """Sorting, tables and row blocks in one call against a call each; offsets beyond the context among them."""
+    from minference_amd.index import _build
+    from minference_amd.ops import _index_from_lists, _sorted_indices
+    print(f"case {n} tokens, {nv} columns, {ns} slashes, {dtype}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(n + ns)
+    v = torch.rand(2, 1, max(n, nv), generator=g, device=gpu).argsort(-1)[..., :nv].to(dtype)
+    s = torch.rand(2, 1, max(n + 100, ns), generator=g, device=gpu).argsort(-1)[..., :ns].to(dtype)
+    s[1, 0] = torch.arange(ns, device=gpu).flip(0).roll(ns // 3)
+    s[:, :, ns // 2] = 0
+    vs, ss = _sorted_indices(v, s, 2, 1)
+    want, got = _build(None, vs, ss, n, zero_fill=False), _index_from_lists(v, s, 2, 1, n)
+    for count, payload in ((0, 1), (2, 3)):
+        assert torch.equal(got[count], want[count])
+        there = torch.arange(want[payload].shape[-1], device=gpu) < want[count][..., None]
+        assert torch.equal(got[payload][there], want[payload][there])
