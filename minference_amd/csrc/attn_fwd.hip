@@ -111,7 +111,7 @@ struct AttnParams {
     // a-shape; query rows >= dense_from attend to every earlier key (tri-shape), INT_MAX = none
     int n_init, n_local, dense_from;
     int descending;          // row blocks are handed out from the last one down
-    int chunk, turn;         // units per deal, whether an XCD takes another place in every round of deals (see launch_hd)
+    int chunk, turn;         // units per deal, whether an XCD takes another place in every round of deals (see plan_launch)
     FastDiv by_deal, by_group, by_groups, by_heads;   // workgroups of a deal; hq / hk; batch x kv groups; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
@@ -286,7 +286,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
     // ---- which (batch, head, row block): XCD-aware remap --------------------
     // Consecutive workgroup ids go round-robin to the 8 XCDs.  Deal number 8 r + x of the launch, the workgroups
     // that share K/V and so an L2 (some neighbouring row-block pairs of the query heads of a kv group), is worked
-    // through by one of them, consecutive deals by different ones (see launch_hd).
+    // through by one of them, consecutive deals by different ones (see plan_launch).
     // (32-bit arithmetic: the launcher refuses grids beyond 2^31 workgroups, and 64-bit divisions of
     // wave-uniform values cost a thousand scalar instructions per workgroup here)
     const int group = (int)p.by_group.d;
@@ -1164,7 +1164,7 @@ __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kerne
 }
 
 // The pattern types of a layer in one launch: workgroups [0, first_bs) walk vertical-slash lists, [first_bs, first_as)
-// block-sparse lists, the rest A-shape windows (each part a multiple of 8 workgroups, see launch_hd).  As three launches
+// block-sparse lists, the rest A-shape windows (each part a multiple of 8 workgroups, see plan_launch).  As three launches
 // each waited for the last walks of the one before on a chip that was emptying.
 // Table of unlike patterns, 32 / 8 heads, whole layer, us: 9000 tokens 774 -> 692, 20000 fp16 1898 -> 1802, of 64 1059 ->
 // 995, 50000 4531 -> 4482, 100000 9316 -> 9243; 28 / 4 heads 20000 tokens 1390 -> 1352; 8 / 2 heads 12000 tokens 331 -> 328.

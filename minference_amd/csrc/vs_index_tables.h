@@ -1,5 +1,5 @@
-// The table pass of the index builder (see vs_index.hip): device code of vs_index_prep_kernel and of the kernel that makes
-// the tables right behind the selection (topk.hip).
+// The table pass of the index builder (see vs_index.hip): device code of vs_index_prep_kernel and of the kernels that make
+// the tables right behind a selection (topk.hip) or a sort (index_sort.hip).
 #pragma once
 #include "minf_common.h"
 
