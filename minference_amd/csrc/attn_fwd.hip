@@ -851,6 +851,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
             probs(1);
             probs(2);
             probs(3);
+            if constexpr (!SUM_LAST) l_i = (l_i * alpha) * alpha + psum;
             if constexpr (VF_AHEAD) {
 #pragma unroll
             for (int s = 0; s < 4; ++s)
@@ -894,12 +895,14 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
         // a v_dot2 as well 41; four in a row 12 in all).  A batch behind each key group's products took, dense, 16384
         // tokens, 32 / 8 heads 1882 us against 1832 (on zeros 1365 : 1315); plain adds of the unpacked halves 2000.
         // (Not at head_dim 256, 7 % slower, whose one wave has nothing else to run meanwhile, and not in the general form
-        // at 64: A-shape, window 512, 1 to 2 % slower.)
+        // at 64: A-shape, window 512, 1 to 2 % slower.  Those add the tile's sum to the row's before the products: behind
+        // them it kept two more values alive through the chain, and tri-shape calls of one 64-wide head that are a chain
+        // of such steps took 22.4 us for 21.3, 1000 tokens, and 54.2 for 51.1, 2816.)
         if constexpr (SUM_LAST) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) psum = pair_sum<T>(pfr[q], psum);
+            l_i = (l_i * alpha) * alpha + psum;
         }
-        l_i = (l_i * alpha) * alpha + psum;
         __builtin_amdgcn_s_setprio(0);
     };
 
@@ -1039,8 +1042,11 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
             for (; it + 1 < split_end; ++it) step(it, std::integral_constant<int, 2>{});
         }
     }
-    // (not in the segments of 64-wide heads: tri-shape, 24000 tokens, 128 dense rows, 117 -> 119 us)
-    if constexpr (!VSP && (HD == 128 || (HD == 64 && !CUT))) {
+    // From one such tile on, at head_dim 64 too: where that form began at eight tiles and was left out of segments, us before
+    // and now, tri-shape with a window of 3968, one head 6000 tokens 75.3 : 64.4, 12000 80.5 : 70.8, 16 heads 24000 461 :
+    // 448; with a window of 512 (five tiles), 16 heads 24000 tokens 116.0 : 115.5; A-shape of that window, 32 / 8 heads,
+    // 48538 tokens 363 : 354.
+    if constexpr (!VSP && HD <= 128) {
         // tiles of which both row blocks see every key, after another such tile and before one that both visit or mask
         const bool causal = MODE == MODE_DENSE || mA * BM >= p.dense_from;
         const bool windowed = MODE == MODE_ASHAPE && mB * BM + BM - 1 < p.dense_from;
@@ -1051,7 +1057,7 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
                 first = max((mB * BM + BM - p.n_local + BN - 1) >> 6, shift + nblk) + 1;
             }
             const int lo = max(first - shift, it_begin + 1), hi = min(mA - 1 - shift, it_end - 1);
-            if (hi - lo >= (HD == 64 ? 8 : 1)) {
+            if (lo < hi) {
                 for (; it < lo; ++it) step(it, std::integral_constant<int, 0>{});
                 for (; it < hi; ++it) step(it, std::integral_constant<int, 3>{});
             }

@@ -30,6 +30,20 @@ def test_split_walks_match_the_oracle(gpu, n, hq, hk, b, d, dtype):
               O.vertical_slash_sparse_attention(q, ke, ve, v_idx.cpu(), s_idx.cpu()), "vertical-slash")
 
 
+@pytest.mark.parametrize("n,hq", [(1300, 1), (1000, 40)])
+@pytest.mark.parametrize("window", [129, 192, 193, 256, 320, 575, 640, 5000])
+def test_short_stretches_of_unmasked_tiles_at_head_dim_64(gpu, n, hq, window):
+    """Windows that leave a walk no, one, a few and more than eight tiles without a masked key, sinks beside them or
+    before them, segments that begin and end among those tiles (one head) and whole walks (forty)."""
+    import minference_amd as M
+    q, k, v = make(1, hq, 1, n, window, torch.float16, 64)
+    qg, kg, vg, one = q.to(gpu), k.to(gpu), v.to(gpu), (slice(None), slice(hq - 1, hq))
+    for n_init in (0, 200):
+        check(M.streaming_forward(qg, kg, vg, n_init, window)[one], O.streaming_forward(q[one], k, v, n_init, window), f"a-shape {n_init}")
+        check(M.tri_shape_forward(qg, kg, vg, n_init, window, 150)[one], O.tri_shape_forward(q[one], k, v, n_init, window, 150), f"tri-shape {n_init}")
+    check(M.dense_causal_attention(qg, kg, vg)[one], sdpa_causal(q[one], k, v), "dense")
+
+
 @pytest.mark.parametrize("op,n,segments", [("ashape", 1024, 2), ("ashape", 2048, 4), ("ashape", 2100, 5), ("ashape", 4000, 8),
                                            ("ashape", 4200, 9), ("ashape", 8192, 16), ("dense", 16000, 6), ("tri", 9000, 18)])
 def test_folds_of_every_number_of_segments(gpu, op, n, segments):
