@@ -112,7 +112,7 @@ struct AttnParams {
     int n_init, n_local, dense_from;
     int descending;          // row blocks are handed out from the last one down
     int chunk, turn;         // units per deal, whether an XCD takes another place in every round of deals (see plan_launch)
-    FastDiv by_deal, by_group, by_groups, by_heads;   // workgroups of a deal; hq / hk; batch x kv groups; kv heads, or chunks of the head list
+    FastDiv by_deal, by_group, by_set, by_chunks, by_heads;   // workgroups of a deal; hq / hk; groups of a set; deals of a group; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
     // every head is processed and index_heads = hq
@@ -293,8 +293,16 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
     unsigned rest = wg >> 3;
     auto next_digit = [&](const FastDiv &f) { const unsigned q = fast_quot(rest, f), r = rest - q * f.d; rest = q; return r; };
     const unsigned in_deal = next_digit(p.by_deal);
+    constexpr bool SETS = MODE == MODE_VS && !CUT;      // (elsewhere all groups are one set)
     rest = 8u * rest + ((wg + rest * (unsigned)p.turn) & 7u);
-    const unsigned gi = next_digit(p.by_groups), first_unit = rest * (unsigned)p.chunk;
+    unsigned gi = next_digit(p.by_set);
+    if constexpr (SETS) {
+        const unsigned deal = next_digit(p.by_chunks);
+        gi += rest * p.by_set.d;
+        if (gi >= (unsigned)p.batch * p.by_heads.d) return false;       // padding of the last round (workgroup-uniform)
+        rest = deal;
+    }
+    const unsigned first_unit = rest * (unsigned)p.chunk;
     rest = in_deal;
     const int hin = (int)next_digit(p.by_group);
     // Dense causal work grows with the row block, so the heavy (late) blocks go first.  The sparse
@@ -1377,7 +1385,7 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.head_list = t->head_list;
     p.index_heads = t->head_list ? t->index_heads : t->heads_q;
     p.chunk = 1; p.turn = 0;      // set by the launcher
-    p.by_deal = p.by_group = p.by_groups = p.by_heads = fast_div(1);      // set by the launcher
+    p.by_deal = p.by_group = p.by_set = p.by_chunks = p.by_heads = fast_div(1);      // set by the launcher
     p.descending = 0;
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
     p.dtype = t->dtype;
@@ -1480,14 +1488,17 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     const int split_pairs = (p.rows + 1) / 2 - p.split_first;
     const long long units = p.split_first + (long long)split_pairs * p.nseg;
     // The launch is a sequence of deals, `chunk` units (row-block pairs, or segments) of one kv group each: the first
-    // units of every group, then the next ones, ...  Consecutive deals go to the 8 XCDs in turn, so every XCD gets an
-    // equal part of every stretch of the sequence, and where it matters (`turn`) of every group: where each worked
-    // through an eighth of the launch (or of a few groups), the one with the longest walks or the densest heads was left
-    // working alone.  32 / 8 heads with a table of unlike patterns, 50000 tokens 5.54 -> 4.60 ms (28 / 4 heads 4.70 ->
+    // units of every group of a set, then the next ones, ..., then the next set.  Consecutive deals go to the 8 XCDs in
+    // turn, so every XCD gets an equal part of every stretch of the sequence, and where it matters (`turn`) of every group:
+    // where each worked through an eighth of the launch (or of a few groups), the one with the longest walks or the densest
+    // heads was left working alone.  32 / 8 heads with a table of unlike patterns, 50000 tokens 5.54 -> 4.60 ms (28 / 4 heads 4.70 ->
     // 3.79), 20000 tokens 2.22 -> 1.86 (1.78 -> 1.40); vertical-slash, 32 / 8 heads, 131072 tokens 14.86 -> 13.96 ms, 500
     // columns and 700 slashes 4.41 -> 4.04 (28 / 4 heads 120000 tokens 3.87 -> 3.08); 9000 tokens, 8 / 2 heads,
     // vertical-slash 359 -> 214 us, block-sparse 318 -> 202, A-shape 224 -> 142.  A launch that fits the chip at
-    // once gains little and may lose (vertical-slash, 4 heads 13000 tokens 214 -> 193 us, 15000 223 -> 220, 16384 212 -> 233).
+    // once gains little and may lose (vertical-slash, 4 heads 13000 tokens 218 -> 186 us, 15000 234 -> 225, 16384 223 -> 232):
+    // there, and at two or three workgroups a slot, it is chance which walks end up last.  In deals of an eighth those three
+    // take 252, 257 and 229, in deals of 8 one group after the other 196, 232 and 201.  8 / 2 heads, 20763 tokens 506 -> 526, in
+    // deals of 8 workgroups 495; but these take 8 heads, 16443 tokens, from 408 to 438 (426 in eighths).  No order serves all.
     // A deal's workgroups share K/V through an L2, but it has to be small beside what an XCD gets in all:
     //  * 32 workgroups for whole layers of vertical-slash lists: 32 / 8 heads, 65000 tokens, 500 columns and 700 slashes, deals
     //    of 16, 32, 64, 128: 2016, 1996, 1991, 1996 us; 16 heads 30000 tokens, of 1, 2, 4, 8, 16: 1710, 1574, 1543, 1523,
@@ -1501,9 +1512,14 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     //  * one unit in dense and split walks.  Dense, 8 / 2 heads 16384 tokens, of 1, 2, 4, 8 units 492, 499, 512, 553 us;
     //  * one head of up to 131072 tokens: an eighth (vertical-slash, 65536 tokens 204 us, in deals of 16 225; 100000
     //    tokens 366 : 394).
-    // turn: an XCD takes another place in every round of deals, so that with 2, 4 or 8 groups it meets all of them.
-    // Heads of a list are unlike, and so are the slashes of a layer's heads: 32 / 8 heads, 65000 tokens, 500 columns, 700
-    // slashes 2.13 -> 1.93 ms.  Equal heads keep an XCD to its groups (A-shape, 70000 tokens 4.44 : 4.58 ms).
+    // turn: an XCD takes another place in every round of deals, so that with 2, 4 or 8 groups it meets all of them.  Heads of a
+    // list are unlike, and so are the slashes of a layer's heads: 32 / 8 heads, 65000 tokens,
+    // 500 columns, 700 slashes 2.13 -> 1.93 ms.  Equal heads keep an XCD to its groups (A-shape, 70000 tokens 4.44 : 4.58 ms).
+    // set: in a batch of more than sixteen groups (of several heads), eight or the next number that divides theirs, where
+    // walks are not split and differ.  An XCD that goes through all the groups with every deal has K/V of as many under way: 8 sequences, 32 / 8
+    // heads, 16000 tokens, 500 columns and 700 slashes 5102 -> 4836 us, 1000 and 6096 11.80 -> 11.42 ms.  The heads of one sequence
+    // go together (32 heads, 100000 tokens, scattered 36.2 : 38.2 ms), so do ungrouped ones (4 times 16, 10000 tokens, 1000 and
+    // 6096 1564 : 1590 us) and split walks (16 heads, 8192 tokens 260 : 281).
     const long long groups = (long long)p.batch * (grid_heads / group);
     const int most = MODE == MODE_BS ? p.max_blocks :
                      MODE == MODE_ASHAPE ? (int)(((long long)p.n_local + p.n_init) / BN) + 2 : p.rows;    // steps of a full walk (lists: unknown)
@@ -1520,11 +1536,16 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     if (MODE != MODE_DENSE && split_pairs == 0 && groups * group == 1 && units <= 1024) chunk = (units + 7) / 8;
     if (chunk > units) chunk = units;
     p.chunk = (int)chunk;
+    const long long deal = chunk * group, chunks = (units + chunk - 1) / chunk, deals = chunks * groups;
+    const bool whole_lists = MODE == MODE_VS && !p.head_list && split_pairs == 0;
+    long long set = groups;
+    if (whole_lists && p.batch > 1 && group > 1 && groups > 16)
+        for (set = 8; groups % set; ++set) {}
     p.turn = p.head_list || MODE == MODE_VS;
-    const long long deal = chunk * group, deals = (units + chunk - 1) / chunk * groups;
     p.by_group = fast_div((unsigned)group);
     p.by_deal = fast_div((unsigned)deal);
-    p.by_groups = fast_div((unsigned)groups);
+    p.by_set = fast_div((unsigned)set);
+    p.by_chunks = fast_div((unsigned)chunks);
     p.by_heads = fast_div((unsigned)(grid_heads / group));
     return (deals + 7) / 8 * 8 * deal;
 }

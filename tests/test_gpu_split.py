@@ -190,11 +190,11 @@ def test_striped_row_blocks_cover_every_row(gpu, hq, hk, n, b):
 
 
 @pytest.mark.parametrize("hq,hk,n,b", [(20, 1, 8300, 1), (6, 3, 8300, 2), (3, 3, 8300, 1), (9, 9, 8500, 1), (1, 1, 66000, 1),
-                                       (2, 1, 66000, 1)])
+                                       (2, 1, 66000, 1), (8, 4, 8300, 6), (6, 3, 8300, 6)])
 def test_heads_do_not_depend_on_how_a_launch_is_dealt(gpu, hq, hk, n, b):
     """Every head of a launch against the head on its own, bit for bit (lengths that are not split): more
-    query heads than a deal has workgroups, batches, deals of an eighth of the launch and of a few pairs, both
-    sides of 512 and 1024 workgroups; the output is full of NaN before, so that no row can be left out."""
+    query heads than a deal has workgroups, batches, groups in two and three sets, deals of an eighth of the launch and
+    of a few pairs, both sides of 512 and 1024 workgroups; the output is full of NaN before, so that no row can be left out."""
     import minference_amd as M
     q, k, v = (t.to(gpu) for t in make(b, hq, hk, n, 7, torch.bfloat16, 64))
     group = hq // hk
