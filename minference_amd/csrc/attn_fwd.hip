@@ -111,7 +111,8 @@ struct AttnParams {
     // a-shape; query rows >= dense_from attend to every earlier key (tri-shape), INT_MAX = none
     int n_init, n_local, dense_from;
     int descending;          // row blocks are handed out from the last one down
-    int chunk, turn;         // units per deal, whether an XCD takes another place in every round of deals (see plan_launch)
+    int chunk, turn;         // units per deal; an XCD takes another place every 2^turn rounds of deals, 31: never (see plan_launch)
+    int far_turn;            // the same where most heads keep more than an eighth of the blocks, 0: as elsewhere
     FastDiv by_deal, by_group, by_set, by_chunks, by_heads;   // workgroups of a deal; hq / hk; groups of a set; deals of a group; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
@@ -294,7 +295,15 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
     auto next_digit = [&](const FastDiv &f) { const unsigned q = fast_quot(rest, f), r = rest - q * f.d; rest = q; return r; };
     const unsigned in_deal = next_digit(p.by_deal);
     constexpr bool SETS = MODE == MODE_VS && !CUT;      // (elsewhere all groups are one set)
-    rest = 8u * rest + ((wg + rest * (unsigned)p.turn) & 7u);
+    int turn = p.turn;
+    if constexpr (SETS) {
+        if (p.far_turn) {                                // up to 64 heads' last rows: the same answer in every workgroup
+            const int heads = min(p.hq, 64), head = minf_lane();
+            const bool far = head < heads && p.bc[(head + 1ll) * p.rows - 1] > p.rows >> 3;
+            if (2 * __builtin_popcountll(__ballot(far)) > heads) turn = p.far_turn;
+        }
+    }
+    rest = 8u * rest + ((wg + (rest >> turn)) & 7u);
     unsigned gi = next_digit(p.by_set);
     if constexpr (SETS) {
         const unsigned deal = next_digit(p.by_chunks);
@@ -1384,7 +1393,7 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.n_init = p.n_local = 0; p.dense_from = 0x7fffffff;
     p.head_list = t->head_list;
     p.index_heads = t->head_list ? t->index_heads : t->heads_q;
-    p.chunk = 1; p.turn = 0;      // set by the launcher
+    p.chunk = 1; p.turn = p.far_turn = 0;      // set by the launcher
     p.by_deal = p.by_group = p.by_set = p.by_chunks = p.by_heads = fast_div(1);      // set by the launcher
     p.descending = 0;
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
@@ -1512,9 +1521,17 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     //  * one unit in dense and split walks.  Dense, 8 / 2 heads 16384 tokens, of 1, 2, 4, 8 units 492, 499, 512, 553 us;
     //  * one head of up to 131072 tokens: an eighth (vertical-slash, 65536 tokens 204 us, in deals of 16 225; 100000
     //    tokens 366 : 394).
-    // turn: an XCD takes another place in every round of deals, so that with 2, 4 or 8 groups it meets all of them.  Heads of a
-    // list are unlike, and so are the slashes of a layer's heads: 32 / 8 heads, 65000 tokens,
+    // turn: an XCD takes another place from time to time, so that with 2, 4 or 8 groups it meets all of them.  Heads of a
+    // list are unlike (another place in every round), and so are the slashes of a layer's heads: 32 / 8 heads, 65000 tokens,
     // 500 columns, 700 slashes 2.13 -> 1.93 ms.  Equal heads keep an XCD to its groups (A-shape, 70000 tokens 4.44 : 4.58 ms).
+    // But while it keeps its place, it works on neighbours of one group, and lists of scattered slashes live on neighbours
+    // that reach a tile at the same time: 600 scattered slashes, 32 / 8 heads, 131072 tokens, another place in every round and
+    // every 2, 4, 8, 16, never: 59.7, 59.2, 59.2, 58.3, 56.5, 56.0 ms.  Lists of neighbouring diagonals gain nothing by it and lose
+    // the balance: 500 columns and 700 slashes, 131072 tokens 3.81, 3.80, 3.80, 3.82, 3.86, 4.00 ms, 100000 tokens 2.63, 2.65,
+    // 2.66, 2.74, 2.78, 2.93 (1000 and 6096, 131072 tokens 13.16, 13.16, 13.19, 13.19, 13.18, 13.35).  So a launch of 48 rounds and
+    // more goes through the eight places once, in steps of a power of two, if most of its heads keep more than an eighth of
+    // the blocks in the last row (scattered 26 % of all blocks, 1000 and 6096 11 %, 500 and 700 3 %): the workgroups see that
+    // from the counts.  Where a place is no single group's it stays as it was (16 heads, scattered, 25.2 : 25.7 ms).
     // set: in a batch of more than sixteen groups (of several heads), eight or the next number that divides theirs, where
     // walks are not split and differ.  An XCD that goes through all the groups with every deal has K/V of as many under way: 8 sequences, 32 / 8
     // heads, 16000 tokens, 500 columns and 700 slashes 5102 -> 4836 us, 1000 and 6096 11.80 -> 11.42 ms.  The heads of one sequence
@@ -1541,7 +1558,10 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     long long set = groups;
     if (whole_lists && p.batch > 1 && group > 1 && groups > 16)
         for (set = 8; groups % set; ++set) {}
-    p.turn = p.head_list || MODE == MODE_VS;
+    p.turn = p.head_list || MODE == MODE_VS ? 0 : 31;
+    p.far_turn = 0;
+    if (whole_lists && 8 % set == 0 && chunks * set >= 8 * 48)
+        while (2ll << p.far_turn <= chunks * set / 64) ++p.far_turn;
     p.by_group = fast_div((unsigned)group);
     p.by_deal = fast_div((unsigned)deal);
     p.by_set = fast_div((unsigned)set);

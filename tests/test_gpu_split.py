@@ -215,6 +215,31 @@ def test_heads_do_not_depend_on_how_a_launch_is_dealt(gpu, hq, hk, n, b):
                 assert torch.equal(f(q[i], k[j], v[j], i, None), out[i]), (name, bb, h)
 
 
+@pytest.mark.parametrize("hq,hk,n,b,far", [(32, 8, 48100, 1, 40), (32, 8, 49000, 1, 40), (32, 8, 49000, 1, 16), (32, 8, 49000, 1, 0), (66, 2, 26000, 1, 66),
+                                           (16, 2, 98400, 1, 9), (24, 24, 66000, 1, 24), (16, 4, 30000, 7, 0)])
+def test_long_launches_are_dealt_whole(gpu, hq, hk, n, b, far):
+    """Launches just below and above 48 rounds of deals, from where on XCDs keep their place for some rounds if more than half of
+    the (first 64) heads keep an eighth of the blocks (`far` heads do), one set of groups and several: some heads
+    on their own, bit for bit, and no row left out."""
+    import minference_amd as M
+    print(f"case {hq} / {hk} heads, {n} tokens, batch {b}, {far} far", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    q, k, v = (torch.randn(b, h, n, 64, generator=g, device=gpu, dtype=torch.bfloat16) for h in (hq, hk, hk))
+    ns = n // 64 // 6
+    vi = torch.arange(40, device=gpu, dtype=torch.int32).repeat(b, hq, 1) * 7
+    si = torch.arange(ns, device=gpu, dtype=torch.int32).flip(0).repeat(b, hq, 1)
+    si[:, :far] *= 256                                  # (blocks of their own, the others of one band)
+    ix = M.index._build(None, vi, si.contiguous(), n, zero_fill=False)
+    assert int((ix[0][0, :, -1] > (n + 63) // 64 // 8).sum()) == min(far, hq)
+    out = torch.full_like(q, float("nan"))
+    M.ops.vertical_slash_attention_from_index(q, k, v, *ix, out=out)
+    assert torch.isfinite(out).all()
+    for bb, h in ((0, 0), (0, hq // 2 + 1), (b - 1, 1), (b - 1, hq - 1)):
+        i, j = (slice(bb, bb + 1), slice(h, h + 1)), (slice(bb, bb + 1), slice(h // (hq // hk), h // (hq // hk) + 1))
+        one = M.ops.vertical_slash_attention_from_index(q[i], k[j], v[j], *(t[i].contiguous() for t in ix))
+        assert torch.equal(one, out[i]), (bb, h)
+
+
 @pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16)])
 def test_a_nan_key_reaches_every_row_that_attends_to_it(gpu, d, dtype):
     """The row sum of a segment with a NaN score is NaN: the fold keeps it, as a whole walk's rows are NaN,
