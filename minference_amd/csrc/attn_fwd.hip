@@ -1532,6 +1532,8 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     // more goes through the eight places once, in steps of a power of two, if most of its heads keep more than an eighth of
     // the blocks in the last row (scattered 26 % of all blocks, 1000 and 6096 11 %, 500 and 700 3 %): the workgroups see that
     // from the counts.  Where a place is no single group's it stays as it was (16 heads, scattered, 25.2 : 25.7 ms).
+    // Split walks: every round, but eight groups of one head, every fourth: 8192 tokens, 500 columns and 700 slashes 101 ->
+    // 89.5 us, 6000 85.9 -> 83.8 (32 / 8 heads, 6000, 187 : 194).
     // set: in a batch of more than sixteen groups (of several heads), eight or the next number that divides theirs, where
     // walks are not split and differ.  An XCD that goes through all the groups with every deal has K/V of as many under way: 8 sequences, 32 / 8
     // heads, 16000 tokens, 500 columns and 700 slashes 5102 -> 4836 us, 1000 and 6096 11.80 -> 11.42 ms.  The heads of one sequence
@@ -1562,6 +1564,7 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     p.far_turn = 0;
     if (whole_lists && 8 % set == 0 && chunks * set >= 8 * 48)
         while (2ll << p.far_turn <= chunks * set / 64) ++p.far_turn;
+    if (MODE == MODE_VS && !p.head_list && split_pairs > 0 && groups == 8 && group == 1) p.turn = 2;
     p.by_group = fast_div((unsigned)group);
     p.by_deal = fast_div((unsigned)deal);
     p.by_set = fast_div((unsigned)set);

@@ -175,11 +175,11 @@ def test_split_walks_of_narrow_lists(gpu, n, hq, top_k, nv, ns):
           O.vertical_slash_sparse_attention(q, k, v, vi, si), "vertical-slash")
 
 
-@pytest.mark.parametrize("hq,hk,n,b", [(3, 1, 900, 1), (6, 3, 700, 2), (10, 5, 13400, 1)])
-def test_striped_row_blocks_cover_every_row(gpu, hq, hk, n, b):
-    """Head counts that do not divide among the eight XCDs: the row-block pairs are dealt out in stripes
-    with a padded last round; with V = 1 every row of every head must come out as exactly 1 (the last
-    size also reaches the striped list walks: ten heads, 105 pairs)."""
+@pytest.mark.parametrize("hq,hk,n,b", [(3, 1, 900, 1), (6, 3, 700, 2), (10, 5, 13400, 1), (8, 8, 1500, 1), (4, 4, 6000, 2), (8, 8, 8192, 1)])
+def test_deals_cover_every_row(gpu, hq, hk, n, b):
+    """Head counts that do not divide among the eight XCDs, whose last round of deals is padded, and eight groups of one
+    head, whose split walks change XCD every fourth round: with V = 1 every row of every head must come out as
+    exactly 1 (ten heads, 105 pairs: list walks that are not split)."""
     import minference_amd as M
     q, k, _ = make(b, hq, hk, n, 3, torch.bfloat16)
     qg, kg = q.to(gpu), k.to(gpu)
