@@ -112,8 +112,7 @@ struct AttnParams {
     int n_init, n_local, dense_from;
     int descending;          // row blocks are handed out from the last one down
     int chunk, turn;         // units per deal; an XCD takes another place every 2^turn rounds of deals, 31: never (see plan_launch)
-    int far_turn;            // the same where most heads keep more than an eighth of the blocks, 0: as elsewhere
-    FastDiv by_deal, by_group, by_set, by_chunks, by_heads;   // workgroups of a deal; hq / hk; groups of a set; deals of a group; kv heads, or chunks of the head list
+    FastDiv by_deal, by_group, by_set, by_heads;   // workgroups of a deal; hq / hk; groups of a set; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
     // every head is processed and index_heads = hq
@@ -125,6 +124,10 @@ struct AttnParams {
     char *part;
     int dtype;               // MINF_BF16, MINF_F16 or MINF_16BIT_SELECT
     const int *select;       // not null: this launch is one of two, and only the one for dtype *select does anything
+    // whole list walks only.  Behind the rest: every workgroup starts with a chain of reads of these arguments, and with
+    // the two in front the others' lay across one more cache line (A-shape, window 64, fp32 tensors, 32 / 8 heads, 65536 tokens 1185 : 1203 us)
+    FastDiv by_chunks;       // deals of a group
+    int far_turn;            // turn where most heads keep more than an eighth of the blocks, 0: as elsewhere
 };
 
 // Split walks.  A launch whose row-block pairs cannot fill the chip, or whose longest walks would outlast
