@@ -3,13 +3,19 @@
 // The attention kernels compute on 16-bit operands with fp32 accumulation (the reference picks fp16 operands for
 // every input that is not bf16, pit_sparse_flash_attention_v2.py:175).  fp32 q/k/v become fp16 when the
 // largest |value| of the three lies in [2^-10, 32768], else bf16 (fp16 would overflow, or flush most of
-// the tensor).  The choice is made here, on the device: a first kernel converts to fp16 and leaves the largest |value|
-// of each of its workgroups, every workgroup of the second one folds those, one of them leaves the dtype code
-// that the attention launches and the widening kernel read (minf_qkvo.dtype_select), and where the code is bf16 they
-// convert once more, over what the first kernel wrote.  Bound by bytes: q, k and v are read and written once.
+// the tensor).  The choice is made here, on the device: a first kernel converts, to fp16 or, in large tensors, to the
+// format that one or two rows of each ask for, and leaves the largest |value| of each of its workgroups, every workgroup of
+// the second one folds those, one of them leaves the dtype code that the attention launches and the widening kernel
+// read (minf_qkvo.dtype_select), and where the code is not the format written they convert once more, over what the first
+// kernel wrote.  Bound by bytes: q, k and v are read and written once.
 // With a pass for the largest |value| alone before the conversion (8192 tokens, 4 heads of 128, 3 x 16.8 MB)
-// the two took 9.0 + 13.4 us, now 13.6 + 3.7; 32768 tokens, 16 heads 365 -> 223, 65536 tokens, 32 / 8 heads 744 -> 446,
-// 5.4 TB/s.  Tensors that do need bf16 pay for the second conversion: 366 -> 450 and 743 -> 1008.
+// the two took 22.2 us, now 15.1; 32768 tokens, 16 heads 363 -> 223, 65536 tokens, 32 / 8 heads 741 -> 447, 5.4 TB/s.
+// Tensors that need bf16 took, with that pass, converted to fp16 whatever the values, and sampled first: 8192 tokens, 4
+// heads 22.2, 26.8, 15.7 us, 32 / 8 heads 75.7, 122, 53.4, 32768 tokens, 16 heads 366, 451, 223, 65536 tokens, 32 / 8 heads
+// 744, 1007, 448.  The sample lengthens a conversion by one to two microseconds all the same (it is on its way behind the first
+// step's loads, at addresses from the host; an operator's call on 5000 tokens, 8 / 2 heads, 123.9 -> 125.8), so smaller
+// tensors, for which a second conversion costs 5 to 12, go without.  Where it does not show what the tensors ask for, one value
+// above 32768, they are converted twice: 102, 443 and 886 us.
 // With the choice read back by the host (three reductions, a synchronisation, three conversions) the GPU
 // idled about 60 us per call.
 #include "minf_common.h"
@@ -20,6 +26,7 @@ constexpr int NARROW_THREADS = 256;
 constexpr int UNDER_WAY = 2;     // steps of 8 elements a thread has under way
 constexpr int NARROW_PARTIALS = MINF_NARROW_WORKSPACE_INTS - 1;      // workgroups of a launch, a third per tensor
 constexpr int NARROW_WGS = NARROW_PARTIALS / 3;
+constexpr long long SAMPLED_FROM = 1 << 20;      // vectors of the largest tensor
 static_assert(NARROW_WGS * 3 == NARROW_PARTIALS, "the same number of workgroups for each tensor");
 
 struct NarrowTensor {
@@ -28,11 +35,13 @@ struct NarrowTensor {
     long long stride[3];         // elements: batch, head, token
     long long rows;              // batch * heads * n
     int heads;
+    const float *sample;         // the rows that are looked at first: the first one, elements from one to the next
+    long long sample_step;
     FastDiv by_n, by_heads;
 };
 struct NarrowParams {
     NarrowTensor t[3];
-    int dim;
+    int dim, sampled, lanes_log2;      // whether rows are looked at first, lanes that read one
     FastDiv by_dim_out;          // vectors of 8 elements per output row
     int *ws;                     // [0]: the dtype code, then the partial maxima (bit patterns)
 };
@@ -59,51 +68,97 @@ __device__ __forceinline__ unsigned wg_max(unsigned m, unsigned (&part)[NARROW_T
     return m;
 }
 
-// One pass over a workgroup's share of a tensor, 8 output elements per thread and step, converted to T and written;
-// the largest bit pattern of |x| read.
-template <typename T, typename I> __device__ __forceinline__ unsigned convert_share(const NarrowParams &p, const NarrowTensor &t) {
-    const I total = (I)t.rows * p.by_dim_out.d, step = (I)NARROW_WGS * NARROW_THREADS;
-    unsigned m = 0;
-    for (I i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x; i < total; i += UNDER_WAY * step) {
-        float4 x[UNDER_WAY][2];
-        I at[UNDER_WAY];
+// bit patterns of the largest and smallest |x| that a tensor's largest may be for fp16
+constexpr unsigned MOST_F16 = 0x47000000u, LEAST_F16 = 0x3a800000u;      // 32768, 2^-10
+
+// Loads of one step: UNDER_WAY vectors of 8 elements from number i on.
+template <typename I> struct Step {
+    float4 x[UNDER_WAY][2];
+    I at[UNDER_WAY];
+};
+template <typename I> __device__ __forceinline__ void load_step(const NarrowParams &p, const NarrowTensor &t, I i, I total, Step<I> &s) {
+    const I step = (I)NARROW_WGS * NARROW_THREADS;
 #pragma unroll
-        for (int u = 0; u < UNDER_WAY; ++u) {
-            at[u] = min(i + u * step, total - 1);      // (the last vector again, past the end)
-            int d;
-            const float *src = vector_ptr<I>(t, p.by_dim_out, 8, at[u], d);
+    for (int u = 0; u < UNDER_WAY; ++u) {
+        s.at[u] = min(i + u * step, total - 1);        // (the last vector again, past the end)
+        int d;
+        const float *src = vector_ptr<I>(t, p.by_dim_out, 8, s.at[u], d);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) x[u][h] = d + 4 * h < p.dim ? *reinterpret_cast<const float4 *>(src + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int h = 0; h < 2; ++h) s.x[u][h] = d + 4 * h < p.dim ? *reinterpret_cast<const float4 *>(src + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+}
+// converted to T and written; -> the largest bit pattern of |x| read, or m
+template <typename T, typename I> __device__ __forceinline__ unsigned store_step(const NarrowTensor &t, const Step<I> &s, unsigned m) {
+#pragma unroll
+    for (int u = 0; u < UNDER_WAY; ++u) {
+        const float v[8] = {s.x[u][0].x, s.x[u][0].y, s.x[u][0].z, s.x[u][0].w, s.x[u][1].x, s.x[u][1].y, s.x[u][1].z, s.x[u][1].w};
+        union { T e[8]; uint4 u4; } o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            o.e[e] = (T)v[e];
+            m = max(m, __float_as_uint(v[e]) & 0x7fffffffu);
         }
-#pragma unroll
-        for (int u = 0; u < UNDER_WAY; ++u) {
-            const float v[8] = {x[u][0].x, x[u][0].y, x[u][0].z, x[u][0].w, x[u][1].x, x[u][1].y, x[u][1].z, x[u][1].w};
-            union { T e[8]; uint4 u4; } o;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                o.e[e] = (T)v[e];
-                m = max(m, __float_as_uint(v[e]) & 0x7fffffffu);
-            }
-            *reinterpret_cast<uint4 *>(t.out + (long long)at[u] * 16) = o.u4;
-        }
+        *reinterpret_cast<uint4 *>(t.out + (long long)s.at[u] * 16) = o.u4;
     }
     return m;
 }
 
+// One pass over a workgroup's share of a tensor from number i on, the step at i loaded; the largest bit pattern of |x| read.
+template <typename T, typename I> __device__ __forceinline__ unsigned convert_share(const NarrowParams &p, const NarrowTensor &t, I i, I total, Step<I> &s) {
+    unsigned m = 0;
+    while (i < total) {
+        m = store_step<T, I>(t, s, m);
+        i += (I)UNDER_WAY * NARROW_WGS * NARROW_THREADS;
+        if (i < total) load_step<I>(p, t, i, total, s);
+    }
+    return m;
+}
+
+// The sampled rows of each tensor (their first 256 values, a vector per lane), and whether they ask for fp16: the same answer
+// in every wavefront.
+struct Sample { uint4 x[3]; };
+__device__ __forceinline__ Sample load_sample(const NarrowParams &p) {
+    Sample s;
+    const int lane = minf_lane(), d = 4 * min(lane & ((1 << p.lanes_log2) - 1), p.dim / 4 - 1);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) s.x[i] = *reinterpret_cast<const uint4 *>(p.t[i].sample + (lane >> p.lanes_log2) * p.t[i].sample_step + d);
+    return s;
+}
+__device__ __forceinline__ bool takes_f16(const Sample &s) {
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        m = max(max(max(m, s.x[i].x & 0x7fffffffu), s.x[i].y & 0x7fffffffu), max(s.x[i].z & 0x7fffffffu, s.x[i].w & 0x7fffffffu));
+    return __any(m >= LEAST_F16) && !__any(m > MOST_F16);
+}
+
+// leaves the largest bit pattern it read, with the sign bit where it wrote bf16
 template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_kernel(const NarrowParams p) {
     __shared__ unsigned part[NARROW_THREADS / 64];
-    const unsigned m = wg_max(convert_share<_Float16, I>(p, p.t[blockIdx.y]), part);
-    if (threadIdx.x == 0) p.ws[1 + blockIdx.y * NARROW_WGS + blockIdx.x] = (int)m;
+    const NarrowTensor &t = p.t[blockIdx.y];
+    const I total = (I)t.rows * p.by_dim_out.d, i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x;
+    Step<I> s;
+    load_step<I>(p, t, min(i, total - 1), total, s);                     // (under way before the sample is looked at)
+    const bool f16 = !p.sampled || takes_f16(load_sample(p));
+    const unsigned m = wg_max(f16 ? convert_share<_Float16, I>(p, t, i, total, s) : convert_share<__bf16, I>(p, t, i, total, s), part);
+    if (threadIdx.x == 0) p.ws[1 + blockIdx.y * NARROW_WGS + blockIdx.x] = (int)(f16 ? m : m | 0x80000000u);
 }
 
 template <typename I> __global__ __launch_bounds__(NARROW_THREADS) void narrow_choose_kernel(const NarrowParams p) {
     __shared__ unsigned part[NARROW_THREADS / 64];
     unsigned m = 0;
-    for (int i = (int)threadIdx.x; i < NARROW_PARTIALS; i += NARROW_THREADS) m = max(m, (unsigned)p.ws[1 + i]);
+    for (int i = (int)threadIdx.x; i < NARROW_PARTIALS; i += NARROW_THREADS) m = max(m, (unsigned)p.ws[1 + i] & 0x7fffffffu);
+    const bool is_f16 = p.ws[1] >= 0;
     m = wg_max(m, part);
-    const bool f16 = m >= __float_as_uint(0x1p-10f) && m <= __float_as_uint(32768.0f);
+    const bool f16 = m >= LEAST_F16 && m <= MOST_F16;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.ws[0] = f16 ? MINF_F16 : MINF_BF16;
-    if (!f16) convert_share<__bf16, I>(p, p.t[blockIdx.y]);
+    if (f16 == is_f16) return;
+    const NarrowTensor &t = p.t[blockIdx.y];
+    const I total = (I)t.rows * p.by_dim_out.d, i = (I)blockIdx.x * NARROW_THREADS + threadIdx.x;
+    Step<I> s;
+    if (i < total) load_step<I>(p, t, i, total, s);
+    if (f16) convert_share<_Float16, I>(p, t, i, total, s);
+    else convert_share<__bf16, I>(p, t, i, total, s);
 }
 
 __global__ __launch_bounds__(NARROW_THREADS) void widen_kernel(const char *__restrict__ in, float *__restrict__ out, long long rows,
@@ -139,6 +194,9 @@ extern "C" int minf_narrow_qkv(const minf_qkvo *t, int dim_in, void *q16, void *
     const void *in[3] = {t->q, t->k, t->v};
     void *out[3] = {q16, k16, v16};
     const int64_t *strides[3] = {t->q_stride, t->k_stride, t->v_stride};
+    p.dim = dim_in;
+    p.lanes_log2 = 0;
+    while (p.lanes_log2 < 6 && 4 << p.lanes_log2 < dim_in) ++p.lanes_log2;
     for (int i = 0; i < 3; ++i) {
         if ((((uintptr_t)in[i]) | ((uintptr_t)out[i])) & 15) return MINF_ERR_ALIGNMENT;
         for (int j = 0; j < 3; ++j) {
@@ -149,15 +207,19 @@ extern "C" int minf_narrow_qkv(const minf_qkvo *t, int dim_in, void *q16, void *
         p.t[i].out = (char *)out[i];
         p.t[i].heads = i == 0 ? t->heads_q : t->heads_kv;
         p.t[i].rows = (long long)t->batch * p.t[i].heads * t->n;
+        // as many rows as a wavefront holds: the middle head's tokens, evenly spread from the middle one to the last
+        const long long head = (long long)t->batch * p.t[i].heads / 2, sampled = 64ll >> p.lanes_log2;
+        p.t[i].sample = p.t[i].in + head / p.t[i].heads * strides[i][0] + head % p.t[i].heads * strides[i][1] + t->n / 2 * strides[i][2];
+        p.t[i].sample_step = sampled > 1 ? (t->n - 1 - t->n / 2) / (sampled - 1) * strides[i][2] : 0;
         p.t[i].by_n = fast_div((unsigned)t->n);
         p.t[i].by_heads = fast_div((unsigned)p.t[i].heads);
     }
-    p.dim = dim_in;
     p.by_dim_out = fast_div((unsigned)t->head_dim / 8u);
     p.ws = workspace;
     hipStream_t st = (hipStream_t)stream;
     // (multiplications place numbers below 2^31, and so must the steps past the end be)
     const long long most = p.t[0].rows > p.t[1].rows ? p.t[0].rows : p.t[1].rows;
+    p.sampled = most * p.by_dim_out.d >= SAMPLED_FROM;
     const bool small = most * p.by_dim_out.d < 0x7fffffffLL - 2ll * UNDER_WAY * NARROW_WGS * NARROW_THREADS;
     const dim3 grid(NARROW_WGS, 3), block(NARROW_THREADS);
     if (small) hipLaunchKernelGGL(narrow_kernel<unsigned>, grid, block, 0, st, p);

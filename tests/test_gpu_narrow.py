@@ -74,6 +74,46 @@ def test_the_largest_value_is_found_wherever_it_lies(gpu, n, layout):
         v[0, h, t, d] = old
 
 
+@pytest.mark.parametrize("where", ["nowhere", "one channel", "all of q", "from the middle of k on", "first rows", "last row", "one wavefront of many steps",
+                                   "a tail", "tiny", "tiny middle head", "zero middle head", "large middle row"])
+def test_the_rows_looked_at_first_do_not_decide(gpu, where):
+    """Nine steps of a workgroup (eight whole ones and a tail), and the middle head's rows, by some of which the first conversion
+    goes: values that ask for bf16 in all of them, in other rows, in them alone, in the vector that several threads write past
+    the end; rows that ask for bf16 in tensors that do not."""
+    import minference_amd as M
+    n = 8 * 1024 + 3
+    g = torch.Generator(device=gpu).manual_seed(3)
+    q, k, v = (torch.randn(1, 8, n, 128, device=gpu, generator=g) for _ in range(3))
+    dtype = torch.float16 if where == "nowhere" else torch.bfloat16
+    if where == "one channel":
+        k[..., 5] *= 1e5
+    elif where == "all of q":
+        q *= 1e6
+    elif where == "from the middle of k on":
+        k[:, 4:] *= 1e6
+    elif where == "first rows":
+        v[:, 0, :3] = 1e5
+    elif where == "last row":
+        v[0, 7, n - 1, 127] = -1e30
+    elif where == "one wavefront of many steps":
+        q[0, 3, 7, 8:16] = float("inf")
+        q[0, 7, 8000, 3] = 5e4
+    elif where == "a tail":
+        q[0, 7, n - 3:] = 4e4
+        v[0, 7, n - 1] = 0
+    elif where == "tiny":
+        q, k, v = q * 1e-6, k * 1e-6, v * 1e-6
+    elif where == "large middle row":
+        k[0, 4, n // 2, 127] = 1e9
+    elif where.endswith("middle head"):
+        dtype = torch.float16
+        for t in (q, k, v):
+            t[0, 4] *= 1e-7 if where.startswith("tiny") else 0
+    want = M.streaming_forward(q.to(dtype), k.to(dtype), v.to(dtype), 16, 100).float()
+    for _ in range(2):
+        assert torch.equal(M.streaming_forward(q, k, v, 16, 100).nan_to_num(7.0), want.nan_to_num(7.0))
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_values_that_are_no_numbers_choose_bf16(gpu, bad):
     import minference_amd as M
