@@ -34,7 +34,8 @@ def test_index_forms_of_the_operator(gpu):
 
 
 @pytest.mark.parametrize("n,nv,ns", [(64, 1, 1), (700, 128, 128), (700, 30, 129), (5000, 1024, 1025), (9000, 2049, 2048), (20001, 500, 8192), (20001, 500, 8193),
-                                     (20001, 16384, 16384), (524160, 60, 300), (524224, 60, 300)])      # (the bitmap shares LDS with the lists up to 524160)
+                                     (20001, 16384, 16384), (524160, 60, 300), (524224, 60, 300),       # (the bitmap shares LDS with the lists up to 524160)
+                                     (524160, 16384, 16384), (524224, 300, 16384), (524160, 8193, 8192)])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 def test_index_of_unsorted_lists(gpu, n, nv, ns, dtype):
     """Sorting, tables and row blocks in one call against a call each; offsets beyond the context among them."""

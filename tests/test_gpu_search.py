@@ -173,6 +173,49 @@ def test_recall_tiles_stripes_and_flag_mixes(gpu, n, hq, hk, begin, d):
     assert np.abs(got[:, 7] - 1.0).max() <= 1e-6             # a window of all offsets keeps everything
 
 
+@pytest.mark.parametrize("n,hq,hk", [(1500, 3, 1), (97, 2, 2), (4100, 1, 1)])
+def test_long_searches_set_the_same_flags(gpu, monkeypatch, n, hq, hk):
+    """Contexts beyond the kernels that write flag bytes at once (32768 tokens; 4096 block rows) set them candidate by
+    candidate in zeroed arrays: the same recall with those limits at zero, two block-sparse candidates (the first one
+    clears) and all kinds among them."""
+    from minference_amd import _lib, pattern_recall
+    q, k = (t.to(gpu) for t in heads(n, hq, hk, 5 + n))
+    cands = [("vertical_and_slash", 40, 60), ("block_sparse", 4, 1), ("stream_llm", 4, 64), ("block_sparse", 16, 1), ("stream_llm", 0, 0),
+             ("vertical_and_slash", n, 30), ("stream_llm", n + 5, 3), ("block_sparse", 2, 1)]
+    cands = [c for c in cands if c[0] != "block_sparse" or c[1] <= (n + 31) // 32]
+    for chosen in (cands, cands[1:2], cands[2:3]):
+        monkeypatch.setattr(_lib, "MINF_SEARCH_FLAGS_MAX", 32768)
+        monkeypatch.setattr(_lib, "MINF_SEARCH_BLOCK_FLAGS_MAX", 4096)
+        want = pattern_recall(q, k, chosen, 10)
+        for name in ("MINF_SEARCH_FLAGS_MAX", "MINF_SEARCH_BLOCK_FLAGS_MAX"):
+            monkeypatch.setattr(_lib, name, 0)
+            assert torch.equal(pattern_recall(q, k, chosen, 10), want), name
+
+
+@pytest.mark.parametrize("n", [32768, 32769])
+def test_recall_on_both_sides_of_the_flag_kernels_limit(gpu, n):
+    """The last 70 rows of one head against fp64 sums over flags made of the same scores with torch.  Both sums of a row are
+    fp32 sums of about n / 64 block sums, each with a rounding of at most 2^-24."""
+    from minference_amd import pattern_recall, vertical_slash_scores
+    g = torch.Generator(device=gpu).manual_seed(n)
+    q, k = (torch.randn(1, 1, n, 128, device=gpu, generator=g).bfloat16() for _ in range(2))
+    begin = n - 70
+    cands = [("vertical_and_slash", 100, 300), ("stream_llm", 9, 1000), ("vertical_and_slash", 1000, 30), ("vertical_and_slash", 31, 6096)]
+    got = pattern_recall(q, k, cands, begin)[0, 0]
+    vertical, slash = (x[0, 0] for x in vertical_slash_scores(q, k, 64, 30, 30, reference_rounding=False))
+    r, c = torch.arange(begin, n, device=gpu)[:, None], torch.arange(n, device=gpu)[None]
+    s = q[0, 0, begin:].double() @ k[0, 0].double().t().contiguous() * 128 ** -0.5
+    p = torch.softmax(s.masked_fill(c > r, float("-inf")), -1)
+    for t, (kind, a, b) in enumerate(cands):
+        col, diag = (torch.zeros(n, dtype=torch.bool, device=gpu) for _ in range(2))
+        if kind == "stream_llm":
+            col[:a], diag[:b + 1] = True, True
+        else:
+            col[torch.topk(vertical, a).indices], diag[n - 1 - torch.topk(slash, b).indices] = True, True
+        want = float((p * (col[None] | diag[(r - c).clamp(min=0)])).sum() / (n - begin))
+        assert abs(float(got[t]) - want) <= 2 * (n / 64 + 64) * 2.0 ** -24 * want, (t, float(got[t]), want)
+
+
 @pytest.mark.parametrize("n,dtype", [(1500, torch.bfloat16), (3001, torch.float16)])
 def test_recall_keeps_fp32_accuracy(gpu, n, dtype):
     """Against fp64 sums on the same operands, all candidates with the largest keys: exponentials of 24 bits, fp32 row sums whose roundings average
