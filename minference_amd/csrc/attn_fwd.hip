@@ -93,6 +93,7 @@ constexpr int QK_AHEAD = 2;
 #endif
 constexpr int VALU_MASK = 0x402;             // sched_group_barrier classes: VALU | transcendental
 
+constexpr int TURN_CHOSEN = 32;              // every round, or every 2^far_turn
 struct AttnParams {
     const char *q, *k, *v;
     char *o;
@@ -111,7 +112,7 @@ struct AttnParams {
     // a-shape; query rows >= dense_from attend to every earlier key (tri-shape), INT_MAX = none
     int n_init, n_local, dense_from;
     int descending;          // row blocks are handed out from the last one down
-    int chunk, turn;         // units per deal; an XCD takes another place every 2^turn rounds of deals, 31: never (see plan_launch)
+    int chunk, turn;         // units per deal; an XCD takes another place every 2^turn rounds of deals, 31: never, or TURN_CHOSEN (see plan_launch)
     FastDiv by_deal, by_group, by_set, by_heads;   // workgroups of a deal; hq / hk; groups of a set; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
@@ -124,10 +125,10 @@ struct AttnParams {
     char *part;
     int dtype;               // MINF_BF16, MINF_F16 or MINF_16BIT_SELECT
     const int *select;       // not null: this launch is one of two, and only the one for dtype *select does anything
-    // whole list walks only.  Behind the rest: every workgroup starts with a chain of reads of these arguments, and with
+    // turn == TURN_CHOSEN only.  Behind the rest: every workgroup starts with a chain of reads of these arguments, and with
     // the two in front the others' lay across one more cache line (A-shape, window 64, fp32 tensors, 32 / 8 heads, 65536 tokens 1185 : 1203 us)
     FastDiv by_chunks;       // deals of a group
-    int far_turn;            // turn where most heads keep more than an eighth of the blocks, 0: as elsewhere
+    int far_turn;            // turn where most of four heads keep more than an eighth of the blocks, 0: no such turn
 };
 
 // Split walks.  A launch whose row-block pairs cannot fill the chip, or whose longest walks would outlast
@@ -297,18 +298,21 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
     unsigned rest = wg >> 3;
     auto next_digit = [&](const FastDiv &f) { const unsigned q = fast_quot(rest, f), r = rest - q * f.d; rest = q; return r; };
     const unsigned in_deal = next_digit(p.by_deal);
-    constexpr bool SETS = MODE == MODE_VS && !CUT;      // (elsewhere all groups are one set)
+    // (only whole list walks come in more than one set of groups, or choose their turn here)
+    const bool choose = MODE == MODE_VS && !CUT && p.turn == TURN_CHOSEN;
     int turn = p.turn;
-    if constexpr (SETS) {
-        if (p.far_turn) {                                // up to 64 heads' last rows: the same answer in every workgroup
-            const int heads = min(p.hq, 64), head = minf_lane();
-            const bool far = head < heads && p.bc[(head + 1ll) * p.rows - 1] > p.rows >> 3;
-            if (2 * __builtin_popcountll(__ballot(far)) > heads) turn = p.far_turn;
+    if (choose) {
+        turn = 0;
+        if (p.far_turn) {                                // four heads' last rows: the same answer in every workgroup
+            int far = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) far += as_const(p.bc)[(((i * p.hq) >> 2) + 1ll) * p.rows - 1] > p.rows >> 3;
+            if (far > 2) turn = p.far_turn;
         }
     }
     rest = 8u * rest + ((wg + (rest >> turn)) & 7u);
     unsigned gi = next_digit(p.by_set);
-    if constexpr (SETS) {
+    if (choose) {
         const unsigned deal = next_digit(p.by_chunks);
         gi += rest * p.by_set.d;
         if (gi >= (unsigned)p.batch * p.by_heads.d) return false;       // padding of the last round (workgroup-uniform)
@@ -1532,7 +1536,7 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     // every 2, 4, 8, 16, never: 59.7, 59.2, 59.2, 58.3, 56.5, 56.0 ms.  Lists of neighbouring diagonals gain nothing by it and lose
     // the balance: 500 columns and 700 slashes, 131072 tokens 3.81, 3.80, 3.80, 3.82, 3.86, 4.00 ms, 100000 tokens 2.63, 2.65,
     // 2.66, 2.74, 2.78, 2.93 (1000 and 6096, 131072 tokens 13.16, 13.16, 13.19, 13.19, 13.18, 13.35).  So a launch of 48 rounds and
-    // more goes through the eight places once, in steps of a power of two, if most of its heads keep more than an eighth of
+    // more goes through the eight places once, in steps of a power of two, if three of four heads keep more than an eighth of
     // the blocks in the last row (scattered 26 % of all blocks, 1000 and 6096 11 %, 500 and 700 3 %): the workgroups see that
     // from the counts.  Where a place is no single group's it stays as it was (16 heads, scattered, 25.2 : 25.7 ms).
     // Split walks: every round, but eight groups of one head, every fourth: 8192 tokens, 500 columns and 700 slashes 101 ->
@@ -1567,6 +1571,7 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     p.far_turn = 0;
     if (whole_lists && 8 % set == 0 && chunks * set >= 8 * 48)
         while (2ll << p.far_turn <= chunks * set / 64) ++p.far_turn;
+    if (p.far_turn || set < groups) p.turn = TURN_CHOSEN;
     if (MODE == MODE_VS && !p.head_list && split_pairs > 0 && groups == 8 && group == 1) p.turn = 2;
     p.by_group = fast_div((unsigned)group);
     p.by_deal = fast_div((unsigned)deal);

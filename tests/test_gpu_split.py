@@ -218,8 +218,8 @@ def test_heads_do_not_depend_on_how_a_launch_is_dealt(gpu, hq, hk, n, b):
 @pytest.mark.parametrize("hq,hk,n,b,far", [(32, 8, 48100, 1, 40), (32, 8, 49000, 1, 40), (32, 8, 49000, 1, 16), (32, 8, 49000, 1, 0), (66, 2, 26000, 1, 66),
                                            (16, 2, 98400, 1, 9), (24, 24, 66000, 1, 24), (16, 4, 30000, 7, 0)])
 def test_long_launches_are_dealt_whole(gpu, hq, hk, n, b, far):
-    """Launches just below and above 48 rounds of deals, from where on XCDs keep their place for some rounds if more than half of
-    the (first 64) heads keep an eighth of the blocks (`far` heads do), one set of groups and several: some heads
+    """Launches just below and above 48 rounds of deals, from where on XCDs keep their place for some rounds if three of four
+    heads keep more than an eighth of the blocks (the first `far` heads do), one set of groups and several: some heads
     on their own, bit for bit, and no row left out."""
     import minference_amd as M
     print(f"case {hq} / {hk} heads, {n} tokens, batch {b}, {far} far", flush=True)
