@@ -342,9 +342,10 @@ int minf_vs_estimate_heads(const void *q, const void *k, const int64_t *q_stride
                            size_t workspace_bytes, void *stream);
 
 /*
- * The whole vertical_and_slash layer (minference/modules/minference_forward.py:599-614) in one call: minf_vs_estimate,
- * minf_topk_indices_pair, minf_vs_index_build_full_ws and minf_vs_attn_fwd, in this order on `stream`.  nnz_v, nnz_s:
- * sizes of the selections, 1 .. n; the other arguments as in minf_vs_estimate.  t->seqlens and t->head_list null, dtype
+ * The whole vertical_and_slash layer (minference/modules/minference_forward.py:599-614) in one call on `stream`, with the
+ * bits of minf_vs_estimate, minf_topk_indices_pair, minf_vs_index_build_full_ws and minf_vs_attn_fwd in this order.  (From
+ * 257 to 16384 tokens, up to 4096 of them for 512 heads at most, one kernel takes the place of the estimation's last one,
+ * of the selections and of the index builder's first one.)  nnz_v, nnz_s: sizes of the selections, 1 .. n; the other arguments as in minf_vs_estimate.  t->seqlens and t->head_list null, dtype
  * bf16 or fp16, t->workspace unused.  workspace: minf_vs_prefill_workspace_bytes() bytes, 16-byte aligned (0 for
  * arguments the call refuses).
  */

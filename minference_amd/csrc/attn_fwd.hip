@@ -947,14 +947,18 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
         copy_tile(cur, k_base, k_row, std::false_type{}, gt_cur, lds_k);
     }
 
-    // One step of the walk, in three forms (the last two for the paired list walks only):
+    // One step of the walk, in four forms (COMMON and SPLIT for the paired list walks only):
     // general (kind 0) -- any tile, any successor, every mode;
+    // PLAIN (kind 3) -- a tile of which both row blocks see every key, after another such tile or as a list's first, and the
+    // next one alike or at least unmasked up to the pair's first row: in list walks both are common entries (the next one may
+    // lie anywhere behind this one), else the next one is this one's neighbour.  Both lie below the pair's first row, hence before
+    // the end of the sequence: they are copied without a look at it, and no mask and, but for a list's, no jump is asked for;
     // COMMON (kind 1) -- this tile and the next one are both on the list of common entries: shared,
     // contiguous, never gathered;
     // SPLIT (kind 2) -- this step and the next one are both split steps in which each row block
     // visits a block entry of its own, fetched a step ahead: a leftover from the split lists in LDS
-    // or, when the lists were not split, an entry of its list in global memory (kind 2).
-    // In the two special forms everything that deals with the other cases drops out of the
+    // or, when the lists were not split, an entry of its list in global memory.
+    // In the special forms everything that deals with the other cases drops out of the
     // instruction stream (the general form costs about 1.7 times a COMMON step).
     [[maybe_unused]] int sp_entry = 0;
     auto step = [&](const int it, auto kind_c) {

@@ -673,7 +673,9 @@ __global__ __launch_bounds__(TK_THREADS) void topk_regs_kernel(const TopkProblem
 // a head, that read what the one before wrote.
 // The three and now, without the gaps between them: one head of 4096 tokens, 500 columns and 700 slashes 2.9 + 7.5 + 5.7 ->
 // 11.7 us, whole layer 68.1 -> 63.9, 1000 and 6096 (all diagonals) 73.3 -> 60.2; 32 heads, 16001 tokens, 1000 and 6096
-// 5.1 + 17.7 + 15.4 -> 31.5.
+// 5.1 + 17.7 + 15.4 -> 31.5.  Each selection has a histogram of its own, 102 KB of LDS in all (137 beyond 8192 entries), so one
+// workgroup a CU; launches of several rounds of them gain all the same: 256 heads, 500 columns and 700 slashes, 5000 tokens
+// 5.4 + 20.3 + 6.5 -> 24.8, 16000 tokens 10.2 + 35.3 + 13.2 -> 45.4, 512 heads 22.5 + 66.3 + 20.0 -> 91.1.
 template <int ITEMS>
 __global__ __launch_bounds__(TK_THREADS) void vs_select_kernel(const EstWindows e, int n, int nnz_v, int32_t *__restrict__ v_idx, int nnz_s,
                                                                int32_t *__restrict__ s_idx, int32_t *__restrict__ tables, int rows, int bm_words) {
@@ -700,7 +702,8 @@ __global__ __launch_bounds__(TK_THREADS) void vs_select_kernel(const EstWindows 
 // topk_regs_kernel, one selection per candidate (the histogram of the top digit is made once), every byte written once.
 // Bound by the selections' barriers and LDS atomics.  A selection, two scatters into zeroed flags per
 // candidate and the zeros before them were fifteen launches: 32 heads, 16384 tokens, the reference's six candidates,
-// 116 -> 39 us, whole search 1885 -> 1810.
+// 116 -> 39 us, whole search 1885 -> 1810.  (Rows of more than 16384 entries take a few registers more than there are; whole
+// search, 24000 tokens, 3564 -> 3422, 8 / 2 heads 32000 tokens 1781 -> 1647.)
 constexpr int FLAG_CANDS = 8;
 struct FlagsProblem {
     const float *scores;         // may be null when every k is zero
