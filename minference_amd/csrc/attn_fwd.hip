@@ -93,7 +93,6 @@ constexpr int QK_AHEAD = 2;
 #endif
 constexpr int VALU_MASK = 0x402;             // sched_group_barrier classes: VALU | transcendental
 
-constexpr int TURN_CHOSEN = 32;              // every round, or every 2^far_turn
 struct AttnParams {
     const char *q, *k, *v;
     char *o;
@@ -112,8 +111,8 @@ struct AttnParams {
     // a-shape; query rows >= dense_from attend to every earlier key (tri-shape), INT_MAX = none
     int n_init, n_local, dense_from;
     int descending;          // row blocks are handed out from the last one down
-    int chunk, turn;         // units per deal; an XCD takes another place every 2^turn rounds of deals, 31: never, or TURN_CHOSEN (see plan_launch)
-    FastDiv by_deal, by_group, by_set, by_heads;   // workgroups of a deal; hq / hk; groups of a set; kv heads, or chunks of the head list
+    int chunk, turn;         // units per deal; an XCD takes another place every 2^turn rounds of deals, 31: never (see plan_launch)
+    FastDiv by_deal, by_group, by_groups, by_heads;   // workgroups of a deal; hq / hk; batch x kv groups; kv heads, or chunks of the head list
     // optional head selection: head_list[i], i < index_heads, are the query heads to process and i is
     // the head's position in the index tensors (which then have index_heads heads); without a list
     // every head is processed and index_heads = hq
@@ -125,9 +124,9 @@ struct AttnParams {
     char *part;
     int dtype;               // MINF_BF16, MINF_F16 or MINF_16BIT_SELECT
     const int *select;       // not null: this launch is one of two, and only the one for dtype *select does anything
-    // turn == TURN_CHOSEN only.  Behind the rest: every workgroup starts with a chain of reads of these arguments, and with
-    // the two in front the others' lay across one more cache line (A-shape, window 64, fp32 tensors, 32 / 8 heads, 65536 tokens 1185 : 1203 us)
-    FastDiv by_chunks;       // deals of a group
+    // CHOSEN launches only.  Behind the rest: every workgroup starts with a chain of reads of these arguments, and with two of
+    // them in front the others' lay across one more cache line (A-shape, window 64, fp32 tensors, 32 / 8 heads, 65536 tokens 1185 : 1203 us)
+    FastDiv by_set, by_chunks;      // groups of a set; deals of a group
     int far_turn;            // turn where most of four heads keep more than an eighth of the blocks, 0: no such turn
 };
 
@@ -298,26 +297,8 @@ __device__ __forceinline__ bool attn_walk(const AttnParams &p, const unsigned wg
     unsigned rest = wg >> 3;
     auto next_digit = [&](const FastDiv &f) { const unsigned q = fast_quot(rest, f), r = rest - q * f.d; rest = q; return r; };
     const unsigned in_deal = next_digit(p.by_deal);
-    // (only whole list walks come in more than one set of groups, or choose their turn here)
-    const bool choose = MODE == MODE_VS && !CUT && p.turn == TURN_CHOSEN;
-    int turn = p.turn;
-    if (choose) {
-        turn = 0;
-        if (p.far_turn) {                                // four heads' last rows: the same answer in every workgroup
-            int far = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) far += as_const(p.bc)[(((i * p.hq) >> 2) + 1ll) * p.rows - 1] > p.rows >> 3;
-            if (far > 2) turn = p.far_turn;
-        }
-    }
-    rest = 8u * rest + ((wg + (rest >> turn)) & 7u);
-    unsigned gi = next_digit(p.by_set);
-    if (choose) {
-        const unsigned deal = next_digit(p.by_chunks);
-        gi += rest * p.by_set.d;
-        if (gi >= (unsigned)p.batch * p.by_heads.d) return false;       // padding of the last round (workgroup-uniform)
-        rest = deal;
-    }
+    rest = 8u * rest + ((wg + (rest >> p.turn)) & 7u);
+    const unsigned gi = next_digit(p.by_groups);
     const unsigned first_unit = rest * (unsigned)p.chunk;
     rest = in_deal;
     const int hin = (int)next_digit(p.by_group);
@@ -1187,14 +1168,40 @@ __device__ __forceinline__ void attn_workgroup(const AttnParams &p, const unsign
     }
 }
 
-template <typename T, int MODE, int HD, bool CUT>
+// CHOSEN: the number under which attn_walk, for which XCDs keep their places and all groups are one set, finds the deal of
+// workgroup `wg` -> false: it has none (padding of the last round).  The choice is every workgroup's own, from four heads'
+// counts, and so the same in all of them.  A form of the kernel of its own: as a branch of the walk's decoding, or before it, it
+// cost launches that choose nothing 1 to 3 % (one head 10555 tokens 217.5 us, 220.3 and 224.7; 4 heads 11055 tokens 183.1, 187.3
+// and 186.3), the compiler then making one loop of the three general steps it makes otherwise, with more spilled scalars.
+__device__ __forceinline__ bool chosen_place(const AttnParams &p, unsigned &wg) {
+    unsigned turn = 0;
+    if (p.far_turn) {
+        const cint_ptr last = as_const(p.bc) + p.rows - 1;       // (four loads on their way together)
+        const int quarter = p.hq >> 2, most = p.rows >> 3;
+        const int c0 = last[0], c1 = last[(long long)quarter * p.rows], c2 = last[2ll * quarter * p.rows], c3 = last[3ll * quarter * p.rows];
+        if ((c0 > most) + (c1 > most) + (c2 > most) + (c3 > most) > 2) turn = (unsigned)p.far_turn;
+    }
+    const unsigned round = fast_quot(wg >> 3, p.by_deal), in_deal = (wg >> 3) - round * p.by_deal.d;
+    const unsigned place = 8u * round + ((wg + (round >> turn)) & 7u);
+    const unsigned row = fast_quot(place, p.by_set), set = fast_quot(row, p.by_chunks);
+    const unsigned groups = (unsigned)p.batch * p.by_heads.d, g = set * p.by_set.d + place - row * p.by_set.d;
+    if (g >= groups) return false;
+    const unsigned deal = (row - set * p.by_chunks.d) * groups + g;
+    wg = (((deal >> 3) * p.by_deal.d + in_deal) << 3) + (deal & 7u);
+    return true;
+}
+
+template <typename T, int MODE, int HD, bool CUT, bool CHOSEN = false>
 __global__ __launch_bounds__(2 * NTHREADS, HD > 128 ? 1 : 2) void attn_fwd_kernel(const AttnParams p) {
     typedef AttnLds<MODE, HD> L;
     if (p.select && *as_const(p.select) != dtype_code<T>()) return;
     __shared__ __attribute__((aligned(16))) char lds_k[L::NK];
     __shared__ __attribute__((aligned(16))) char lds_v[L::NV];
     __shared__ int vs_only[L::NONLY];        // paired list walks: [row block][entries the other list lacks]
-    attn_workgroup<T, MODE, HD, CUT>(p, blockIdx.x, lds_k, lds_v, vs_only);
+    unsigned wg = blockIdx.x;
+    if constexpr (CHOSEN)
+        if (!chosen_place(p, wg)) return;
+    attn_workgroup<T, MODE, HD, CUT>(p, wg, lds_k, lds_v, vs_only);
 }
 
 // The pattern types of a layer in one launch: workgroups [0, first_bs) walk vertical-slash lists, [first_bs, first_as)
@@ -1405,7 +1412,7 @@ void fill_params(AttnParams &p, const minf_qkvo *t) {
     p.head_list = t->head_list;
     p.index_heads = t->head_list ? t->index_heads : t->heads_q;
     p.chunk = 1; p.turn = p.far_turn = 0;      // set by the launcher
-    p.by_deal = p.by_group = p.by_set = p.by_chunks = p.by_heads = fast_div(1);      // set by the launcher
+    p.by_deal = p.by_group = p.by_groups = p.by_heads = p.by_set = p.by_chunks = fast_div(1);      // set by the launcher
     p.descending = 0;
     p.split_first = (p.rows + 1) / 2; p.nseg = 1; p.seg_len = 1; p.part = nullptr;
     p.dtype = t->dtype;
@@ -1575,10 +1582,11 @@ template <int MODE, int HD> long long plan_launch(AttnParams &p, const minf_qkvo
     p.far_turn = 0;
     if (whole_lists && 8 % set == 0 && chunks * set >= 8 * 48)
         while (2ll << p.far_turn <= chunks * set / 64) ++p.far_turn;
-    if (p.far_turn || set < groups) p.turn = TURN_CHOSEN;
+    if (p.far_turn || set < groups) p.turn = 31;               // (lists: a CHOSEN launch)
     if (MODE == MODE_VS && !p.head_list && split_pairs > 0 && groups == 8 && group == 1) p.turn = 2;
     p.by_group = fast_div((unsigned)group);
     p.by_deal = fast_div((unsigned)deal);
+    p.by_groups = fast_div((unsigned)groups);
     p.by_set = fast_div((unsigned)set);
     p.by_chunks = fast_div((unsigned)chunks);
     p.by_heads = fast_div((unsigned)(grid_heads / group));
@@ -1593,9 +1601,11 @@ template <int MODE, int HD> int launch_hd(AttnParams p, const minf_qkvo *t, void
     const int split_pairs = (p.rows + 1) / 2 - p.split_first;
     const dim3 block(2 * NTHREADS);
     hipStream_t st = (hipStream_t)stream;
+    const bool chosen = MODE == MODE_VS && p.turn == 31;
 #define MINF_LAUNCH_ATTN(T)                                                                                      \
     do {                                                                                                         \
         if (p.nseg > 1) hipLaunchKernelGGL((attn_fwd_kernel<T, MODE, HD, true>), dim3((unsigned)grid), block, 0, st, p); \
+        else if (chosen) hipLaunchKernelGGL((attn_fwd_kernel<T, MODE, HD, false, MODE == MODE_VS>), dim3((unsigned)grid), block, 0, st, p); \
         else hipLaunchKernelGGL((attn_fwd_kernel<T, MODE, HD, false>), dim3((unsigned)grid), block, 0, st, p);   \
     } while (0)
     if (dtype != MINF_F16) MINF_LAUNCH_ATTN(__bf16);
@@ -1684,6 +1694,7 @@ template <typename T, int HD> bool launch_mixed(const AttnParams &vs, const minf
     memset(&m, 0, sizeof(m));
     long long vs_wgs = 0, bs_wgs = 0, as_wgs = 0;
     if (vs_t) { m.vs = vs; vs_wgs = plan_launch<MODE_VS, HD>(m.vs, vs_t); }
+    if (m.vs.turn == 31) m.vs.turn = 0;           // (no CHOSEN form of this kernel)
     if (bs_t) { m.bs = bs; bs_wgs = plan_launch<MODE_BS, HD>(m.bs, bs_t); }
     if (as_t) { m.as = as; as_wgs = plan_launch<MODE_ASHAPE, HD>(m.as, as_t); }
     if ((vs_t && m.vs.nseg > 1) || (bs_t && m.bs.nseg > 1) || (as_t && m.as.nseg > 1)) return false;
