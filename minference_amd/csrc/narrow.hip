@@ -11,10 +11,10 @@
 // With a pass for the largest |value| alone before the conversion (8192 tokens, 4 heads of 128, 3 x 16.8 MB)
 // the two took 22.2 us, now 15.1; 32768 tokens, 16 heads 363 -> 223, 65536 tokens, 32 / 8 heads 741 -> 447, 5.4 TB/s.
 // Tensors that need bf16 took, with that pass, converted to fp16 whatever the values, and sampled first: 8192 tokens, 4
-// heads 22.2, 26.8, 15.7 us, 32 / 8 heads 75.7, 122, 53.4, 32768 tokens, 16 heads 366, 451, 223, 65536 tokens, 32 / 8 heads
-// 744, 1007, 448.  The sample lengthens a conversion by one to two microseconds all the same (it is on its way behind the first
-// step's loads, at addresses from the host; an operator's call on 5000 tokens, 8 / 2 heads, 123.9 -> 125.8), so smaller
-// tensors, for which a second conversion costs 5 to 12, go without.  Where it does not show what the tensors ask for, one value
+// heads 22.2, 26.8, 15.7 us, 14 heads 65.5, 78.3, 44, 32 / 8 heads 75.7, 122, 53.4, 32768 tokens, 16 heads 366, 451, 223,
+// 65536 tokens, 32 / 8 heads 744, 1007, 448.  The sample lengthens a call by one to two microseconds all the same (it is on its
+// way behind the first step's loads, at addresses from the host; operator, 5000 tokens, 8 / 2 heads, 123.9 -> 125.8, two times
+// 1427 tokens, 28 / 4 heads, 100.4 -> 101.8), so smaller tensors, which lose 4 to 13 to the second conversion, go without.  Where it does not show what the tensors ask for, one value
 // above 32768, they are converted twice: 102, 443 and 886 us.
 // With the choice read back by the host (three reductions, a synchronisation, three conversions) the GPU
 // idled about 60 us per call.
@@ -26,7 +26,7 @@ constexpr int NARROW_THREADS = 256;
 constexpr int UNDER_WAY = 2;     // steps of 8 elements a thread has under way
 constexpr int NARROW_PARTIALS = MINF_NARROW_WORKSPACE_INTS - 1;      // workgroups of a launch, a third per tensor
 constexpr int NARROW_WGS = NARROW_PARTIALS / 3;
-constexpr long long SAMPLED_FROM = 1 << 20;      // vectors of the largest tensor
+constexpr long long SAMPLED_FROM = 1 << 21;      // vectors of the largest tensor
 static_assert(NARROW_WGS * 3 == NARROW_PARTIALS, "the same number of workgroups for each tensor");
 
 struct NarrowTensor {

@@ -77,11 +77,11 @@ def test_the_largest_value_is_found_wherever_it_lies(gpu, n, layout):
 @pytest.mark.parametrize("where", ["nowhere", "one channel", "all of q", "from the middle of k on", "first rows", "last row", "one wavefront of many steps",
                                    "a tail", "tiny", "tiny middle head", "zero middle head", "large middle row"])
 def test_the_rows_looked_at_first_do_not_decide(gpu, where):
-    """Nine steps of a workgroup (eight whole ones and a tail), and the middle head's rows, by some of which the first conversion
+    """Seventeen steps of a workgroup (sixteen whole ones and a tail), and the middle head's rows, by some of which the first conversion
     goes: values that ask for bf16 in all of them, in other rows, in them alone, in the vector that several threads write past
     the end; rows that ask for bf16 in tensors that do not."""
     import minference_amd as M
-    n = 8 * 1024 + 3
+    n = 16 * 1024 + 3
     g = torch.Generator(device=gpu).manual_seed(3)
     q, k, v = (torch.randn(1, 8, n, 128, device=gpu, generator=g) for _ in range(3))
     dtype = torch.float16 if where == "nowhere" else torch.bfloat16
@@ -97,7 +97,7 @@ def test_the_rows_looked_at_first_do_not_decide(gpu, where):
         v[0, 7, n - 1, 127] = -1e30
     elif where == "one wavefront of many steps":
         q[0, 3, 7, 8:16] = float("inf")
-        q[0, 7, 8000, 3] = 5e4
+        q[0, 7, 16000, 3] = 5e4
     elif where == "a tail":
         q[0, 7, n - 3:] = 4e4
         v[0, 7, n - 1] = 0
